@@ -539,7 +539,7 @@ class Synapses:
             np.cumsum(np.bincount(pos_post, minlength=self.target.N), out=ptr_[1:])
             self.csr["post_ptr"] = dev(ptr_.astype(np.uint32).view(np.int32))
             self.csr["post_syn"] = dev(perm.astype(np.int32))
-            self.csr["pre_of"] = dev(self.pre[order].astype(np.int32))
+            self.csr["post_pre"] = dev(self.pre[order][perm].astype(np.int32))
 
     @property
     def n_events(self):
@@ -1329,13 +1329,14 @@ class Network:
             host = {"dt": self.dt}
             host.update(getattr(s, "namespace", {}) or {})
             sc = scalar_values(sp, host, g.float_t)
-            K = SummedKernel(f"{s.name}_{tv}", sp.vector, used, pre_r, post_r, var_types, g.vars[tv], sc, g.float_t)
+            t0, t1 = s.tgt_range
+            K = SummedKernel(f"{s.name}_{tv}", sp.vector, used, pre_r, post_r, var_types, g.vars[tv], sc, g.float_t,
+                             lanes=SummedKernel.lanes_for(s.csr["n_syn"], t1 - t0))
             fn = self.device.function(K.source, K.kernel_name)
             cls = K.struct.ctypes_struct()
-            t0, t1 = s.tgt_range
             v = {"clock": self.clock.data_ptr(), "step_off": 0, "dt": self.dt, "t0": t0, "t1": t1,
                  "post_ptr": s.csr["post_ptr"].data_ptr(), "post_syn": s.csr["post_syn"].data_ptr(),
-                 "pre_of": s.csr["pre_of"].data_ptr(), "target": g._dev[tv].data_ptr()}
+                 "post_pre": s.csr["post_pre"].data_ptr(), "target": g._dev[tv].data_ptr()}
             for n in used:
                 v[f"s_{n}"] = s.csr["syn"][n].data_ptr()
             for n, gv in pre_r.items():
@@ -1349,7 +1350,7 @@ class Network:
                 if name in v:
                     setattr(a, name, v[name])
             s.summed_kernels.append(K)
-            self._add_launch(fn, max(1, (t1 - t0 + K.BLOCK - 1) // K.BLOCK), K.BLOCK, a, cls)
+            self._add_launch(fn, K.grid(t1 - t0), K.BLOCK, a, cls)
 
     def _build_post(self, s):
         host = {"dt": self.dt}
