@@ -1,23 +1,19 @@
 """Batched parameter sweeps: many independent networks in one persistent kernel.
 
 A sweep (e.g. 1024 CUBA networks of uneven size, each with its own
-connectivity and parameters) is advanced by one kernel per launch in which
-every workgroup owns one network and steps it through ``steps_per_launch``
-time steps without any grid-wide synchronisation.  Per step and network the
-workgroup
+connectivity and parameters) is advanced by launches in which every workgroup
+owns one network and steps it through ``steps_per_launch`` time steps without
+any grid-wide synchronisation: its state in registers, its spikes and the
+events of its targets in LDS (resident.ResidentKernel).  A pathway's events
+carry one constant per network, so counting them per target gives the sums of
+the cython runtime's left fold over the spike queue
+(brian2/synapses/spikequeue.h:151-191 with delay 0) bit for bit.  Networks are
+launched by size, so that small ones share a compute unit; the launches of the
+sizes run side by side.
 
-  1. updates its neurons (Brian's stateupdate / threshold / reset statements,
-     fused; the reset only touches variables no pathway writes),
-  2. compacts the spikes in ascending neuron order into LDS (wave ballot +
-     prefix over waves),
-  3. propagates the spikes in that order, one source row at a time with a
-     barrier in between, so that every target receives its events in the order
-     of Brian's spike queue (brian2/synapses/spikequeue.h:151-191 with delay 0)
-     and the per-target sums are bit-identical to the cython runtime's.
-
-Launches of the step kernel are replayed from a hipGraph.  The block size and
-the number of steps per launch are chosen by a small autotuner that times the
-candidates on the real networks (results do not depend on either).
+Launches are replayed from a hipGraph.  The largest block size and the number
+of steps per launch are chosen by a small autotuner that times the candidates
+on the real networks (results do not depend on either).
 """
 import ctypes
 import time
@@ -25,8 +21,16 @@ import time
 import numpy as np
 
 from . import _lib
-from .codegen import HostEval, ParamStruct, cast_value, ctype_of, source_header, translate_block
-from .kernels import identifiers
+from .codegen import HostEval, ParamStruct, Renderer, cast_value, ctype_of, translate_block
+from .kernels import _rename, identifiers
+from .resident import (
+    MAX_NEURONS,
+    ResidentKernel,
+    lds_plan,
+    neurons_in_registers,
+    refractory_form,
+    timestep_bound,
+)
 from .runtime import Device, Model, dev, ptr, zeros
 
 L = _lib.lib
@@ -72,6 +76,7 @@ class BatchedCUBA:
         self.spike_capacity_hz = spike_capacity_hz
         self.horizon_steps = horizon_steps
         self._built = False
+        self.counts = None  # events per neuron, where they do not fit a workgroup's LDS
         self.block = 256
         self.steps_per_launch = 100
 
@@ -111,19 +116,24 @@ class BatchedCUBA:
                 self.scalar_types = {key: row[key][1] for key in names}
             table.append([float(row[key][0]) for key in names])
         self.scalar_names = names
-        return np.array(table, np.float64)
+        table = np.array(table, np.float64)
+        # refractory periods in steps: compared through their bound (resident.timestep_bound)
+        self.bounds = {}
+        for k, (tg, n) in enumerate(names):
+            steps = table[:, k]
+            if self.scalar_types[(tg, n)] == "long long" and tg == "su" and np.all(steps >= 1):
+                self.bounds[f"{tg}_{n}"] = f"tb_{n}"
+                of = {int(x): timestep_bound(int(x), self.dt) for x in np.unique(steps)}
+                table = np.column_stack([table, [of[int(x)] for x in steps]])
+        return table
 
-    def _source(self):
-        T = self.block
-        NW = T // 64
-        NS = len(self.scalar_names)
-        nmax = max(n.N for n in self.nets)
+    def _struct(self):
         ps = ParamStruct("hbb_params")
         ps.ptr("clock", "long long", const=True)
         ps.val("step_off", "long long")
         ps.val("dt", "double")
         ps.val("n_steps", "int")
-        ps.val("n_nets", "int")
+        ps.val("first", "int")  # the launch's networks: order[first + workgroup]
         ps.ptr("order", "int", const=True)
         ps.ptr("n_off", "int", const=True)
         ps.ptr("ne", "int", const=True)
@@ -132,146 +142,130 @@ class BatchedCUBA:
         ps.ptr("scal", "double", const=True)
         for v, ct in self.vars.items():
             ps.ptr(f"a_{v}", "unsigned char" if ct == "bool" else ct)
+        ps.ptr("counts", "unsigned int")
         ps.ptr("spk_i", "int")
         ps.ptr("spk_step", "int")
         ps.ptr("spk_off", "long long", const=True)
         ps.ptr("spk_cap", "long long", const=True)
         ps.ptr("spk_n", "long long")
         ps.ptr("status", "int")
-        self.struct = ps
+        return ps
+
+    def _kernel(self, rows_in_lds, counts_in_lds):
+        """The step kernel (resident.ResidentKernel): the networks' scalars are read per
+        workgroup, the pathway of an event is that of its source (exc below NE)."""
+        names = {}
+        for (tg, n) in self.scalar_types:
+            names.setdefault(tg, {})[n] = f"{tg}_{n}"
 
         def block(tag, spec, extra=None):
             types = dict(self.vars)
             types.update({"t": "double", "dt": "double", "N": "int", "i": "int", "_idx": "int"})
             types.update(extra or {})
-            names = {}
-            for (tg, n), ct in self.scalar_types.items():
-                if tg == tag:
-                    types[n] = ct
-                    names[n] = f"{tg}_{n}"
-            lines = translate_block(spec.vector, spec.conditional_write, types, set(), self.float_t)
-            import re
+            types.update({n: ct for (tg, n), ct in self.scalar_types.items() if tg == tag})
+            return _rename(translate_block(spec.vector, spec.conditional_write, types, set(), self.float_t, select=True),
+                           names.get(tag, {}))
 
-            if names:
-                pat = re.compile(r"(?<![\w.])(" + "|".join(re.escape(k) for k in sorted(names, key=len, reverse=True))
-                                 + r")(?!\w)")
-                lines = [pat.sub(lambda m: names[m.group(1)], ln) for ln in lines]
-            return lines
-
-        from .codegen import Renderer
-
-        def value_expr(tag, spec):
-            types = {}
-            names = {}
-            for (tg, n), ct in self.scalar_types.items():
-                if tg == tag:
-                    types[n] = ct
-                    names[n] = f"{tg}_{n}"
+        def operand(tag, spec, var):
+            types = {n: ct for (tg, n), ct in self.scalar_types.items() if tg == tag}
             c, _ = Renderer(types).render(spec.vector[-1]["expr"])
-            import re
+            ct = self.vars[var]
+            return f"const {ct} {tag}_val = ({ct})({_rename([c], names.get(tag, {}))[0]});"
 
-            if names:
-                pat = re.compile(r"(?<![\w.])(" + "|".join(re.escape(k) for k in sorted(names, key=len, reverse=True))
-                                 + r")(?!\w)")
-                c = pat.sub(lambda m: names[m.group(1)], c)
-            return c
-
-        k = [source_header(T), ps.c_decl()]
-        k.append(f'extern "C" __global__ void __launch_bounds__({T}) batched_step(const hbb_params p) {{')
-        k.append("    const int net = p.order[blockIdx.x];")
-        k.append("    const int off = p.n_off[net];")
-        k.append("    const int N = p.n_off[net + 1] - off;")
-        k.append("    const int NE = p.ne[net];")
-        k.append("    const double dt = p.dt;")
+        update, spike = [], []
+        if self.su is not None:
+            update += ["{"] + block("su", self.su) + ["}"]
+        if self.th is not None:
+            update += ["{"] + block("th", self.th, {"_cond": "bool"}) + ["hb_cond = _cond;", "}"]
+        if self.rs is not None:
+            if {st["var"] for st in self.rs.vector} & {self.exc_var, self.inh_var}:
+                raise NotImplementedError("reset writes a synaptic target variable")
+            spike = block("rs", self.rs)
+        test = refractory_form(update, spike, self.vars)
+        prologue = [
+            "const int net = p.order[p.first + (int)blockIdx.x];",
+            "const int hb_off = p.n_off[net];",
+            "const int N = p.n_off[net + 1] - hb_off;",
+            "const int NE = p.ne[net];",
+            "const unsigned int* hb_rp = p.row_ptr + hb_off + net;  // N + 1 entries per network",
+            "// the plan's clock counts launches of n_steps steps each",
+            "const long long hb_step0 = (p.clock[0] + p.step_off) * p.n_steps;",
+            "const long long hb_so = p.spk_off[net], hb_sc = p.spk_cap[net];",
+            "long long hb_sn = p.spk_n[net];",
+        ]
+        row = len(self.scalar_names) + len(self.bounds)
         for idx, (tg, n) in enumerate(self.scalar_names):
             ct = self.scalar_types[(tg, n)]
-            k.append(f"    const {ct} {tg}_{n} = ({ct})p.scal[(size_t)net * {NS} + {idx}];")
-        k.append(f"    __shared__ int s_spk[{nmax}];")
-        k.append(f"    __shared__ int s_w[{NW + 1}];")
-        k.append("    __shared__ int s_n;")
-        k.append("    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;")
-        k.append("    const unsigned int* rp = p.row_ptr + off + net;  // N + 1 entries per network")
-        for (tag, spec, var) in (("pe", self.exc_spec, self.exc_var), ("pi", self.inh_spec, self.inh_var)):
-            k.append(f"    const {self.vars[var]} {tag}_val = ({self.vars[var]})({value_expr(tag, spec)});")
-        k.append("    for (int s = 0; s < p.n_steps; s++) {")
-        k.append("        // the plan's clock counts launches of n_steps steps each")
-        k.append("        const long long step = (p.clock[0] + p.step_off) * p.n_steps + s;")
-        k.append("        const double t = (double)step * dt;")
-        k.append("        if (threadIdx.x == 0) s_n = 0;")
-        k.append("        __syncthreads();")
-        k.append(f"        for (int j0 = 0; j0 < N; j0 += {T}) {{")
-        k.append("            const int i = j0 + threadIdx.x;")
-        k.append("            const int _idx = i;")
-        k.append("            (void)_idx; (void)t;")
-        k.append("            bool hb_cond = false;")
-        k.append("            if (i < N) {")
-        body = []
-        for v, ct in self.vars.items():
-            body.append(f"bool {v} = p.a_{v}[off + i] != 0;" if ct == "bool" else f"{ct} {v} = p.a_{v}[off + i];")
-        if self.su is not None:
-            body.append("{")
-            body += ["    " + x for x in block("su", self.su)]
-            body.append("}")
-        if self.th is not None:
-            body.append("{")
-            body += ["    " + x for x in block("th", self.th, {"_cond": "bool"})]
-            body.append("    hb_cond = _cond;")
-            body.append("}")
-            if self.uses_refractory:
-                body.append("if (hb_cond) { not_refractory = false; lastspike = t; }")
-        if self.rs is not None:
-            written = {st["var"] for st in self.rs.vector}
-            if written & {self.exc_var, self.inh_var}:
-                raise NotImplementedError("reset writes a synaptic target variable")
-            body.append("if (hb_cond) {")
-            body += ["    " + x for x in block("rs", self.rs)]
-            body.append("}")
-        for v, ct in self.vars.items():
-            body.append(f"p.a_{v}[off + i] = {v} ? 1 : 0;" if ct == "bool" else f"p.a_{v}[off + i] = {v};")
-        k += ["                " + x for x in body]
-        k.append("            }")
-        k.append("            const unsigned long long bal = __ballot(hb_cond);")
-        k.append("            if (lane == 0) s_w[wid] = __popcll(bal);")
-        k.append("            __syncthreads();")
-        k.append("            if (threadIdx.x == 0) {")
-        k.append("                int acc = s_n;")
-        k.append(f"                for (int w = 0; w < {NW}; w++) {{ const int c = s_w[w]; s_w[w] = acc; acc += c; }}")
-        k.append(f"                s_w[{NW}] = acc;")
-        k.append("            }")
-        k.append("            __syncthreads();")
-        k.append("            if (hb_cond) s_spk[s_w[wid] + __popcll(bal & ((1ull << lane) - 1ull))] = i;")
-        k.append(f"            if (threadIdx.x == 0) s_n = s_w[{NW}];")
-        k.append("            __syncthreads();")
-        k.append("        }")
-        k.append("        const int nspk = s_n;")
-        # record
-        k.append("        if (nspk) {")
-        k.append("            const long long base = p.spk_n[net];")
-        k.append("            const long long cap = p.spk_cap[net];")
-        k.append(f"            for (int q = threadIdx.x; q < nspk; q += {T}) {{")
-        k.append("                if (base + q < cap) {")
-        k.append("                    p.spk_i[p.spk_off[net] + base + q] = s_spk[q];")
-        k.append("                    p.spk_step[p.spk_off[net] + base + q] = (int)step;")
-        k.append("                }")
-        k.append("            }")
-        k.append("            __syncthreads();")
-        k.append("            if (threadIdx.x == 0) { p.spk_n[net] = base + nspk; if (base + nspk > cap) atomicOr(p.status, 2); }")
-        k.append("        }")
-        # propagate in ascending source order, one row at a time
-        ev, iv = self.exc_var, self.inh_var
-        k.append("        for (int q = 0; q < nspk; q++) {")
-        k.append("            const int src = s_spk[q];")
-        k.append("            const unsigned int a = rp[src], b = rp[src + 1];")
-        k.append("            if (src < NE) {")
-        k.append(f"                for (unsigned int e = a + threadIdx.x; e < b; e += {T}) p.a_{ev}[off + p.post[e]] += pe_val;")
-        k.append("            } else {")
-        k.append(f"                for (unsigned int e = a + threadIdx.x; e < b; e += {T}) p.a_{iv}[off + p.post[e]] += pi_val;")
-        k.append("            }")
-        k.append("            __syncthreads();")
-        k.append("        }")
-        k.append("    }")
-        k.append("}")
-        return "\n".join(k) + "\n"
+            prologue.append(f"const {ct} {tg}_{n} = ({ct})p.scal[(size_t)net * {row} + {idx}];")
+        for idx, b in enumerate(self.bounds.values()):
+            prologue.append(f"const double {b} = p.scal[(size_t)net * {row} + {len(self.scalar_names) + idx}];")
+        prologue += [operand("pe", self.exc_spec, self.exc_var), operand("pi", self.inh_spec, self.inh_var)]
+        shared = [
+            "// spikes as bits by neuron and the spikes before each word (steps of many spikes)",
+            "unsigned long long* const s_bit = (unsigned long long*)(hb_lds + (((unsigned char*)(s_spk + N) - hb_lds + 7) & ~7));",
+            "int* const s_pre = (int*)(s_bit + (N + 63) / 64);",
+        ]
+        store = ("if (hb_sn + {r} < hb_sc) {{ p.spk_i[hb_so + hb_sn + {r}] = {i}; "
+                 "p.spk_step[hb_so + hb_sn + {r}] = (int)step; }}")
+        record = [
+            "// the record keeps a step's spikes in ascending order",
+            "if (hb_nsp <= 64) {",
+            "    if (wid == NW - 1) {  // rank by counting the smaller ones",
+            "        const int id_ = lane < hb_nsp ? (int)s_spk[lane] : 0;",
+            "        int r_ = 0;",
+            "        for (int j = 0; j < hb_nsp; j++) r_ += (int)s_spk[j] < id_ ? 1 : 0;",
+            "        if (lane < hb_nsp) { " + store.format(r="r_", i="id_") + " }",
+            "    }",
+            "} else {  // rank by the set bits below",
+            "    const int nw_ = (N + 63) / 64;",
+            "    for (int w = threadIdx.x; w < nw_; w += T) s_bit[w] = 0ull;",
+            "    __syncthreads();",
+            "    for (int j = threadIdx.x; j < hb_nsp; j += T)",
+            "        atomicOr((unsigned int*)s_bit + (s_spk[j] >> 5), 1u << (s_spk[j] & 31));",
+            "    __syncthreads();",
+            "    if (wid == 0) {",
+            "        int c_ = 0;",
+            "        for (int w0 = 0; w0 < nw_; w0 += 64) {",
+            "            const int n_ = w0 + lane < nw_ ? __popcll(s_bit[w0 + lane]) : 0;",
+            "            const int x_ = hb_wave_incl_scan(n_);",
+            "            if (w0 + lane < nw_) s_pre[w0 + lane] = c_ + x_ - n_;",
+            "            c_ += __builtin_amdgcn_readlane(x_, 63);",
+            "        }",
+            "    }",
+            "    __syncthreads();",
+            "    for (int j = threadIdx.x; j < hb_nsp; j += T) {",
+            "        const int id_ = (int)s_spk[j];",
+            "        const int r_ = s_pre[id_ >> 6] + __popcll(s_bit[id_ >> 6] & ((1ull << (id_ & 63)) - 1ull));",
+            "        " + store.format(r="r_", i="id_"),
+            "    }",
+            "}",
+            "hb_sn += hb_nsp;",
+        ]
+        finish = ["if (threadIdx.x == 0) { p.spk_n[net] = hb_sn; if (hb_sn > hb_sc) atomicOr(p.status, 2); }"]
+        return ResidentKernel(
+            "batched_step", self._struct(), self.vars, update,
+            [(self.exc_var, "+=", "pe_val"), (self.inh_var, "+=", "pi_val")], prologue,
+            ["const int hb_tgt = (int)hb_syn;", "const int hb_path = hb_src < NE ? 0 : 1;"], spike=spike,
+            refractory=self.uses_refractory and self.th is not None, record=record, finish=finish, rows_in_lds=rows_in_lds, counts_in_lds=counts_in_lds, shared=shared,
+            bound=self.bounds.get(test))
+
+    def _classes(self):
+        """The networks by workgroup size, largest first: [(threads, first, networks)].
+
+        A thread holds up to `resident` neurons, so a network takes the fewest threads (a
+        power of two from 128 to `block`) that hold it, and small networks share a compute
+        unit.  The launches of the sizes run side by side, so there are at most four."""
+        R = neurons_in_registers(self.vars)
+        out = []
+        for k, n in enumerate(sorted((n.N for n in self.nets), reverse=True)):
+            t = 128
+            while t < self.block and t * R < n:
+                t *= 2
+            t = min(t, self.block)
+            if not out or out[-1][0] != t:
+                out.append([t, k, 0, n])
+            out[-1][2] += 1
+        return out
 
     def build(self):
         import torch
@@ -348,29 +342,37 @@ class BatchedCUBA:
         D = self.device
         if self.t_step % self.steps_per_launch:
             raise ValueError("the current step is not a multiple of steps_per_launch")
-        src = self._source()
-        self.source = src
-        self.fn = D.function(src, "batched_step")
-        cls = self.struct.ctypes_struct()
         self.launch_clock = torch.full((1,), self.t_step // self.steps_per_launch, dtype=torch.int64, device="cuda")
         v = dict(clock=self.launch_clock.data_ptr(), step_off=0, dt=self.dt, n_steps=self.steps_per_launch,
-                 n_nets=len(self.nets), order=self.order.data_ptr(), n_off=self.n_off_d.data_ptr(),
+                 order=self.order.data_ptr(), n_off=self.n_off_d.data_ptr(),
                  ne=self.ne_d.data_ptr(), row_ptr=self.row_ptr.data_ptr(), post=self.post.data_ptr(),
                  scal=self.scal.data_ptr(), spk_i=self.spk_i.data_ptr(), spk_step=self.spk_step.data_ptr(),
                  spk_off=self.spk_off.data_ptr(), spk_cap=self.spk_cap.data_ptr(), spk_n=self.spk_n.data_ptr(),
                  status=self.status.data_ptr())
         for n in self.vars:
             v[f"a_{n}"] = self.state[n].data_ptr()
-        a = cls()
-        for name, _ in cls._fields_:
-            if name in v:
-                setattr(a, name, v[name])
-        self.cls, self.args = cls, a
         self.plan = ctypes.c_void_p()
         _lib.check(L.hb_plan_create(D.ctx, ptr(self.launch_clock), ctypes.byref(self.plan)))
-        buf = bytes(a)
-        _lib.check(L.hb_plan_add(self.plan, self.fn, len(self.nets), self.block, 0, buf, len(buf),
-                                 cls.step_off.offset))
+        # one launch per workgroup size, side by side
+        for k, (threads, first, count, nmax) in enumerate(self._classes()):
+            extra = 8 + 12 * ((nmax + 63) // 64)
+            if nmax > MAX_NEURONS:
+                raise NotImplementedError(f"networks of more than {MAX_NEURONS} neurons")
+            K = self._kernel(*lds_plan(nmax, 1, extra))
+            fn = D.function(K.source, K.kernel_name)
+            if not K.counts_in_lds and self.counts is None:
+                self.counts = zeros(int(self.n_off[-1]), "int")
+            cls = K.struct.ctypes_struct()
+            a = cls()
+            v.update(first=first, counts=0 if self.counts is None else self.counts.data_ptr())
+            for name, _ in cls._fields_:
+                if name in v:
+                    setattr(a, name, v[name])
+            buf = bytes(a)
+            _lib.check(L.hb_plan_add(self.plan, fn, count, threads, K.lds_bytes(nmax, threads, extra), buf, len(buf),
+                                     cls.step_off.offset))
+            if k:
+                _lib.check(L.hb_plan_set_lane(self.plan, k, 1 + (k - 1) % 3))
 
     # ------------------------------------------------------------------ run
     def run(self, n_steps, graph_launches=10):

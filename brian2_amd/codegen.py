@@ -325,8 +325,22 @@ def cast_value(v, ctype):
 # ---------------------------------------------------------------------------
 # statements -> C (CPPCodeGenerator.translate_statement, cpp_generator.py:251-312)
 # ---------------------------------------------------------------------------
-def translate_statement(st, types, declared, float_t):
-    """One statement dict (captured from Brian) -> list of C lines."""
+_CHEAP = (ast.Expression, ast.BinOp, ast.UnaryOp, ast.BoolOp, ast.Compare, ast.Name, ast.Constant, ast.Load, ast.Add,
+          ast.Sub, ast.Mult, ast.USub, ast.UAdd, ast.Not, ast.And, ast.Or, ast.Lt, ast.LtE, ast.Gt, ast.GtE, ast.Eq,
+          ast.NotEq)
+
+
+def is_cheap(expr):
+    """Whether an expression has additions, products and comparisons only."""
+    return all(isinstance(n, _CHEAP) for n in ast.walk(ast.parse(expr.strip(), mode="eval")))
+
+
+def translate_statement(st, types, declared, float_t, select=False):
+    """One statement dict (captured from Brian) -> list of C lines.
+
+    select: the two variants of an expression with one boolean variable are both
+    evaluated and one is taken, where both are cheap: the lanes of a wave mostly need
+    both, and a branch costs more than a few operations."""
     var, op, dtype = st["var"], st["op"], st["dtype"]
     R = Renderer(types)
     lines = []
@@ -341,6 +355,13 @@ def translate_statement(st, types, declared, float_t):
             c, _ = R.render(st["expr"])
             lines.append(f"const {ct} {var} = ({ct})({c});" if st.get("constant") else f"{ct} {var} = ({ct})({c});")
             return lines
+    be = st.get("bool_exprs")
+    if select and be and len(be) == 2 and len(st["bool_vars"]) == 1 and op == "=" and all(is_cheap(e) for _, e in be):
+        vals = {bool(a[0][1]): R.render(e)[0] for a, e in be}
+        if len(vals) == 2:
+            v = st["bool_vars"][0]
+            return lines + [f"{{ const {ct} hb_t = ({ct})({vals[True]}), hb_f = ({ct})({vals[False]}); "
+                            f"{var} = {v} ? hb_t : hb_f; }}"]
     if st.get("bool_exprs"):
         first = True
         nb = len(st["bool_vars"])
@@ -358,12 +379,14 @@ def translate_statement(st, types, declared, float_t):
     return lines
 
 
-def translate_block(statements, conditional_write, types, declared, float_t):
+def translate_block(statements, conditional_write, types, declared, float_t, select=False):
     out = []
     for st in statements:
-        ls = translate_statement(st, types, declared, float_t)
+        ls = translate_statement(st, types, declared, float_t, select)
         cw = conditional_write.get(st["var"])
-        if cw is not None:
+        if cw is not None and select and st["op"] == "=" and not st.get("bool_exprs") and is_cheap(st["expr"]):
+            out.append(f"{st['var']} = {cw} ? {ls[0][len(st['var']) + 3:-1]} : {st['var']};")
+        elif cw is not None:
             out.append(f"if ({cw}) {{")
             out.extend("    " + x for x in ls)
             out.append("}")

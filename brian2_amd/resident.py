@@ -1,0 +1,477 @@
+"""Networks that one workgroup steps on its own: the resident step kernel.
+
+A network without delays whose synapses all carry the same constant per pathway
+(`on_pre: x += c`) and whose neurons fit a workgroup's registers needs no other
+workgroup and no memory between its steps.  One workgroup per network runs any
+number of steps in a launch:
+
+* neuron q*T + x (thread x of T) keeps its state in thread x's registers, for
+  q < R; the neurons beyond R*T (networks larger than the register file) keep
+  theirs in memory;
+* the spikes of a step go to a list in LDS (one LDS atomic per wave that has
+  any);
+* a spike's synapses are read from the CSR by source, 64 per wave, and counted
+  per target and pathway in LDS (integer atomics, two 16-bit counts per word).
+  Every event of a pathway applies the same operation with the same operand, so
+  the count alone fixes the result: the owner applies the operation that many
+  times at its next update, pathway by pathway in schedule order, which is the
+  cython runtime's left fold over the queue
+  (brian2/codegen/runtime/cython_rt/templates/synapses.pyx:42-50) bit for bit.
+
+A step has one barrier (the spike list is complete) and, when there were spikes,
+a second one (the counts are complete).
+"""
+import math
+import re
+
+from .codegen import source_header
+
+LDS_BYTES = 163840       # LDS of one CU
+STATE_REGISTERS = 80     # 32-bit registers of a thread that may hold neuron state
+MAX_RESIDENT = 8         # neurons per thread in registers, at most
+MAX_PATHWAYS = 4         # pathways of a network (two counts per LDS word)
+UNITS_IN_FLIGHT = 4      # 64-synapse pieces a wave reads before it counts them
+MAX_NEURONS = 65535      # spike lists hold 16-bit indices
+
+_REFRACTORY = re.compile(r"not_refractory = \(bool\)\(\(hb_timestep\(\(double\)\(\(t - lastspike\)\), "
+                         r"\(double\)\(dt\)\) >= ([\w.]+)\)\);")
+
+
+def timestep_bound(k, dt):
+    """The smallest y whose quotient int(y / dt) reaches k, for k >= 1 (hb_timestep's
+    comparison with k).  y / dt rounds monotonically, so it is within a few units in the
+    last place of k * dt."""
+    y = k * dt
+    while int(math.nextafter(y, 0.0) / dt) >= k:
+        y = math.nextafter(y, 0.0)
+    while int(y / dt) < k:
+        y = math.nextafter(y, math.inf)
+    return y
+
+
+def refractory_form(update, spike, var_types):
+    """The name compared with in the refractoriness test `timestep(t - lastspike, dt) >= K`,
+    when that test is the only use of lastspike and the only assignment of not_refractory
+    in the lines of a neuron's update and spike; else None.
+
+    The test is then true from one step on until the neuron's next spike: the kernel keeps
+    that step instead of lastspike and not_refractory, compares integers, and forms the
+    step anew only when the neuron spikes."""
+    if var_types.get("lastspike") != "double" or var_types.get("not_refractory") != "bool":
+        return None
+    use = [ln for ln in list(update) + list(spike) if re.search(r"\blastspike\b|\bnot_refractory =[^=]", ln)]
+    if len(use) != 1 or use[0] not in update:
+        return None
+    m = _REFRACTORY.fullmatch(use[0].strip())
+    return None if m is None else m.group(1)
+
+
+def neurons_in_registers(var_types):
+    """Neurons per thread whose state the registers hold (1 to MAX_RESIDENT)."""
+    words = sum(2 if ct in ("double", "long long") else 1 for ct in var_types.values())
+    return max(1, min(MAX_RESIDENT, STATE_REGISTERS // max(1, words)))
+
+
+class ResidentKernel:
+    """Source of a resident step kernel.
+
+    name        kernel name
+    struct      its ParamStruct; fields used here: clock, step_off, dt, n_steps, status
+    var_types   {state variable: C type}
+    update      lines of one neuron's step: they read and write the variables by name and
+                set hb_cond (the neuron spikes)
+    spike       lines of a neuron that spikes (its reset), after the update
+    refractory  whether a spike also sets not_refractory = false and lastspike = t
+    pathways    [(variable, operator, C expression of the operand)] in schedule order
+    prologue    lines that define, per workgroup: N, hb_off (the network's first neuron in
+                the state arrays), hb_rp (row pointers by source), hb_step0
+    event       lines that, for the synapse word hb_syn of source hb_src, define the target
+                hb_tgt and the pathway's number hb_path
+    events      further lines per event
+    record      lines run for a step's spikes (s_spk[0 .. hb_nsp), any order) by every
+                thread; may contain barriers
+    begin/start lines that set hb_recq[q] of neuron i, and lines run before its every step
+                with hb_rec = hb_recq[q] (state monitors)
+    finish      lines run once at the end by every thread
+    resident    neurons per thread in registers
+    bound       C expression of timestep_bound(K, dt) when K >= 1 is the refractory period
+                in steps, so that the release step may be kept (refractory_form)
+    rows_in_lds, counts_in_lds   where row pointers and counts are kept
+
+    What bounds it.  A step is a chain: the update of R neurons per thread, a barrier, the
+    spikes' rows, their synapses (one memory round trip), LDS atomics, a barrier.  The update
+    is straight-line code, so that a wave works on several neurons at a time: what few
+    neurons need (a second event of a pathway, the spike itself) is tested once for all R
+    and handled apart.  Measured on MI355X, cycles per step: a network of 7996 neurons
+    (fp64, 16 waves, two spikes a step) 5070 for the update (2250 of them per wave alone;
+    with branches per neuron 8000), 500 for the rows, 1150 for the synapses, 200 at the
+    second barrier.  1024 networks of 500 to 8000 neurons: 42.9 -> 9.4 us per step against
+    the state in memory and one spike's row at a time behind a barrier; 48 networks (fp32):
+    9.5 -> 2.3.
+    """
+
+    def __init__(self, name, struct, var_types, update, pathways, prologue, event, spike=(), refractory=False,
+                 record=(), start=(), begin=(), finish=(), events=(), max_threads=1024, resident=None,
+                 rows_in_lds=True, counts_in_lds=True, shared=(), bound=None):
+        if not 1 <= len(pathways) <= MAX_PATHWAYS:
+            raise NotImplementedError(f"1 to {MAX_PATHWAYS} pathways")
+        self.kernel_name, self.struct = name, struct
+        self.words = W = (len(pathways) + 1) // 2
+        self.resident = R = resident or neurons_in_registers(var_types)
+        self.rows_in_lds, self.counts_in_lds = rows_in_lds, counts_in_lds
+        period = refractory_form(update, spike, var_types) if refractory else None
+        released = bound is not None and period is not None
+        # what the registers hold: with the release step, neither lastspike nor not_refractory
+        held = {v: ct for v, ct in var_types.items() if not (released and v in ("lastspike", "not_refractory"))}
+        pt = {v: ("unsigned char" if ct == "bool" else ct) for v, ct in var_types.items()}
+        load = {v: (f"p.a_{v}[hb_off + i] != 0" if ct == "bool" else f"p.a_{v}[hb_off + i]") for v, ct in var_types.items()}
+        save = {v: (f"{v} ? 1 : 0" if ct == "bool" else v) for v, ct in var_types.items()}
+        regs = ", ".join(f"r_{v}[q]" for v in held)
+        held_args, all_args = ", ".join(held), ", ".join(var_types)
+        mem_load = " ".join(f"{ct} {v} = {load[v]};" for v, ct in var_types.items())
+        mem_save = " ".join(f"p.a_{v}[hb_off + i] = ({pt[v]})({save[v]});" for v in var_types)
+        # a neuron's events: counted by anybody, read and cleared by its owner (in memory: past
+        # the caches, as the atomics go)
+        pitch = "hb_np" if counts_in_lds else "N"
+        at = f"s_cnt[(size_t){{w}} * {pitch} + i]"
+        if counts_in_lds:
+            read, clear = at, at + " = 0u;"
+        else:
+            read = f"(i < N ? __hip_atomic_load(&{at}, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u)"
+            clear = f"if (i < N) __hip_atomic_store(&{at}, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);"
+        reads = [f"const unsigned int hb_c{w} = {read.format(w=w)};" for w in range(W)]
+        clears = [clear.format(w=w) for w in range(W)]
+
+        def decl(vs):
+            return ", ".join(f"{ct}& {v}" for v, ct in vs.items())
+
+        def field(r, c="hb_c{w}"):
+            c = c.format(w=r // 2)
+            return f"({c} & 0xffffu)" if r % 2 == 0 else f"({c} >> 16)"
+
+        def each_event():  # every event of neuron i, pathway by pathway
+            return [f"for (unsigned int n_ = {field(r)}; n_ > 0u; n_--) {var} {op} {val};"
+                    for r, (var, op, val) in enumerate(pathways)]
+
+        k = [source_header(max_threads), struct.c_decl()]
+        k.append(f'extern "C" __global__ void __launch_bounds__({max_threads}) {name}(const {struct.name} p) {{')
+        k += ["    " + x for x in prologue]
+        k += [
+            "    // the waves that the network's neurons fill: the others end here (barriers count the",
+            "    // waves that run)",
+            f"    const int NW = min((int)blockDim.x >> 6, max(1, (N + {64 * R - 1}) / {64 * R})), T = NW * 64;",
+            "    if ((int)threadIdx.x >= T) return;",
+            "    const int lane = threadIdx.x & 63;",
+            "    const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));",
+            "    const double dt = p.dt;",
+            f"    const int hb_np = N > {R} * T ? N : {R} * T;  // counts of a pathway pair",
+            "    extern __shared__ __align__(16) unsigned char hb_lds[];",
+        ]
+        lds = "hb_lds"
+        if counts_in_lds:
+            k.append(f"    unsigned int* const s_cnt = (unsigned int*)hb_lds;  // [{W}][hb_np], two counts a word")
+            lds = f"(s_cnt + {W} * hb_np)"
+        else:
+            k.append(f"    unsigned int* const s_cnt = p.counts + (size_t)hb_off * {W};")
+        if rows_in_lds:
+            k.append(f"    unsigned int* const s_rp = (unsigned int*){lds};")
+            lds = "(s_rp + N + 1)"
+        row = "s_rp[{}]" if rows_in_lds else "hb_rp[{}]"
+        k += [
+            f"    unsigned short* const s_spk = (unsigned short*){lds};",
+            "    __shared__ int s_n[3];  // spikes of steps s % 3: added to, read, cleared in turn",
+        ]
+        k += ["    " + x for x in shared]
+        if released:
+            k += [
+                f"    const double hb_tb = {bound};",
+                "    // a neuron that last spiked at time x is not refractory from the step k on (a double:",
+                "    // exact) at which (k * dt - x) + 1e-3 * dt >= hb_tb, which grows with k",
+                "    auto hb_free = [&](const double x, const double k) { return (k * dt - x) + 1e-3 * dt >= hb_tb; };",
+                "    auto hb_release = [&](const double x) {  // that step, counted from hb_step0 and 0 at least",
+                "        const double k0 = (double)hb_step0;",
+                "        if (hb_free(x, k0)) return 0;",
+                "        double k = floor((hb_tb + x) / dt);",
+                "        for (int j = 0; j < 8 && hb_free(x, k - 1.0); j++) k -= 1.0;",
+                "        for (int j = 0; j < 8 && !hb_free(x, k); j++) k += 1.0;",
+                "        k -= k0;",
+                "        return k < 2147483647.0 ? (int)k : 0x7fffffff;",
+                "    };",
+            ]
+        # the update of a neuron in registers, and of one in memory where they differ
+        for fn, vs in (("hb_update", held), ("hb_update_mem", var_types)):
+            reg = released and fn == "hb_update"
+            lines = ["not_refractory = s >= hb_rel;" if reg and _REFRACTORY.fullmatch(x.strip()) else x for x in update]
+            k += [
+                "    // one step of neuron i after the events of the step before: whether it spikes",
+                f"    auto {fn} = [&](const int i, const int s, const double t, {decl(vs)}"
+                f"{', const int hb_rel' if reg else ''}) __attribute__((always_inline)) {{",
+                "        const int _idx = i;",
+                "        (void)_idx; (void)s; (void)t;",
+                "        bool hb_cond = false;",
+            ]
+            k += ["        bool not_refractory;"] if reg else []
+            k += ["        " + x for x in lines]
+            k += ["        return hb_cond;", "    };"]
+            if not released:
+                break
+        k += [f"    auto hb_spike = [&](const int i, const double t, {decl(held)}) __attribute__((always_inline)) {{",
+              "        const int _idx = i;", "        (void)_idx; (void)t;"]
+        if refractory and not released:
+            k.append("        not_refractory = false; lastspike = t;")
+        k += ["        " + x for x in spike]
+        k.append("    };")
+        if rows_in_lds:
+            k.append("    for (int i = threadIdx.x; i <= N; i += T) s_rp[i] = hb_rp[i];")
+        k.append("    if (threadIdx.x < 3) s_n[threadIdx.x] = 0;")
+        first = "hb_release(p.a_lastspike[hb_off + i])"
+        if released and counts_in_lds:  # formed one by one (the code is long), passed through the counts
+            k += [
+                "    #pragma unroll 1",
+                f"    for (int i = threadIdx.x; i < {R} * T; i += T)",
+                f"        s_cnt[i] = i < N ? (unsigned int){first} : 0x7fffffffu;",
+            ]
+            first = "(int)s_cnt[i]"
+        for v, ct in held.items():
+            k.append(f"    {ct} r_{v}[{R}];")
+        if released:
+            k.append(f"    int r_rel[{R}];")
+        if start:
+            k.append(f"    int hb_recq[{R}];")
+        k += [
+            f"    unsigned long long hb_act[{R}];  // lanes with a neuron (scalars)",
+            "    #pragma unroll",
+            f"    for (int q = 0; q < {R}; q++) {{",
+            "        const int i = q * T + (int)threadIdx.x;",
+            "        const bool act = i < N;",
+            "        hb_act[q] = __builtin_amdgcn_ballot_w64(act);",
+        ]
+        for v, ct in held.items():
+            k.append(f"        r_{v}[q] = act ? {load[v]} : ({ct})0;")
+        if released:
+            k.append(f"        r_rel[q] = act ? {first} : 0x7fffffff;")
+        k += ["        " + x for x in begin]
+        k.append("        // waited for here: a wait inside the loop would be for the step's stores as well")
+        k += [f'        asm volatile("" : "+v"(r_{v}[q]));' for v, ct in held.items() if ct != "bool"]
+        k.append("    }")
+        if counts_in_lds:
+            k.append(f"    for (int i = threadIdx.x; i < {W} * hb_np; i += T) s_cnt[i] = 0u;")
+        k.append("    __syncthreads();")
+        fence = [] if counts_in_lds else ["__threadfence();  // the counts are in memory"]
+        put = [
+            "if (b_ != 0ull) {  // the wave's spikes to the list",
+            "    int o_ = 0;",
+            "    if (lane == 0) o_ = atomicAdd(&s_n[hb_cur], __popcll(b_));",
+            "    o_ = __builtin_amdgcn_readfirstlane(o_);",
+            "    if ((b_ >> lane) & 1ull) {",
+            "        s_spk[o_ + __popcll(b_ & ((1ull << lane) - 1ull))] = (unsigned short)i;",
+        ]
+        k += [
+            "    int hb_cur = 0, hb_old = 2;",
+            "    double hb_k = (double)hb_step0;  // the step (exact)",
+            "    for (int s = 0; s < p.n_steps; s++, hb_k += 1.0) {",
+            "        const long long step = hb_step0 + s;",
+            "        const double t = hb_k * dt;  // (double)step * dt",
+            "        (void)step;",
+        ]
+        k += [f"        unsigned int hb_c{w}[{R}], hb_o{w} = 0u;" for w in range(W)]
+        k += ["        #pragma unroll", f"        for (int q = 0; q < {R}; q++) {{  // all reads in flight together",
+              "            const int i = q * T + (int)threadIdx.x;"]
+        k += [f"            hb_c{w}[q] = {read.format(w=w)};" for w in range(W)]
+        k += [f"            hb_o{w} |= hb_c{w}[q];" for w in range(W)]
+        k.append("        }")
+        more = " | ".join(f"(hb_o{w} & 0xfffefffeu)" for w in range(W))
+        same = len({v for v, _, _ in pathways}) < len(pathways)
+        # pathways into one variable follow each other, so only the last of them may leave its
+        # last event to the selection below
+        last = {v: r for r, (v, _, _) in enumerate(pathways)}
+        rest = " | ".join(f"hb_o{w}" for w in range(W)) if same else more
+        k += [f"        if (__builtin_amdgcn_ballot_w64(({rest}) != 0u) != 0ull) {{  // more events than one of a pathway",
+              "            #pragma unroll", f"            for (int q = 0; q < {R}; q++) {{"]
+        k += [f"                {held[v]}& {v} = r_{v}[q];" for v in dict.fromkeys(v for v, _, _ in pathways)]
+        for r_, (var, op, val) in enumerate(pathways):
+            k.append(f"                for (unsigned int n_ = {field(r_, 'hb_c{w}[q]')}; n_ > "
+                     f"{1 if last[var] == r_ else 0}u; n_--) {var} {op} {val};")
+        k += ["            }", "        }",
+              f"        unsigned long long hb_b[{R}], hb_any = 0ull;  // the wave's spikes (scalars)",
+              "        #pragma unroll",
+              f"        for (int q = 0; q < {R}; q++) {{  // lanes without a neuron compute on zeros",
+              "            const int i = q * T + (int)threadIdx.x;"]
+        for r_, (var, op, val) in enumerate(pathways):
+            if last[var] == r_:
+                k += [f"            {{ {held[var]} x_ = r_{var}[q]; x_ {op} {val}; "
+                      f"r_{var}[q] = {field(r_, 'hb_c{w}[q]')} != 0u ? x_ : r_{var}[q]; }}"]
+        k += ["            " + x for x in clears]
+        if start:
+            k += ["            if (i < N) {"] + [f"                const {ct}& {v} = r_{v}[q];" for v, ct in held.items()]
+            k += ["                const int hb_rec = hb_recq[q];"]
+            k += ["                " + x for x in start] + ["            }"]
+        k += [
+            f"            hb_b[q] = __builtin_amdgcn_ballot_w64(hb_update(i, s, t, {regs}"
+            f"{', r_rel[q]' if released else ''})) & hb_act[q];",
+            "            hb_any |= hb_b[q];",
+            "        }",
+            "        if (hb_any != 0ull) {",
+            "            int hb_x = (int)threadIdx.x;  // hidden: see the end",
+            '            asm volatile("" : "+v"(hb_x));',
+        ]
+        if released:
+            k += [
+                "            // the release step of a neuron that spikes now: K steps on, or one beside it by rounding",
+                f"            const double k_ = hb_k + (double)({period});",
+                f"            const int rel_ = s + (int)({period}) + (hb_free(t, k_ - 1.0) ? -1 : hb_free(t, k_) ? 0 : 1);",
+            ]
+        k += ["            #pragma unroll", f"            for (int q = 0; q < {R}; q++) {{",
+              "                const int i = q * T + hb_x;", "                const unsigned long long b_ = hb_b[q];"]
+        k += ["                " + x for x in put]
+        if released:
+            k.append("                        r_rel[q] = rel_; p.a_lastspike[hb_off + i] = t;")
+        k += [f"                        hb_spike(i, t, {regs});", "                    }", "                }",
+              "            }", "        }",
+              f"        for (int j0 = {R} * T; j0 < N; j0 += T) {{  // neurons beyond the registers",
+              "            const int i = j0 + (int)threadIdx.x;",
+              "            bool sp = false;",
+              "            if (i < N) {",
+              f"                {mem_load}"]
+        k += ["                " + x for x in reads + each_event() + clears]
+        if start:
+            k += ["                {"] + ["                " + x for x in self._search(begin)]
+            k += ["                " + x for x in start] + ["                }"]
+        k += [f"                sp = {'hb_update_mem' if released else 'hb_update'}(i, s, t, {all_args});",
+              "                if (sp) {"]
+        if released:
+            k.append("                    not_refractory = false; lastspike = t;")
+        k += [f"                    hb_spike(i, t, {held_args});", "                }",
+              f"                {mem_save}", "            }",
+              "            const unsigned long long b_ = __builtin_amdgcn_ballot_w64(sp);"]
+        k += ["            " + x for x in put] + ["                }", "            }"]
+        k += ["        }"] + ["        " + x for x in fence] + [
+            "        __syncthreads();",
+            "        const int hb_nsp = s_n[hb_cur];",
+            "        // the last step's counter: every wave has read it, and it is added to again only",
+            "        // behind the next step's barrier",
+            "        if (threadIdx.x == 0) s_n[hb_old] = 0;",
+            "        hb_old = hb_cur;",
+            "        hb_cur = hb_cur == 2 ? 0 : hb_cur + 1;",
+            "        if (hb_nsp > 0) {",
+        ]
+        k += ["            " + x for x in record]
+
+        def unit(u, ok, x, src, ind):
+            return [ind + ln for ln in (
+                f"const int l_ = __builtin_ctzll(__builtin_amdgcn_ballot_w64(in_ > {u}));",
+                "const int first_ = __builtin_amdgcn_readlane(in_ - nu_, l_);",
+                "const unsigned int a_ = (unsigned int)__builtin_amdgcn_readlane((int)ra_, l_);",
+                "const unsigned int z_ = (unsigned int)__builtin_amdgcn_readlane((int)rb_, l_);",
+                f"{src} = __builtin_amdgcn_readlane(sp_, l_);",
+                f"const unsigned int e_ = a_ + (unsigned int)({u} - first_) * 64u + (unsigned int)lane;",
+                f"{ok} = e_ < z_;",
+                f"{x} = p.post[e_ < z_ ? e_ : z_ - 1u];",
+            )]
+
+        def count(x, src, ind):
+            return [ind + ln for ln in (
+                f"const unsigned int hb_syn = {x};", f"const int hb_src = {src};", "(void)hb_src;", *event,
+                f"atomicAdd(&s_cnt[(hb_path >> 1) * {pitch} + hb_tgt], hb_path & 1 ? 0x10000u : 1u);", *events)]
+
+        F = UNITS_IN_FLIGHT
+        k += [
+            "            // 64 spikes at a time: lane l holds spike l's row; the rows' pieces of 64 synapses",
+            "            // are dealt to the waves",
+            "            for (int c0 = 0; c0 < hb_nsp; c0 += 64) {",
+            "                const int sp_ = c0 + lane < hb_nsp ? (int)s_spk[c0 + lane] : -1;",
+            f"                const unsigned int ra_ = sp_ >= 0 ? {row.format('sp_')} : 0u, "
+            f"rb_ = sp_ >= 0 ? {row.format('sp_ + 1')} : 0u;",
+            "                const int nu_ = (int)((rb_ - ra_ + 63u) >> 6);",
+            "                const int in_ = hb_wave_incl_scan(nu_);",
+            "                const int U = __builtin_amdgcn_readlane(in_, 63);",
+            "                if (U <= NW) {  // at most one piece per wave",
+            "                    if (wid < U) {",
+            "                        int g_; bool ok_; unsigned int x_;",
+        ]
+        k += unit("wid", "ok_", "x_", "g_", " " * 24)
+        k += ["                        if (ok_) {"] + count("x_", "g_", " " * 28) + ["                        }"]
+        k += [
+            "                    }",
+            "                } else {",
+            f"                    for (int u0 = wid; u0 < U; u0 += {F} * NW) {{",
+            f"                        unsigned int x_[{F}];",
+            f"                        int g_[{F}];",
+            f"                        bool ok_[{F}];",
+            "                        #pragma unroll",
+            f"                        for (int j = 0; j < {F}; j++) {{",
+            "                            const int u = u0 + j * NW;",
+            "                            ok_[j] = false; x_[j] = 0u; g_[j] = 0;",
+            "                            if (u < U) {  // the same for the wave",
+        ]
+        k += unit("u", "ok_[j]", "x_[j]", "g_[j]", " " * 32)
+        k += [
+            "                            }",
+            "                        }",
+            "                        #pragma unroll",
+            f"                        for (int j = 0; j < {F}; j++)",
+            "                            if (ok_[j]) {",
+        ]
+        k += count("x_[j]", "g_[j]", " " * 32)
+        k += [
+            "                            }",
+            "                    }",
+            "                }",
+            "            }",
+        ] + ["            " + x for x in fence] + [
+            "            __syncthreads();",
+            "        }",
+            "    }",
+            "    // the last step's events, and the state back to memory (the index is hidden from the",
+            "    // compiler, which would keep the addresses of the first loads in registers for it)",
+            "    int hb_x = (int)threadIdx.x;",
+            '    asm volatile("" : "+v"(hb_x));',
+            "    #pragma unroll",
+            f"    for (int q = 0; q < {R}; q++) {{",
+            "        const int i = q * T + hb_x;",
+            "        if (i < N) {",
+        ]
+        k += ["            " + x for x in reads]
+        k += [f"            {held[v]}& {v} = r_{v}[q];" for v in dict.fromkeys(v for v, _, _ in pathways)]
+        k += ["            " + x for x in each_event() + clears]
+        for v, ct in held.items():
+            val = f"r_{v}[q] ? 1 : 0" if ct == "bool" else f"r_{v}[q]"
+            k.append(f"            p.a_{v}[hb_off + i] = ({pt[v]})({val});")
+        if released:
+            k.append("            p.a_not_refractory[hb_off + i] = p.n_steps - 1 >= r_rel[q] ? 1 : 0;")
+        k += [
+            "        }",
+            "    }",
+            f"    for (int i = {R} * T + hb_x; i < N; i += T) {{",
+            f"        {mem_load}",
+        ]
+        k += ["        " + x for x in reads + each_event() + clears]
+        k += [f"        {mem_save}", "    }"]
+        k += ["    " + x for x in finish]
+        k.append("}")
+        self.source = "\n".join(k) + "\n"
+
+    @staticmethod
+    def _search(begin):
+        """The begin lines for a neuron outside the registers (hb_rec instead of hb_recq[q])."""
+        return ["int hb_recm[1]; { const int q = 0; const bool act = true;"] + [
+            x.replace("hb_recq", "hb_recm") for x in begin] + ["}", "const int hb_rec = hb_recm[0];"]
+
+    def lds_bytes(self, N, threads, extra=0):
+        """Dynamic LDS of a workgroup of that many threads for a network of N neurons."""
+        b = 2 * N + extra
+        if self.counts_in_lds:
+            b += 4 * self.words * max(N, self.resident * threads)
+        if self.rows_in_lds:
+            b += 4 * (N + 1)
+        return (b + 15) // 16 * 16
+
+
+def lds_plan(N, words, extra=0):
+    """(rows_in_lds, counts_in_lds) for networks of up to N neurons: the counts first (they
+    are written), then the row pointers (read, once per spike)."""
+    room = LDS_BYTES - 2048 - 2 * N - extra
+    c = 4 * words * max(N, 1024 * MAX_RESIDENT)
+    counts = c <= room
+    rows = counts and c + 4 * (N + 1) <= room
+    return rows, counts

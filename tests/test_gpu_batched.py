@@ -115,3 +115,35 @@ def test_batched_fp32_equals_the_plain_fp32_path():
         o = np.lexsort((i, s))
         assert np.array_equal(i[o], c["mon"].i) and np.array_equal(s[o], c["mon"].step), net.N
         assert np.array_equal(B.get("v", k), c["G"].get("v")), net.N
+
+
+@pytest.mark.parametrize("variant", ["registers", "lastspike kept", "rows in memory", "counts in memory"])
+def test_resident_forms_at_the_edges_of_a_workgroup(variant, monkeypatch):
+    """Networks of sizes around a wave, a workgroup and the registers' share of it (the last
+    two have neurons in memory), first a step in which every second neuron spikes, then
+    ordinary ones: every form of the kernel equals the plain path's staged fold."""
+    from brian2_amd import batched, resident, synth
+
+    if variant == "lastspike kept":
+        monkeypatch.setattr(batched, "refractory_form", lambda *a: None)
+    elif variant != "registers":
+        monkeypatch.setattr(batched, "lds_plan", lambda *a: (False, variant == "rows in memory"))
+    sizes = [63, 64, 65, 511, 512, 513, 1025, 2049, 8192, 8193]
+    nets = [batched.SweepNetwork(n, n * 4 // 5, 7 + k, {"we": 1.62e-3 * (0.5 + 0.2 * k)}) for k, n in enumerate(sizes)]
+    B = batched.BatchedCUBA(nets)
+    B.block, B.steps_per_launch = 1024, 10
+    B.build()
+    B.state["v"][::2] = -0.0495
+    B.run(150)
+    for k, net in enumerate(nets):
+        c = synth.cuba_network(N=net.N, NE=net.NE, seed=net.seed, we=net.namespace["we"],
+                               network_options={"tile": 256})
+        v = c["G"].get("v")
+        a = int(B.n_off[k])
+        v[a % 2::2] = -0.0495
+        c["G"].v = v
+        c["net"].run(150)
+        i, s = B.spikes(k)
+        assert len(i) > 0 and np.array_equal(i, c["mon"].i) and np.array_equal(s, c["mon"].step), net.N
+        for x in ("v", "ge", "gi", "lastspike", "not_refractory"):
+            assert np.array_equal(B.get(x, k), c["G"].get(x)), (net.N, x)
