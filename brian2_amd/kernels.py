@@ -475,6 +475,21 @@ def _fold_passes(T, U, W, cap, vt, apply_lines, npt=1):
     return k
 
 
+def group_block(tag, spec, arrays, scalars, float_t, extra_types=(), select=False):
+    """C lines of one of a group's code objects: state variables by their names, scalars
+    ({(tag, name): (value, ctype)}) as fields p.<tag>_<name> of the parameter struct."""
+    types = dict(arrays)
+    types.update({"t": "double", "dt": "double", "N": "int", "i": "int", "_idx": "int"})
+    types.update(extra_types)
+    names = {}
+    for (tg, n), (_, ct) in scalars.items():
+        if tg == tag:
+            types[n] = ct
+            names[n] = f"p.{tag}_{n}"
+    lines = translate_block(spec.vector, spec.conditional_write, types, set(), float_t, select)
+    return _rename(lines, names)
+
+
 # ---------------------------------------------------------------------------
 class NeuronKernel:
     """Fused per-group step kernel (or the end-of-run flush kernel)."""
@@ -514,16 +529,7 @@ class NeuronKernel:
         self._build()
 
     def _block(self, tag, spec, extra_types):
-        types = dict(self.arrays)
-        types.update({"t": "double", "dt": "double", "N": "int", "i": "int", "_idx": "int"})
-        types.update(extra_types)
-        names = {}
-        for (tg, n), (_, ct) in self.scalars.items():
-            if tg == tag:
-                types[n] = ct
-                names[n] = f"p.{tag}_{n}"
-        lines = translate_block(spec.vector, spec.conditional_write, types, set(), self.float_t)
-        return _rename(lines, names)
+        return group_block(tag, spec, self.arrays, self.scalars, self.float_t, extra_types)
 
     def _build(self):
         ps = ParamStruct(f"hbp_{self.name}")

@@ -21,10 +21,12 @@ number of steps in a launch:
 A step has one barrier (the spike list is complete) and, when there were spikes,
 a second one (the counts are complete).
 """
+import ast
 import math
 import re
 
-from .codegen import source_header
+from .codegen import ParamStruct, Renderer, source_header
+from .kernels import _rename, group_block
 
 LDS_BYTES = 163840       # LDS of one CU
 STATE_REGISTERS = 80     # 32-bit registers of a thread that may hold neuron state
@@ -60,7 +62,7 @@ def refractory_form(update, spike, var_types):
     if var_types.get("lastspike") != "double" or var_types.get("not_refractory") != "bool":
         return None
     use = [ln for ln in list(update) + list(spike) if re.search(r"\blastspike\b|\bnot_refractory =[^=]", ln)]
-    if len(use) != 1 or use[0] not in update:
+    if len(use) != 1 or use[0] not in update or any("not_refractory" in ln for ln in spike):
         return None
     m = _REFRACTORY.fullmatch(use[0].strip())
     return None if m is None else m.group(1)
@@ -475,3 +477,215 @@ def lds_plan(N, words, extra=0):
     counts = c <= room
     rows = counts and c + 4 * (N + 1) <= room
     return rows, counts
+
+
+def heavy_operations(specs):
+    """Exponentials, powers and the like in the vector code of code objects."""
+    n = 0
+    for spec in specs:
+        for st in spec.vector if spec is not None else ():
+            exprs = [e for _, e in st.get("bool_exprs") or []] or [st["expr"]]
+            n += max(sum(isinstance(x, ast.Call) and x.func.id not in ("int", "float", "abs", "timestep", "sign", "clip")
+                         or isinstance(x, ast.Pow) for x in ast.walk(ast.parse(e.strip(), mode="eval")))
+                     for e in exprs)
+    return n
+
+
+class GroupStep:
+    """The resident step of a neuron group with synapses onto itself (Network's small
+    networks): the ResidentKernel with the group's monitors.
+
+    group      its NeuronGroup; scalars {(tag, name): (value, ctype)} of its code objects
+    pathways   [(Synapses, {name: (value, ctype)})] in schedule order
+    val_t      type in which the pathways' values are held before they are applied"""
+
+    MAX_SYNAPSES = 1 << 25
+    MAX_HEAVY = {"double": 16384, "float": 36864}  # neurons x heavy operations of an update
+
+    def __init__(self, group, scalars, pathways, val_t, n_syn, dt):
+        g = group
+        # as few neurons per thread as 1024 threads allow: 500 neurons one / two / eight per
+        # thread 0.81 / 1.07 / 1.62 us per step, 4000 four / eight 2.03 / 2.39
+        self.rows = -(-g.N // 1024)
+        waves = -(-g.N // 64)
+        self.threads = 64 * -(-waves // self.rows)
+        ps = ParamStruct(f"hbr_{g.name}")
+        ps.ptr("clock", "long long")
+        ps.val("step_off", "long long")
+        ps.val("dt", "double")
+        ps.val("n_steps", "int")
+        ps.val("N", "int")
+        for v, ct in g.vars.items():
+            ps.ptr(f"a_{v}", "unsigned char" if ct == "bool" else ct)
+        for (tg, n), (_, ct) in sorted(scalars.items()):
+            ps.val(f"{tg}_{n}", ct)
+        for r, (_, sc) in enumerate(pathways):
+            for n, (_, ct) in sorted(sc.items()):
+                ps.val(f"c{r}_{n}", ct)
+        ps.val("bound", "double")
+        ps.ptr("row_ptr", "unsigned int", const=True)
+        ps.ptr("post", "unsigned int", const=True)
+        ps.ptr("events", "unsigned long long")
+        ps.ptr("counts", "unsigned int")
+        ps.ptr("status", "int")
+        if g.smon:
+            ps.ptr("mon_i", "int")
+            ps.ptr("mon_step", "int")
+            ps.ptr("mon_n", "unsigned long long")
+            ps.ptr("mon_count", "int")
+            ps.val("mon_cap", "long long")
+            ps.val("mon_start", "int")
+            ps.val("mon_stop", "int")
+        if g.rmon:
+            ps.ptr("rate_cnt", "int")
+            ps.val("rate_row0", "long long")
+            ps.val("rate_rows", "long long")
+            ps.val("rate_start", "int")
+            ps.val("rate_stop", "int")
+        if g.stmon:
+            ps.ptr("rec_idx", "int", const=True)
+            ps.ptr("rec_buf", "double")
+            ps.val("rec_row0", "long long")
+            ps.val("rec_rows", "long long")
+            ps.val("n_rec", "int")
+            ps.val("pad_rec", "int")
+        self.struct = ps
+
+        def block(tag, spec, extra=()):
+            return group_block(tag, spec, g.vars, scalars, g.float_t, extra, select=True)
+
+        update, spike = [], []
+        if g.su is not None:
+            update += ["{"] + block("su", g.su) + ["}"]
+        if g.th is not None:
+            update += ["{"] + block("th", g.th, {"_cond": "bool"}) + ["hb_cond = _cond;", "}"]
+        if g.rs is not None:
+            spike = block("rs", g.rs)
+        # the refractory period in steps, compared through its bound
+        recorded = set(g.stmon.variables) if g.stmon else set()
+        self.bound = None
+        name = refractory_form(update, spike, g.vars)
+        if name is not None and not recorded & {"lastspike", "not_refractory"}:
+            value, ct = scalars.get(("su", name[len("p.su_"):]), (0, None))
+            if ct == "long long" and value >= 1:
+                self.bound = timestep_bound(value, dt)
+        ops, events = [], []
+        for r, (s, sc) in enumerate(pathways):
+            c, _ = Renderer({n: ct for n, (_, ct) in sc.items()}).render(s.spec.vector[0]["expr"])
+            c, = _rename([c], {n: f"p.c{r}_{n}" for n in sc})
+            ops.append((s.target_var, s.op, f"(({val_t})({c}))"))
+            events.append(f"hb_ev{r} += hb_path == {r} ? 1u : 0u;")
+        prologue = [
+            "const int N = p.N, hb_off = 0;",
+            "const unsigned int* hb_rp = p.row_ptr;",
+            "const long long hb_step0 = p.clock[0] + p.step_off;",
+        ] + [f"unsigned long long hb_ev{r} = 0ull;" for r in range(len(ops))]
+        record, finish, shared, begin, start = [], [], [], [], []
+        # the record is the last waves' work: the first ones have the spikes' synapses
+        each = "for (int j = T - 1 - (int)threadIdx.x; j < {n}; j += T) {{"
+        if g.smon:
+            add = ["if (o_ < (unsigned long long)p.mon_cap) { p.mon_i[o_] = id_; p.mon_step[o_] = (int)step; }",
+                   "atomicAdd(&p.mon_count[id_ - p.mon_start], 1);"]
+            if g.smon.range == (0, g.N):
+                prologue.append("unsigned long long hb_mn = p.mon_n[0];")
+                record += [each.format(n="hb_nsp"), "    const int id_ = (int)s_spk[j];",
+                           "    const unsigned long long o_ = hb_mn + (unsigned long long)j;"]
+                record += ["    " + x for x in add] + ["}", "hb_mn += (unsigned long long)hb_nsp;"]
+            else:
+                prologue.append("const unsigned long long hb_m0 = p.mon_n[0];")
+                shared += ["__shared__ unsigned int s_mon;  // records of the launch", "if (threadIdx.x == 0) s_mon = 0u;"]
+                record += [each.format(n="hb_nsp"), "    const int id_ = (int)s_spk[j];",
+                           "    if (id_ >= p.mon_start && id_ < p.mon_stop) {",
+                           "        const unsigned long long o_ = hb_m0 + (unsigned long long)atomicAdd(&s_mon, 1u);"]
+                record += ["        " + x for x in add] + ["    }", "}"]
+                finish += ["const unsigned long long hb_mn = hb_m0 + (unsigned long long)s_mon;"]
+            finish += ["if (threadIdx.x == 0) {", "    p.mon_n[0] = hb_mn;",
+                       "    if (hb_mn > (unsigned long long)p.mon_cap) atomicOr(p.status, 2);", "}"]
+        if g.rmon:
+            record += [
+                "if (p.rate_cnt && step - p.rate_row0 >= 0 && step - p.rate_row0 < p.rate_rows) {",
+                "    " + each.format(n="hb_nsp"),
+                "        const int id_ = (int)s_spk[j];",
+                "        if (id_ >= p.rate_start && id_ < p.rate_stop) atomicAdd(&p.rate_cnt[step - p.rate_row0], 1);",
+                "    }",
+                "}",
+            ]
+        if g.stmon:  # recorded neurons: their place in rec_idx, or -1
+            begin += [
+                "hb_recq[q] = -1;",
+                "if (act) {",
+                "    int lo = 0, hi = p.n_rec;",
+                "    while (lo < hi) { const int m = (lo + hi) >> 1; if (p.rec_idx[m] < i) lo = m + 1; else hi = m; }",
+                "    if (lo < p.n_rec && p.rec_idx[lo] == i) hb_recq[q] = lo;",
+                "}",
+            ]
+            nv = len(g.stmon.variables)
+            start += ["if (hb_rec >= 0 && step - p.rec_row0 >= 0 && step - p.rec_row0 < p.rec_rows) {",
+                      f"    double* const o_ = p.rec_buf + (size_t)(step - p.rec_row0) * {nv} * p.n_rec + hb_rec;"]
+            start += [f"    o_[(size_t){a} * p.n_rec] = (double){v};" for a, v in enumerate(g.stmon.variables)] + ["}"]
+        finish += [f"if (hb_ev{r}) atomicAdd(&p.events[{r}], hb_ev{r});" for r in range(len(ops))]
+        finish.append("if (threadIdx.x == 0) p.clock[0] = hb_step0 + p.n_steps;")
+        self.ops, self.n_syn = ops, n_syn
+        self.kernel = ResidentKernel(
+            f"resident_{g.name}", ps, g.vars, update, ops, prologue,
+            ["const int hb_tgt = (int)(hb_syn & 0xffffu);", "const int hb_path = (int)(hb_syn >> 16);"], spike=spike,
+            refractory=g.uses_refractory and g.th is not None, record=record, start=start, begin=begin, finish=finish,
+            events=events, max_threads=self.threads, resident=self.rows, shared=shared,
+            bound="p.bound" if self.bound is not None else None)
+        self.lds_bytes = self.kernel.lds_bytes(g.N, self.threads)
+
+    @classmethod
+    def takes(cls, net, groups, paths, summed):
+        """Whether Network net is stepped this way: one group whose neurons fit a workgroup's
+        registers, synapses from it onto itself without delays or variables of their own,
+        default launch shapes, an update that one compute unit can carry.
+
+        Measured on MI355X, us per step, this step against a launch for the group and one
+        per pathway: CUBA with 500 / 4000 / 8192 neurons 0.83 / 2.0 / 3.9 against
+        12.7 / 16.0 / 18.9; 8000 neurons with 19 million synapses 3.9 against 23.7 (in a
+        volley one compute unit has all the events, hence the bound on them).  An update
+        with exponentials is throughput: COBAHH (29 of them) with 400 / 600 / 1000 neurons
+        18.7 / 26.2 / 42.6 against 23.7 / 25.9 / 29.7 in fp64, with 1000 / 2000 neurons
+        18.2 / 38.6 against 23.8 / 27.8 in fp32."""
+        if len(groups) != 1 or summed or not 1 <= len(paths) <= MAX_PATHWAYS:
+            return False
+        if any(x is not None for x in (net.tile, net.npt, net.gather_pairs, net.bucket_cap)):
+            return False
+        g = groups[0]
+        if getattr(g, "su", None) is None or not 1 <= g.N <= 1024 * neurons_in_registers(g.vars):
+            return False
+        if g.N * heavy_operations((g.su, g.th, g.rs)) > cls.MAX_HEAVY[g.float_t]:
+            return False
+        for s in paths:
+            if s.source is not g or s.target is not g or s.syn_vars or s.plastic or s.post_spec is not None:
+                return False
+            if s.count_events or s.carry is not None or s.csr["dmin"] != 0 or s.csr["n_seg"] != 1:
+                return False
+            if len(s.spec.vector) != 1 or g.vars[s.target_var] not in ("double", "float"):
+                return False
+        return sum(int(s.csr["n_syn"]) for s in paths) <= cls.MAX_SYNAPSES
+
+    @staticmethod
+    def merged_rows(group, paths):
+        """The pathways' synapses as one CSR by source: row pointers and, per synapse, the
+        target and the pathway's number (bits 16 and up).  None when a target has more than
+        65535 synapses of a pathway (its count would not fit)."""
+        import torch
+
+        N, words, src = group.N, [], []
+        for r, s in enumerate(paths):
+            ptr = s.csr["seg_ptr"].long()
+            a = s.src_range[0]
+            n = int(s.csr["n_syn"])
+            post = s.csr["post"][:n]
+            if n > 65535 and int(torch.bincount(post, minlength=N).max()) > 65535:
+                return None
+            words.append(post | (r << 16))
+            src.append(torch.repeat_interleave(torch.arange(a, a + len(ptr) - 1, device=post.device), ptr[1:] - ptr[:-1],
+                                               output_size=n))
+        src, words = torch.cat(src), torch.cat(words)
+        order = torch.argsort(src, stable=True)
+        rows = torch.zeros(N + 1, dtype=torch.int64, device=src.device)
+        rows[1:] = torch.bincount(src, minlength=N).cumsum(0)
+        post = words[order] if len(words) else torch.zeros(1, dtype=torch.int32, device=src.device)
+        return rows.int(), post.int().contiguous()

@@ -19,6 +19,7 @@ import numpy as np
 
 from . import _lib
 from . import kernels as _kernels
+from . import resident as _resident
 from .codegen import ctype_of
 from .kernels import (
     LDS_BYTES,
@@ -36,6 +37,7 @@ from .kernels import (
 )
 
 L = _lib.lib
+RESIDENT_STEPS = 2000  # steps of one launch of the resident step (some ms)
 S_POISSON_GROUP = 17  # generator stream of PoissonGroup draws (hb_rng.h)
 SPEC_DIR = os.path.join(os.path.dirname(os.path.abspath(__file__)), "specs")
 
@@ -823,20 +825,20 @@ class Network:
             g.ring_cnt = zeros(g.ring_slots * len(g.ring_parts), "int")
             if isinstance(g, NeuronGroup):
                 g._dev = {n: dev(g._host[n], ct) for n, ct in g.vars.items()}
+        for g in groups:
+            g.incoming = [s for s in paths if s.target is g]
+        self.resident = None
+        if self._build_resident(groups, paths):
+            self._built = True
+            return
         # incoming pathways -> buckets
         for g in groups:
-            incoming = [s for s in paths if s.target is g]
-            g.incoming = incoming
+            incoming = g.incoming
             if not incoming:
                 continue
             if not isinstance(g, NeuronGroup):
                 raise NotImplementedError("pathways into a spike source")
-            vts = {self._value_type(s) for s in incoming}
-            if len(vts & {"int", "long long"}) and len(vts) > 1:
-                raise NotImplementedError("integer and floating-point pathway targets in one group")
-            val_t = "double" if "double" in vts else ("long long" if "long long" in vts else
-                                                        ("int" if "int" in vts else "float"))
-            g.val_t = val_t
+            g.val_t = self._group_value_type(incoming)
             self._alloc_staging(g, incoming)
         self._plan = ctypes.c_void_p()
         _lib.check(L.hb_plan_create(D.ctx, ptr(self.clock), ctypes.byref(self._plan)), "hb_plan_create")
@@ -857,12 +859,13 @@ class Network:
         for s in self.summed_syn:
             self._build_summed(s)
         for g in groups:
-            rm = [m for m in self.rmons if m.source is g]
-            if len(rm) > 1:
-                raise NotImplementedError("more than one PopulationRateMonitor per group")
-            g.rmon = rm[0] if rm else None
-            if g.rmon is not None:
-                g.rmon.buf = None
+            if not isinstance(g, NeuronGroup):
+                rm = [m for m in self.rmons if m.source is g]
+                if len(rm) > 1:
+                    raise NotImplementedError("more than one PopulationRateMonitor per group")
+                g.rmon = rm[0] if rm else None
+                if g.rmon is not None:
+                    g.rmon.buf = None
             if isinstance(g, NeuronGroup):
                 self._build_group(g)
             elif isinstance(g, PoissonGroup):
@@ -882,6 +885,114 @@ class Network:
                 if s.carry is not None:
                     _lib.check(L.hb_plan_set_lane(self._plan, s.carry_index, 1 + i % 3), "hb_plan_set_lane")
         self._built = True
+
+    def _monitors(self, g):
+        """The group's monitors (g.smon, g.stmon, g.rmon)."""
+        smon = [m for m in self.smons if m.source is g]
+        if len(smon) > 1:
+            raise NotImplementedError("more than one SpikeMonitor per group")
+        stmon = [m for m in self.stmons if m.source is g]
+        if len(stmon) > 1:
+            raise NotImplementedError("more than one StateMonitor per group")
+        rmon = [m for m in self.rmons if m.source is g]
+        if len(rmon) > 1:
+            raise NotImplementedError("more than one PopulationRateMonitor per group")
+        g.smon = smon[0] if smon else None
+        g.stmon = stmon[0] if stmon else None
+        g.rmon = rmon[0] if rmon else None
+        if g.rmon is not None:
+            g.rmon.buf = None
+        if g.stmon is not None and isinstance(g, NeuronGroup):
+            for v in g.stmon.variables:
+                if v not in g.vars:
+                    raise KeyError(f"StateMonitor variable {v!r} is not a state variable of {g.name}")
+
+    # -- networks that one workgroup steps (resident.GroupStep) ------------------
+    def _build_resident(self, groups, paths):
+        """Builds the resident step when the network takes it (resident.GroupStep.takes)."""
+        if not _resident.GroupStep.takes(self, groups, paths, self.summed_syn):
+            return False
+        g = groups[0]
+        if self._reset_mode(g) == "deferred":
+            return False
+        self._monitors(g)
+        if g.stmon is not None and g.stmon.when != "start":
+            return False
+        consts = []
+        for s in paths:
+            host = {"dt": self.dt}
+            host.update(getattr(s, "namespace", {}) or {})
+            sc = scalar_values(s.spec, host, g.float_t)
+            names = identifiers([{"var": "_value", "expr": s.spec.vector[0]["expr"]}]) - {"_value"}
+            if any(n not in sc and (n not in s.spec.variables or s.spec.variables[n]["kind"] != "Function")
+                   for n in names):
+                return False
+            consts.append((s, sc))
+        merged = _resident.GroupStep.merged_rows(g, paths)
+        if merged is None:
+            return False
+        scalars = self._group_scalars(g)
+        g.val_t = self._group_value_type(g.incoming)
+        n_syn = sum(int(s.csr["n_syn"]) for s in paths)
+        R = _resident.GroupStep(g, scalars, consts, g.val_t, n_syn, self.dt)
+        R.group, R.scalars, R.consts = g, scalars, consts
+        R.row_ptr, R.post = merged
+        R.fn = self.device.function(R.kernel.source, R.kernel.kernel_name)
+        R.cls = R.struct.ctypes_struct()
+        R.events = _torch().zeros(len(paths), dtype=_torch().int64, device="cuda")
+        for r, s in enumerate(paths):
+            s.events_dev = R.events[r:r + 1]
+            s.fused_into = None
+        g.flush_fn = None
+        if g.smon:
+            self._alloc_spike_monitor(g, g.smon)
+        if g.stmon:
+            g.stmon.rec_idx = dev(g.stmon.sorted_idx, "int")
+            g.stmon.rec_buf = None
+        self._plan = ctypes.c_void_p()
+        _lib.check(L.hb_plan_create(self.device.ctx, ptr(self.clock), ctypes.byref(self._plan)), "hb_plan_create")
+        self._launches = []
+        self.resident = R
+        return True
+
+    def _run_resident(self, n_steps):
+        """Launches the resident step for n_steps steps on the current stream."""
+        R, g = self.resident, self.resident.group
+        v = {"clock": self.clock.data_ptr(), "step_off": 0, "dt": self.dt, "n_steps": n_steps, "N": g.N,
+             "bound": R.bound or 0.0, "row_ptr": R.row_ptr.data_ptr(), "post": R.post.data_ptr(),
+             "events": R.events.data_ptr(), "status": self.status.data_ptr()}
+        for n in g.vars:
+            v[f"a_{n}"] = g._dev[n].data_ptr()
+        for (tg, n), (val, _) in R.scalars.items():
+            v[f"{tg}_{n}"] = val
+        for r, (_, sc) in enumerate(R.consts):
+            for n, (val, _) in sc.items():
+                v[f"c{r}_{n}"] = val
+        v.update(self._monitor_args(g))
+        a = R.cls()
+        for name, _ in R.cls._fields_:
+            if name in v:
+                setattr(a, name, v[name])
+        buf = bytes(a)
+        _lib.check(L.hb_launch(R.fn, 1, R.threads, R.lds_bytes, self.device.stream, buf, len(buf)), "resident step")
+
+    @staticmethod
+    def _monitor_args(g, flush=False):
+        """Parameter fields of a group's monitors."""
+        v = {}
+        if not flush and g.smon:
+            m = g.smon
+            v.update(mon_i=m.mon_i.data_ptr(), mon_step=m.mon_step.data_ptr(), mon_n=m.mon_n.data_ptr(),
+                     mon_count=m.count_dev.data_ptr(), mon_cap=m.cap, mon_start=m.range[0], mon_stop=m.range[1])
+        if not flush and g.rmon is not None:
+            m = g.rmon
+            v.update(rate_cnt=m.buf.data_ptr() if m.buf is not None else 0, rate_row0=getattr(m, "row0", 0),
+                     rate_rows=getattr(m, "rows", 0), rate_start=m.range[0], rate_stop=m.range[1])
+        if g.stmon and (not flush or g.stmon.when == "end"):
+            m = g.stmon
+            v.update(rec_idx=m.rec_idx.data_ptr(), rec_buf=m.rec_buf.data_ptr() if m.rec_buf is not None else 0,
+                     rec_row0=getattr(m, "row0", 0), rec_rows=getattr(m, "rows", 0), n_rec=len(m.sorted_idx))
+        return v
 
     def _alloc_staging(self, g, incoming):
         """Event staging of one target group.
@@ -955,6 +1066,14 @@ class Network:
         s.pairs = int(self.gather_pairs or pc)
         s.units_max = -(-pairs_max // s.pairs)
 
+    def _group_value_type(self, incoming):
+        """The type in which the values of a group's incoming pathways are staged."""
+        vts = {self._value_type(s) for s in incoming}
+        if len(vts & {"int", "long long"}) and len(vts) > 1:
+            raise NotImplementedError("integer and floating-point pathway targets in one group")
+        return "double" if "double" in vts else ("long long" if "long long" in vts else
+                                                 ("int" if "int" in vts else "float"))
+
     def _value_type(self, s):
         from .codegen import Renderer
 
@@ -1007,18 +1126,8 @@ class Network:
         mode = self._reset_mode(g)
         if mode == "deferred":
             g.spiked = zeros(g.N, "bool")
-        smon = [m for m in self.smons if m.source is g]
-        if len(smon) > 1:
-            raise NotImplementedError("more than one SpikeMonitor per group")
-        stmon = [m for m in self.stmons if m.source is g]
-        if len(stmon) > 1:
-            raise NotImplementedError("more than one StateMonitor per group")
-        g.smon = smon[0] if smon else None
-        g.stmon = stmon[0] if stmon else None
-        for st in (g.stmon,) if g.stmon else ():
-            for v in st.variables:
-                if v not in g.vars:
-                    raise KeyError(f"StateMonitor variable {v!r} is not a state variable of {g.name}")
+        self._monitors(g)
+
         def step_kernel(waves):
             return NeuronKernel(g.name, g.N, g.vars, g.float_t, g.su, g.th, g.rs, mode, scalars, fold,
                                 getattr(g, "lds_cap", 0), getattr(g, "val_t", "double"),
@@ -1152,18 +1261,7 @@ class Network:
                      tile_cap=g.tile_cap, stg_stride=g.stg_cap)
         if getattr(g, "spiked", None) is not None:
             v["spiked"] = g.spiked.data_ptr()
-        if not flush and g.smon:
-            m = g.smon
-            v.update(mon_i=m.mon_i.data_ptr(), mon_step=m.mon_step.data_ptr(), mon_n=m.mon_n.data_ptr(),
-                     mon_count=m.count_dev.data_ptr(), mon_cap=m.cap, mon_start=m.range[0], mon_stop=m.range[1])
-        if not flush and g.rmon is not None:
-            m = g.rmon
-            v.update(rate_cnt=m.buf.data_ptr() if m.buf is not None else 0, rate_row0=getattr(m, "row0", 0),
-                     rate_rows=getattr(m, "rows", 0), rate_start=m.range[0], rate_stop=m.range[1])
-        if g.stmon and (not flush or g.stmon.when == "end"):
-            m = g.stmon
-            v.update(rec_idx=m.rec_idx.data_ptr(), rec_buf=m.rec_buf.data_ptr() if m.rec_buf is not None else 0,
-                     rec_row0=getattr(m, "row0", 0), rec_rows=getattr(m, "rows", 0), n_rec=len(m.sorted_idx))
+        v.update(self._monitor_args(g, flush))
         s = cls()
         for name, _ in cls._fields_:
             if name in v:
@@ -1676,14 +1774,17 @@ class Network:
                 m.row0 = self.t_step
                 m.rec_buf = torch.zeros(max(n_steps, 1) * len(m.variables) * len(m.sorted_idx), dtype=torch.float64,
                                         device="cuda")
-                self._set_launch_args(g.launch_index, self._launch_args(g))
+                if self.resident is None:
+                    self._set_launch_args(g.launch_index, self._launch_args(g))
             # population rate monitors: spike counts of this run's steps
             m = getattr(g, "rmon", None)
             if m is not None and not isinstance(g, SpikeGeneratorGroup):
                 m.rows, m.row0 = n_steps, self.t_step
                 m.buf = zeros(max(n_steps, 1), "int")
-                self._set_launch_args(g.launch_index, self._launch_args(g))
+                if self.resident is None:
+                    self._set_launch_args(g.launch_index, self._launch_args(g))
         done = 0
+        timers = []
         if timing:  # HIP events on the plan's stream around each chunk's launches
             _lib.check(L.hb_plan_timing(self._plan, 1, None, None), "hb_plan_timing")
         while done < n_steps:
@@ -1694,8 +1795,18 @@ class Network:
                     chunk = min(chunk, self._ensure_monitor_room(g, m, gs))
             # whole graphs of gs steps, then the rest as one graph of its own length (a run
             # shorter than gs steps is still replayed from a captured graph)
-            k = gs * (chunk // gs) if chunk >= gs else chunk
-            _lib.check(L.hb_plan_run(self._plan, stream, k, gs if k >= gs else k), "hb_plan_run")
+            if self.resident is not None:
+                k = min(chunk, RESIDENT_STEPS)
+                ev = [torch.cuda.Event(enable_timing=True) for _ in range(2)] if timing else []
+                for e in ev[:1]:
+                    e.record()
+                self._run_resident(k)
+                for e in ev[1:]:
+                    e.record()
+                timers += [ev] if ev else []
+            else:
+                k = gs * (chunk // gs) if chunk >= gs else chunk
+                _lib.check(L.hb_plan_run(self._plan, stream, k, gs if k >= gs else k), "hb_plan_run")
             done += k
             self.t_step += k
             st = int(self.status.cpu().item())  # synchronises
@@ -1704,7 +1815,7 @@ class Network:
         if timing:
             ms, nr = ctypes.c_double(), ctypes.c_int64()
             _lib.check(L.hb_plan_timing(self._plan, 0, ctypes.byref(ms), ctypes.byref(nr)), "hb_plan_timing")
-            self.last_run_gpu_ms = ms.value
+            self.last_run_gpu_ms = ms.value + sum(a.elapsed_time(b) for a, b in timers)
         # fold the events delivered by the last step into the state (end of run)
         for g in self.groups:
             if getattr(g, "flush_fn", None) is not None:
@@ -1759,6 +1870,9 @@ class Network:
                 raise NotImplementedError("profile() of a network with a StateMonitor")
             if getattr(g, "rmon", None) is not None:
                 raise NotImplementedError("profile() of a network with a PopulationRateMonitor")
+        if self.resident is not None:
+            self.run(n_steps, timing=True)
+            return [("resident", self.resident.group.name, self.last_run_gpu_ms)]
         ms = (ctypes.c_float * len(self._launches))()
         _lib.check(L.hb_plan_profile(self._plan, self.device.stream, int(n_steps), ms), "hb_plan_profile")
         self.t_step += int(n_steps)
@@ -1817,7 +1931,8 @@ class Network:
             ni[:n] = m.mon_i[:n]
             ns[:n] = m.mon_step[:n]
             m.mon_i, m.mon_step, m.cap = ni, ns, newcap
-            self._set_launch_args(g.launch_index, self._launch_args(g))
+            if self.resident is None:
+                self._set_launch_args(g.launch_index, self._launch_args(g))
             free = m.cap - n
         return max(1, free // max(g.N, 1))
 
