@@ -40,7 +40,7 @@ import numpy as np
 
 from . import _lib
 from .codegen import ParamStruct, source_header, translate_block
-from .kernels import _rename, scalar_values
+from .kernels import LDS_BYTES, _rename, scalar_values
 from .runtime import Device, Model
 
 L = _lib.lib
@@ -84,12 +84,6 @@ def lif_inputs(trials, seed=SEED, c=LIF):
     targets = 0.02 + 0.16 * uniform(seed, S_TARGET, np.arange(c["n_readout"], dtype=np.uint64))
     return dict(rates=rates, pre_in=pre_in, post_in=post_in, pre_rec=pre_rec, post_rec=post_rec,
                 w_in=w_in, w_rec=w_rec, v0=v0, targets=targets, sigma=sigma)
-
-
-def _csr_ptr(pre, n_src):
-    ptr = np.zeros(n_src + 1, np.int64)
-    np.cumsum(np.bincount(pre, minlength=n_src), out=ptr[1:])
-    return ptr.astype(np.uint32)
 
 
 def linear_map(spec, consts, dt, float_t="double"):
@@ -156,26 +150,51 @@ class LIFNetwork:
         self.seed = int(seed)
         self.dt = 1e-4
         self.wt = weight_dtype
+        self._shape()
         self._kernels()
         inp = lif_inputs(self.B, seed, c)
         self.inp = inp
         self.D = Device.get()
         dev = lambda a, dt: torch.from_numpy(np.ascontiguousarray(a).astype(dt)).to("cuda")  # noqa: E731
-        self.r_dt = dev(inp["rates"] * self.dt, np.float64)
-        self.in_ptr = dev(_csr_ptr(inp["pre_in"], self.n_in).view(np.int32), np.int32)
-        self.in_post = dev(inp["post_in"], np.int32)
-        self.rec_ptr = dev(_csr_ptr(inp["pre_rec"], self.N).view(np.int32), np.int32)
-        self.rec_post = dev(inp["post_rec"], np.int32)
+        # U < rate dt for a U of 53 bits over 2^53: the bits below ceil(rate dt 2^53), exactly
+        self.r_dt = dev(np.ceil(np.ldexp(inp["rates"] * self.dt, 53)), np.int64)
         self.n_syn_in, self.n_syn_rec = len(inp["pre_in"]), len(inp["pre_rec"])
+        # places of the synapses in the dense matrix; first synapse and synapses of each row
+        niw, nsw = self._words()
+        width = self.block * self.per_thread
+        self.dense_size = (niw + nsw) * 64 * width
+        self.in_at = dev(inp["pre_in"].astype(np.int64) * width + inp["post_in"], np.int64)
+        self.rec_at = dev((inp["pre_rec"].astype(np.int64) + niw * 64) * width + inp["post_rec"], np.int64)
+        rows = np.zeros(((niw + nsw) * 64, 2), np.int32)
+        for pre, first in ((inp["pre_in"], 0), (inp["pre_rec"], niw * 64)):
+            n = np.bincount(pre, minlength=1) if len(pre) else np.zeros(1, np.int64)
+            rows[first:first + len(n), 0], rows[first:first + len(n), 1] = np.where(n > 0, np.cumsum(n) - n, 0), n
+        self.row_at = dev(rows, np.int32)
+        self.post_in = dev(inp["post_in"] if len(inp["post_in"]) else [0], np.int32)
+        self.post_rec = dev(inp["post_rec"] if len(inp["post_rec"]) else [0], np.int32)
         npw = np.float32 if weight_dtype == "float" else np.float64
         self.w_in0 = dev(inp["w_in"].astype(npw), npw)
         self.w_rec0 = dev(inp["w_rec"].astype(npw), npw)
         self.v0 = dev(inp["v0"], np.float64)
         self.targets = dev(inp["targets"], np.float64)
+        self._inp_fn = self.D.function(self.fwd_source, "lif_inputs")
         self._fwd_fn = self.D.function(self.fwd_source, "lif_forward")
         self._bwd_fn = self.D.function(self.bwd_source, "lif_backward")
 
     # ------------------------------------------------------------------ kernels
+    def _shape(self):
+        """Threads of a trial's workgroup and neurons per thread: eight waves at most, two per
+        SIMD.  1000 neurons, 2000 steps with 4 / 8 / 16 waves, ms: 256 trials forward 2.08 /
+        2.00 / 2.15, backward 4.28 / 4.04 / 4.02; 9 trials, double weights, 600 steps forward
+        0.61 / 0.53 / 0.50, backward 0.99 / 0.93 / 0.84."""
+        self.block = 64 * min(8, -(-self.N // 64))
+        self.per_thread = -(-self.N // self.block)
+        # steps of a block of the backward pass: what its LDS holds (16 bytes per neuron and step,
+        # 2 per possible event), a raster word per thread, at most 8
+        words = sum(self._words())
+        step = 16 * self.block * self.per_thread + 2 * 64 * words
+        self.sub = max(1, min(8, self.block // words, (LDS_BYTES - 4096) // step))
+
     def _kernels(self):
         """Loads the model's statements and generates both kernel sources."""
         self.model = Model.load("lif")
@@ -194,6 +213,7 @@ class LIFNetwork:
         self = cls.__new__(cls)
         self.c = dict(LIF if config is None else config)
         self.N, self.dt, self.wt = self.c["N"], 1e-4, weight_dtype
+        self._shape()
         self._kernels()
         return self.fwd_source, self.bwd_source
 
@@ -214,33 +234,28 @@ class LIFNetwork:
     def _struct(self, name, backward):
         WT = self.wt
         ps = ParamStruct(name)
-        ps.val("k0", "long long")
-        ps.val("n_steps", "int")
+        ps.val("n_seg", "int")    # checkpoint intervals of a run
+        ps.val("n_steps", "int")  # steps of an interval
         ps.val("T_total", "int")
         ps.val("seed", "unsigned long long")
         ps.val("n_in", "int")
         ps.val("N", "int")
         ps.val("R", "int")
         ps.val("trial0", "int")
+        ps.val("n_trials", "int")
         ps.val("theta", "double")
         ps.val("dt", "double")
         for n in self.su_scalars:
             ps.val(f"su_{n}", "double")
-        ps.ptr("r_dt", "double", const=True)
-        ps.ptr("in_ptr", "unsigned int", const=True)
-        ps.ptr("in_post", "int", const=True)
-        ps.ptr("rec_ptr", "unsigned int", const=True)
-        ps.ptr("rec_post", "int", const=True)
-        ps.ptr("hist_v", "double")
-        ps.ptr("hist_I", "double")
-        ps.ptr("fs_step", "int")
+        ps.ptr("dense", WT, const=True)  # weights by (source, target), 0 where there is no synapse
+        ps.ptr("raster", "unsigned long long", const=backward)  # [trial][step][words]
+        ps.ptr("ckpt_v", "double", const=backward)
+        ps.ptr("ckpt_I", "double", const=backward)
+        ps.ptr("fs_step", "int", const=backward)
         if not backward:
-            ps.ptr("in_w", WT, const=True)
-            ps.ptr("rec_w", WT, const=True)
+            ps.ptr("r_dt", "unsigned long long", const=True)
             ps.ptr("v", "double")
             ps.ptr("I", "double")
-            ps.ptr("ckpt_v", "double")
-            ps.ptr("ckpt_I", "double")
             ps.ptr("fs_vprev", "double")
             ps.ptr("fs_u", "double")
             ps.ptr("l2", "double")
@@ -255,230 +270,491 @@ class LIFNetwork:
             ps.val("coef_fs", "double")
             ps.val("coef_v", "double")
             ps.ptr("targets", "double", const=True)
-            ps.ptr("lam_v", "double")
-            ps.ptr("lam_I", "double")
+            ps.ptr("row_at", "int", const=True)  # first synapse and synapses of each row
+            ps.ptr("post_in", "int", const=True)
+            ps.ptr("post_rec", "int", const=True)
+            ps.ptr("sub_v", "double")
+            ps.ptr("sub_I", "double")
+            ps.val("n_syn_in", "long long")
+            ps.val("n_syn_rec", "long long")
             ps.ptr("g_in", "double")
             ps.ptr("g_rec", "double")
             ps.ptr("gacc", "double")
         return ps
 
-    def _common(self, ps):
-        NW = BLOCK // 64
-        k = [source_header(BLOCK), _rng_header(), ps.c_decl()]
-        return k, self.su_code, NW
+    def _words(self):
+        """64-bit words of a step's spikes: the inputs', then the neurons'."""
+        return max(1, -(-self.c["n_in"] // 64)), -(-self.N // 64)
 
-    def _compaction(self, cond, arr, count):
-        """Ordered compaction of `cond` over the threads into LDS `arr`, total in `count`."""
-        NW = BLOCK // 64
+    def _head(self, ps, name):
+        """What both kernels begin with.
+
+        Thread x of the trial's workgroup has the neurons q*T + x, q < Q (few waves, so
+        that what every wave does alike is done few times).  Rows of the dense matrices
+        are numbered by the raster's bits (inputs, then neurons, in schedule order), with
+        a column per neuron: every thread reads its own columns of each spiking source's
+        row and adds them up itself, in (pathway, source) order, without a barrier
+        between the rows."""
+        NIW, NSW = self._words()
+        T, Q = self.block, self.per_thread
+        return [source_header(T), _rng_header(), ps.c_decl(), f"""
+#define HB_NIW {NIW}          // words of a step's input spikes
+#define HB_NW {NIW + NSW}           // words of a step
+#define HB_Q {Q}             // neurons per thread
+#define HB_ROWS 4            // rows in flight
+// a step's rows, loaded at once: {Q} columns of each
+template <typename V> struct hb_rows {{
+    V x[HB_ROWS][HB_Q];
+    __device__ __forceinline__ void load(const int u, const int row, const V* col) {{
+        #pragma unroll
+        for (int q = 0; q < HB_Q; q++) x[u][q] = col[(size_t)row * {T * Q} + q * {T}];
+    }}
+    __device__ __forceinline__ void add(double (&I)[HB_Q], const int m) const {{
+        #pragma unroll
+        for (int u = 0; u < HB_ROWS; u++)
+            if (u < m)
+                #pragma unroll
+                for (int q = 0; q < HB_Q; q++) I[q] += (double)x[u][q];
+    }}
+}};
+""", f'extern "C" __global__ void __launch_bounds__({T}) {name}(const {ps.name} p) {{',
+            "    const int b = blockIdx.x;",
+            "    const int lane = threadIdx.x & 63;",
+            "    const int wid = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);",
+            "    const int N = p.N;",
+            "    const double dt = p.dt;",
+            "    const size_t bo = (size_t)b * N;",
+            f"    const {self.wt}* const col = p.dense + threadIdx.x;",
+            f"#define HB_EACH_Q _Pragma(\"unroll\") for (int q = 0; q < HB_Q; q++)",
+            f"#define HB_J (q * {T} + (int)threadIdx.x)  // neuron q of the thread",
+            "    // stateupdate of neuron j at step k (Brian's statements)",
+            "    auto hb_update = [&](const int j, const int k, double& v, double& I) __attribute__((always_inline)) {",
+            "        const double t = (double)k * dt;",
+            "        const int i = j, _idx = j;",
+            "        (void)t; (void)i; (void)_idx;",
+            ] + ["        " + x for x in self.su_code] + ["    };"]
+
+    def _sum_lines(self, what, into, n):
+        """Lines that add up a value per neuron: wave shuffles over 64 neurons, then the groups
+        of 64 in order (n values side by side)."""
+        NSW = self._words()[1]
+        W = self.block // 64
         return [
-            "        {",
-            f"            const unsigned long long bal_ = __ballot({cond});",
-            "            if (lane == 0) s_w[wid] = __popcll(bal_);",
-            "            __syncthreads();",
-            "            if (threadIdx.x == 0) {",
-            "                int acc_ = 0;",
-            f"                for (int w_ = 0; w_ < {NW}; w_++) {{ const int c_ = s_w[w_]; s_w[w_] = acc_; acc_ += c_; }}",
-            f"                s_w[{NW}] = acc_;",
+            "            HB_EACH_Q {",
+            f"                double x[{n}] = {{{', '.join(f'HB_J < N ? {w} : 0.0' for w in what)}}};",
+            "                #pragma unroll",
+            f"                for (int c = 0; c < {n}; c++) {{",
+            "                    for (int o = 32; o > 0; o >>= 1) x[c] += __shfl_down(x[c], o, 64);",
+            f"                    if (lane == 0 && q * {W} + wid < {NSW}) s_red[q * {W} + wid][c] = x[c];",
+            "                }",
             "            }",
             "            __syncthreads();",
-            f"            if ({cond}) {arr}[s_w[wid] + __popcll(bal_ & ((1ull << lane) - 1ull))] = (int)threadIdx.x;",
-            f"            {count} = s_w[{NW}];",
+            f"            if ((int)threadIdx.x < {n}) {{",
+            "                double acc = 0.0;",
+            f"                for (int w = 0; w < {NSW}; w++) acc += s_red[w][threadIdx.x];",
+            f"                {into} += acc;",
+            "            }",
             "            __syncthreads();",
-            "        }",
         ]
 
     def _fwd_source(self):
+        """Forward pass of a trial per workgroup, all steps in one launch.
+
+        A step is one barrier: every wave puts its neurons' spikes as words into LDS (two
+        buffers in turn), and behind the barrier reads all words and adds its columns of
+        the spiking sources' rows.  The inputs' spikes are drawn by a kernel of its own
+        before (lif_inputs), which the whole chip shares; both end up in the raster, from
+        which the backward pass knows every spike.  Bound by the chain of a step: update,
+        barrier, words, one row fetch (L2).  256 trials of 1000 neurons (fp32 weights):
+        2.05 us per step with ordered compactions and a barrier per row (ten barriers a
+        step), 1.00 now and 0.05 for the draws."""
         ps = self._struct("hba_fwd", False)
         self.fwd_struct = ps
-        k, su, NW = self._common(ps)
-        T = BLOCK
+        NIW, NSW = self._words()
+        T, Q = self.block, self.per_thread
+        W = T // 64
+        k = self._head(ps, "lif_forward")
         k += [
-            f'extern "C" __global__ void __launch_bounds__({T}) lif_forward(const hba_fwd p) {{',
-            "    const int b = blockIdx.x;",
-            "    const int j = threadIdx.x;",
-            "    const int lane = j & 63, wid = j >> 6;",
-            "    const int N = p.N;",
-            "    const bool act = j < N;",
-            "    const double dt = p.dt;",
-            f"    __shared__ double s_I[{T}];",
-            f"    __shared__ int s_spk[{T}];",
-            f"    __shared__ int s_inp[{T}];",
-            f"    __shared__ int s_w[{NW + 1}];",
-            f"    __shared__ double s_red[{NW}];",
-            "    const size_t bo = (size_t)b * N;",
-            "    double v = act ? p.v[bo + j] : 0.0;",
-            "    double I = act ? p.I[bo + j] : 0.0;",
-            "    if (p.ckpt_v && act) {",
-            "        const size_t co = ((size_t)(p.k0 / p.n_steps) * gridDim.x + b) * N + j;",
-            "        p.ckpt_v[co] = v; p.ckpt_I[co] = I;",
+            f"    __shared__ unsigned long long s_ras[64][HB_NW];  // words of the last steps, and the inputs' ahead",
+            f"    __shared__ double s_red[{NSW}][1];",
+            "    double v[HB_Q], I[HB_Q], l2[HB_Q];",
+            "    bool fs_open[HB_Q];",
+            "    HB_EACH_Q {",
+            "        v[q] = HB_J < N ? p.v[bo + HB_J] : 0.0;",
+            "        I[q] = HB_J < N ? p.I[bo + HB_J] : 0.0;",
+            "        fs_open[q] = HB_J < p.R && p.fs_step[b * p.R + (HB_J < p.R ? HB_J : 0)] < 0;",
+            "        l2[q] = 0.0;",
+            "        // waited for here: a wait inside the loop would be for the checkpoints' stores as well",
+            "        asm volatile(\"\" : \"+v\"(v[q]), \"+v\"(I[q]));",
             "    }",
-            "    const unsigned long long rng_base = ((unsigned long long)(p.trial0 + b) * p.n_in + j) * (unsigned long long)p.T_total;",
-            "    double l2 = 0.0;",
-            "    for (int s = 0; s < p.n_steps; s++) {",
-            "        const long long k = p.k0 + s;",
-            "        const double t = (double)k * dt;",
-            "        (void)t;",
-            "        if (p.hist_v && act) {",
-            "            const size_t ho = ((size_t)b * p.n_steps + s) * N + j;",
-            "            p.hist_v[ho] = v; p.hist_I[ho] = I;",
+            "    double l2_all = p.l2[b];",
+            "    long long n_spk = p.spk_i ? p.spk_n[b] : 0;",
+            "    const int T = p.n_seg * p.n_steps;",
+            "    unsigned long long* const ras = p.raster + (size_t)b * T * HB_NW;",
+            "    // the spikes of n steps from k to the raster",
+            "    auto hb_flush = [&](const int k, const int n) {",
+            f"        for (int x = threadIdx.x; x < n * {NSW}; x += {T})",
+            f"            ras[(size_t)(k + x / {NSW}) * HB_NW + HB_NIW + x % {NSW}] = s_ras[(k + x / {NSW}) & 63][HB_NIW + x % {NSW}];",
+            "    };",
+            "    // the inputs' words of the next 32 steps, read 32 steps ahead (every memory access in",
+            "    // flight is waited for with a step's rows)",
+            f"    constexpr int AHEAD = (32 * HB_NIW + {T - 1}) / {T};",
+            "    unsigned long long ahead[AHEAD];",
+            "    auto hb_ahead = [&](const int k) {",
+            "        #pragma unroll",
+            "        for (int a = 0; a < AHEAD; a++) {",
+            f"            const int x = a * {T} + (int)threadIdx.x, s = k + x / HB_NIW;",
+            "            ahead[a] = ras[s < T && x < 32 * HB_NIW ? (size_t)s * HB_NW + x % HB_NIW : 0];",
             "        }",
-            "        const double v_prev = v;",
-            "        const int i = j, _idx = j;",
-            "        (void)i; (void)_idx;",
-            "        if (act) { // stateupdate (Brian's statements)",
-        ]
-        k += ["            " + x for x in su]
-        k += [
+            "    };",
+            "    hb_ahead(0);",
+            "    for (int k = 0, c = 0, sg = 0; k < T; k++) {",
+            "        if ((k & 31) == 0) {",
+            "            #pragma unroll",
+            "            for (int a = 0; a < AHEAD; a++) {",
+            f"                const int x = a * {T} + (int)threadIdx.x;",
+            "                if (x < 32 * HB_NIW) s_ras[(k + x / HB_NIW) & 63][x % HB_NIW] = ahead[a];",
+            "            }",
+            "            hb_ahead(k + 32);",
+            "            if (k > 0) hb_flush(k - 32, 32);",
             "        }",
-            "        const bool cond = act && (v > p.theta);",
-            "        const bool cin = j < p.n_in && hb_uniform01(hb_rand64(p.seed, "
-            f"{S_POISSON}ull, rng_base + (unsigned long long)k)) < p.r_dt[j < p.n_in ? j : 0];",
-            "        int nspk, ninp;",
-        ]
-        k += self._compaction("cond", "s_spk", "nspk")
-        k += self._compaction("cin", "s_inp", "ninp")
-        k += [
-            "        if (cond && j < p.R && p.fs_step && p.fs_step[b * p.R + j] < 0) {",
-            "            p.fs_step[b * p.R + j] = (int)k;",
-            "            if (p.fs_vprev) { p.fs_vprev[b * p.R + j] = v_prev; p.fs_u[b * p.R + j] = v; }",
+            "        if (c == 0)",
+            "            HB_EACH_Q if (HB_J < N) {",
+            "                const size_t co = ((size_t)sg * gridDim.x + b) * N + HB_J;",
+            "                p.ckpt_v[co] = v[q]; p.ckpt_I[co] = I[q];",
+            "            }",
+            "        bool cond[HB_Q], fs_any = false;",
+            "        double v_prev[HB_Q];",
+            "        unsigned long long mine[HB_Q], word = 0ull;",
+            "        HB_EACH_Q {",
+            "            v_prev[q] = v[q];",
+            "            hb_update(HB_J, k, v[q], I[q]);",
+            "            cond[q] = HB_J < N && v[q] > p.theta;",
+            "            mine[q] = __builtin_amdgcn_ballot_w64(cond[q]);",
+            "            fs_any = fs_any || (cond[q] && fs_open[q]);",
+            "            word = lane == q ? mine[q] : word;",
             "        }",
-            "        // propagation, in schedule order: syn_in_pre, then syn_rec_pre; each a left fold",
-            "        // in (source, synapse) order",
-            "        s_I[j] = I;",
+            f"        if (lane < HB_Q && lane * {W} + wid < {NSW}) s_ras[k & 63][HB_NIW + lane * {W} + wid] = word;",
+            "        if (__builtin_amdgcn_ballot_w64(fs_any) != 0ull)",
+            "            HB_EACH_Q if (cond[q] && fs_open[q]) { // first spike of a readout",
+            "                fs_open[q] = false;",
+            "                p.fs_step[b * p.R + HB_J] = k; p.fs_vprev[b * p.R + HB_J] = v_prev[q]; p.fs_u[b * p.R + HB_J] = v[q];",
+            "            }",
             "        __syncthreads();",
-            "        for (int q = 0; q < ninp; q++) {",
-            "            const int src = s_inp[q];",
-            "            const unsigned int a = p.in_ptr[src], e_ = p.in_ptr[src + 1];",
-            f"            for (unsigned int e = a + j; e < e_; e += {T}) s_I[p.in_post[e]] += (double)p.in_w[e];",
-            "            __syncthreads();",
+            "        const unsigned long long rd = s_ras[k & 63][lane < HB_NW ? lane : 0];",
+            "        const unsigned long long rw = lane < HB_NW ? rd : 0ull;",
+            "        // propagation, in schedule order: syn_in_pre, then syn_rec_pre; each a left fold in",
+            "        // (source, synapse) order.  Everything about the sources is the same for the wave",
+            "        unsigned long long nz = __builtin_amdgcn_ballot_w64(rw != 0ull);",
+            "        if (nz != 0ull) {",
+            f"            hb_rows<{self.wt}> r;",
+            "            const int one = (lane << 6) + __builtin_ctzll(rw | 1ull << 63);  // the word's first source",
+            "            const int n_nz = __popcll(nz);",
+            "            if (n_nz <= HB_ROWS && __builtin_amdgcn_ballot_w64((rw & (rw - 1ull)) != 0ull && rw != 0ull) == 0ull) {",
+            "                // few words of one source each (most steps); a missing one repeats the last:",
+            "                // loads without a branch stay in flight",
+            "                int l = 0;",
+            "                #pragma unroll",
+            "                for (int u = 0; u < HB_ROWS; u++) {",
+            "                    l = nz != 0ull ? __builtin_ctzll(nz) : l;",
+            "                    nz &= nz - 1ull;",
+            "                    r.load(u, __builtin_amdgcn_readlane(one, l), col);",
+            "                }",
+            "                r.add(I, n_nz);",
+            "            } else {  // word by word, bit by bit",
+            "                for (; nz; nz &= nz - 1ull) {",
+            "                    const int l = __builtin_ctzll(nz);",
+            "                    unsigned long long bits = ((unsigned long long)(unsigned int)",
+            "                        __builtin_amdgcn_readlane((int)(rw >> 32), l) << 32) | (unsigned int)__builtin_amdgcn_readlane((int)rw, l);",
+            "                    while (bits) {",
+            "                        int m = 0, row = 0;",
+            "                        #pragma unroll",
+            "                        for (int u = 0; u < HB_ROWS; u++) {",
+            "                            m += bits != 0ull ? 1 : 0;",
+            "                            row = bits != 0ull ? (l << 6) + __builtin_ctzll(bits) : row;",
+            "                            bits &= bits - 1ull;",
+            "                            r.load(u, row, col);",
+            "                        }",
+            "                        r.add(I, m);",
+            "                    }",
+            "                }",
+            "            }",
             "        }",
-            "        for (int q = 0; q < nspk; q++) {",
-            "            const int src = s_spk[q];",
-            "            const unsigned int a = p.rec_ptr[src], e_ = p.rec_ptr[src + 1];",
-            f"            for (unsigned int e = a + j; e < e_; e += {T}) s_I[p.rec_post[e]] += (double)p.rec_w[e];",
-            "            __syncthreads();",
+            "        HB_EACH_Q {",
+            "            if (cond[q]) v[q] = 0.0; // reset",
+            "            l2[q] += v[q] * v[q];",
             "        }",
-            "        I = s_I[j];",
-            "        if (cond) v = 0.0; // reset",
-            "        l2 += v * v;",
-            "        if (p.spk_i && nspk) {",
-            "            const long long base = p.spk_n[b];",
-            f"            for (int q = j; q < nspk; q += {T})",
-            "                if (base + q < p.spk_cap) { p.spk_i[(size_t)b * p.spk_cap + base + q] = s_spk[q]; "
-            "p.spk_step[(size_t)b * p.spk_cap + base + q] = (int)k; }",
-            "            __syncthreads();",
-            "            if (j == 0) p.spk_n[b] = base + nspk;",
+            "        if (p.spk_i) { // the step's spikes in ascending order",
+            "            const int n_ = lane >= HB_NIW && lane < HB_NW ? __popcll(rw) : 0;",
+            "            const int x_ = hb_wave_incl_scan(n_);",
+            f"            HB_EACH_Q if (q * {W} + wid < {NSW}) {{",
+            f"                const long long at = n_spk + __builtin_amdgcn_readlane(x_ - n_, HB_NIW + q * {W} + wid) "
+            "+ __popcll(mine[q] & ((1ull << lane) - 1ull));",
+            "                if (cond[q] && at < p.spk_cap) { p.spk_i[(size_t)b * p.spk_cap + at] = HB_J; "
+            "p.spk_step[(size_t)b * p.spk_cap + at] = k; }",
+            "            }",
+            "            n_spk += __builtin_amdgcn_readlane(x_, 63);",
             "        }",
-            "        __syncthreads();",
+            "        if (++c == p.n_steps) { // an interval's sum",
+            "            c = 0; sg++;",
+        ]
+        k += self._sum_lines(["l2[q]"], "l2_all", 1)
+        k += [
+            "            HB_EACH_Q l2[q] = 0.0;",
+            "        }",
             "    }",
-            "    if (act) { p.v[bo + j] = v; p.I[bo + j] = I; }",
-            "    if (p.l2) {",
-            "        // fixed-order reduction: wave shuffles, then the waves in order",
-            "        double x = act ? l2 : 0.0;",
-            "        for (int o = 32; o > 0; o >>= 1) x += __shfl_down(x, o, 64);",
-            "        if (lane == 0) s_red[wid] = x;",
-            "        __syncthreads();",
-            f"        if (j == 0) {{ double acc = 0.0; for (int w_ = 0; w_ < {NW}; w_++) acc += s_red[w_]; p.l2[b] += acc; }}",
+            "    hb_flush((T - 1) & ~31, T - ((T - 1) & ~31));  // (behind the last interval's barriers)",
+            "    HB_EACH_Q if (HB_J < N) { p.v[bo + HB_J] = v[q]; p.I[bo + HB_J] = I[q]; }",
+            "    if (threadIdx.x == 0) { p.l2[b] = l2_all; if (p.spk_i) p.spk_n[b] = n_spk; }",
+            "}",
+            "// input spikes of every trial and step: input i of trial b spikes at step k iff",
+            "// U(seed, stream, ((trial0 + b) n_in + i) T_total + k) < rate dt, compared as integers",
+            "// (U is 53 bits over 2^53; r_dt: the bound ceil(rate dt 2^53)).  A wave draws a word of",
+            "// DRAWS steps one after the other",
+            "#define DRAWS 16",
+            f'extern "C" __global__ void __launch_bounds__({T}) lif_inputs(const {ps.name} p) {{',
+            "    const int lane = threadIdx.x & 63, T = p.n_seg * p.n_steps;",
+            f"    const long long u = (long long)blockIdx.x * {W} + (threadIdx.x >> 6);",
+            "    const int nk = (T + DRAWS - 1) / DRAWS;",
+            "    const int b = (int)(u / (nk * HB_NIW)), w = (int)(u % HB_NIW), k0 = (int)(u / HB_NIW % nk) * DRAWS;",
+            "    if (b >= p.n_trials) return;",
+            "    const int i = w * 64 + lane;",
+            "    const unsigned long long bound = i < p.n_in ? p.r_dt[i] : 0ull;",
+            f"    const unsigned long long key = hb_mix64(p.seed ^ hb_mix64({S_POISSON}ull + 0x9e3779b97f4a7c15ULL));",
+            "    unsigned long long z = key + (((unsigned long long)(p.trial0 + b) * p.n_in + i) * (unsigned long long)p.T_total"
+            " + (unsigned long long)k0 + 1ull) * 0x9e3779b97f4a7c15ULL;",
+            "    unsigned long long* const ras = p.raster + ((size_t)b * T + k0) * HB_NW + w;",
+            "    for (int s = 0; s < DRAWS && k0 + s < T; s++, z += 0x9e3779b97f4a7c15ULL) {",
+            "        const unsigned long long m = __builtin_amdgcn_ballot_w64((hb_mix64(z) >> 11) < bound);",
+            "        if (lane == 0) ras[(size_t)s * HB_NW] = m;",
             "    }",
             "}",
         ]
         return "\n".join(k) + "\n"
 
     def _bwd_source(self):
+        """Backward pass of a trial per workgroup, all intervals in one launch.
+
+        With the raster the recomputation of an interval is each thread's own: no spike has
+        to be exchanged, and the rows of a step are fetched while the step before it is
+        computed.  The steps are taken in blocks of SUB: a block's raster words become a
+        list of its events in LDS (step and source, in order; a word per thread).  From the
+        interval's checkpoint the states at every block's start are kept (sub_v, sub_I);
+        from the last block to the first, its steps' states are recomputed into LDS (a
+        column per neuron) and walked in reverse.  The adjoint of I is kept in the
+        state's place, and the block's weight gradients follow: a wave adds it to the
+        synapses of its sources that spiked, in descending step order.
+        Bound by the latency of the rows and of the gradients.  256 trials: 5.05 us per
+        step with the recomputation through a history of 16 bytes per neuron and step in
+        memory, 2.02 now."""
         ps = self._struct("hba_bwd", True)
         self.bwd_struct = ps
-        k, su, NW = self._common(ps)
-        T = BLOCK
+        NIW, NSW = self._words()
+        NW = NIW + NSW
+        T, Q, SB = self.block, self.per_thread, self.sub
+        W = T // 64
+        # events of a batch of weight gradients and pieces of 64 synapses of each (longer rows in
+        # a loop behind it)
+        GP = max(1, min(4, -(-int(1.1 * self.c["p"] * self.N) // 64)))
+        GB = max(2, 12 // GP)
+        k = self._head(ps, "lif_backward")
         k += [
-            f'extern "C" __global__ void __launch_bounds__({T}) lif_backward(const hba_bwd p) {{',
-            "    const int b = blockIdx.x;",
-            "    const int j = threadIdx.x;",
-            "    const int lane = j & 63, wid = j >> 6;",
-            "    const int N = p.N;",
-            "    const bool act = j < N;",
-            "    const double dt = p.dt;",
-            f"    __shared__ double s_lam[{T}];",
-            f"    __shared__ int s_spk[{T}];",
-            f"    __shared__ int s_inp[{T}];",
-            f"    __shared__ int s_w[{NW + 1}];",
-            f"    __shared__ double s_red[{NW}][4];",
-            "    const size_t bo = (size_t)b * N;",
-            "    double lam_v = act ? p.lam_v[bo + j] : 0.0;",
-            "    double lam_I = act ? p.lam_I[bo + j] : 0.0;",
-            "    double gA = 0.0, gB = 0.0, gC = 0.0, gbeta = 0.0;",
-            "    const int fs_k = (j < p.R) ? p.fs_step[b * p.R + j] : -1;",
-            "    const unsigned long long rng_base = ((unsigned long long)(p.trial0 + b) * p.n_in + j) * (unsigned long long)p.T_total;",
-            "    double* g_in = p.g_in + (size_t)b * p.in_ptr[p.n_in];",
-            "    double* g_rec = p.g_rec + (size_t)b * p.rec_ptr[N];",
-            "    for (int s = p.n_steps - 1; s >= 0; s--) {",
-            "        const long long k = p.k0 + s;",
-            "        const double t = (double)k * dt;",
-            "        (void)t;",
-            "        const size_t ho = ((size_t)b * p.n_steps + s) * N + j;",
-            "        const double v_prev = act ? p.hist_v[ho] : 0.0;",
-            "        const double I_prev = act ? p.hist_I[ho] : 0.0;",
-            "        double v = v_prev, I = I_prev;",
-            "        const int i = j, _idx = j;",
-            "        (void)i; (void)_idx;",
-            "        if (act) { // the step's update again (identical statements and values)",
-        ]
-        k += ["            " + x for x in su]
-        k += [
-            "        }",
-            "        const double u = v;",
-            "        const bool cond = act && (u > p.theta);",
-            "        const bool cin = j < p.n_in && hb_uniform01(hb_rand64(p.seed, "
-            f"{S_POISSON}ull, rng_base + (unsigned long long)k)) < p.r_dt[j < p.n_in ? j : 0];",
-            "        const double v_post = cond ? 0.0 : u;",
-            "        double dLdu = cond ? 0.0 : (lam_v + p.coef_v * 2.0 * v_post);",
-            "        double extra = 0.0;",
-            "        if (fs_k == (int)k) { // first spike of a readout: interpolated crossing time",
-            "            const double d = u - v_prev;",
-            "            const double tc = dt * ((double)k + (p.theta - v_prev) / d);",
-            "            const double dLdt = p.coef_fs * 2.0 * (tc - p.targets[j]);",
-            "            dLdu += dLdt * (-dt * (p.theta - v_prev) / (d * d));",
-            "            extra = dLdt * (dt * (p.theta - u) / (d * d));",
-            "        }",
-            "        int nspk, ninp;",
-        ]
-        k += self._compaction("cond", "s_spk", "nspk")
-        k += self._compaction("cin", "s_inp", "ninp")
-        k += [
-            "        // event-based weight gradients: lam of I after this step at every target of a source",
-            "        // that spiked in it (rows of different sources never share a synapse)",
-            "        s_lam[j] = lam_I;",
+            f"    __shared__ double s_hv[{SB}][{T * Q}], s_hi[{SB}][{T * Q}];",
+            f"    __shared__ unsigned short s_ev[{SB * NW * 64}];  // events of a block: step << 11 | row",
+            f"    __shared__ int s_of[{SB + 1}], s_sh[{max(1, T // 64)}];",
+            f"    __shared__ double s_red[{NSW}][4];",
+            "    double lam_v[HB_Q], lam_I[HB_Q], gA[HB_Q], gB[HB_Q], gC[HB_Q], gbeta[HB_Q], v[HB_Q], I[HB_Q];",
+            "    int fs_k[HB_Q];",
+            "    HB_EACH_Q {",
+            "        lam_v[q] = lam_I[q] = gA[q] = gB[q] = gC[q] = gbeta[q] = 0.0;",
+            "        fs_k[q] = HB_J < p.R ? p.fs_step[b * p.R + (HB_J < p.R ? HB_J : 0)] : -1;",
+            "    }",
+            "    double g_all = threadIdx.x < 4 ? p.gacc[b * 4 + (threadIdx.x & 3)] : 0.0;",
+            "    const int C = p.n_steps, T = p.n_seg * C;",
+            f"    const int n_sub = (C + {SB - 1}) / {SB};",
+            "    const unsigned long long* const ras = p.raster + (size_t)b * T * HB_NW;",
+            "    double* const g_in = p.g_in + (size_t)b * p.n_syn_in;",
+            "    double* const g_rec = p.g_rec + (size_t)b * p.n_syn_rec;",
+            f"    auto hb_len = [&](const int sb) {{ return C - sb * {SB} < {SB} ? C - sb * {SB} : {SB}; }};",
+            "    // this thread's word of block sb of interval sg",
+            "    const int ws = (int)threadIdx.x / HB_NW;  // its step",
+            "    auto hb_word = [&](const int sg, const int sb) {",
+            "        const bool in = sg >= 0 && ws < hb_len(sb);",
+            f"        const unsigned long long w = ras[in ? (size_t)(sg * C + sb * {SB}) * HB_NW + threadIdx.x : 0];",
+            "        return in ? w : 0ull;",
+            "    };",
+            "    // a block's list of events from the threads' words; returns their number",
+            "    auto hb_list = [&](unsigned long long w) {",
+            "        int n;",
+            "        int x = hb_block_exscan(__popcll(w), s_sh, &n);",
+            f"        if (threadIdx.x % HB_NW == 0 && ws < {SB}) s_of[ws] = x;",
+            f"        if (threadIdx.x == 0) s_of[{SB}] = n;",
+            "        for (; w; w &= w - 1ull) s_ev[x++] = (unsigned short)(ws << 11 | ((int)threadIdx.x % HB_NW * 64 + __builtin_ctzll(w)));",
             "        __syncthreads();",
-            "        for (int q = 0; q < ninp; q++) {",
-            "            const int src = s_inp[q];",
-            "            const unsigned int a = p.in_ptr[src], e_ = p.in_ptr[src + 1];",
-            f"            for (unsigned int e = a + j; e < e_; e += {T}) g_in[e] += s_lam[p.in_post[e]];",
+            "        return n;",
+            "    };",
+            "    // the first n steps (from step k0) of the block in the list of n_ev events; before step",
+            "    // s, keep(s).  Lane l holds event l and the events before step l; the rows of a step are",
+            "    // loaded two steps ahead",
+            "    auto hb_steps = [&](const int k0, const int n, const int n_ev, auto keep) __attribute__((always_inline)) {",
+            "        const int ev = (int)s_ev[lane < n_ev ? lane : 0];",
+            f"        const int of = s_of[lane < {SB} ? lane : {SB}];",
+            "        auto event = [&](const int x) {",
+            "            return (x < 64 ? __builtin_amdgcn_readlane(ev, x) : __builtin_amdgcn_readfirstlane((int)s_ev[x])) & 2047;",
+            "        };",
+            f"        hb_rows<{self.wt}> r[{SB + 2}];",
+            f"        int x[{SB + 2}], m[{SB + 2}];",
+            "        auto first = [&](const int s) {  // a step's events and its first rows (a missing one repeats",
+            "            x[s] = __builtin_amdgcn_readlane(of, s);  // the last, or row 0: no branch around a load)",
+            "            m[s] = __builtin_amdgcn_readlane(of, s + 1) - x[s];",
+            "            #pragma unroll",
+            "            for (int u = 0; u < HB_ROWS; u++) r[s].load(u, m[s] > 0 ? event(x[s] + (u < m[s] ? u : m[s] - 1)) : 0, col);",
+            "        };",
+            "        first(0);",
+            f"        if ({SB} > 1) first({1 if SB > 1 else 0});",
+            "        #pragma unroll",
+            f"        for (int s = 0; s < {SB}; s++)",
+            "            if (s < n) {",
+            "                const int k = k0 + s;",
+            "                keep(s);",
+            f"                if (s + 2 < {SB}) first(s + 2);",
+            "                bool cond[HB_Q];",
+            "                HB_EACH_Q { hb_update(HB_J, k, v[q], I[q]); cond[q] = v[q] > p.theta; }",
+            "                r[s].add(I, m[s]);",
+            "                for (int u = HB_ROWS; u < m[s]; u++) {",
+            f"                    hb_rows<{self.wt}> g;",
+            "                    g.load(0, event(x[s] + u), col);",
+            "                    g.add(I, 1);",
+            "                }",
+            "                HB_EACH_Q if (cond[q]) v[q] = 0.0;",
+            "            }",
+            "    };",
+            "    // weight gradients.  A wave has the rows whose number is its own modulo the waves (so that",
+            "    // a synapse is always added to by the same lane); its events of a block, the latest first,",
+            f"    // in batches of {GB}: their synapses' gradients and targets are loaded (hb_take) before the",
+            "    // adjoint of the block is known, and added to and stored behind it (hb_give)",
+            f"    double gy[{GB}][{GP}];",
+            f"    int gt[{GB}][{GP}], ge[{GB}], gn[{GB}], gs[{GB}], g_m = 0, g_c = 0;",
+            "    unsigned long long g_left = 0ull;  // the wave's events of the 64 from g_c on still to come",
+            "    auto hb_mine = [&](const int n_ev) {",
+            "        const int ev = (int)s_ev[g_c + lane < n_ev ? g_c + lane : 0];",
+            f"        return __builtin_amdgcn_ballot_w64(g_c + lane < n_ev && (ev & 2047) % {W} == wid);",
+            "    };",
+            "    auto hb_take = [&](const int n_ev) __attribute__((always_inline)) {",
+            "        g_m = 0;",
+            "        while (g_left == 0ull && g_c > 0) { g_c -= 64; g_left = hb_mine(n_ev); }",
+            f"        int row[{GB}];",
+            "        bool again = false;  // a row's second event waits for the next batch",
+            "        #pragma unroll",
+            f"        for (int u = 0; u < {GB}; u++) {{",
+            "            const bool more = g_left != 0ull && !again;",
+            "            const int x = more ? 63 - __builtin_clzll(g_left) : 0;",
+            "            const int ev = __builtin_amdgcn_readfirstlane((int)s_ev[g_c + x]);",
+            "            row[u] = ev & 2047;",
+            "            #pragma unroll",
+            "            for (int w = 0; w < u; w++) again = again || (more && row[w] == row[u]);",
+            "            const bool ok = more && !again;",
+            "            g_left = ok ? g_left & ~(1ull << x) : g_left;",
+            "            g_m += ok ? 1 : 0;",
+            "            gs[u] = ev >> 11;",
+            "            ge[u] = ok ? p.row_at[2 * row[u]] : 0;",
+            "            gn[u] = ok ? p.row_at[2 * row[u] + 1] : 0;",
             "        }",
-            "        for (int q = 0; q < nspk; q++) {",
-            "            const int src = s_spk[q];",
-            "            const unsigned int a = p.rec_ptr[src], e_ = p.rec_ptr[src + 1];",
-            f"            for (unsigned int e = a + j; e < e_; e += {T}) g_rec[e] += s_lam[p.rec_post[e]];",
+            "        #pragma unroll",
+            f"        for (int u = 0; u < {GB}; u++) {{",
+            "            const bool in = row[u] < HB_NIW * 64;",
+            "            double* const g = in ? g_in : g_rec;",
+            "            const int* const post = in ? p.post_in : p.post_rec;",
+            "            #pragma unroll",
+            f"            for (int c = 0; c < {GP}; c++) {{",
+            "                const int e = ge[u] + (c * 64 + lane < gn[u] ? c * 64 + lane : 0);",
+            "                gy[u][c] = g[e];",
+            "                gt[u][c] = post[e];",
+            "            }",
+            "            ge[u] = in ? ge[u] : ~ge[u];",
             "        }",
-            "        const double lamJ = lam_I;",
-            "        gA += dLdu * v_prev;",
-            "        gB += dLdu * I_prev;",
-            "        gC += dLdu;",
-            "        gbeta += lamJ * I_prev;",
-            "        lam_v = p.A * dLdu + extra;",
-            "        lam_I = p.B * dLdu + p.beta * lamJ;",
-            "        __syncthreads();",
+            "    };",
+            "    auto hb_give = [&]() __attribute__((always_inline)) {",
+            "        #pragma unroll",
+            f"        for (int u = 0; u < {GB}; u++)",
+            "            if (u < g_m) {",
+            "                double* const g = ge[u] >= 0 ? g_in : g_rec;",
+            "                const int* const post = ge[u] >= 0 ? p.post_in : p.post_rec;",
+            "                const int e = (ge[u] >= 0 ? ge[u] : ~ge[u]) + lane;",
+            "                #pragma unroll",
+            f"                for (int c = 0; c < {GP}; c++)",
+            "                    if (c * 64 + lane < gn[u]) g[e + c * 64] = gy[u][c] + s_hi[gs[u]][gt[u][c]];",
+            f"                for (int y = {GP} * 64 + lane; y < gn[u]; y += 64) g[e - lane + y] += s_hi[gs[u]][post[e - lane + y]];",
+            "            }",
+            "    };",
+            "    unsigned long long w_next = hb_word(p.n_seg - 1, 0);  // of the block to come (read ahead)",
+            "    for (int sg = p.n_seg - 1; sg >= 0; sg--) {",
+            "        const size_t co = ((size_t)sg * gridDim.x + b) * N + threadIdx.x;",
+            f"        HB_EACH_Q {{ v[q] = HB_J < N ? p.ckpt_v[co + q * {T}] : 0.0; I[q] = HB_J < N ? p.ckpt_I[co + q * {T}] : 0.0; }}",
+            "        const size_t so = (size_t)b * n_sub * N + threadIdx.x;",
+            "        for (int sb = 0; sb < n_sub - 1; sb++) {",
+            "            const int n_ev = hb_list(w_next);",
+            "            w_next = hb_word(sg, sb + 1);",
+            "            HB_EACH_Q if (HB_J < N) {",
+            f"                p.sub_v[so + (size_t)sb * N + q * {T}] = v[q]; p.sub_I[so + (size_t)sb * N + q * {T}] = I[q];",
+            "            }",
+            f"            hb_steps(sg * C + sb * {SB}, {SB}, n_ev, [](const int) {{}});",
+            "        }",
+            "        for (int sb = n_sub - 1; sb >= 0; sb--) {",
+            f"            const int k0 = sg * C + sb * {SB}, n = hb_len(sb);",
+            "            const int n_ev = hb_list(w_next);",
+            "            w_next = sb > 0 ? hb_word(sg, sb - 1) : hb_word(sg - 1, 0);",
+            "            if (sb < n_sub - 1)",
+            "                HB_EACH_Q {",
+            f"                    v[q] = HB_J < N ? p.sub_v[so + (size_t)sb * N + q * {T}] : 0.0;",
+            f"                    I[q] = HB_J < N ? p.sub_I[so + (size_t)sb * N + q * {T}] : 0.0;",
+            "                }",
+            "            hb_steps(k0, n - 1, n_ev, [&](const int s) { HB_EACH_Q { s_hv[s][HB_J] = v[q]; s_hi[s][HB_J] = I[q]; } });",
+            "            HB_EACH_Q { s_hv[n - 1][HB_J] = v[q]; s_hi[n - 1][HB_J] = I[q]; }",
+            "            g_c = n_ev > 0 ? (n_ev - 1) & ~63 : 0;",
+            "            g_left = hb_mine(n_ev);",
+            "            hb_take(n_ev);",
+            "            for (int s = n - 1; s >= 0; s--) {",
+            "                const int k = k0 + s;",
+            "                HB_EACH_Q {",
+            "                    const double v_prev = s_hv[s][HB_J], I_prev = s_hi[s][HB_J];",
+            "                    double u = v_prev, In = I_prev;",
+            "                    hb_update(HB_J, k, u, In);  // the step's update again (identical statements and values)",
+            "                    const bool cond = HB_J < N && u > p.theta;",
+            "                    const double v_post = cond ? 0.0 : u;",
+            "                    double dLdu = cond ? 0.0 : __builtin_fma(p.coef_v * 2.0, v_post, lam_v[q]);",
+            "                    double extra = 0.0;",
+            "                    if (fs_k[q] == k) { // first spike of a readout: interpolated crossing time",
+            "                        const double d = u - v_prev;",
+            "                        const double tc = dt * ((double)k + (p.theta - v_prev) / d);",
+            "                        const double dLdt = p.coef_fs * 2.0 * (tc - p.targets[HB_J]);",
+            "                        dLdu += dLdt * (-dt * (p.theta - v_prev) / (d * d));",
+            "                        extra = dLdt * (dt * (p.theta - u) / (d * d));",
+            "                    }",
+            "                    const double lamJ = lam_I[q];",
+            "                    s_hi[s][HB_J] = lamJ;  // for the weight gradients below",
+            "                    gA[q] = __builtin_fma(dLdu, v_prev, gA[q]);",
+            "                    gB[q] = __builtin_fma(dLdu, I_prev, gB[q]);",
+            "                    gC[q] += dLdu;",
+            "                    gbeta[q] = __builtin_fma(lamJ, I_prev, gbeta[q]);",
+            "                    lam_v[q] = __builtin_fma(p.A, dLdu, extra);",
+            "                    lam_I[q] = __builtin_fma(p.B, dLdu, p.beta * lamJ);",
+            "                }",
+            "            }",
+            "            // event-based weight gradients: lam of I after a step at the targets of a source that",
+            "            // spiked in it",
+            "            __syncthreads();",
+            "            hb_give();",
+            "            while (g_left != 0ull || g_c > 0) { hb_take(n_ev); hb_give(); }",
+            "        }",
+            "        {  // the interval's sums",
+        ]
+        k += self._sum_lines(["gA[q]", "gB[q]", "gC[q]", "gbeta[q]"], "g_all", 4)
+        k += [
+            "            HB_EACH_Q gA[q] = gB[q] = gC[q] = gbeta[q] = 0.0;",
+            "        }",
             "    }",
-            "    if (act) { p.lam_v[bo + j] = lam_v; p.lam_I[bo + j] = lam_I; }",
-            "    double x[4] = {act ? gA : 0.0, act ? gB : 0.0, act ? gC : 0.0, act ? gbeta : 0.0};",
-            "    for (int c = 0; c < 4; c++) {",
-            "        for (int o = 32; o > 0; o >>= 1) x[c] += __shfl_down(x[c], o, 64);",
-            "        if (lane == 0) s_red[wid][c] = x[c];",
-            "    }",
-            "    __syncthreads();",
-            "    if (j < 4) {",
-            "        double acc = 0.0;",
-            f"        for (int w_ = 0; w_ < {NW}; w_++) acc += s_red[w_][j];",
-            "        p.gacc[b * 4 + j] += acc;",
-            "    }",
+            "    if (threadIdx.x < 4) p.gacc[b * 4 + threadIdx.x] = g_all;",
             "}",
         ]
         return "\n".join(k) + "\n"
@@ -489,19 +765,18 @@ class LIFNetwork:
         sc = scalar_values(self.su, {"dt": self.dt, "N": self.N, **consts}, "double")
         return {n: sc[n][0] for n in self.su_scalars}, consts
 
-    def _launch(self, fn, cls, vals):
+    def _launch(self, fn, cls, vals, grid=None):
         a = cls()
         for name, _ in cls._fields_:
             if name in vals:
                 setattr(a, name, vals[name])
         buf = bytes(a)
         stream = ctypes.c_void_p(_torch().cuda.current_stream().cuda_stream)
-        _lib.check(L.hb_launch(fn, self.B, BLOCK, 0, stream, buf, len(buf)), "lif launch")
+        _lib.check(L.hb_launch(fn, self.B if grid is None else grid, self.block, 0, stream, buf, len(buf)), "lif launch")
 
     def _base_vals(self, sc):
-        v = dict(T_total=self.T, seed=self.seed, n_in=self.n_in, N=self.N, R=self.R, trial0=0,
-                 theta=self.c["theta"], dt=self.dt, r_dt=self.r_dt.data_ptr(), in_ptr=self.in_ptr.data_ptr(),
-                 in_post=self.in_post.data_ptr(), rec_ptr=self.rec_ptr.data_ptr(), rec_post=self.rec_post.data_ptr())
+        v = dict(n_seg=self.S, n_steps=self.C, T_total=self.T, seed=self.seed, n_in=self.n_in, N=self.N, R=self.R,
+                 trial0=0, n_trials=self.B, theta=self.c["theta"], dt=self.dt)
         for n, x in sc.items():
             v[f"su_{n}"] = x
         return v
@@ -523,8 +798,12 @@ class LIFNetwork:
         fs_u = torch.zeros_like(fs_vprev)
         l2 = torch.zeros(B, dtype=torch.float64, device="cuda")
         vals = self._base_vals(sc)
-        vals.update(n_steps=self.C, in_w=w_in.data_ptr(), rec_w=w_rec.data_ptr(), v=v.data_ptr(), I=I.data_ptr(),
-                    ckpt_v=ckpt_v.data_ptr(), ckpt_I=ckpt_I.data_ptr(), fs_step=fs_step.data_ptr(),
+        dense = torch.zeros(self.dense_size, dtype=w_in.dtype, device="cuda")
+        dense[self.in_at] = w_in
+        dense[self.rec_at] = w_rec
+        raster = torch.empty((B, self.T, sum(self._words())), dtype=torch.int64, device="cuda")
+        vals.update(dense=dense.data_ptr(), raster=raster.data_ptr(), r_dt=self.r_dt.data_ptr(), v=v.data_ptr(),
+                    I=I.data_ptr(), ckpt_v=ckpt_v.data_ptr(), ckpt_I=ckpt_I.data_ptr(), fs_step=fs_step.data_ptr(),
                     fs_vprev=fs_vprev.data_ptr(), fs_u=fs_u.data_ptr(), l2=l2.data_ptr())
         if record_spikes:
             spk_i = torch.zeros((B, spike_cap), dtype=torch.int32, device="cuda")
@@ -533,11 +812,11 @@ class LIFNetwork:
             vals.update(spk_i=spk_i.data_ptr(), spk_step=spk_step.data_ptr(), spk_n=spk_n.data_ptr(),
                         spk_cap=spike_cap)
         cls = self.fwd_struct.ctypes_struct()
-        for sg in range(self.S):
-            vals["k0"] = sg * self.C
-            self._launch(self._fwd_fn, cls, vals)
+        waves = B * -(-self.T // 16) * self._words()[0]  # of lif_inputs
+        self._launch(self._inp_fn, cls, vals, -(-waves // (self.block // 64)))
+        self._launch(self._fwd_fn, cls, vals)
         loss, parts = self._loss(fs_step, fs_vprev, fs_u, l2)
-        saved = dict(w_in=w_in, w_rec=w_rec, tau_m=tau_m, tau_s=tau_s, ckpt_v=ckpt_v, ckpt_I=ckpt_I,
+        saved = dict(w_in=w_in, w_rec=w_rec, dense=dense, raster=raster, tau_m=tau_m, tau_s=tau_s, ckpt_v=ckpt_v, ckpt_I=ckpt_I,
                      fs_step=fs_step, fs_vprev=fs_vprev, fs_u=fs_u, v=v, I=I, parts=parts)
         if record_spikes:
             n = spk_n.cpu().numpy()
@@ -566,34 +845,25 @@ class LIFNetwork:
         tau_m, tau_s = saved["tau_m"], saved["tau_s"]
         sc, consts = self._scalars(tau_m, tau_s)
         lin = linear_map(self.su, consts, self.dt)
-        hist_v = torch.empty((B, self.C, N), dtype=torch.float64, device="cuda")
-        hist_I = torch.empty_like(hist_v)
-        lam_v = torch.zeros((B, N), dtype=torch.float64, device="cuda")
-        lam_I = torch.zeros_like(lam_v)
-        g_in = torch.zeros((B, self.n_syn_in), dtype=torch.float64, device="cuda")
-        g_rec = torch.zeros((B, self.n_syn_rec), dtype=torch.float64, device="cuda")
+        sub_v = torch.empty((B, -(-self.C // self.sub), N), dtype=torch.float64, device="cuda")
+        sub_I = torch.empty_like(sub_v)
+        # (a pathway without synapses keeps a place to read)
+        g_in = torch.zeros((B, max(1, self.n_syn_in)), dtype=torch.float64, device="cuda")
+        g_rec = torch.zeros((B, max(1, self.n_syn_rec)), dtype=torch.float64, device="cuda")
         gacc = torch.zeros((B, 4), dtype=torch.float64, device="cuda")
-        v = torch.empty((B, N), dtype=torch.float64, device="cuda")
-        I = torch.empty_like(v)
-        fvals = self._base_vals(sc)
-        fvals.update(n_steps=self.C, in_w=saved["w_in"].data_ptr(), rec_w=saved["w_rec"].data_ptr(),
-                     v=v.data_ptr(), I=I.data_ptr(), hist_v=hist_v.data_ptr(), hist_I=hist_I.data_ptr())
-        bvals = self._base_vals(sc)
-        bvals.update(n_steps=self.C, hist_v=hist_v.data_ptr(), hist_I=hist_I.data_ptr(),
-                     fs_step=saved["fs_step"].data_ptr(), A=lin["A"], B=lin["B"], beta=lin["beta"],
-                     coef_fs=grad_out / (B * c["t_ref"] ** 2),
-                     coef_v=grad_out * c["c_v"] / (N * self.T * c["theta"] ** 2) / B,
-                     targets=self.targets.data_ptr(), lam_v=lam_v.data_ptr(), lam_I=lam_I.data_ptr(),
-                     g_in=g_in.data_ptr(), g_rec=g_rec.data_ptr(), gacc=gacc.data_ptr())
-        fcls, bcls = self.fwd_struct.ctypes_struct(), self.bwd_struct.ctypes_struct()
-        for sg in reversed(range(self.S)):
-            v.copy_(saved["ckpt_v"][sg])
-            I.copy_(saved["ckpt_I"][sg])
-            fvals["k0"] = bvals["k0"] = sg * self.C
-            self._launch(self._fwd_fn, fcls, fvals)
-            self._launch(self._bwd_fn, bcls, bvals)
-        gw_in = g_in.sum(0)
-        gw_rec = g_rec.sum(0)
+        vals = self._base_vals(sc)
+        vals.update(dense=saved["dense"].data_ptr(), raster=saved["raster"].data_ptr(),
+                    ckpt_v=saved["ckpt_v"].data_ptr(), ckpt_I=saved["ckpt_I"].data_ptr(),
+                    fs_step=saved["fs_step"].data_ptr(), A=lin["A"], B=lin["B"], beta=lin["beta"],
+                    coef_fs=grad_out / (B * c["t_ref"] ** 2),
+                    coef_v=grad_out * c["c_v"] / (N * self.T * c["theta"] ** 2) / B,
+                    targets=self.targets.data_ptr(), row_at=self.row_at.data_ptr(), post_in=self.post_in.data_ptr(),
+                    post_rec=self.post_rec.data_ptr(), sub_v=sub_v.data_ptr(),
+                    sub_I=sub_I.data_ptr(), n_syn_in=g_in.shape[1], n_syn_rec=g_rec.shape[1], g_in=g_in.data_ptr(),
+                    g_rec=g_rec.data_ptr(), gacc=gacc.data_ptr())
+        self._launch(self._bwd_fn, self.bwd_struct.ctypes_struct(), vals)
+        gw_in = g_in.sum(0)[:self.n_syn_in]
+        gw_rec = g_rec.sum(0)[:self.n_syn_rec]
         ga = gacc.sum(0).cpu().numpy()
         g_coef = {"A": ga[0], "B": ga[1], "C": ga[2], "beta": ga[3]}
         g_tau_m = sum(g_coef[k] * lin[f"d{k}"][0] for k in g_coef)

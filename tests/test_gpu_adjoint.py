@@ -130,3 +130,40 @@ def test_full_configuration_is_deterministic():
     assert np.isfinite(a[0]) and a[0] == b[0]
     assert np.array_equal(a[1], b[1]) and np.array_equal(a[2], b[2]) and a[3] == b[3] and a[4] == b[4]
     assert np.isfinite(a[1]).all() and np.abs(a[2]).max() > 0
+
+
+@pytest.mark.parametrize("n, n_in, p, rate, steps, every, wt", [
+    (64, 1, 0.1, 500.0, 60, 20, "double"),      # one wave, one input, blocks of 8 and a rest of 4
+    (65, 64, 1e-9, 500.0, 50, 50, "float"),     # a second word of one neuron; no synapses
+    (300, 65, 1.0, 300.0, 70, 7, "double"),    # rows longer than their pieces, an interval within a block
+    (513, 200, 0.1, 1500.0, 60, 30, "float"),  # many events: several per word, row and block
+    (1024, 1024, 0.05, 100.0, 40, 1, "float"),  # the largest
+])
+def test_shapes_at_the_edges_of_words_blocks_and_batches(n, n_in, p, rate, steps, every, wt):
+    """Loss and gradients against autograd of the tensor reference (both double beyond the
+    weights' rounding; sums of at most 1e5 terms, so 1e-9)."""
+    import torch
+
+    from brian2_amd.adjoint import LIF, LIFNetwork
+    from lif_reference import reference_loss
+
+    c = dict(LIF, N=n, NE=n * 4 // 5, n_in=n_in, p=p, rate_lo=rate / 2, rate_hi=rate, n_steps=steps, tau_m=0.004, bias=0.012)
+    net = LIFNetwork(trials=3, config=c, weight_dtype=wt, ckpt_every=every)
+    loss, saved = net.forward(net.w_in0, net.w_rec0, c["tau_m"], c["tau_s"])
+    g_in, g_rec, g_m, g_s = net.backward(saved)
+    sc, _ = net._scalars(c["tau_m"], c["tau_s"])
+    leaf = lambda x: torch.tensor(x, dtype=torch.float64, requires_grad=True)  # noqa: E731
+    w_in, w_rec = leaf(net.w_in0.cpu().numpy().astype(np.float64)), leaf(net.w_rec0.cpu().numpy().astype(np.float64))
+    tm, ts = leaf(c["tau_m"]), leaf(c["tau_s"])
+    ref, _, raster = reference_loss(net.inp, O.lif_inputs(3, c=c)["trains"], net.inp["v0"], w_in, w_rec, tm, ts, c,
+                                    lio_values=tuple(sc[f"_lio_{k}"] for k in (1, 2, 3, 4)))
+    ref.backward()
+    assert raster.sum() > 3 * n // 10
+    assert abs(loss - float(ref)) <= 1e-11 * abs(float(ref))
+    for got, want in ((g_in, w_in), (g_rec, w_rec)):
+        got = got.cpu().numpy()
+        assert got.shape == tuple(want.shape)
+        if len(got) and want.grad is not None and float(want.grad.abs().max()) > 0:
+            assert _rel(got, want.grad.numpy()) < 1e-9
+    assert abs(g_m - float(tm.grad)) <= 1e-9 * abs(float(tm.grad))
+    assert abs(g_s - float(ts.grad)) <= 1e-9 * abs(float(ts.grad))
