@@ -732,7 +732,8 @@ class Network:
         """bucket_cap: events of a tile sorted in LDS at a time (default: what fits two
         workgroups per CU); bucket_mem_frac: share of free device memory the event
         staging may use; tile: threads per workgroup of the step kernels (default:
-        1024 for groups of at least 65536 neurons, else 256); npt: neurons per thread
+        1024 for groups of at least 65536 neurons, and for groups from 5121 whose launches
+        fuse and whose update is a light one, else 256); npt: neurons per thread
         (default 1); overlap: run the gathers concurrently with the group updates when
         every delay is at least one step (default True); fuse: with overlap, run a
         group of 1024-thread tiles and the gathers into it as one launch per step
@@ -807,7 +808,7 @@ class Network:
         # per group: device state, spike ring
         for g in groups:
             # threads per workgroup, neurons per thread; a workgroup owns a tile of block * npt neurons
-            g.block = int(self.tile or (1024 if g.N >= 65536 else 256))
+            g.block = int(self.tile or (1024 if g.N >= 65536 or self._fuses_early(g, paths) else 256))
             g.npt = int(self.npt or 1)
             g.tile = g.block * g.npt
             dmax = max([s.csr["dmin"] + s.csr["n_seg"] - 1 for s in paths if s.source is g]
@@ -846,8 +847,7 @@ class Network:
         # with every delay at least one step, the gathers of step s read only spikes of earlier
         # steps: they run concurrently with the group updates of step s and with each other
         # (three side lanes, taken in turn), or inside the target group's launch
-        self.concurrent_gathers = (bool(paths) and all(s.csr["dmin"] >= 1 for s in paths) and self.overlap
-                                   and not any(s.plastic for s in paths))
+        self.concurrent_gathers = self._gathers_concur(paths)
         for g in groups:
             g.fused = None
             g.fuse_ok = (self.fuse and self.concurrent_gathers and isinstance(g, NeuronGroup)
@@ -885,6 +885,25 @@ class Network:
                 if s.carry is not None:
                     _lib.check(L.hb_plan_set_lane(self._plan, s.carry_index, 1 + i % 3), "hb_plan_set_lane")
         self._built = True
+
+    def _gathers_concur(self, paths):
+        return (bool(paths) and all(s.csr["dmin"] >= 1 for s in paths) and self.overlap
+                and not any(s.plastic for s in paths))
+
+    def _fuses_early(self, g, paths):
+        """Whether a group of fewer than 65536 neurons takes tiles of 1024 threads, so that its
+        update and its gathers are one launch (kernels.FusedStepKernel).
+
+        A step of separate launches is bound by the launches, a fork to the lanes and a join:
+        8192 neurons (in-degree 1000) 16.4 us per step against 6.2 fused, 20000 17.0 against
+        6.3, 60000 (in-degree 300) 18.3 against 12.4.  Tiles of 1024 leave compute units
+        without work, which an update of many exponentials and powers pays for (35 of them:
+        6000 neurons 28.5 against 39.0, 30000 36.9 against 39.3; none: 18.4 against 9.1), so
+        they are for updates of few; groups of up to five such tiles keep the launch per
+        pathway, which profile() times one by one."""
+        return (self.fuse and self.npt in (None, 1) and isinstance(g, NeuronGroup) and g.N > 5 * _kernels.GATHER_BLOCK
+                and any(s.target is g for s in paths) and self._gathers_concur(paths)
+                and _resident.heavy_operations([g.su, g.th, g.rs]) < 8)
 
     def _monitors(self, g):
         """The group's monitors (g.smon, g.stmon, g.rmon)."""
@@ -1012,8 +1031,9 @@ class Network:
         g.n_tiles = (g.N + T - 1) // T
         vbytes = 8 if g.val_t in ("double", "long long") else 4
         # tiles of 1024 neurons, one per thread: two workgroups per CU when the step kernel fits
-        # in 64 VGPRs (checked when it is built), so each gets half the LDS
-        g.two_per_cu = g.block == 1024 and g.npt == 1
+        # in 64 VGPRs (checked when it is built), so each gets half the LDS.  Groups of fewer tiles
+        # than a quarter of the CUs have one to themselves
+        g.two_per_cu = g.block == 1024 and g.npt == 1 and (bool(self.tile) or g.N >= 65536)
         cap = fold_capacity(g.block, g.val_t, g.npt, wgs_per_cu=2 if g.two_per_cu else None)
         g.lds_cap = int(min(self.bucket_cap, cap) if self.bucket_cap else cap)
         window = _kernels.GATHER_BLOCK * _kernels.GATHER_EVENTS_PER_THREAD

@@ -106,3 +106,19 @@ def test_store_restore_replays_bit_identically(shape):
     net.run(0)  # folds the events of the last profiled step
     assert np.array_equal(mon.i[n0:], a_i) and np.array_equal(mon.step[n0:], a_s)
     assert all(np.array_equal(c["G"].get(v), x) for v, x in zip(("v", "ge", "gi"), a_state))
+
+
+@pytest.mark.parametrize("n, float_t", [(5120, "double"), (5121, "double"), (7168, "float")])
+def test_groups_that_fuse_below_65536(n, float_t):
+    """Beyond five tiles of 1024 a group with delays takes one launch per step: the same spikes
+    and state as separate launches of 256-thread tiles."""
+    from brian2_amd import synth
+
+    out = []
+    for shape in ({}, {"tile": 256}):
+        c = synth.cuba_synw_network(N=n, K=70, float_t=float_t, ginh=0.4, network_options=shape)
+        c["net"].run(400)
+        assert (c["G"].fused is not None) == (n > 5120 and not shape)
+        out.append([c["mon"].i, c["mon"].step, c["net"].n_events] + [c["G"].get(v) for v in ("v", "ge", "gi")])
+    assert len(out[0][0]) > 0
+    assert all(np.array_equal(a, b) for a, b in zip(*out))
