@@ -491,6 +491,26 @@ def heavy_operations(specs):
     return n
 
 
+def plain_network(net, groups, paths, summed):
+    """Whether Network net is one group with synapses onto itself whose events are no more than
+    their number: no delays, no variables of the synapses; default launch shapes."""
+    if len(groups) != 1 or summed or not 1 <= len(paths) <= MAX_PATHWAYS:
+        return False
+    if any(x is not None for x in (net.tile, net.npt, net.gather_pairs, net.bucket_cap)):
+        return False
+    g = groups[0]
+    if getattr(g, "su", None) is None or g.N < 1:
+        return False
+    for s in paths:
+        if s.source is not g or s.target is not g or s.syn_vars or s.plastic or s.post_spec is not None:
+            return False
+        if s.count_events or s.carry is not None or s.csr["dmin"] != 0 or s.csr["n_seg"] != 1:
+            return False
+        if len(s.spec.vector) != 1 or g.vars[s.target_var] not in ("double", "float"):
+            return False
+    return True
+
+
 class GroupStep:
     """The resident step of a neuron group with synapses onto itself (Network's small
     networks): the ResidentKernel with the group's monitors.
@@ -500,7 +520,7 @@ class GroupStep:
     val_t      type in which the pathways' values are held before they are applied"""
 
     MAX_SYNAPSES = 1 << 25
-    MAX_HEAVY = {"double": 16384, "float": 36864}  # neurons x heavy operations of an update
+    MAX_HEAVY = {"double": 8192, "float": 16384}  # neurons x heavy operations of an update
 
     def __init__(self, group, scalars, pathways, val_t, n_syn, dt):
         g = group
@@ -640,29 +660,20 @@ class GroupStep:
         registers, synapses from it onto itself without delays or variables of their own,
         default launch shapes, an update that one compute unit can carry.
 
-        Measured on MI355X, us per step, this step against a launch for the group and one
-        per pathway: CUBA with 500 / 4000 / 8192 neurons 0.83 / 2.0 / 3.9 against
-        12.7 / 16.0 / 18.9; 8000 neurons with 19 million synapses 3.9 against 23.7 (in a
-        volley one compute unit has all the events, hence the bound on them).  An update
-        with exponentials is throughput: COBAHH (29 of them) with 400 / 600 / 1000 neurons
-        18.7 / 26.2 / 42.6 against 23.7 / 25.9 / 29.7 in fp64, with 1000 / 2000 neurons
-        18.2 / 38.6 against 23.8 / 27.8 in fp32."""
-        if len(groups) != 1 or summed or not 1 <= len(paths) <= MAX_PATHWAYS:
-            return False
-        if any(x is not None for x in (net.tile, net.npt, net.gather_pairs, net.bucket_cap)):
+        Measured on MI355X, us per step, this step against one launch per step over the whole
+        chip (kernels.PulledEvents): CUBA with 500 / 4000 / 8192 neurons 0.84 / 2.2 / 3.9
+        against 3.8 / 4.6 / 5.3; 8000 neurons with 19 million synapses 3.9 (in a volley one
+        compute unit has all the events, hence the bound on them).  An update with
+        exponentials is throughput: COBAHH (29 of them) with 200 / 400 neurons 8.6 / 15.7
+        against 11.8 / 12.0 in fp64, with 400 / 600 neurons 6.4 / 9.3 against 8.4 / 8.4 in
+        fp32."""
+        if not plain_network(net, groups, paths, summed):
             return False
         g = groups[0]
-        if getattr(g, "su", None) is None or not 1 <= g.N <= 1024 * neurons_in_registers(g.vars):
+        if g.N > 1024 * neurons_in_registers(g.vars):
             return False
         if g.N * heavy_operations((g.su, g.th, g.rs)) > cls.MAX_HEAVY[g.float_t]:
             return False
-        for s in paths:
-            if s.source is not g or s.target is not g or s.syn_vars or s.plastic or s.post_spec is not None:
-                return False
-            if s.count_events or s.carry is not None or s.csr["dmin"] != 0 or s.csr["n_seg"] != 1:
-                return False
-            if len(s.spec.vector) != 1 or g.vars[s.target_var] not in ("double", "float"):
-                return False
         return sum(int(s.csr["n_syn"]) for s in paths) <= cls.MAX_SYNAPSES
 
     @staticmethod

@@ -1,0 +1,77 @@
+"""Groups whose step counts its own events from the last step's spikes
+(kernels.PulledEvents), against the staged launches (tile given), bit for bit."""
+import numpy as np
+import pytest
+
+from test_gpu_resident import _const_spec
+
+pytestmark = pytest.mark.gpu
+
+E = ("ge", "+=", 1.62e-3)
+I = ("gi", "+=", -9e-3)
+CASES = {
+    "one neuron": (1, "double", [((0, 1), (0, 1)) + E + (1.0,)], "start"),
+    "a word": (64, "double", [((0, 64), (0, 64)) + E + (0.5,), ((0, 64), (0, 64)) + I + (0.2,)], None),
+    "a word and one": (65, "float", [((3, 65), (0, 65)) + E + (0.5,), ((0, 7), (1, 60)) + I + (1.0,)], "end"),
+    "a chunk of words": (4096, "double", [((0, 3000), (0, 4096)) + E + (0.01,), ((3000, 4096), (0, 4096)) + I + (0.01,)],
+                         "start"),
+    "a chunk and one": (4097, "float", [((0, 4097), (7, 4090)) + E + (0.01,)], None),
+    "the largest": (16384, "double", [((0, 13000), (0, 16384)) + E + (0.004,), ((13000, 16384), (0, 16384)) + I + (0.004,)],
+                    "end"),
+    "one variable, a pathway without synapses": (700, "double", [
+        ((0, 700), (0, 700), "ge", "+=", 1.1e-3, 0.03), ((0, 300), (0, 700), "ge", "*=", 0.9, 0.02),
+        ((0, 700), (0, 700)) + I + (0.0,), ((200, 700), (0, 400), "ge", "-=", 1e-4, 0.03)], None),
+}
+
+
+def _run(n, float_t, paths, state, model="cuba", twice=False, **options):
+    from brian2_amd import (Model, Network, NeuronGroup, PopulationRateMonitor, SpikeMonitor, StateMonitor, Synapses)
+
+    rng = np.random.default_rng(5)
+    G = NeuronGroup(n, Model.load(model), float_t=float_t, name="g")
+    G.v = -0.06 + 0.02 * rng.random(n) if model == "cuba" else -0.06 + 0.05 * rng.random(n)
+    G.lastspike = np.where(rng.random(n) < 0.3, -3.3e-3 * rng.random(n), -1e4)
+    syn = []
+    for k, (src, tgt, var, op, value, p) in enumerate(paths):
+        a, b = G[src[0]:src[1]], G[tgt[0]:tgt[1]]
+        S = Synapses(a, b, _const_spec(var, op, value), name=f"s{k}")
+        i, j = np.nonzero(rng.random((a.N, b.N)) < p)
+        S.connect(np.append(i, i[:1]), np.append(j, j[:1])) if twice else S.connect(i, j)
+        syn.append(S)
+    spikes, rate = SpikeMonitor(G[n // 3:]), PopulationRateMonitor(G[:max(1, n // 2)])
+    mons = [StateMonitor(G, ["v", "ge"], record=sorted({0, n // 2, n - 1}), when=state)] if state else []
+    net = Network(G, *syn, spikes, rate, *mons, dt=1e-4, **options)
+    for k in (1, 40, 19):
+        net.run(k)
+    net.store()
+    net.run(30)
+    net.restore()
+    net.run(20)
+    net.run(10, dt=5e-5)
+    out = [G.get(v) for v in G.vars] + [np.array([s.n_events for s in syn])]
+    return G, out + [spikes.i, spikes.step, spikes.count, rate.count] + [m.values() for m in mons]
+
+
+@pytest.mark.parametrize("name", sorted(CASES))
+def test_pulled_events_equal_the_staged_launches(name, monkeypatch):
+    from brian2_amd import resident
+
+    monkeypatch.setattr(resident.GroupStep, "takes", classmethod(lambda *a: False))
+    G, got = _run(*CASES[name])
+    H, want = _run(*CASES[name], tile=256)
+    assert G.pull is not None and H.pull is None
+    assert CASES[name][0] == 1 or want[0].std() > 0
+    for x, y in zip(got, want):
+        assert np.array_equal(x, y)
+
+
+def test_cobahh_pulls_and_what_is_not_taken():
+    """The example with exponentials by default; pairs with two synapses and launch shapes stay."""
+    paths = [((0, 900), (0, 1100), "ge", "+=", 6e-9, 0.02), ((900, 1100), (0, 1100), "gi", "+=", 6.7e-8, 0.02)]
+    G, got = _run(1100, "double", paths, "start", model="cobahh")
+    H, want = _run(1100, "double", paths, "start", model="cobahh", tile=128)
+    assert G.pull is not None and H.pull is None
+    assert len(want[-4]) > 0
+    for x, y in zip(got, want):
+        assert np.array_equal(x, y)
+    assert _run(1100, "double", paths, None, model="cobahh", twice=True)[0].pull is None
