@@ -20,6 +20,7 @@ import numpy as np
 from . import _lib
 from . import kernels as _kernels
 from . import resident as _resident
+from . import targets as _targets
 from .codegen import Renderer, ctype_of
 from .kernels import (
     LDS_BYTES,
@@ -831,7 +832,7 @@ class Network:
         for g in groups:
             g.incoming = [s for s in paths if s.target is g]
         self.resident = None
-        if self._build_resident(groups, paths):
+        if self._build_resident(groups, paths) or self._build_targets(groups, paths):
             self._built = True
             return
         for g in groups:
@@ -1049,8 +1050,78 @@ class Network:
         self.resident = R
         return True
 
+    # -- targets of a spike generator (targets.TargetSteps) ----------------------
+    def _build_targets(self, groups, paths):
+        """Builds the targets' kernel when the network takes it (targets.TargetSteps.takes)."""
+        gen = [g for g in groups if isinstance(g, SpikeGeneratorGroup)]
+        tgt = [g for g in groups if isinstance(g, NeuronGroup)]
+        if len(gen) != 1 or len(tgt) != 1 or len(groups) != 2 or len(paths) != 1 or self.summed_syn:
+            return False
+        src, g, s = gen[0], tgt[0], paths[0]
+        self._monitors(g)
+        if g.stmon is not None or g.rmon is not None or any(m.source is src for m in self.smons + self.stmons + self.rmons):
+            return False
+        if src.times is not None:
+            src.rebin(self.dt)
+        if not _targets.TargetSteps.takes(self, src, g, s):
+            return False
+        sc = []
+        for spec in (s.spec, s.post_spec):
+            host = {"dt": self.dt}
+            host.update(getattr(s, "namespace", {}) or {})
+            sc.append(scalar_values(spec, host, g.float_t))
+        g.val_t = self._group_value_type(paths)
+        R = _targets.TargetSteps(g, self._group_scalars(g), s.syn_ctypes(), s.plastic, s.spec.vector, s.target_index,
+                                 sc[0], s.post_spec.vector, sc[1], s.target_var, s.op, g.val_t)
+        R.path, R.gen = s, src
+        R.fn = self.device.function(R.source, R.kernel_name)
+        R.cls = R.struct.ctypes_struct()
+        ptr_ = s.csr["post_ptr"].long()
+        R.deg = int((ptr_[1:] - ptr_[:-1]).max())
+        R.lds = R.lds_bytes(R.syn_arrays, R.deg, s.src_range[1] - s.src_range[0])
+        s.events_dev = _torch().zeros(g.N, dtype=_torch().int64, device="cuda")
+        s.fused_into = None
+        src.gen_tb, src.gen_idx = dev(src.timebins, "int"), dev(src.indices, "int")
+        src.smon = src.stmon = src.rmon = src.flush_fn = g.flush_fn = None
+        if g.smon:
+            self._alloc_spike_monitor(g, g.smon)
+        self._plan = ctypes.c_void_p()
+        _lib.check(L.hb_plan_create(self.device.ctx, ptr(self.clock), ctypes.byref(self._plan)), "hb_plan_create")
+        self._launches = []
+        self.resident = R
+        return True
+
+    def _run_targets(self, n_steps):
+        """Launches the targets' kernel for n_steps steps on the current stream."""
+        R, g, s, src = self.resident, self.resident.group, self.resident.path, self.resident.gen
+        v = {"step0": self.t_step, "dt": self.dt, "n_steps": n_steps, "N": g.N, "deg": R.deg, "src0": s.src_range[0],
+             "n_src": s.src_range[1] - s.src_range[0], "gen_tb": src.gen_tb.data_ptr(), "gen_idx": src.gen_idx.data_ptr(),
+             "gen_at": int(np.searchsorted(src.timebins, self.t_step, side="left")), "gen_n": len(src.timebins),
+             "events": s.events_dev.data_ptr(), "status": self.status.data_ptr()}
+        for n in ("post_ptr", "post_syn", "post_pre"):
+            v[n] = s.csr[n].data_ptr()
+        for n in g.vars:
+            v[f"a_{n}"] = g._dev[n].data_ptr()
+        for n in R.syn_arrays:
+            v[f"s_{n}"] = s.csr["syn"][n].data_ptr()
+        for (tg, n), (val, _) in R.scalars.items():
+            v[f"{tg}_{n}"] = val
+        for x, sc in (("c", R.pre_scalars), ("q", R.post_scalars)):
+            for n, (val, _) in sc.items():
+                v[f"{x}_{n}"] = val
+        v.update(self._monitor_args(g))
+        a = R.cls()
+        for name, _ in R.cls._fields_:
+            if name in v:
+                setattr(a, name, v[name])
+        buf = bytes(a)
+        _lib.check(L.hb_launch(R.fn, g.N, 64, R.lds, self.device.stream, buf, len(buf)), "targets' steps")
+        self.clock.fill_(self.t_step + n_steps)
+
     def _run_resident(self, n_steps):
         """Launches the resident step for n_steps steps on the current stream."""
+        if isinstance(self.resident, _targets.TargetSteps):
+            return self._run_targets(n_steps)
         R, g = self.resident, self.resident.group
         v = {"clock": self.clock.data_ptr(), "step_off": 0, "dt": self.dt, "n_steps": n_steps, "N": g.N,
              "bound": R.bound or 0.0, "row_ptr": R.row_ptr.data_ptr(), "post": R.post.data_ptr(),
