@@ -176,9 +176,10 @@ def fold_capacity(T, val_t, npt=1, wgs_per_cu=None):
     return int(max(128, cap - cap % 64))
 
 
-def _fold_source(T, cap, vt, flush, npt=1):
+def _fold_source(T, cap, vt, flush, npt=1, share=1):
     """Fold of the events staged by the previous step's gathers, for a tile of
-    T*npt targets (thread x owns targets q*T + x, q < npt).
+    T*npt/share targets (thread x owns targets q*T + x, q < npt; with share > 1 the
+    first T/share threads own one each, and all of them work on the events).
 
     The tile's events are contiguous in its region of the staging buffer (in the
     order the gathers' atomics gave them; the keys fix the delivery order).
@@ -195,7 +196,8 @@ def _fold_source(T, cap, vt, flush, npt=1):
     U = FOLD_EVENTS_PER_THREAD
     XW = T * U
     W = cap // 2
-    TN = T * npt
+    own, end, if_own = (f"(int)threadIdx.x < {T // share} ? ", " : 0", f"if ((int)threadIdx.x < {T // share}) ") if share > 1 else ("",) * 3
+    TN = T * npt // share
     k = [
         "    // ---- events delivered by propagate(step - 1): this tile's region of the staging ----",
         "    // staging buffers rotate over three steps: step s's gathers write buffer s % 3 (possibly",
@@ -263,7 +265,7 @@ def _fold_source(T, cap, vt, flush, npt=1):
         f"    bool hb_bigt[{npt}];",
         "    int hb_ct = 0;",
         "    #pragma unroll",
-        f"    for (int q = 0; q < {npt}; q++) {{ hb_c[q] = s_fill[q * {T} + threadIdx.x]; hb_b[q] = hb_ct; hb_ct += hb_c[q]; }}",
+        f"    for (int q = 0; q < {npt}; q++) {{ hb_c[q] = {own}s_fill[q * {T} + threadIdx.x]{end}; hb_b[q] = hb_ct; hb_ct += hb_c[q]; }}",
         "    // segments in LDS: an allocation, waves in any order (the passes need no particular order)",
         "    const int hb_tb = hb_block_alloc(hb_ct, &s_alloc);",
         f"    const bool hb_one = hb_tot <= {cap};",
@@ -273,8 +275,7 @@ def _fold_source(T, cap, vt, flush, npt=1):
         f"    for (int q = 0; q < {npt}; q++) {{",
         "        hb_b[q] += hb_tb;",
         f"        hb_bigt[q] = !hb_one && hb_c[q] > {W};",
-        f"        s_beg[q * {T} + threadIdx.x] = hb_bigt[q] ? ~hb_b[q] : hb_b[q];",
-        f"        s_fill[q * {T} + threadIdx.x] = 0;",
+        f"        {if_own}{{ s_beg[q * {T} + threadIdx.x] = hb_bigt[q] ? ~hb_b[q] : hb_b[q]; s_fill[q * {T} + threadIdx.x] = 0; }}",
         "        hb_anyb = hb_anyb || hb_bigt[q];",
         "        if (!hb_bigt[q] && hb_c[q] > hb_cm) hb_cm = hb_c[q];",
         "    }",
@@ -312,7 +313,7 @@ def _fold_source(T, cap, vt, flush, npt=1):
     return pro, k, U, W
 
 
-def _fold_passes(T, U, W, cap, vt, apply_lines, npt=1):
+def _fold_passes(T, U, W, cap, vt, apply_lines, npt=1, share=1):
     """Phase C of the fold (see _fold_source).  `apply_lines` apply (hb_k, hb_v) to
     target q's registers.
 
@@ -325,7 +326,7 @@ def _fold_passes(T, U, W, cap, vt, apply_lines, npt=1):
     segment of a target of the pass, which the pass wrote in full.  Targets
     sorted in global memory come last."""
     XW = T * U
-    TN = T * npt
+    TN = T * npt // share
     RU, AB = FOLD_RANK_UNROLL, FOLD_APPLY_BATCH
     k = [
         f"    const int hb_lim = hb_one ? hb_tot : {cap};  // LDS positions a pass may have written",
@@ -497,7 +498,7 @@ class NeuronKernel:
     def __init__(self, name, N, arrays, float_t, stateupdate=None, threshold=None, reset=None,
                  reset_mode="none", scalars=None, fold=None, lds_cap=0, val_t="double",
                  spikemon=None, statemon=None, flush=False, uses_refractory=False, statemon_when="start",
-                 tile=256, npt=1, ratemon=None, waves_per_eu=0, ring_parts=None, pull=None):
+                 tile=256, npt=1, ratemon=None, waves_per_eu=0, ring_parts=None, pull=None, share=1):
         self.name = name
         self.N = N
         self.pull = pull              # PulledEvents: incoming events from the last step's spikes, or None
@@ -527,8 +528,11 @@ class NeuronKernel:
             raise ValueError("ring parts must be ascending neuron indices starting at 0")
         self.T = tile                 # threads per workgroup
         self.npt = npt                # neurons per thread: a workgroup owns tile * npt neurons
+        self.share = share            # threads per neuron (npt 1): tile / share neurons
         if npt < 1 or tile * npt > 65536:
             raise ValueError("a tile holds at most 65536 neurons")
+        if share < 1 or tile % share or (share > 1 and (npt > 1 or tile // share < 64)):
+            raise ValueError("share divides the tile's threads, of one neuron each")
         self._build()
 
     def _block(self, tag, spec, extra_types):
@@ -587,7 +591,7 @@ class NeuronKernel:
 
     def _source(self, ps):
         T, NPT = self.T, self.npt
-        TN = T * NPT
+        TN = T * NPT // self.share
         k = [source_header(T), DECL_MARK, ps.c_decl()]
         kname = f"{'flush' if self.flush else 'step'}_{self.name}"
         self.kernel_name = kname
@@ -598,9 +602,10 @@ class NeuronKernel:
         k.append("    const double dt = p.dt;")
         k.append("    const int N = p.N;")
         k.append("    const int hb_tile = blockIdx.x;")
-        k += [
-            f"    const int hb_i0 = hb_tile * {TN} + threadIdx.x;  // neuron q*{T} + hb_i0 for q < {NPT}",
-        ]
+        if self.share > 1:  # the threads that only work on the events have no neuron
+            k.append(f"    const int hb_i0 = (int)threadIdx.x < {TN} ? hb_tile * {TN} + (int)threadIdx.x : 0x7fffffff;")
+        else:
+            k.append(f"    const int hb_i0 = hb_tile * {TN} + threadIdx.x;  // neuron q*{T} + hb_i0 for q < {NPT}")
         k.append("    (void)t; (void)dt;")
         if self.pull:
             k += self.pull.load_lines()
@@ -611,7 +616,7 @@ class NeuronKernel:
                 R = len(self.ring_parts)
                 k += [f"    __shared__ int s_npart[{R}], s_pbase[{R}];",
                       f"    if (threadIdx.x < {R}) s_npart[threadIdx.x] = 0;"]
-        fold = _fold_source(T, self.cap, self.val_t, self.flush, NPT) if self.fold else None
+        fold = _fold_source(T, self.cap, self.val_t, self.flush, NPT, self.share) if self.fold else None
         if fold:
             k += fold[0]  # the tile's event count first: phase A's loads depend on it, not on the state
         # state of this thread's neurons in registers (the fold updates them)
@@ -641,7 +646,7 @@ class NeuronKernel:
             for rank, var, op in self.fold:
                 apply.append(f"case {rank}: hb_a_{var}[q] {op} hb_v; break;")
             apply += ["default: break;", "}"]
-            k += _fold_passes(T, U, W, self.cap, self.val_t, apply, NPT)
+            k += _fold_passes(T, U, W, self.cap, self.val_t, apply, NPT, self.share)
             k += ["    } else {", "    __syncthreads();  // the workgroup's counters, cleared at the start", "    }"]
         if self.statemon and (not self.flush or self.statemon_when == "end"):
             # the recorded neurons of this tile: rec_idx[hb_rlo, hb_rhi), found by two searches
@@ -1792,7 +1797,7 @@ class FusedStepKernel:
     def __init__(self, step, gathers, gather_blocks, n_tiles, tiles_first=False):
         if step.flush or any(g.block != step.T for g in gathers):
             raise ValueError("a fused launch needs a step kernel and gathers of one workgroup size")
-        if int(n_tiles) != -(-step.N // (step.T * step.npt)) or len(gather_blocks) != len(gathers):
+        if int(n_tiles) != -(-step.N // (step.T * step.npt // step.share)) or len(gather_blocks) != len(gathers):
             raise ValueError("the fused launch's tiles or gather workgroups do not match its kernels")
         self.step, self.gathers = step, list(gathers)
         self.gather_blocks = [int(b) for b in gather_blocks]

@@ -813,7 +813,8 @@ class Network:
             # threads per workgroup, neurons per thread; a workgroup owns a tile of block * npt neurons
             g.block = int(self.tile or (1024 if g.N >= 65536 or self._fuses_early(g, paths) else 256))
             g.npt = int(self.npt or 1)
-            g.tile = g.block * g.npt
+            g.share = self._share(g, paths)
+            g.tile = g.block * g.npt // g.share
             dmax = max([s.csr["dmin"] + s.csr["n_seg"] - 1 for s in paths if s.source is g]
                        + [s.post_delay_steps for s in paths if s.target is g and s.post_spec is not None] + [0])
             g.ring_slots = dmax + 2
@@ -911,6 +912,22 @@ class Network:
                 and any(s.target is g for s in paths) and self._gathers_concur(paths)
                 and _resident.heavy_operations([g.su, g.th, g.rs]) < 8)
 
+    def _share(self, g, paths):
+        """Threads per neuron of the tiles of a group below 65536 neurons that fuses (1, 2 or 4:
+        the most with which the tiles, one per CU, run beside the gathers' 3/8 all at once).
+
+        A tile's events are one workgroup's work, and in a volley that is what a step waits for:
+        20000 neurons (in-degree 1000) 46 us for the 18000 events of a tile of 1024 neurons, the
+        gathers 14.  us per step on average, share 1 / 2 / 4: 5500 neurons (in-degree 500) 8.1 /
+        7.4 / 7.2, 20000 10.4 / 8.1 / 7.8, 50000 (98 and 196 tiles for 2 and 4) 11.2 / 9.0 / 10.1.
+        Larger groups, of two workgroups per CU, keep tiles of 1024."""
+        if self.tile or g.N >= 65536 or not self._fuses_early(g, paths):
+            return 1
+        slots, share = self.device.n_cu * 5 // 8, 1
+        while share < 4 and -(-2 * share * g.N // _kernels.GATHER_BLOCK) <= slots:
+            share *= 2
+        return share
+
     def _monitors(self, g):
         """The group's monitors (g.smon, g.stmon, g.rmon)."""
         smon = [m for m in self.smons if m.source is g]
@@ -968,7 +985,7 @@ class Network:
         rows = [self._bit_rows(s, n_words) for s in paths]
         if any(x is None for x in rows):
             return False
-        g.block, g.npt, g.tile = 64, 1, 64
+        g.block, g.npt, g.tile, g.share = 64, 1, 64, 1
         g.val_t = self._group_value_type(paths)
         ops, fields, args = [], [], {"n_words": n_words}
         for r, ((s, sc), (first, count, bits)) in enumerate(zip(consts, rows)):
@@ -1302,7 +1319,7 @@ class Network:
                                 uses_refractory=g.uses_refractory,
                                 statemon_when=g.stmon.when if g.stmon else "start", tile=g.block, npt=g.npt,
                                 ratemon=g.rmon.range if g.rmon else None, waves_per_eu=waves,
-                                ring_parts=g.ring_parts, pull=g.pull)
+                                ring_parts=g.ring_parts, pull=g.pull, share=g.share)
 
         # two workgroups of 1024 threads per CU need at most 64 VGPRs: keep that build only
         # if the compiler fits it without spilling
@@ -1344,7 +1361,7 @@ class Network:
                              getattr(g, "lds_cap", 0), getattr(g, "val_t", "double"), flush=True,
                              uses_refractory=g.uses_refractory,
                              statemon=g.stmon.variables if end_mon else None, statemon_when="end", tile=g.block,
-                             npt=g.npt, waves_per_eu=g.waves, pull=g.pull)
+                             npt=g.npt, waves_per_eu=g.waves, pull=g.pull, share=g.share)
             g.flush_fn = D.function(F.source, F.kernel_name)
             g.flush_struct_cls = F.struct.ctypes_struct()
         else:

@@ -95,3 +95,16 @@ def test_burst_trace_bitexact_unsorted_gather_windows(case, shape, monkeypatch):
     print(f"burst case with delays >= 1, unsorted gather windows, launch shape {shape}", flush=True)
     got = device_trace(pre, post, w, d1, **shape)
     assert np.array_equal(got, exp)
+
+
+def test_burst_trace_with_threads_beyond_the_neurons(case, monkeypatch):
+    """Tiles of four threads per neuron, fused and separate (the hubs' index lists, several
+    passes and the ragged last tile included): the same traces."""
+    from brian2_amd.runtime import Network
+
+    pre, post, w, d, exp0 = case
+    exp1 = expected_trace(pre, post, w, d + 1)
+    monkeypatch.setattr(Network, "_share", lambda self, g, paths: 4)
+    for shape in ({"tile": 1024}, {"tile": 1024, "bucket_cap": 128}, {"tile": 256}):
+        assert np.array_equal(device_trace(pre, post, w, d, **shape), exp0)
+        assert np.array_equal(device_trace(pre, post, w, d + 1, **shape), exp1)

@@ -108,10 +108,12 @@ def test_store_restore_replays_bit_identically(shape):
     assert all(np.array_equal(c["G"].get(v), x) for v, x in zip(("v", "ge", "gi"), a_state))
 
 
-@pytest.mark.parametrize("n, float_t", [(5120, "double"), (5121, "double"), (7168, "float")])
+@pytest.mark.parametrize("n, float_t", [(5120, "double"), (5121, "double"), (7168, "float"), (40961, "double"),
+                                        (65535, "float")])
 def test_groups_that_fuse_below_65536(n, float_t):
-    """Beyond five tiles of 1024 a group with delays takes one launch per step: the same spikes
-    and state as separate launches of 256-thread tiles."""
+    """Beyond five tiles of 1024 a group with delays takes one launch per step, in tiles of four,
+    two or one threads per neuron: the same spikes and state as separate launches of 256-thread
+    tiles."""
     from brian2_amd import synth
 
     out = []
@@ -119,6 +121,8 @@ def test_groups_that_fuse_below_65536(n, float_t):
         c = synth.cuba_synw_network(N=n, K=70, float_t=float_t, ginh=0.4, network_options=shape)
         c["net"].run(400)
         assert (c["G"].fused is not None) == (n > 5120 and not shape)
+        if not shape:
+            assert c["G"].tile == (256 if n <= 40960 else 512)
         out.append([c["mon"].i, c["mon"].step, c["net"].n_events] + [c["G"].get(v) for v in ("v", "ge", "gi")])
     assert len(out[0][0]) > 0
     assert all(np.array_equal(a, b) for a, b in zip(*out))
