@@ -21,12 +21,12 @@ number of steps in a launch:
 A step has one barrier (the spike list is complete) and, when there were spikes,
 a second one (the counts are complete).
 """
-import ast
 import math
 import re
 
 from .codegen import ParamStruct, Renderer, source_header
 from .kernels import _rename, group_block
+from .kernels import heavy_operations as _heavy
 
 LDS_BYTES = 163840       # LDS of one CU
 STATE_REGISTERS = 80     # 32-bit registers of a thread that may hold neuron state
@@ -481,14 +481,8 @@ def lds_plan(N, words, extra=0):
 
 def heavy_operations(specs):
     """Exponentials, powers and the like in the vector code of code objects."""
-    n = 0
-    for spec in specs:
-        for st in spec.vector if spec is not None else ():
-            exprs = [e for _, e in st.get("bool_exprs") or []] or [st["expr"]]
-            n += max(sum(isinstance(x, ast.Call) and x.func.id not in ("int", "float", "abs", "timestep", "sign", "clip")
-                         or isinstance(x, ast.Pow) for x in ast.walk(ast.parse(e.strip(), mode="eval")))
-                     for e in exprs)
-    return n
+    return sum(max(_heavy(e) for e in [e for _, e in st.get("bool_exprs") or []] or [st["expr"]])
+               for spec in specs for st in (spec.vector if spec is not None else ()))
 
 
 def plain_network(net, groups, paths, summed):
@@ -520,7 +514,10 @@ class GroupStep:
     val_t      type in which the pathways' values are held before they are applied"""
 
     MAX_SYNAPSES = 1 << 25
-    MAX_HEAVY = {"double": 8192, "float": 16384}  # neurons x heavy operations of an update
+    # neurons x heavy operations of an update: where one launch per step over the whole chip is
+    # faster, and where staged launches are
+    PULL_HEAVY = {"double": 2048, "float": 7168}
+    MAX_HEAVY = {"double": 16384, "float": 36864}
 
     def __init__(self, group, scalars, pathways, val_t, n_syn, dt):
         g = group
@@ -655,6 +652,14 @@ class GroupStep:
         self.lds_bytes = self.kernel.lds_bytes(g.N, self.threads)
 
     @classmethod
+    def too_heavy(cls, groups):
+        """Whether the only group's update is rather for the whole chip (see takes)."""
+        g = groups[0] if len(groups) == 1 else None
+        if getattr(g, "su", None) is None:
+            return False
+        return g.N * heavy_operations((g.su, g.th, g.rs)) > cls.PULL_HEAVY[g.float_t]
+
+    @classmethod
     def takes(cls, net, groups, paths, summed):
         """Whether Network net is stepped this way: one group whose neurons fit a workgroup's
         registers, synapses from it onto itself without delays or variables of their own,
@@ -664,9 +669,11 @@ class GroupStep:
         chip (kernels.PulledEvents): CUBA with 500 / 4000 / 8192 neurons 0.84 / 2.2 / 3.9
         against 3.8 / 4.6 / 5.3; 8000 neurons with 19 million synapses 3.9 (in a volley one
         compute unit has all the events, hence the bound on them).  An update with
-        exponentials is throughput: COBAHH (29 of them) with 200 / 400 neurons 8.6 / 15.7
-        against 11.8 / 12.0 in fp64, with 400 / 600 neurons 6.4 / 9.3 against 8.4 / 8.4 in
-        fp32."""
+        exponentials is throughput: COBAHH (29 of them) with 100 / 200 neurons 8.1 / 8.7
+        against 6.2 / 7.4 in fp64, with 200 / 300 neurons 5.1 / 6.1 against 5.7 / 5.5 in fp32
+        (too_heavy).  Networks that cannot count their events that way (a pair with two
+        synapses) are staged otherwise: 400 / 600 neurons 15.8 / 31.8 against 22.7 / 24.2 in
+        fp64, 1000 neurons 15.7 against 22.4 in fp32."""
         if not plain_network(net, groups, paths, summed):
             return False
         g = groups[0]

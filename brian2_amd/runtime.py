@@ -833,12 +833,15 @@ class Network:
         for g in groups:
             g.incoming = [s for s in paths if s.target is g]
         self.resident = None
-        if self._build_resident(groups, paths) or self._build_targets(groups, paths):
-            self._built = True
-            return
         for g in groups:
             g.pull = None
-        self._build_pull(groups, paths)
+        # heavy updates rather over the whole chip than in one workgroup (GroupStep.takes)
+        pulled = _resident.GroupStep.too_heavy(groups) and self._build_pull(groups, paths)
+        if not pulled and (self._build_resident(groups, paths) or self._build_targets(groups, paths)):
+            self._built = True
+            return
+        if not pulled:
+            self._build_pull(groups, paths)
         # incoming pathways -> buckets
         for g in groups:
             incoming = g.incoming
@@ -972,8 +975,8 @@ class Network:
         neurons that has two synapses of a pathway.
 
         Against a launch for the group and one per pathway, us per step in fp64 / fp32: COBAHH
-        with 1000 neurons 12.2 against 24.3 / 8.4 against 22.3, 16384 neurons 14.7 against
-        34.0 / 11.5 against 32.4; CUBA with 9000 neurons 4.9 against 16.6 / 5.2 against 18.8,
+        with 1000 neurons 7.8 against 24.6 / 6.0 against 22.4, 16384 neurons 10.8 against
+        34.1 / 9.4 against 32.3; CUBA with 9000 neurons 4.9 against 16.6 / 5.2 against 18.8,
         16384 neurons 6.0 against 19.7 / 5.8 against 21.0."""
         if not _resident.plain_network(self, groups, paths, self.summed_syn) or groups[0].N > PULL_NEURONS:
             return False
@@ -985,7 +988,10 @@ class Network:
         rows = [self._bit_rows(s, n_words) for s in paths]
         if any(x is None for x in rows):
             return False
-        g.block, g.npt, g.tile, g.share = 64, 1, 64, 1
+        # the waves of a tile: one per independent heavy part of the update, four at most
+        parts = _kernels.split_update(g.su, 4) if self._reset_mode(g) != "deferred" else []
+        g.npt, g.tile, g.share = 1, 64, max(1, len(parts))
+        g.block = 64 * g.share
         g.val_t = self._group_value_type(paths)
         ops, fields, args = [], [], {"n_words": n_words}
         for r, ((s, sc), (first, count, bits)) in enumerate(zip(consts, rows)):

@@ -75,3 +75,19 @@ def test_cobahh_pulls_and_what_is_not_taken():
     for x, y in zip(got, want):
         assert np.array_equal(x, y)
     assert _run(1100, "double", paths, None, model="cobahh", twice=True)[0].pull is None
+
+
+def test_parts_of_an_update():
+    """The parts that waves may take read nothing that the update has written before, and
+    temporaries that read each other stay together."""
+    from brian2_amd.kernels import CodeSpec, split_update
+
+    def st(var, op, expr):
+        return dict(var=var, op=op, expr=expr, dtype="float64")
+
+    code = [st("a", ":=", "exp(x)"), st("b", ":=", "exp(a) + x"), st("c", ":=", "y ** 3"), st("x", "=", "b"),
+            st("d", ":=", "exp(x)"), st("e", ":=", "c + exp(z)"), st("f", ":=", "z + y"), st("y", "=", "d + e + f")]
+    spec = CodeSpec({"name": "u", "template": "stateupdate", "owner": "g", "variables": {}, "indices": {},
+                     "blocks": {"None": {"scalar": [], "vector": code, "conditional_write": {}}}})
+    assert split_update(spec, 4) == [[0, 1], [2, 5]]
+    assert split_update(spec, 1) == [[0, 1, 2, 5]]
