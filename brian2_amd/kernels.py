@@ -537,7 +537,7 @@ class NeuronKernel:
     def __init__(self, name, N, arrays, float_t, stateupdate=None, threshold=None, reset=None,
                  reset_mode="none", scalars=None, fold=None, lds_cap=0, val_t="double",
                  spikemon=None, statemon=None, flush=False, uses_refractory=False, statemon_when="start",
-                 tile=256, npt=1, ratemon=None, waves_per_eu=0, ring_parts=None, pull=None, share=1):
+                 tile=256, npt=1, ratemon=None, waves_per_eu=0, ring_parts=None, pull=None, share=1, summed=None):
         self.name = name
         self.N = N
         self.pull = pull              # PulledEvents: incoming events from the last step's spikes, or None
@@ -574,8 +574,11 @@ class NeuronKernel:
         self.share = share            # threads per neuron (npt 1): tile / share neurons
         if npt < 1 or tile * npt > 65536:
             raise ValueError("a tile holds at most 65536 neurons")
-        if share < 1 or tile % share or (share > 1 and (npt > 1 or tile // share < 64)):
+        self.summed = summed          # OwnSum: a summed variable of this group formed here, or None
+        if share < 1 or tile % share or (share > 1 and (npt > 1 or (fold and tile // share < 64))):
             raise ValueError("share divides the tile's threads, of one neuron each")
+        if summed is not None and share != 64:
+            raise ValueError("a summed variable takes a wave per neuron")
         self._build()
 
     def _block(self, tag, spec, extra_types):
@@ -605,6 +608,8 @@ class NeuronKernel:
             ps.val("stg_stride", "unsigned long long")
         if self.pull:
             self.pull.fields(ps)
+        if self.summed:
+            self.summed.fields(ps)
         if self.reset_mode == "deferred":
             ps.ptr("spiked", "unsigned char")
         ps.ptr("status", "int")
@@ -684,6 +689,8 @@ class NeuronKernel:
             k += self._split_lines() if self.parts else []
             if self.share > 1:
                 k.append("    if (threadIdx.x >= 64) return;  // the rest is the first wave's")
+        if self.summed:
+            k += self.summed.lines(T)
         if self.fold:
             fk, U, W = fold[1], fold[2], fold[3]
             # hb_tot is the same for every thread of the workgroup: a tile without events skips
@@ -774,6 +781,8 @@ class NeuronKernel:
             body.append("p.spiked[i] = 0;")
         for v, ct in self.arrays.items():
             body.append(f"p.a_{v}[i] = {v} ? 1 : 0;" if ct == "bool" else f"p.a_{v}[i] = {v};")
+        if self.summed:
+            body += [f"p.z_x_{v}[(size_t)((step + 1) & 1) * N + i] = {v};" for v in self.summed.shared]
         body.append("hb_condq[q] = hb_cond;")
         k += ["            " + x for x in body]
         k.append("        }")
@@ -1743,14 +1752,14 @@ class SummedKernel:
         ]
         reads = [f"const {ct} {v} = p.s_{v}[e];" for v, ct in syn_arrays.items()]
         reads += [f"const {var_types[n]} {n} = p.a_{n}[_presynaptic_idx];" for n in sorted(pre_reads)]
-        posts = [f"    const {var_types[n]} {n} = p.a_{n}[_postsynaptic_idx];" for n in sorted(post_reads)]
+        posts = [f"const {var_types[n]} {n} = p.a_{n}[_postsynaptic_idx];" for n in sorted(post_reads)]
         if self.lanes == 1:
             k += [
                 f"    const int j = p.t0 + (int)(blockIdx.x * {B} + threadIdx.x);",
                 "    if (j >= p.t1) return;",
                 "    const int _postsynaptic_idx = j;",
                 "    (void)_postsynaptic_idx;",
-            ] + posts + [
+            ] + ["    " + x for x in posts] + [
                 f"    {target_t} hb_acc = ({target_t})0;",
                 "    for (unsigned int k_ = p.post_ptr[j]; k_ < p.post_ptr[j + 1]; k_++) {",
                 "        const unsigned int e = p.post_syn[k_];",
@@ -1761,62 +1770,139 @@ class SummedKernel:
             k += ["        " + x for x in reads + lines]
             k += ["        hb_acc += _synaptic_var;", "    }", "    p.target[j] = hb_acc;", "}"]
         else:
-            U = self.CHUNK // 64
             k += [
                 f"    __shared__ __align__(16) {vt} s_sum[{B // 64}][{self.CHUNK}];",
                 "    const int lane = threadIdx.x & 63;",
                 "    const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));",
                 f"    const int j = p.t0 + (int)blockIdx.x * {B // 64} + wid;  // the same for the whole wave",
                 "    if (j >= p.t1) return;",
-                "    const int _postsynaptic_idx = j;",
-                "    (void)_postsynaptic_idx;",
-                "    const unsigned int lo = p.post_ptr[j], hi = p.post_ptr[j + 1];",
-            ] + posts + [
-                f"    {target_t} hb_acc = ({target_t})0;",
-                f"    for (unsigned int c_ = lo; c_ < hi; c_ += {self.CHUNK}u) {{",
-                "        // positions and sources, then the variables: loads at a clamped index, so that those",
-                "        // of a chunk are issued together (one under a condition is waited for in its branch)",
-                f"        unsigned int hb_e[{U}];",
-                f"        int hb_p[{U}];",
-                "        #pragma unroll",
-                f"        for (int u = 0; u < {U}; u++) {{",
-                "            const unsigned int q_ = c_ + u * 64u + lane;",
-                "            const unsigned int k_ = q_ < hi ? q_ : hi - 1u;",
-                "            hb_e[u] = p.post_syn[k_];",
-                "            hb_p[u] = p.post_pre[k_];",
-                "        }",
-                "        #pragma unroll",
-                f"        for (int u = 0; u < {U}; u++) {{",
-                "            const unsigned int e = hb_e[u];",
-                "            const int _idx = (int)e;",
-                "            const int _presynaptic_idx = hb_p[u];",
-                "            (void)_idx; (void)_presynaptic_idx;",
             ]
-            k += ["            " + x for x in reads + lines]
-            k += [
-                "            s_sum[wid][u * 64 + lane] = _synaptic_var;",
-                "        }",
-                "        // the wave's own LDS accesses stay in order: only the compiler must keep it",
-                "        __builtin_amdgcn_wave_barrier();",
-                f"        const unsigned int n_ = hi - c_ < {self.CHUNK}u ? hi - c_ : {self.CHUNK}u;",
-                "        unsigned int q_ = 0u;",
-                "        for (; q_ + 16u <= n_; q_ += 16u) {",
-                f"            {vt} hb_x[16];",
-                "            #pragma unroll",
-                "            for (int u = 0; u < 16; u++) hb_x[u] = s_sum[wid][q_ + u];",
-                "            #pragma unroll",
-                "            for (int u = 0; u < 16; u++) hb_acc += hb_x[u];",
-                "        }",
-                "        for (; q_ < n_; q_++) hb_acc += s_sum[wid][q_];",
-                "        __builtin_amdgcn_wave_barrier();",
-                "    }",
-                "    if (lane == 0) p.target[j] = hb_acc;",
-                "}",
-            ]
+            k += ["    " + x for x in wave_sum_lines(self.CHUNK, "p.", vt, target_t, posts, reads, lines)]
+            k += ["    if (lane == 0) p.target[j] = hb_acc;", "}"]
         self.source = "\n".join(k) + "\n"
 
     def grid(self, n_targets):
         return max(1, -(-n_targets * self.lanes // self.BLOCK))
+
+
+def wave_sum_lines(chunk, P, vt, target_t, posts, reads, lines, own=None):
+    """Lines by which a wave (lane, wid, target j) forms hb_acc, the sum over j's synapses in
+    order, through s_sum[wid][chunk] (SummedKernel).  P: prefix of the connectivity's fields;
+    posts, reads: the target's and a synapse's variables; lines: the expression; own: the
+    synapses' variables that are stored by target ({name: C type}; then no place in the
+    storage by source is read)."""
+    U = chunk // 64
+    decl = ["unsigned int hb_e[{U}];"] if own is None else [f"{ct} hb_s_{v}[{{U}}];" for v, ct in own.items()]
+    load = [f"hb_e[u] = {P}post_syn[k_];"] if own is None else [f"hb_s_{v}[u] = {P}s_{v}[k_];" for v in own]
+    at = ["const unsigned int e = hb_e[u];", "const int _idx = (int)e;", "(void)_idx;"] if own is None else []
+    return [
+        "const int _postsynaptic_idx = j;",
+        "(void)_postsynaptic_idx;",
+        f"const unsigned int lo = {P}post_ptr[j], hi = {P}post_ptr[j + 1];",
+    ] + posts + [
+        f"{target_t} hb_acc = ({target_t})0;",
+        f"for (unsigned int c_ = lo; c_ < hi; c_ += {chunk}u) {{",
+        "    // positions and sources, then the variables: loads at a clamped index, so that those",
+        "    // of a chunk are issued together (one under a condition is waited for in its branch)",
+    ] + ["    " + x.format(U=U) for x in decl] + [
+        f"    int hb_p[{U}];",
+        "    #pragma unroll",
+        f"    for (int u = 0; u < {U}; u++) {{",
+        "        const unsigned int q_ = c_ + u * 64u + lane;",
+        "        const unsigned int k_ = q_ < hi ? q_ : hi - 1u;",
+    ] + ["        " + x for x in load] + [
+        f"        hb_p[u] = {P}post_pre[k_];",
+        "    }",
+        "    #pragma unroll",
+        f"    for (int u = 0; u < {U}; u++) {{",
+    ] + ["        " + x for x in at] + [
+        "        const int _presynaptic_idx = hb_p[u];",
+        "        (void)_presynaptic_idx;",
+    ] + ["        " + x for x in reads + lines] + [
+        "        // past the end -0.0, which changes no sum",
+        f"        s_sum[wid][u * 64 + lane] = c_ + u * 64u + lane < hi ? _synaptic_var : ({vt})-0.0;",
+        "    }",
+        "    // the wave's own LDS accesses stay in order: only the compiler must keep it",
+        "    __builtin_amdgcn_wave_barrier();",
+        f"    const unsigned int n_ = hi - c_ < {chunk}u ? hi - c_ : {chunk}u;",
+        "    // sixteen at a time, the next sixteen on their way",
+        f"    {vt} hb_x[16], hb_y[16];",
+        "    #pragma unroll",
+        "    for (int u = 0; u < 16; u++) hb_x[u] = s_sum[wid][u];",
+        "    for (unsigned int q_ = 0u; q_ < n_; q_ += 32u) {",
+        "        #pragma unroll",
+        "        for (int u = 0; u < 16; u++) hb_y[u] = s_sum[wid][q_ + 16u + u];",
+        "        #pragma unroll",
+        "        for (int u = 0; u < 16; u++) hb_acc += hb_x[u];",
+        "        if (q_ + 16u >= n_) break;",
+        f"        const unsigned int z_ = q_ + 32u < {chunk}u ? q_ + 32u : 0u;",
+        "        #pragma unroll",
+        "        for (int u = 0; u < 16; u++) hb_x[u] = s_sum[wid][z_ + u];",
+        "        #pragma unroll",
+        "        for (int u = 0; u < 16; u++) hb_acc += hb_y[u];",
+        "    }",
+        "    __builtin_amdgcn_wave_barrier();",
+        "}",
+    ]
+
+
+class OwnSum:
+    """A summed variable over synapses of a group onto itself, formed in the group's own step
+    (SummedKernel's wave per target, then the neuron), so that a step is one launch.
+
+    The sources' variables are read while other workgroups write them: they come from copies of
+    the last step's values, of which there are two in turn, written with the state.  The
+    synapses' variables come from copies by target, made when a run begins.
+    MEASURED_OWNSUM"""
+
+    CHUNK = 512
+
+    def __init__(self, statements, syn_arrays, pre_reads, post_reads, var_types, target, target_t, scalars, float_t,
+                 t0, t1):
+        self.syn_arrays, self.scalars, self.target, self.target_t = syn_arrays, scalars, target, target_t
+        self.pre_reads, self.post_reads, self.var_types, self.t0, self.t1 = pre_reads, post_reads, var_types, t0, t1
+        self.shared = sorted(set(pre_reads.values()))
+        types = dict(syn_arrays)
+        types.update({n: var_types[n] for n in list(pre_reads) + list(post_reads)})
+        types.update({"_idx": "int", "_presynaptic_idx": "int", "_postsynaptic_idx": "int", "t": "double"})
+        types.update({n: ct for n, (_, ct) in scalars.items()})
+        self.code = _rename(translate_block(statements, {}, types, set(), float_t), {n: f"p.z_c_{n}" for n in scalars})
+        self.vt = types["_synaptic_var"]
+
+    def fields(self, ps):
+        ps.ptr("z_post_ptr", "unsigned int", const=True)
+        ps.ptr("z_post_pre", "int", const=True)
+        for v, ct in self.syn_arrays.items():
+            ps.ptr(f"z_s_{v}", ct, const=True)
+        for n, (_, ct) in sorted(self.scalars.items()):
+            ps.val(f"z_c_{n}", ct)
+        for n, v in sorted({v: n for n, v in self.pre_reads.items()}.items()):
+            ps.ptr(f"z_x_{n}", self.var_types[v])  # [2][N]
+
+    def lines(self, T):
+        TN = T // 64
+        reads = [f"const {ct} {v} = hb_s_{v}[u];" for v, ct in self.syn_arrays.items()]
+        reads += [f"const {self.var_types[n]} {n} = p.z_x_{v}[hb_at + _presynaptic_idx];" for n, v in sorted(self.pre_reads.items())]
+        posts = [f"const {self.var_types[n]} {n} = p.a_{v}[j];" for n, v in sorted(self.post_reads.items())]
+        k = [
+            "    {",
+            f"    __shared__ __align__(16) {self.vt} s_sum[{TN}][{self.CHUNK}];",
+            f"    __shared__ {self.target_t} s_tgt[{TN}];",
+            "    const int lane = threadIdx.x & 63;",
+            "    const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));",
+            f"    const int j = hb_tile * {TN} + wid;",
+            "    const size_t hb_at = (size_t)(step & 1) * N;",
+            f"    if (j >= {self.t0} && j < {self.t1}) {{",
+        ]
+        k += ["        " + x for x in wave_sum_lines(self.CHUNK, "p.z_", self.vt, self.target_t, posts, reads, self.code,
+                                                  own=self.syn_arrays)]
+        return k + [
+            "        if (lane == 0) s_tgt[wid] = hb_acc;",
+            "    }",
+            "    __syncthreads();",
+            f"    if ((int)threadIdx.x < {TN} && hb_i0 >= {self.t0} && hb_i0 < {self.t1}) hb_a_{self.target}[0] = s_tgt[threadIdx.x];",
+            "    }",
+        ]
 
 
 __all__ = ["CodeSpec", "NeuronKernel", "GatherKernel", "PostPathKernel", "SummedKernel", "scalar_values",

@@ -67,3 +67,40 @@ def test_summed_fold_at_the_chunk_edges(lanes, float_t, monkeypatch):
     for i, j, x in zip(pre, post, w):
         want[j] = want[j] + ft(x * np.float64(v[i] - v[j]))
     assert np.array_equal(G.get("Igap"), want)
+
+
+@pytest.mark.parametrize("n, t, float_t, when", [(20, (0, 20), "double", "start"), (257, (3, 250), "float", "end"),
+                                                 (301, (0, 301), "double", "end")])
+def test_a_groups_own_sum_equals_two_launches(n, t, float_t, when):
+    """A summed variable that the group forms in its own step: as with a launch of its own
+    (tile given), over runs in pieces, restore, state set between runs and a change of dt."""
+    from brian2_amd import Model, Network, NeuronGroup, PopulationRateMonitor, SpikeMonitor, StateMonitor, Synapses
+
+    def run(**options):
+        rng = np.random.default_rng(n)
+        m = Model.load("gap")
+        G = NeuronGroup(n, m, float_t=float_t)
+        G.v = 1.3 * rng.random(n)  # some above the threshold
+        S = Synapses(G, G[t[0]:t[1]], summed={"Igap": m.summed["Igap"]})
+        i, j = np.nonzero((rng.random((n, t[1] - t[0])) < 0.95) & (np.arange(t[1] - t[0]) != 7))
+        o = rng.permutation(len(i))
+        S.connect(i[o], j[o])
+        S.set("w", 6.0 / n * rng.random(len(i)))
+        mons = [SpikeMonitor(G), StateMonitor(G, ["v", "Igap"], record=[0, 7, n - 1], when=when), PopulationRateMonitor(G)]
+        net = Network(G, S, *mons, dt=1e-4, **options)
+        net.run(3)
+        net.run(150)
+        net.store()
+        net.run(1)
+        net.restore()
+        G.v = G.get("v")[::-1].copy()
+        net.run(70)
+        net.run(40, dt=5e-5)
+        return G, [G.get("v"), G.get("Igap"), mons[0].i, mons[0].step, mons[1].values(), mons[2].count]
+
+    G, got = run()
+    H, want = run(tile=256)
+    assert G.own_sum is not None and H.own_sum is None
+    assert len(want[2]) > 0
+    for x, y in zip(got, want):
+        assert np.array_equal(x, y)
