@@ -1691,7 +1691,7 @@ class SummedKernel:
     the values go to LDS in synapse order; then the wave adds them up one by one
     (every lane the same sum, broadcast reads).  What is left is one chain of
     three dependent loads and the chain of additions (300 neurons all-to-all: 98.2 us
-    per step with a thread per target, 8.5 with a wave, two launches a step).
+    per step with a thread per target, 8.2 with a wave, two launches a step).
     lanes = 1: a thread per target, whose loads are a chain per synapse."""
 
     BLOCK = 256
@@ -1853,7 +1853,10 @@ class OwnSum:
     The sources' variables are read while other workgroups write them: they come from copies of
     the last step's values, of which there are two in turn, written with the state.  The
     synapses' variables come from copies by target, made when a run begins.
-    MEASURED_OWNSUM"""
+
+    What bounds it: the launch, three dependent loads (1 us) and the chain of additions, whose
+    order is the result (300 neurons all-to-all: 300 additions, 1.5 us).  300 neurons: 8.2 us
+    per step with a launch of its own for the sum, 5.8 in one."""
 
     CHUNK = 512
 
