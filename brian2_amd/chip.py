@@ -1,0 +1,296 @@
+"""A network without delays over the whole chip, many steps in a launch.
+
+Networks of one group with synapses onto itself whose events carry no more than their number
+(resident.plain_network), too large or too heavy for the one workgroup of resident.py: a
+workgroup has 64 neurons, whose state its registers hold through all steps of the launch, and
+what the workgroups tell each other after a step is one word of spikes each.
+"""
+import re
+
+from .codegen import ParamStruct, source_header
+from .kernels import _rename, group_block, group_statements, identifiers, split_update
+
+SPINS = 1 << 22  # polls of the others' words before a launch gives up (seconds)
+
+
+class ChipSteps:
+    """Source of the kernel (a workgroup per 64 neurons; all of them have to run at once).
+
+    A step's word goes into the exchange as two 8-byte atomics, each a half of the word and the
+    step's number: what is read is complete or not there yet, so neither fences nor a counter are
+    needed (a barrier with fences of 63 workgroups takes 4.7 us, one with a counter 2.1).  There
+    are two places per workgroup in turn: who writes step s + 2 has read everybody's s + 1, which
+    they write when they have read s.  The words' set bits become a list of sources in LDS; a
+    lane per source loads the word of this workgroup's 64 targets from the source's row of the
+    pathway's bit matrix; a neuron's events are counted bit by bit, with the words in scalar
+    registers, and applied pathway by pathway.
+
+    waves: an update's independent heavy parts (kernels.split_update) have a wave each, which
+    hands its results to the others through LDS; all else every wave does alike, so that each
+    has the state.  An update of many exponentials is bound by the instructions that one wave
+    issues, and the other SIMDs would be idle.
+
+    What bounds it: the chain words -> rows -> update -> words.  4000 COBAHH neurons, us per
+    step: 36.8 as three launches that stage the events (29.2 with functions without branches),
+    12.8 as one launch a step that counts its events itself, 8.6 with the update's parts on
+    waves, 6.4 with all steps in a launch.
+
+    group, scalars {(tag, name): (value, ctype)}; pathways [(variable, operator, C expression
+    of the operand, first source, sources)]; consts [(field, C type)] of the operands'
+    constants; mode: when a reset happens ('fused': at once, 'deferred': after the events)"""
+
+    def __init__(self, group, scalars, pathways, consts, n_words, mode):
+        g = self.group = group
+        self.scalars, self.pathways, self.n_words = scalars, list(pathways), int(n_words)
+        NW, R = self.n_words, len(self.pathways)
+        C = -(-NW // 64)
+        parts = split_update(g.su, 4)
+        parts = parts if len(parts) > 1 else []
+        W = self.waves = max(1, len(parts))
+        ps = ParamStruct(f"hbc_{g.name}")
+        ps.val("step0", "long long")
+        ps.val("dt", "double")
+        ps.val("n_steps", "int")
+        ps.val("N", "int")
+        for v, ct in g.vars.items():
+            ps.ptr(f"a_{v}", "unsigned char" if ct == "bool" else ct)
+        for (tg, n), (_, ct) in sorted(scalars.items()):
+            ps.val(f"{tg}_{n}", ct)
+        for n, ct in consts:
+            ps.val(n, ct)
+        for r in range(R):
+            ps.ptr(f"bits{r}", "unsigned long long", const=True)  # [sources][n_words]
+            ps.ptr(f"events{r}", "unsigned long long")  # per workgroup
+        ps.ptr("xch", "unsigned long long")  # [2][n_words][2]
+        ps.ptr("status", "int")
+        if g.smon:
+            ps.ptr("mon_i", "int")
+            ps.ptr("mon_step", "int")
+            ps.ptr("mon_n", "unsigned long long")
+            ps.ptr("mon_count", "int")
+            ps.val("mon_cap", "long long")
+            ps.val("mon_start", "int")
+            ps.val("mon_stop", "int")
+        if g.rmon:
+            ps.ptr("rate_cnt", "int")
+            ps.val("rate_row0", "long long")
+            ps.val("rate_rows", "long long")
+            ps.val("rate_start", "int")
+            ps.val("rate_stop", "int")
+        if g.stmon:
+            ps.ptr("rec_idx", "int", const=True)
+            ps.ptr("rec_buf", "double")
+            ps.val("rec_row0", "long long")
+            ps.val("rec_rows", "long long")
+            ps.val("n_rec", "int")
+            ps.val("pad_rec", "int")
+        self.struct = ps
+        self.kernel_name = f"chip_{g.name}"
+
+        def block(tag, spec, extra=()):
+            return group_block(tag, spec, g.vars, scalars, g.float_t, extra)
+
+        first = "threadIdx.x < 64"
+        k = [source_header(64 * W), ps.c_decl()]
+        k.append(f'extern "C" __global__ void __launch_bounds__({64 * W}) {self.kernel_name}(const {ps.name} p) {{')
+        k += [
+            "    const int hb_lane = threadIdx.x & 63, hb_blk = blockIdx.x;",
+            "    const int hb_wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);",
+            "    const int i = hb_blk * 64 + hb_lane, N = p.N, _idx = i;",
+            "    const bool hb_act = i < N;",
+            "    const double dt = p.dt;",
+            "    (void)_idx; (void)hb_wave; (void)dt;",
+            "    __shared__ unsigned short s_src[4096];",
+            f"    __shared__ unsigned int s_cnt[2][{R}][64];",
+            "    __shared__ int s_late[2];",
+        ]
+        sts = group_statements("su", g.su, g.vars, scalars, g.float_t)
+        done = {x for w in parts for x in w}
+        read = set().union(*(identifiers([st]) for x, (st, _) in enumerate(sts) if x not in done), set())
+        handed = sorted(x for x in done if sts[x][0]["var"] in read)
+        for x in handed:
+            ct = re.match(r"(?:const )?(\w+(?: long)?) ", sts[x][1][0]).group(1)
+            k.append(f"    __shared__ {ct} s_part_{sts[x][0]['var']}[2][64];")
+        for v, ct in g.vars.items():
+            k.append(f"    {ct} {v} = hb_act ? p.a_{v}[i]{' != 0' if ct == 'bool' else ''} : ({ct})0;")
+            if ct != "bool":
+                k.append(f'    asm volatile("" : "+v"({v}));  // waited for here, not in the loop behind its stores')
+        k += [
+            f"    unsigned int hb_e[{R}];",
+            f"    for (int r = 0; r < {R}; r++) hb_e[r] = 0u;",
+            "    bool hb_cond = false, hb_ok = true;",
+        ]
+        if g.stmon:
+            k += [
+                "    int hb_rec = -1;  // this neuron's place among the recorded",
+                "    if (hb_act) {",
+                "        int lo = 0, hi = p.n_rec;",
+                "        while (lo < hi) { const int m = (lo + hi) >> 1; if (p.rec_idx[m] < i) lo = m + 1; else hi = m; }",
+                "        if (lo < p.n_rec && p.rec_idx[lo] == i) hb_rec = lo;",
+                "    }",
+            ]
+
+        def record(row):
+            nv = len(g.stmon.variables)
+            return [f"if ({first} && hb_rec >= 0 && {row} >= 0 && {row} < p.rec_rows) {{",
+                    f"    double* const o_ = p.rec_buf + (size_t)({row}) * {nv} * p.n_rec + hb_rec;"] + [
+                f"    o_[(size_t){a} * p.n_rec] = (double){v};" for a, v in enumerate(g.stmon.variables)] + ["}"]
+
+        # events of the step whose number from the launch's start, plus one, is tag
+        k += [
+            f"    auto hb_pull = [&](const unsigned int tag, unsigned int (&n)[{R}]) {{",
+            f"        const unsigned long long* const x = p.xch + (size_t)(tag & 1u) * {2 * NW};",
+            f"        unsigned long long lo[{C}], hi[{C}];",
+            "        for (int spin = 0;; spin++) {",
+            "            bool there = true;",
+            "            #pragma unroll",
+            f"            for (int c = 0; c < {C}; c++) {{",
+            f"                const int w = c * 64 + hb_lane < {NW} ? c * 64 + hb_lane : {NW - 1};",
+            "                lo[c] = __hip_atomic_load(x + 2 * w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);",
+            "                hi[c] = __hip_atomic_load(x + 2 * w + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);",
+            "            }",
+            "            #pragma unroll",
+            f"            for (int c = 0; c < {C}; c++)",
+            "                there = there && (unsigned int)(lo[c] >> 32) == tag && (unsigned int)(hi[c] >> 32) == tag;",
+            "            if (__builtin_amdgcn_ballot_w64(!there) == 0ull) break;",
+            f"            if (spin == {SPINS}) {{ hb_ok = false; if (hb_lane == 0) atomicOr(p.status, 16); break; }}",
+            "        }",
+            f"        for (int r = 0; r < {R}; r++) n[r] = 0u;",
+            "        #pragma unroll",
+            f"        for (int c = 0; c < {C}; c++) {{",
+            f"            unsigned long long w = c * 64 + hb_lane < {NW} && hb_ok ? hi[c] << 32 | (unsigned int)lo[c] : 0ull;",
+            "            if (__builtin_amdgcn_ballot_w64(w != 0ull) == 0ull) continue;",
+            "            // the chunk's sources, in order (this wave's own list: its accesses stay in order)",
+            "            const int in_ = hb_wave_incl_scan(__popcll(w));",
+            "            const int m = __builtin_amdgcn_readlane(in_, 63);",
+            "            for (int o = in_ - __popcll(w); w; w &= w - 1ull) s_src[o++] = (unsigned short)(hb_lane << 6 | __builtin_ctzll(w));",
+            "            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, \"wavefront\");",
+            "            for (int s0 = 0; s0 < m; s0 += 64) {",
+            "                const int src = s0 + hb_lane < m ? c * 4096 + (int)s_src[s0 + hb_lane < m ? s0 + hb_lane : 0] : -1;",
+        ]
+        for r, (_, _, _, a, cnt) in enumerate(self.pathways):
+            k += [
+                f"                const bool ok{r} = (unsigned int)(src - {a}) < {cnt}u;",
+                f"                const unsigned long long x{r} = p.bits{r}[ok{r} ? (size_t)(src - {a}) * {NW} + hb_blk : (size_t)0];",
+            ]
+        for r in range(R):
+            k += [
+                "                {",
+                f"                    const unsigned long long x = ok{r} ? x{r} : 0ull;",
+                f"                    hb_e[{r}] += (unsigned int)__popcll(x);",
+                "                    for (unsigned long long m = __builtin_amdgcn_ballot_w64(x != 0ull); m; m &= m - 1ull) {",
+                "                        const int l = __builtin_ctzll(m);",
+                "                        const unsigned int lo_ = (unsigned int)__builtin_amdgcn_readlane((int)x, l);",
+                "                        const unsigned int hi_ = (unsigned int)__builtin_amdgcn_readlane((int)(x >> 32), l);",
+                f"                        n[{r}] += ((hb_lane < 32 ? lo_ : hi_) >> (hb_lane & 31)) & 1u;",
+                "                    }",
+                "                }",
+            ]
+        k += [
+            "            }",
+            "            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, \"wavefront\");",
+            "        }",
+            "    };",
+            "    // the events of the step before step hb_s of the launch, applied (hb_ok: no workgroup missing)",
+            "    auto hb_events = [&](const int hb_s, const double t) {",
+            "        (void)t;",
+            f"        unsigned int hb_n[{R}];",
+        ]
+        if W > 1:
+            k += [
+                "        if (hb_wave == 0) {",
+                "            hb_pull((unsigned int)hb_s, hb_n);",
+                "            #pragma unroll",
+                f"            for (int r = 0; r < {R}; r++) s_cnt[hb_s & 1][r][hb_lane] = hb_n[r];",
+                "            if (hb_lane == 0) s_late[hb_s & 1] = hb_ok ? 0 : 1;",
+                "        }",
+                "        __syncthreads();",
+                "        #pragma unroll",
+                f"        for (int r = 0; r < {R}; r++) hb_n[r] = s_cnt[hb_s & 1][r][hb_lane];",
+                "        hb_ok = s_late[hb_s & 1] == 0;",
+            ]
+        else:
+            k.append("        hb_pull((unsigned int)hb_s, hb_n);")
+        for r, (var, op, val, _, _) in enumerate(self.pathways):
+            k.append(f"        for (unsigned int n_ = hb_n[{r}]; n_ > 0u; n_--) {var} {op} {val};")
+        if mode == "deferred":
+            k += ["        if (hb_cond) { // reset of the step before, after its propagation"]
+            k += ["            " + x for x in block("rs", g.rs)] + ["        }"]
+        k += ["    };", "    for (int hb_s = 0; hb_s < p.n_steps; hb_s++) {", "        const long long hb_step = p.step0 + hb_s;",
+              "        const double t = (double)hb_step * dt;", "        (void)t;",
+              "        if (hb_s > 0) { hb_events(hb_s, t); if (!hb_ok) return; }"]
+        if g.stmon:
+            row = "(hb_step - p.rec_row0)" if g.stmon.when == "start" else "(hb_step - 1 - p.rec_row0)"
+            k += ["        " + x for x in record(row)]
+        for w, part in enumerate(parts):
+            k.append(f"        {'else ' if w else ''}if (hb_wave == {w}) {{")
+            for x in part:
+                k += ["            " + y for y in sts[x][1]]
+                if x in handed:
+                    k.append(f"            s_part_{sts[x][0]['var']}[hb_s & 1][hb_lane] = {sts[x][0]['var']};")
+            k.append("        }")
+        if W > 1:
+            k.append("        __syncthreads();  // (two sets of results in turn: one barrier is enough)")
+        k += ["        hb_cond = false;", "        {"]
+        for x, (st, ls) in enumerate(sts):
+            if x not in done:
+                k += ["            " + y for y in ls]
+            elif x in handed:
+                k.append(f"            const auto {st['var']} = s_part_{st['var']}[hb_s & 1][hb_lane];")
+        k.append("        }")
+        if g.th is not None:
+            k += ["        {"] + ["            " + x for x in block("th", g.th, {"_cond": "bool"})]
+            k += ["            hb_cond = _cond && hb_act;", "        }"]
+            if g.uses_refractory:
+                k.append("        if (hb_cond) { not_refractory = false; lastspike = t; }")
+        if mode == "fused":
+            k += ["        if (hb_cond) {"] + ["            " + x for x in block("rs", g.rs)] + ["        }"]
+        k += [
+            "        const unsigned long long hb_w = __builtin_amdgcn_ballot_w64(hb_cond);",
+            f"        if ({first}) {{",
+            "            if (hb_lane < 2) {  // first of all: the others wait for it",
+            "                const unsigned long long x = hb_lane == 0 ? hb_w & 0xffffffffull : hb_w >> 32;",
+            f"                __hip_atomic_store(p.xch + ((size_t)((hb_s + 1) & 1) * {NW} + hb_blk) * 2 + hb_lane,",
+            "                                   (unsigned long long)(hb_s + 1) << 32 | x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);",
+            "            }",
+        ]
+        if g.smon:
+            k += [
+                "            const bool in_ = hb_cond && i >= p.mon_start && i < p.mon_stop;",
+                "            const unsigned long long m_ = __builtin_amdgcn_ballot_w64(in_);",
+                "            if (m_ != 0ull) {",
+                "                unsigned long long o_ = 0ull;",
+                "                if (hb_lane == 0) {",
+                "                    o_ = atomicAdd(p.mon_n, (unsigned long long)__popcll(m_));",
+                "                    if (o_ + (unsigned long long)__popcll(m_) > (unsigned long long)p.mon_cap) atomicOr(p.status, 2);",
+                "                }",
+                "                o_ = __shfl(o_, 0, 64) + (unsigned long long)__popcll(m_ & ((1ull << hb_lane) - 1ull));",
+                "                if (in_ && o_ < (unsigned long long)p.mon_cap) { p.mon_i[o_] = i; p.mon_step[o_] = (int)hb_step; }",
+                "                if (in_) p.mon_count[i - p.mon_start] += 1;",
+                "            }",
+            ]
+        if g.rmon:
+            k += [
+                "            const int c_ = __popcll(__builtin_amdgcn_ballot_w64(hb_cond && i >= p.rate_start && i < p.rate_stop));",
+                "            if (hb_lane == 0 && c_ && p.rate_cnt && hb_step - p.rate_row0 >= 0 && hb_step - p.rate_row0 < p.rate_rows)",
+                "                atomicAdd(&p.rate_cnt[hb_step - p.rate_row0], c_);",
+            ]
+        k += [
+            "        }",
+            "    }",
+            "    {  // the last step's events, and the state back to memory",
+            "        const long long hb_step = p.step0 + p.n_steps;",
+            "        hb_events(p.n_steps, (double)hb_step * dt);",
+            "        if (!hb_ok) return;",
+        ]
+        if g.stmon and g.stmon.when == "end":
+            k += ["        " + x for x in record("(hb_step - 1 - p.rec_row0)")]
+        k += ["    }", f"    if ({first}) {{", "        if (hb_act) {"]
+        for v, ct in g.vars.items():
+            k.append(f"            p.a_{v}[i] = {v}{' ? 1 : 0' if ct == 'bool' else ''};")
+        k.append("        }")
+        for r in range(R):
+            k += [f"        const int e{r} = __builtin_amdgcn_readlane(hb_wave_incl_scan((int)hb_e[{r}]), 63);",
+                  f"        if (hb_lane == 0) p.events{r}[hb_blk] += (unsigned long long)e{r};"]
+        k += ["    }", "}"]
+        self.source = "\n".join(k) + "\n"

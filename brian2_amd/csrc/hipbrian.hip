@@ -291,6 +291,16 @@ extern "C" int hb_launch(void* fn, unsigned grid, unsigned block, unsigned shmem
     return launch_fn((const hb_fn*)fn, grid, block, shmem, (hipStream_t)stream, args, argsize);
 }
 
+// A launch whose workgroups all run at once (they wait for each other), or an error.
+extern "C" int hb_launch_together(void* fn, unsigned grid, unsigned block, unsigned shmem, void* stream, const void* args) {
+    const hb_fn* f = (const hb_fn*)fn;
+    if (!f || !f->mfn) return set_err("hb_launch_together: not a generated kernel");
+    if (grid == 0) return 0;
+    void* argv[] = {const_cast<void*>(args)};
+    HB_HIP(hipModuleLaunchCooperativeKernel(f->mfn, grid, 1, 1, block, 1, 1, shmem, (hipStream_t)stream, argv));
+    return 0;
+}
+
 // ---------------------------------------------------------------------------
 // step plans
 // ---------------------------------------------------------------------------

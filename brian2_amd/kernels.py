@@ -492,6 +492,19 @@ def group_block(tag, spec, arrays, scalars, float_t, extra_types=(), select=Fals
     return _rename(lines, names)
 
 
+def group_statements(tag, spec, arrays, scalars, float_t):
+    """[(statement, its C lines)] of one of a group's code objects (group_block, one by one)."""
+    types = dict(arrays)
+    types.update({"t": "double", "dt": "double", "N": "int", "i": "int", "_idx": "int"})
+    names = {}
+    for (tg, n), (_, ct) in scalars.items():
+        if tg == tag:
+            types[n], names[n] = ct, f"p.{tag}_{n}"
+    declared = set()
+    return [(st, _rename(translate_block([st], spec.conditional_write, types, declared, float_t), names))
+            for st in spec.vector]
+
+
 def heavy_operations(expr):
     """Exponentials, powers and the like in an expression."""
     return sum(isinstance(x, ast.Call) and x.func.id not in ("int", "float", "abs", "timestep", "sign", "clip")
@@ -537,16 +550,9 @@ class NeuronKernel:
     def __init__(self, name, N, arrays, float_t, stateupdate=None, threshold=None, reset=None,
                  reset_mode="none", scalars=None, fold=None, lds_cap=0, val_t="double",
                  spikemon=None, statemon=None, flush=False, uses_refractory=False, statemon_when="start",
-                 tile=256, npt=1, ratemon=None, waves_per_eu=0, ring_parts=None, pull=None, share=1, summed=None):
+                 tile=256, npt=1, ratemon=None, waves_per_eu=0, ring_parts=None, share=1, summed=None):
         self.name = name
         self.N = N
-        self.pull = pull              # PulledEvents: incoming events from the last step's spikes, or None
-        if pull is not None and (tile // share != 64 or npt != 1 or fold):
-            raise ValueError("a group that pulls its events has tiles of 64 neurons and no staged events")
-        # a group that pulls its events: the update's independent parts, one of share waves each
-        self.parts = split_update(stateupdate, share) if pull is not None and share > 1 and not flush else []
-        if self.parts and (reset_mode == "deferred" or len(self.parts) != share):
-            raise ValueError("the update does not split into that many parts")
         self.arrays = arrays          # {var: ctype} of the group's state arrays
         self.float_t = float_t
         self.su, self.th, self.rs = stateupdate, threshold, reset
@@ -606,8 +612,6 @@ class NeuronKernel:
             ps.val("n_tiles", "long long")
             ps.val("tile_cap", "long long")
             ps.val("stg_stride", "unsigned long long")
-        if self.pull:
-            self.pull.fields(ps)
         if self.summed:
             self.summed.fields(ps)
         if self.reset_mode == "deferred":
@@ -650,16 +654,12 @@ class NeuronKernel:
         k.append("    const double dt = p.dt;")
         k.append("    const int N = p.N;")
         k.append("    const int hb_tile = blockIdx.x;")
-        if self.pull:
-            k.append(f"    const int hb_lane = threadIdx.x & 63, hb_i0 = hb_tile * {TN} + hb_lane;")
-        elif self.share > 1:  # the threads that only work on the events have no neuron
+        if self.share > 1:  # the threads that only work on the events have no neuron
             k.append(f"    const int hb_i0 = (int)threadIdx.x < {TN} ? hb_tile * {TN} + (int)threadIdx.x : 0x7fffffff;")
         else:
             k.append(f"    const int hb_i0 = hb_tile * {TN} + threadIdx.x;  // neuron q*{T} + hb_i0 for q < {NPT}")
         k.append("    (void)t; (void)dt;")
-        if self.pull:
-            k += self.pull.load_lines()
-        elif not self.flush:
+        if not self.flush:
             # spike counts of the workgroup (cleared here, before the first barrier)
             k += ["    __shared__ int s_nsp, s_nspm, s_nrt;", "    if (threadIdx.x == 0) { s_nsp = 0; s_nspm = 0; s_nrt = 0; }"]
             if len(self.ring_parts) > 1:
@@ -684,11 +684,6 @@ class NeuronKernel:
                 k.append(f"        hb_a_{v}[q] = act ? p.a_{v}[i] : ({ct})0;")
         k.append("        hb_condq[q] = false;")
         k.append("    }")
-        if self.pull:
-            k += self.pull.lines()
-            k += self._split_lines() if self.parts else []
-            if self.share > 1:
-                k.append("    if (threadIdx.x >= 64) return;  // the rest is the first wave's")
         if self.summed:
             k += self.summed.lines(T)
         if self.fold:
@@ -752,15 +747,7 @@ class NeuronKernel:
         if not self.flush:
             if self.su is not None:
                 body.append("{ // stateupdate")
-                if self.parts:
-                    done = {k_ for w in self.parts for k_ in w}
-                    for k_, (st, ls) in enumerate(self._statements()):
-                        if k_ not in done:
-                            body += ["    " + x for x in ls]
-                        elif k_ in self._handed:
-                            body.append(f"    const auto {st['var']} = s_part_{st['var']}[hb_lane];")
-                else:
-                    body += ["    " + x for x in self._block("su", self.su, {})]
+                body += ["    " + x for x in self._block("su", self.su, {})]
                 body.append("}")
             if self.th is not None:
                 body.append("{ // threshold")
@@ -792,9 +779,6 @@ class NeuronKernel:
         k.append("    }")
         if self.flush:
             k.append("}")
-            return "\n".join(k) + "\n"
-        if self.pull:
-            k += self._pull_spikes() + ["}"]
             return "\n".join(k) + "\n"
         # ---- spikes of this step -> ring slot (workgroup allocation + one atomic per workgroup)
         k += [
@@ -921,8 +905,6 @@ class NeuronKernel:
         """(state variables that this kernel changes, those of them only at a spike): the rest
         is not stored.  1M CUBA neurons: 66 to 58 bytes of state per neuron and step."""
         out = {var for _, var, _ in self.fold}
-        if self.pull:
-            out |= {x[0] for x in self.pull.pathways}
         if self.summed:
             out.add(self.summed.target)
         specs = [self.rs] if self.reset_mode == "deferred" or not self.flush else []
@@ -937,172 +919,6 @@ class NeuronKernel:
         if not self.flush and self.uses_refractory and self.th is not None:
             out |= {"not_refractory", "lastspike"}
         return out, out - every
-
-    def _statements(self):
-        """[(statement, its C lines)] of the state update."""
-        types = dict(self.arrays)
-        types.update({"t": "double", "dt": "double", "N": "int", "i": "int", "_idx": "int"})
-        names = {}
-        for (tg, n), (_, ct) in self.scalars.items():
-            if tg == "su":
-                types[n], names[n] = ct, f"p.su_{n}"
-        declared = set()
-        return [(st, _rename(translate_block([st], self.su.conditional_write, types, declared, self.float_t), names))
-                for st in self.su.vector]
-
-    def _split_lines(self):
-        """The update's parts (split_update), a wave each; their results to LDS for the first
-        wave, which does the rest of the step.
-
-        An update of many exponentials is bound by the instructions that one wave issues; with
-        so few neurons that a SIMD has no second wave, the other SIMDs are idle.  4000 COBAHH
-        neurons (four parts: the gates h, m, n and the voltage): 12.8 to 8.6 us per step."""
-        sts = self._statements()
-        done = {k for w in self.parts for k in w}
-        read = set()
-        for k, (st, _) in enumerate(sts):
-            if k not in done:
-                read |= identifiers([st])
-        self._handed = {k for k in done if sts[k][0]["var"] in read}
-        ct = {k: re.match(r"(?:const )?(\w+(?: long)?) ", sts[k][1][0]).group(1) for k in self._handed}
-        k = [f"    __shared__ {ct[x]} s_part_{sts[x][0]['var']}[64];" for x in sorted(self._handed)]
-        k += ["    {", "        const int hb_wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);",
-              "        const int i = hb_i0, _idx = i;", "        (void)_idx;"]
-        k += [f"        const {c} {v} = hb_a_{v}[0]; (void){v};" for v, c in self.arrays.items()]
-        for w, part in enumerate(self.parts):
-            k.append(f"        {'else ' if w else ''}if (hb_wave == {w}) {{")
-            for x in part:
-                k += ["            " + y for y in sts[x][1]]
-                if x in self._handed:
-                    k.append(f"            s_part_{sts[x][0]['var']}[hb_lane] = {sts[x][0]['var']};")
-            k.append("        }")
-        return k + ["    }", "    __syncthreads();"]
-
-    def _pull_spikes(self):
-        """The tile's spikes as a word for the next step, and to the monitors."""
-        k = [
-            "    const unsigned long long hb_w = __builtin_amdgcn_ballot_w64(hb_condq[0]);",
-            "    if (threadIdx.x == 0) p.words[(size_t)(step & 1) * gridDim.x + blockIdx.x] = hb_w;",
-        ]
-        if self.spikemon:
-            k += [
-                "    {",
-                "        const bool in_ = hb_condq[0] && hb_i0 >= p.mon_start && hb_i0 < p.mon_stop;",
-                "        const unsigned long long m_ = __builtin_amdgcn_ballot_w64(in_);",
-                "        if (m_ != 0ull) {",
-                "            unsigned long long o_ = 0ull;",
-                "            if (threadIdx.x == 0) {",
-                "                o_ = atomicAdd(p.mon_n, (unsigned long long)__popcll(m_));",
-                "                if (o_ + (unsigned long long)__popcll(m_) > (unsigned long long)p.mon_cap) atomicOr(p.status, 2);",
-                "            }",
-                "            o_ = __shfl(o_, 0, 64) + (unsigned long long)__popcll(m_ & ((1ull << threadIdx.x) - 1ull));",
-                "            if (in_ && o_ < (unsigned long long)p.mon_cap) { p.mon_i[o_] = hb_i0; p.mon_step[o_] = (int)step; }",
-                "        }",
-                "    }",
-            ]
-        if self.ratemon:
-            k += [
-                "    {",
-                "        const int n_ = __popcll(__builtin_amdgcn_ballot_w64(hb_condq[0] && hb_i0 >= p.rate_start && hb_i0 < p.rate_stop));",
-                "        if (threadIdx.x == 0 && n_ && p.rate_cnt && step - p.rate_row0 >= 0 && step - p.rate_row0 < p.rate_rows)",
-                "            atomicAdd(&p.rate_cnt[step - p.rate_row0], n_);",
-                "    }",
-            ]
-        return k
-
-
-class PulledEvents:
-    """A group's incoming events, taken by its own step from the last step's spikes.
-
-    For pathways without delay from the group onto itself whose events all carry the same
-    value: then a neuron needs only their number per pathway, and its step can count them
-    itself, so that a step is one launch.  Each wave (64 neurons) writes its spikes as a
-    word; the next step's waves make a list of the set bits in LDS, take from each source's
-    row of the pathway's bit matrix the word of their own 64 targets (a lane per source, one
-    load each), and count bit by bit with the word in scalar registers.
-
-    What bounds it: the launch, the chain words -> rows (two memory round trips), then the
-    update.  4000 COBAHH neurons: 36.8 us per step with a launch per pathway that stages the
-    events for the next step to sort and fold, 8.6 now.
-
-    pathways   [(variable, operator, C expression of the operand, first source, sources)]
-    consts     [(field, C type)] of the operands' constants
-    n_words    words of a step's spikes (tiles of the group)"""
-
-    def __init__(self, pathways, consts, n_words):
-        self.pathways, self.consts, self.n_words = list(pathways), list(consts), int(n_words)
-
-    def fields(self, ps):
-        ps.ptr("words", "unsigned long long")  # [2][n_words]: spikes of steps s % 2
-        for r in range(len(self.pathways)):
-            ps.ptr(f"bits{r}", "unsigned long long", const=True)  # [sources][n_words]
-            ps.ptr(f"events{r}", "unsigned long long")  # per tile
-        for n, ct in self.consts:
-            ps.val(n, ct)
-
-    def load_lines(self):
-        NW = self.n_words
-        C = -(-NW // 64)
-        return [
-            "    // the words of both parities before the step is known; an atomic's result aside, nothing",
-            "    // in this kernel waits for a store",
-            f"    unsigned long long hb_w0[{C}], hb_w1[{C}];",
-            "    #pragma unroll",
-            f"    for (int c = 0; c < {C}; c++) {{",
-            f"        const int w = c * 64 + hb_lane < {NW} ? c * 64 + hb_lane : {NW - 1};",
-            f"        hb_w0[c] = p.words[w]; hb_w1[c] = p.words[{NW} + w];",
-            "    }",
-        ]
-
-    def lines(self):
-        NW, R = self.n_words, len(self.pathways)
-        C = -(-NW // 64)
-        k = [
-            "    {",
-            "    __shared__ unsigned short s_src[4096];",
-            f"    unsigned int hb_n[{R}], hb_e[{R}];",
-            f"    for (int r = 0; r < {R}; r++) hb_n[r] = hb_e[r] = 0u;",
-            "    const int lane = hb_lane;",
-            "    #pragma unroll",
-            f"    for (int c = 0; c < {C}; c++) {{",
-            f"        unsigned long long w = c * 64 + lane < {NW} ? ((step - 1) & 1 ? hb_w1[c] : hb_w0[c]) : 0ull;",
-            "        if (__builtin_amdgcn_ballot_w64(w != 0ull) == 0ull) continue;",
-            "        // the chunk's sources, in order (with several waves each writes the same)",
-            "        const int in_ = hb_wave_incl_scan(__popcll(w));",
-            "        const int n = __builtin_amdgcn_readlane(in_, 63);",
-            "        for (int o = in_ - __popcll(w); w; w &= w - 1ull) s_src[o++] = (unsigned short)(lane << 6 | __builtin_ctzll(w));",
-            "        __syncthreads();",
-            "        for (int s0 = 0; s0 < n; s0 += 64) {",
-            "            const int src = s0 + lane < n ? c * 4096 + (int)s_src[s0 + lane < n ? s0 + lane : 0] : -1;",
-        ]
-        for r, (_, _, _, a, cnt) in enumerate(self.pathways):
-            k += [
-                f"            const bool ok{r} = (unsigned int)(src - {a}) < {cnt}u;",
-                f"            const unsigned long long x{r} = p.bits{r}[ok{r} ? (size_t)(src - {a}) * {NW} + blockIdx.x : (size_t)0];",
-            ]
-        for r in range(R):
-            k += [
-                "            {",
-                f"                const unsigned long long x = ok{r} ? x{r} : 0ull;",
-                f"                hb_e[{r}] += (unsigned int)__popcll(x);",
-                "                for (unsigned long long m = __builtin_amdgcn_ballot_w64(x != 0ull); m; m &= m - 1ull) {",
-                "                    const int l = __builtin_ctzll(m);",
-                "                    const unsigned int lo = (unsigned int)__builtin_amdgcn_readlane((int)x, l);",
-                "                    const unsigned int hi = (unsigned int)__builtin_amdgcn_readlane((int)(x >> 32), l);",
-                f"                    hb_n[{r}] += ((lane < 32 ? lo : hi) >> (lane & 31)) & 1u;",
-                "                }",
-                "            }",
-            ]
-        k += ["        }", "        __syncthreads();  // before the list is written again", "    }"]
-        for r, (var, op, val, _, _) in enumerate(self.pathways):
-            k += [
-                f"    for (unsigned int n_ = hb_n[{r}]; n_ > 0u; n_--) hb_a_{var}[0] {op} {val};",
-                "    {",
-                f"        const int e_ = __builtin_amdgcn_readlane(hb_wave_incl_scan((int)hb_e[{r}]), 63);",
-                f"        if (threadIdx.x == 0 && e_ > 0) p.events{r}[blockIdx.x] += (unsigned long long)e_;",
-                "    }",
-            ]
-        return k + ["    }"]
 
 
 # ---------------------------------------------------------------------------

@@ -514,9 +514,10 @@ class GroupStep:
     val_t      type in which the pathways' values are held before they are applied"""
 
     MAX_SYNAPSES = 1 << 25
-    # neurons x heavy operations of an update: where one launch per step over the whole chip is
-    # faster, and where staged launches are
-    PULL_HEAVY = {"double": 2048, "float": 7168}
+    # heavy operations of an update, and neurons x these, from which steps over the whole chip
+    # are faster; neurons x these from which staged launches are
+    CHIP_HEAVY = 8
+    CHIP_WORK = {"double": 1024, "float": 2560}
     MAX_HEAVY = {"double": 16384, "float": 36864}
 
     def __init__(self, group, scalars, pathways, val_t, n_syn, dt):
@@ -657,7 +658,8 @@ class GroupStep:
         g = groups[0] if len(groups) == 1 else None
         if getattr(g, "su", None) is None:
             return False
-        return g.N * heavy_operations((g.su, g.th, g.rs)) > cls.PULL_HEAVY[g.float_t]
+        heavy = heavy_operations((g.su, g.th, g.rs))
+        return heavy >= cls.CHIP_HEAVY or g.N * heavy > cls.CHIP_WORK[g.float_t]
 
     @classmethod
     def takes(cls, net, groups, paths, summed):
@@ -665,12 +667,14 @@ class GroupStep:
         registers, synapses from it onto itself without delays or variables of their own,
         default launch shapes, an update that one compute unit can carry.
 
-        Measured on MI355X, us per step, this step against one launch per step over the whole
-        chip (kernels.PulledEvents): CUBA with 500 / 4000 / 8192 neurons 0.84 / 2.2 / 3.9
-        against 3.8 / 4.6 / 5.3; 8000 neurons with 19 million synapses 3.9 (in a volley one
-        compute unit has all the events, hence the bound on them).  An update with
-        exponentials is throughput: COBAHH (29 of them) with 100 / 200 neurons 8.1 / 8.7
-        against 6.2 / 7.4 in fp64, with 200 / 300 neurons 5.1 / 6.1 against 5.7 / 5.5 in fp32
+        Measured on MI355X, us per step, against a launch for the group and one per pathway: CUBA
+        with 500 / 4000 / 8192 neurons 0.84 / 2.2 / 3.9 against 12.3 / 15.7 / 18.0; 8000 neurons
+        with 19 million synapses 3.9 (in a volley one compute unit has all the events, hence the
+        bound on them); over the whole chip (chip.ChipSteps) 1.7 / 3.1 / 3.8.  An update with
+        exponentials is throughput, and latency where the waves are few: COBAHH (29 of them)
+        with 20 / 100 / 400 / 1000 neurons 7.7 / 8.1 / 15.6 / 49.8 against 4.0 / 4.0 / 4.9 / 5.1
+        over the whole chip in fp64, 3.9 / 4.5 / 6.3 / 15.6 against 2.8 / 2.8 / 3.6 / 3.9 in
+        fp32: 0.2 us per heavy operation of a wave, 1.7 (fp64) and 0.5 per 1000 neurons
         (too_heavy).  Networks that cannot count their events that way (a pair with two
         synapses) are staged otherwise: 400 / 600 neurons 15.8 / 31.8 against 22.7 / 24.2 in
         fp64, 1000 neurons 15.7 against 22.4 in fp32."""

@@ -18,6 +18,7 @@ import os
 import numpy as np
 
 from . import _lib
+from . import chip as _chip
 from . import kernels as _kernels
 from . import resident as _resident
 from . import targets as _targets
@@ -834,15 +835,15 @@ class Network:
         for g in groups:
             g.incoming = [s for s in paths if s.target is g]
         self.resident = None
+        self.in_launch = None  # what runs many steps in a launch, or None
         for g in groups:
             g.pull = None
         # heavy updates rather over the whole chip than in one workgroup (GroupStep.takes)
-        pulled = _resident.GroupStep.too_heavy(groups) and self._build_pull(groups, paths)
-        if not pulled and (self._build_resident(groups, paths) or self._build_targets(groups, paths)):
+        if ((_resident.GroupStep.too_heavy(groups) and self._build_pull(groups, paths))
+                or self._build_resident(groups, paths) or self._build_targets(groups, paths)
+                or self._build_pull(groups, paths)):
             self._built = True
             return
-        if not pulled:
-            self._build_pull(groups, paths)
         for g in groups:
             g.own_sum = None
             if self._sums_itself(g, groups, paths):
@@ -851,7 +852,7 @@ class Network:
         # incoming pathways -> buckets
         for g in groups:
             incoming = g.incoming
-            if not incoming or g.pull is not None:
+            if not incoming:
                 continue
             if not isinstance(g, NeuronGroup):
                 raise NotImplementedError("pathways into a spike source")
@@ -869,7 +870,7 @@ class Network:
             g.fuse_ok = (self.fuse and self.concurrent_gathers and isinstance(g, NeuronGroup)
                          and bool(g.incoming) and g.block == _kernels.GATHER_BLOCK)
         for s in paths:
-            s.fused_into = s.target if s.target.fuse_ok or s.target.pull is not None else None
+            s.fused_into = s.target if s.target.fuse_ok else None
         # summed variables first: their updaters run in the 'groups' slot before the target's
         # state update (synapses.py:146-160, order target.order - 1)
         for s in self.summed_syn:
@@ -973,17 +974,17 @@ class Network:
             consts.append((s, sc))
         return consts
 
-    # -- groups that count their events themselves (kernels.PulledEvents) --------
+    # -- networks over the whole chip (chip.ChipSteps) ---------------------------
     def _build_pull(self, groups, paths):
-        """Sets up the only group's pulled events when the network takes them: the networks that
-        one workgroup would step, but for their size or the weight of their update, up to
-        PULL_NEURONS neurons (the bit matrices grow with their square) and with no pair of
-        neurons that has two synapses of a pathway.
+        """Builds the steps over the whole chip when the network takes them: the networks that one
+        workgroup would step, but for their size or the weight of their update, up to
+        PULL_NEURONS neurons (a workgroup of 64 per compute unit; the bit matrices grow with their
+        square) and with no pair of neurons that has two synapses of a pathway.
 
         Against a launch for the group and one per pathway, us per step in fp64 / fp32: COBAHH
-        with 1000 neurons 7.8 against 24.6 / 6.0 against 22.4, 16384 neurons 10.8 against
-        34.1 / 9.4 against 32.3; CUBA with 9000 neurons 4.9 against 16.6 / 5.2 against 18.8,
-        16384 neurons 6.0 against 19.7 / 5.8 against 21.0."""
+        with 100 neurons 4.0 against 18.2 / 2.8 against 15.0, 1000 neurons 5.1 against 24.6 /
+        3.9 against 22.5, 16384 neurons 8.6 against 33.9 / 7.8 against 32.3; CUBA with 9000
+        neurons 3.6 against 16.7 / 4.0 against 18.3."""
         if not _resident.plain_network(self, groups, paths, self.summed_syn) or groups[0].N > PULL_NEURONS:
             return False
         g = groups[0]
@@ -994,12 +995,9 @@ class Network:
         rows = [self._bit_rows(s, n_words) for s in paths]
         if any(x is None for x in rows):
             return False
-        # the waves of a tile: one per independent heavy part of the update, four at most
-        parts = _kernels.split_update(g.su, 4) if self._reset_mode(g) != "deferred" else []
-        g.npt, g.tile, g.share = 1, 64, max(1, len(parts))
-        g.block = 64 * g.share
+        self._monitors(g)
         g.val_t = self._group_value_type(paths)
-        ops, fields, args = [], [], {"n_words": n_words}
+        ops, fields, args = [], [], {}
         for r, ((s, sc), (first, count, bits)) in enumerate(zip(consts, rows)):
             c, _ = Renderer({n: ct for n, (_, ct) in sc.items()}).render(s.spec.vector[0]["expr"])
             c, = _kernels._rename([c], {n: f"p.c{r}_{n}" for n in sc})
@@ -1010,9 +1008,16 @@ class Network:
             s.events_dev = _torch().zeros(n_words, dtype=_torch().int64, device="cuda")
             s.pull_bits = bits
             args[f"bits{r}"], args[f"events{r}"] = bits.data_ptr(), s.events_dev.data_ptr()
-        g.spike_words = zeros(2 * n_words, "long long")
-        args["words"] = g.spike_words.data_ptr()
-        g.pull, g.pull_args = _kernels.PulledEvents(ops, fields, n_words), args
+        R = g.pull = _chip.ChipSteps(g, self._group_scalars(g), ops, fields, n_words, self._reset_mode(g))
+        R.xch = zeros(4 * n_words, "long long")
+        args["xch"] = R.xch.data_ptr()
+        R.args = args
+        R.fn = self.device.function(R.source, R.kernel_name)
+        R.cls = R.struct.ctypes_struct()
+        for s in paths:
+            s.fused_into = None
+        g.flush_fn = None
+        self._step_in_launches(R)
         return True
 
     @staticmethod
@@ -1037,6 +1042,19 @@ class Network:
         if int(ones[bits.view(torch.uint8).int()].sum()) != n:
             return None
         return s.src_range[0] + a, b - a, bits
+
+    def _step_in_launches(self, R):
+        """The network's steps come from R, many in a launch: its monitors, and an empty plan."""
+        g = R.group
+        if g.smon:
+            self._alloc_spike_monitor(g, g.smon)
+        if g.stmon:
+            g.stmon.rec_idx = dev(g.stmon.sorted_idx, "int")
+            g.stmon.rec_buf = None
+        self._plan = ctypes.c_void_p()
+        _lib.check(L.hb_plan_create(self.device.ctx, ptr(self.clock), ctypes.byref(self._plan)), "hb_plan_create")
+        self._launches = []
+        self.in_launch = R
 
     # -- networks that one workgroup steps (resident.GroupStep) ------------------
     def _build_resident(self, groups, paths):
@@ -1068,14 +1086,7 @@ class Network:
             s.events_dev = R.events[r:r + 1]
             s.fused_into = None
         g.flush_fn = None
-        if g.smon:
-            self._alloc_spike_monitor(g, g.smon)
-        if g.stmon:
-            g.stmon.rec_idx = dev(g.stmon.sorted_idx, "int")
-            g.stmon.rec_buf = None
-        self._plan = ctypes.c_void_p()
-        _lib.check(L.hb_plan_create(self.device.ctx, ptr(self.clock), ctypes.byref(self._plan)), "hb_plan_create")
-        self._launches = []
+        self._step_in_launches(R)
         self.resident = R
         return True
 
@@ -1112,13 +1123,27 @@ class Network:
         s.fused_into = None
         src.gen_tb, src.gen_idx = dev(src.timebins, "int"), dev(src.indices, "int")
         src.smon = src.stmon = src.rmon = src.flush_fn = g.flush_fn = None
-        if g.smon:
-            self._alloc_spike_monitor(g, g.smon)
-        self._plan = ctypes.c_void_p()
-        _lib.check(L.hb_plan_create(self.device.ctx, ptr(self.clock), ctypes.byref(self._plan)), "hb_plan_create")
-        self._launches = []
+        self._step_in_launches(R)
         self.resident = R
         return True
+
+    def _run_chip(self, n_steps):
+        """Launches the steps over the whole chip for n_steps steps on the current stream."""
+        R, g = self.in_launch, self.in_launch.group
+        v = {"step0": self.t_step, "dt": self.dt, "n_steps": n_steps, "N": g.N, "status": self.status.data_ptr(), **R.args}
+        for n in g.vars:
+            v[f"a_{n}"] = g._dev[n].data_ptr()
+        for (tg, n), (val, _) in R.scalars.items():
+            v[f"{tg}_{n}"] = val
+        v.update(self._monitor_args(g))
+        a = R.cls()
+        for name, _ in R.cls._fields_:
+            if name in v:
+                setattr(a, name, v[name])
+        R.xch.zero_()  # no step's number
+        buf = bytes(a)
+        _lib.check(L.hb_launch_together(R.fn, R.n_words, 64 * R.waves, 0, self.device.stream, buf), "steps over the chip")
+        self.clock.fill_(self.t_step + n_steps)
 
     def _run_targets(self, n_steps):
         """Launches the targets' kernel for n_steps steps on the current stream."""
@@ -1149,8 +1174,10 @@ class Network:
 
     def _run_resident(self, n_steps):
         """Launches the resident step for n_steps steps on the current stream."""
-        if isinstance(self.resident, _targets.TargetSteps):
+        if isinstance(self.in_launch, _targets.TargetSteps):
             return self._run_targets(n_steps)
+        if isinstance(self.in_launch, _chip.ChipSteps):
+            return self._run_chip(n_steps)
         R, g = self.resident, self.resident.group
         v = {"clock": self.clock.data_ptr(), "step_off": 0, "dt": self.dt, "n_steps": n_steps, "N": g.N,
              "bound": R.bound or 0.0, "row_ptr": R.row_ptr.data_ptr(), "post": R.post.data_ptr(),
@@ -1316,7 +1343,7 @@ class Network:
         D = self.device
         scalars = self._group_scalars(g)
         fold = []
-        for rank, s in enumerate(g.incoming if g.pull is None else ()):
+        for rank, s in enumerate(g.incoming):
             fold.append((rank, s.target_var, s.op))
         mode = self._reset_mode(g)
         if mode == "deferred":
@@ -1331,7 +1358,7 @@ class Network:
                                 uses_refractory=g.uses_refractory,
                                 statemon_when=g.stmon.when if g.stmon else "start", tile=g.block, npt=g.npt,
                                 ratemon=g.rmon.range if g.rmon else None, waves_per_eu=waves,
-                                ring_parts=g.ring_parts, pull=g.pull, share=g.share, summed=g.own_sum)
+                                ring_parts=g.ring_parts, share=g.share, summed=g.own_sum)
 
         # two workgroups of 1024 threads per CU need at most 64 VGPRs: keep that build only
         # if the compiler fits it without spilling
@@ -1373,7 +1400,7 @@ class Network:
                              getattr(g, "lds_cap", 0), getattr(g, "val_t", "double"), flush=True,
                              uses_refractory=g.uses_refractory,
                              statemon=g.stmon.variables if end_mon else None, statemon_when="end", tile=g.block,
-                             npt=g.npt, waves_per_eu=g.waves, pull=g.pull, share=g.share)
+                             npt=g.npt, waves_per_eu=g.waves, share=g.share)
             g.flush_fn = D.function(F.source, F.kernel_name)
             g.flush_struct_cls = F.struct.ctypes_struct()
         else:
@@ -1452,9 +1479,7 @@ class Network:
             v[f"{tg}_{n}"] = val
         if g.own_sum is not None:
             v.update(g.sum_args)
-        if g.pull is not None:
-            v.update(g.pull_args)
-        elif g.incoming:
+        if g.incoming:
             v.update(stg_rec=g.stg_rec.data_ptr(), stg_ord=g.stg_ord.data_ptr(),
                      tile_off=g.tile_off.data_ptr(), tile_cnt=g.tile_cnt.data_ptr(), n_tiles=g.n_tiles,
                      tile_cap=g.tile_cap, stg_stride=g.stg_cap)
@@ -1747,7 +1772,7 @@ class Network:
         out = [(self, "clock"), (self, "status")]
         for g in self.groups:
             out += [(g, "ring_spk"), (g, "ring_cnt")]
-            for a in ("spiked", "gen_state", "tile_cnt", "spike_words"):
+            for a in ("spiked", "gen_state", "tile_cnt"):
                 if getattr(g, a, None) is not None:
                     out.append((g, a))
             m = getattr(g, "smon", None)
@@ -2011,14 +2036,14 @@ class Network:
                 m.row0 = self.t_step
                 m.rec_buf = torch.zeros(max(n_steps, 1) * len(m.variables) * len(m.sorted_idx), dtype=torch.float64,
                                         device="cuda")
-                if self.resident is None:
+                if self.in_launch is None:
                     self._set_launch_args(g.launch_index, self._launch_args(g))
             # population rate monitors: spike counts of this run's steps
             m = getattr(g, "rmon", None)
             if m is not None and not isinstance(g, SpikeGeneratorGroup):
                 m.rows, m.row0 = n_steps, self.t_step
                 m.buf = zeros(max(n_steps, 1), "int")
-                if self.resident is None:
+                if self.in_launch is None:
                     self._set_launch_args(g.launch_index, self._launch_args(g))
         self._copy_read_state()
         done = 0
@@ -2033,7 +2058,7 @@ class Network:
                     chunk = min(chunk, self._ensure_monitor_room(g, m, gs))
             # whole graphs of gs steps, then the rest as one graph of its own length (a run
             # shorter than gs steps is still replayed from a captured graph)
-            if self.resident is not None:
+            if self.in_launch is not None:
                 k = min(chunk, RESIDENT_STEPS)
                 ev = [torch.cuda.Event(enable_timing=True) for _ in range(2)] if timing else []
                 for e in ev[:1]:
@@ -2064,9 +2089,7 @@ class Network:
                 grid = (g.N + g.tile - 1) // g.tile
                 _lib.check(L.hb_launch(g.flush_fn, grid, g.block, 0, stream, buf, len(buf)), "flush")
                 # the flushed events are not folded again by the next run
-                if getattr(g, "pull", None) is not None:
-                    g.spike_words.zero_()
-                elif getattr(g, "incoming", None):
+                if getattr(g, "incoming", None):
                     g.tile_cnt.zero_()
         for g in self.groups:
             m = getattr(g, "stmon", None)
@@ -2111,9 +2134,9 @@ class Network:
                 raise NotImplementedError("profile() of a network with a StateMonitor")
             if getattr(g, "rmon", None) is not None:
                 raise NotImplementedError("profile() of a network with a PopulationRateMonitor")
-        if self.resident is not None:
+        if self.in_launch is not None:
             self.run(n_steps, timing=True)
-            return [("resident", self.resident.group.name, self.last_run_gpu_ms)]
+            return [("resident", self.in_launch.group.name, self.last_run_gpu_ms)]
         self._copy_read_state()
         ms = (ctypes.c_float * len(self._launches))()
         _lib.check(L.hb_plan_profile(self._plan, self.device.stream, int(n_steps), ms), "hb_plan_profile")
@@ -2158,6 +2181,8 @@ class Network:
                        "list holds); build the Network with a larger bucket_mem_frac")
         if st & 2:
             msg.append("spike monitor buffer overflow")
+        if st & 16:
+            msg.append("a workgroup did not hear from the others (their launch was interrupted)")
         if st & 8:
             msg.append("synapse data names a target index outside the target group")
         return "; ".join(msg) or f"device status {st}"
@@ -2173,7 +2198,7 @@ class Network:
             ni[:n] = m.mon_i[:n]
             ns[:n] = m.mon_step[:n]
             m.mon_i, m.mon_step, m.cap = ni, ns, newcap
-            if self.resident is None:
+            if self.in_launch is None:
                 self._set_launch_args(g.launch_index, self._launch_args(g))
             free = m.cap - n
         return max(1, free // max(g.N, 1))

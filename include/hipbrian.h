@@ -83,6 +83,9 @@ int hb_code_object_spills(const void* code, size_t nbytes, int* vgpr_spills, int
  * one struct by value whose bytes are `args`). */
 int hb_launch(void* fn, unsigned grid, unsigned block, unsigned shmem, void* stream, const void* args,
               size_t argsize);
+/* The same for a kernel whose workgroups wait for each other: a cooperative launch,
+ * which runs all of them at once or fails.  Not for a captured graph. */
+int hb_launch_together(void* fn, unsigned grid, unsigned block, unsigned shmem, void* stream, const void* args);
 
 /* ---- step plans (Network.run hot loop + Clock.advance) ------------------ */
 /* A plan is the ordered list of launches of one time step.  `clock` points to a

@@ -1,5 +1,5 @@
-"""Groups whose step counts its own events from the last step's spikes
-(kernels.PulledEvents), against the staged launches (tile given), bit for bit."""
+"""Networks stepped over the whole chip, whose neurons count their own events
+(brian2_amd/chip.py), against the staged launches (tile given), bit for bit."""
 import numpy as np
 import pytest
 
