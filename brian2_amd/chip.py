@@ -8,9 +8,54 @@ what the workgroups tell each other after a step is one word of spikes each.
 import re
 
 from .codegen import ParamStruct, source_header
-from .kernels import _rename, group_block, group_statements, identifiers, split_update
+from .kernels import chain_lines, group_block, group_statements, identifiers, split_update
 
 SPINS = 1 << 22  # polls of the others' words before a launch gives up (seconds)
+
+
+def monitor_fields(ps, g):
+    """Fields of a group's monitors."""
+    if g.smon:
+        ps.ptr("mon_i", "int")
+        ps.ptr("mon_step", "int")
+        ps.ptr("mon_n", "unsigned long long")
+        ps.ptr("mon_count", "int")
+        ps.val("mon_cap", "long long")
+        ps.val("mon_start", "int")
+        ps.val("mon_stop", "int")
+    if g.rmon:
+        ps.ptr("rate_cnt", "int")
+        ps.val("rate_row0", "long long")
+        ps.val("rate_rows", "long long")
+        ps.val("rate_start", "int")
+        ps.val("rate_stop", "int")
+    if g.stmon:
+        ps.ptr("rec_idx", "int", const=True)
+        ps.ptr("rec_buf", "double")
+        ps.val("rec_row0", "long long")
+        ps.val("rec_rows", "long long")
+        ps.val("n_rec", "int")
+        ps.val("pad_rec", "int")
+
+
+def place_lines(first):
+    """The place of neuron i among the recorded ones (hb_rec, -1: not recorded)."""
+    return [
+        "int hb_rec = -1;",
+        f"if ({first}) {{",
+        "    int lo = 0, hi = p.n_rec;",
+        "    while (lo < hi) { const int m = (lo + hi) >> 1; if (p.rec_idx[m] < i) lo = m + 1; else hi = m; }",
+        "    if (lo < p.n_rec && p.rec_idx[lo] == i) hb_rec = lo;",
+        "}",
+    ]
+
+
+def record_lines(g, first, row):
+    """The recorded variables' values to row `row`, by the threads for which `first` holds."""
+    nv = len(g.stmon.variables)
+    return [f"if ({first} && hb_rec >= 0 && {row} >= 0 && {row} < p.rec_rows) {{",
+            f"    double* const o_ = p.rec_buf + (size_t)({row}) * {nv} * p.n_rec + hb_rec;"] + [
+        f"    o_[(size_t){a} * p.n_rec] = (double){v};" for a, v in enumerate(g.stmon.variables)] + ["}"]
 
 
 class ChipSteps:
@@ -63,27 +108,7 @@ class ChipSteps:
             ps.ptr(f"events{r}", "unsigned long long")  # per workgroup
         ps.ptr("xch", "unsigned long long")  # [2][n_words][2]
         ps.ptr("status", "int")
-        if g.smon:
-            ps.ptr("mon_i", "int")
-            ps.ptr("mon_step", "int")
-            ps.ptr("mon_n", "unsigned long long")
-            ps.ptr("mon_count", "int")
-            ps.val("mon_cap", "long long")
-            ps.val("mon_start", "int")
-            ps.val("mon_stop", "int")
-        if g.rmon:
-            ps.ptr("rate_cnt", "int")
-            ps.val("rate_row0", "long long")
-            ps.val("rate_rows", "long long")
-            ps.val("rate_start", "int")
-            ps.val("rate_stop", "int")
-        if g.stmon:
-            ps.ptr("rec_idx", "int", const=True)
-            ps.ptr("rec_buf", "double")
-            ps.val("rec_row0", "long long")
-            ps.val("rec_rows", "long long")
-            ps.val("n_rec", "int")
-            ps.val("pad_rec", "int")
+        monitor_fields(ps, g)
         self.struct = ps
         self.kernel_name = f"chip_{g.name}"
 
@@ -121,20 +146,7 @@ class ChipSteps:
             "    bool hb_cond = false, hb_ok = true;",
         ]
         if g.stmon:
-            k += [
-                "    int hb_rec = -1;  // this neuron's place among the recorded",
-                "    if (hb_act) {",
-                "        int lo = 0, hi = p.n_rec;",
-                "        while (lo < hi) { const int m = (lo + hi) >> 1; if (p.rec_idx[m] < i) lo = m + 1; else hi = m; }",
-                "        if (lo < p.n_rec && p.rec_idx[lo] == i) hb_rec = lo;",
-                "    }",
-            ]
-
-        def record(row):
-            nv = len(g.stmon.variables)
-            return [f"if ({first} && hb_rec >= 0 && {row} >= 0 && {row} < p.rec_rows) {{",
-                    f"    double* const o_ = p.rec_buf + (size_t)({row}) * {nv} * p.n_rec + hb_rec;"] + [
-                f"    o_[(size_t){a} * p.n_rec] = (double){v};" for a, v in enumerate(g.stmon.variables)] + ["}"]
+            k += ["    " + x for x in place_lines("hb_act")]
 
         # events of the step whose number from the launch's start, plus one, is tag
         k += [
@@ -221,7 +233,7 @@ class ChipSteps:
               "        if (hb_s > 0) { hb_events(hb_s, t); if (!hb_ok) return; }"]
         if g.stmon:
             row = "(hb_step - p.rec_row0)" if g.stmon.when == "start" else "(hb_step - 1 - p.rec_row0)"
-            k += ["        " + x for x in record(row)]
+            k += ["        " + x for x in record_lines(g, first, row)]
         for w, part in enumerate(parts):
             k.append(f"        {'else ' if w else ''}if (hb_wave == {w}) {{")
             for x in part:
@@ -284,7 +296,7 @@ class ChipSteps:
             "        if (!hb_ok) return;",
         ]
         if g.stmon and g.stmon.when == "end":
-            k += ["        " + x for x in record("(hb_step - 1 - p.rec_row0)")]
+            k += ["        " + x for x in record_lines(g, first, "(hb_step - 1 - p.rec_row0)")]
         k += ["    }", f"    if ({first}) {{", "        if (hb_act) {"]
         for v, ct in g.vars.items():
             k.append(f"            p.a_{v}[i] = {v}{' ? 1 : 0' if ct == 'bool' else ''};")
@@ -292,5 +304,209 @@ class ChipSteps:
         for r in range(R):
             k += [f"        const int e{r} = __builtin_amdgcn_readlane(hb_wave_incl_scan((int)hb_e[{r}]), 63);",
                   f"        if (hb_lane == 0) p.events{r}[hb_blk] += (unsigned long long)e{r};"]
+        k += ["    }", "}"]
+        self.source = "\n".join(k) + "\n"
+
+
+class SumSteps:
+    """Source of the kernel for a group whose only synapses are a summed variable of itself
+    (kernels.OwnSum for larger groups): a wave per neuron, all steps in a launch.
+
+    As in ChipSteps, what the workgroups tell each other goes through memory in 8-byte atomics
+    tagged with the step: here the values of the variables that the sum reads of its sources.
+    Each workgroup gathers all of them in LDS; a wave's lanes evaluate its neuron's synapses
+    (kept in registers where they fit) and the wave adds them up in order; all lanes do the
+    neuron's step alike.
+
+    What bounds it: the exchange (2.6 us: a read of all values takes 0.8 and is done three times
+    before all are there) and the chain of additions, whose order is the result (300: 1.8 us)."""
+
+    CHUNK = 512
+    WAVES = 4  # neurons of a workgroup: 300 neurons 6.0 / 5.6 / 5.9 / 8.4 us per step with 2 / 4 / 8 / 16
+    WORDS = 768
+
+    @classmethod
+    def takes(cls, n, types):
+        """Whether a group of n neurons, whose sum reads variables of these types of its sources,
+        is stepped this way: with few values to exchange, as everyone reads them all.
+
+        us per step all-to-all against a launch each, fp64 / fp32 (two words or one per neuron):
+        50 neurons 3.4 against 4.4 / 2.3 against 4.2, 150 4.1 against 5.5 / 3.3 against 5.0, 300
+        5.6 against 5.9 / 4.4 against 5.5, 500 7.5 against 7.2 / 5.7 against 6.9, 1000 13.4
+        against 11.0 / 10.2 against 10.1."""
+        return n * sum(2 if ct == "double" else 1 for ct in types) <= cls.WORDS
+
+    def __init__(self, group, scalars, own, max_degree):
+        g = self.group = group
+        self.scalars, self.own = scalars, own
+        T, CH, W = 64 * self.WAVES, self.CHUNK, self.WAVES
+        self.grid = -(-g.N // W)
+        kept = max_degree <= CH
+        words = [(v, h) for v in own.shared for h in ((0, 1) if g.vars[v] == "double" else (0,))]
+        self.n_words = len(words)
+        K = -(-g.N // T)  # neurons whose values a thread gathers
+        U = CH // 64
+        ps = ParamStruct(f"hbw_{g.name}")
+        ps.val("step0", "long long")
+        ps.val("dt", "double")
+        ps.val("n_steps", "int")
+        ps.val("N", "int")
+        for v, ct in g.vars.items():
+            ps.ptr(f"a_{v}", "unsigned char" if ct == "bool" else ct)
+        for (tg, n), (_, ct) in sorted(scalars.items()):
+            ps.val(f"{tg}_{n}", ct)
+        own.fields(ps)  # (z_x_<variable>: the values when the launch begins)
+        ps.ptr("xch", "unsigned long long")  # [2][words][N]
+        ps.ptr("status", "int")
+        monitor_fields(ps, g)
+        self.struct = ps
+        self.kernel_name = f"sums_{g.name}"
+
+        def block(tag, spec, extra=()):
+            return group_block(tag, spec, g.vars, scalars, g.float_t, extra)
+
+        first = "hb_lane == 0"
+        k = [source_header(T), ps.c_decl()]
+        k.append(f'extern "C" __global__ void __launch_bounds__({T}) {self.kernel_name}(const {ps.name} p) {{')
+        k += [
+            "    const int hb_lane = threadIdx.x & 63;",
+            "    const int hb_wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);",
+            f"    const int i = (int)blockIdx.x * {W} + hb_wave, N = p.N, _idx = i;  // the same for the wave",
+            "    const bool hb_act = i < N;",
+            "    const double dt = p.dt;",
+            "    (void)_idx; (void)dt;",
+            f"    __shared__ __align__(16) {own.vt} s_sum[{W}][{CH}];",
+        ] + [f"    __shared__ {g.vars[v]} s_x_{v}[2][{g.N}];" for v in own.shared]
+        k += ["    __shared__ int s_late[2];", "    if (threadIdx.x < 2) s_late[threadIdx.x] = 0;", "    __syncthreads();"]
+        for v, ct in g.vars.items():
+            k.append(f"    {ct} {v} = hb_act ? p.a_{v}[i]{' != 0' if ct == 'bool' else ''} : ({ct})0;")
+            if ct != "bool":
+                k.append(f'    asm volatile("" : "+v"({v}));  // waited for here, not in the loop behind its stores')
+        k += [
+            f"    const bool hb_sums = hb_act && i >= {own.t0} && i < {own.t1};",
+            "    const unsigned int hb_lo = hb_sums ? p.z_post_ptr[i] : 0u, hb_hi = hb_sums ? p.z_post_ptr[i + 1] : 0u;",
+            "    bool hb_cond = false;",
+        ]
+        sl = [f"{ct} hb_s_{v}[{U}];" for v, ct in own.syn_arrays.items()] + [f"int hb_p[{U}];"]
+        ld = ["#pragma unroll", f"for (int u = 0; u < {U}; u++) {{",
+              "    const unsigned int q_ = hb_c + u * 64u + hb_lane, k_ = q_ < hb_hi ? q_ : hb_hi - 1u;"]
+        ld += [f"    hb_s_{v}[u] = p.z_s_{v}[k_];" for v in own.syn_arrays] + ["    hb_p[u] = p.z_post_pre[k_];", "}"]
+        if kept:
+            k += ["    " + x for x in sl]
+            k += ["    if (hb_hi > hb_lo) {", "        const unsigned int hb_c = hb_lo;"] + ["        " + x for x in ld] + ["    }"]
+        if g.stmon:
+            k += ["    " + x for x in place_lines("hb_act")]
+        k += [
+            "    for (int hb_s = 0; hb_s < p.n_steps; hb_s++) {",
+            "        const long long hb_step = p.step0 + hb_s;",
+            "        const double t = (double)hb_step * dt;",
+            "        (void)t;",
+            "        // the sources' values: of the launch's beginning, or of the step before",
+            "        if (hb_s == 0) {",
+            f"            for (int x = threadIdx.x; x < {g.N}; x += {T}) {{",
+        ] + [f"                s_x_{v}[0][x] = p.z_x_{v}[x];" for v in own.shared] + [
+            "            }",
+            "        } else {",
+            f"            const unsigned long long* const x = p.xch + (size_t)(hb_s & 1) * {len(words) * g.N};",
+            f"            unsigned long long hb_v[{K}][{len(words)}];",
+            "            for (int spin = 0;; spin++) {",
+            "                bool there = true;",
+            "                #pragma unroll",
+            f"                for (int c = 0; c < {K}; c++) {{",
+            f"                    const int j = c * {T} + (int)threadIdx.x < {g.N} ? c * {T} + (int)threadIdx.x : {g.N - 1};",
+            "                    #pragma unroll",
+            f"                    for (int h = 0; h < {len(words)}; h++) {{",
+            f"                        hb_v[c][h] = __hip_atomic_load(x + h * {g.N} + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);",
+            "                    }",
+            "                }",
+            "                #pragma unroll",
+            f"                for (int c = 0; c < {K}; c++)",
+            "                    #pragma unroll",
+            f"                    for (int h = 0; h < {len(words)}; h++) there = there && (int)(hb_v[c][h] >> 32) == hb_s;",
+            "                if (__builtin_amdgcn_ballot_w64(!there) == 0ull) break;",
+            f"                if (spin == {SPINS}) {{ if (hb_lane == 0) {{ s_late[hb_s & 1] = 1; atomicOr(p.status, 16); }} break; }}",
+            "            }",
+            "            #pragma unroll",
+            f"            for (int c = 0; c < {K}; c++) {{",
+            f"                const int j = c * {T} + (int)threadIdx.x;",
+            f"                if (j < {g.N}) {{",
+        ]
+        at = {x: n for n, x in enumerate(words)}
+        for v in own.shared:
+            if g.vars[v] == "double":
+                k.append(f"                    s_x_{v}[hb_s & 1][j] = __builtin_bit_cast(double, hb_v[c][{at[(v, 1)]}] << 32 | "
+                         f"(unsigned int)hb_v[c][{at[(v, 0)]}]);")
+            else:
+                k.append(f"                    s_x_{v}[hb_s & 1][j] = __builtin_bit_cast(float, (unsigned int)hb_v[c][{at[(v, 0)]}]);")
+        k += [
+            "                }",
+            "            }",
+            "        }",
+            "        __syncthreads();  // (two sets of values in turn: one barrier is enough)",
+            "        if (s_late[hb_s & 1] != 0) return;",
+            "        if (hb_sums) {",
+            f"            {own.target_t} hb_acc = ({own.target_t})0;",
+            f"            for (unsigned int hb_c = hb_lo; hb_c < hb_hi; hb_c += {CH}u) {{",
+        ]
+        if not kept:
+            k += ["                " + x for x in sl + ld]
+        k += ["                #pragma unroll", f"                for (int u = 0; u < {U}; u++) {{",
+              "                    const int _presynaptic_idx = hb_p[u], _postsynaptic_idx = i;",
+              "                    (void)_presynaptic_idx; (void)_postsynaptic_idx;"]
+        k += [f"                    const {ct} {v} = hb_s_{v}[u];" for v, ct in own.syn_arrays.items()]
+        k += [f"                    const {own.var_types[n]} {n} = s_x_{v}[hb_s & 1][_presynaptic_idx];"
+              for n, v in sorted(own.pre_reads.items())]
+        k += [f"                    const {own.var_types[n]} {n} = {v};" for n, v in sorted(own.post_reads.items())]
+        k += ["                    " + x for x in own.code]
+        k += [
+            "                    // past the end -0.0, which changes no sum",
+            f"                    s_sum[hb_wave][u * 64 + hb_lane] = hb_c + u * 64u + hb_lane < hb_hi ? _synaptic_var : ({own.vt})-0.0;",
+            "                }",
+        ]
+        k += ["                " + x for x in chain_lines(CH, own.vt, "hb_wave", f"(hb_hi - hb_c < {CH}u ? hb_hi - hb_c : {CH}u)")]
+        k += ["            }", f"            {own.target} = hb_acc;", "        }"]
+        if g.stmon:
+            row = "(hb_step - p.rec_row0)" if g.stmon.when == "start" else "(hb_step - 1 - p.rec_row0)"
+            rec = ["        " + x for x in record_lines(g, first, row)]
+            k += rec
+        k += ["        hb_cond = false;", "        {"] + ["            " + x for x in block("su", g.su)] + ["        }"]
+        if g.th is not None:
+            k += ["        {"] + ["            " + x for x in block("th", g.th, {"_cond": "bool"})]
+            k += ["            hb_cond = _cond && hb_act;", "        }"]
+            if g.uses_refractory:
+                k.append("        if (hb_cond) { not_refractory = false; lastspike = t; }")
+        if g.rs is not None:
+            k += ["        if (hb_cond) {"] + ["            " + x for x in block("rs", g.rs)] + ["        }"]
+        k += ["        if (hb_lane == 0 && hb_act) {  // first of all: the others wait for it",
+              f"            unsigned long long* const hb_o = p.xch + (size_t)((hb_s + 1) & 1) * {len(words) * g.N} + i;",
+              "            const unsigned long long hb_tag = (unsigned long long)(hb_s + 1) << 32;"]
+        for n, (v, h) in enumerate(words):
+            if g.vars[v] == "double":
+                bits = f"(__builtin_bit_cast(unsigned long long, {v}) {'>> 32' if h else '& 0xffffffffull'})"
+            else:
+                bits = f"__builtin_bit_cast(unsigned int, {v})"
+            k.append(f"            __hip_atomic_store(hb_o + {n * g.N}, hb_tag | {bits}, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);")
+        if g.smon:
+            k += [
+                "            if (hb_cond && i >= p.mon_start && i < p.mon_stop) {",
+                "                const unsigned long long o_ = atomicAdd(p.mon_n, 1ull);",
+                "                if (o_ < (unsigned long long)p.mon_cap) { p.mon_i[o_] = i; p.mon_step[o_] = (int)hb_step; }",
+                "                else atomicOr(p.status, 2);",
+                "                p.mon_count[i - p.mon_start] += 1;",
+                "            }",
+            ]
+        if g.rmon:
+            k += [
+                "            if (hb_cond && i >= p.rate_start && i < p.rate_stop && p.rate_cnt && hb_step - p.rate_row0 >= 0 && "
+                "hb_step - p.rate_row0 < p.rate_rows)",
+                "                atomicAdd(&p.rate_cnt[hb_step - p.rate_row0], 1);",
+            ]
+        k += ["        }", "    }"]
+        if g.stmon and g.stmon.when == "end":
+            k += ["    {", "        const long long hb_step = p.step0 + p.n_steps;"]
+            k += ["        " + x for x in record_lines(g, first, "(hb_step - 1 - p.rec_row0)")] + ["    }"]
+        k += ["    if (hb_lane == 0 && hb_act) {"]
+        for v, ct in g.vars.items():
+            k.append(f"        p.a_{v}[i] = {v}{' ? 1 : 0' if ct == 'bool' else ''};")
         k += ["    }", "}"]
         self.source = "\n".join(k) + "\n"

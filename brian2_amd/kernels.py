@@ -1625,6 +1625,33 @@ class SummedKernel:
         return max(1, -(-n_targets * self.lanes // self.BLOCK))
 
 
+def chain_lines(chunk, vt, wid, n):
+    """Lines that add the first n of s_sum[wid][chunk] to hb_acc, one by one (every lane the same;
+    behind them up to a multiple of 32: values that change no sum)."""
+    return [
+        "// the wave's own LDS accesses stay in order: only the compiler must keep it",
+        "__builtin_amdgcn_wave_barrier();",
+        f"const unsigned int n_ = {n};",
+        "// sixteen at a time, the next sixteen on their way",
+        f"{vt} hb_x[16], hb_y[16];",
+        "#pragma unroll",
+        f"for (int u = 0; u < 16; u++) hb_x[u] = s_sum[{wid}][u];",
+        "for (unsigned int q_ = 0u; q_ < n_; q_ += 32u) {",
+        "    #pragma unroll",
+        f"    for (int u = 0; u < 16; u++) hb_y[u] = s_sum[{wid}][q_ + 16u + u];",
+        "    #pragma unroll",
+        "    for (int u = 0; u < 16; u++) hb_acc += hb_x[u];",
+        "    if (q_ + 16u >= n_) break;",
+        f"    const unsigned int z_ = q_ + 32u < {chunk}u ? q_ + 32u : 0u;",
+        "    #pragma unroll",
+        f"    for (int u = 0; u < 16; u++) hb_x[u] = s_sum[{wid}][z_ + u];",
+        "    #pragma unroll",
+        "    for (int u = 0; u < 16; u++) hb_acc += hb_y[u];",
+        "}",
+        "__builtin_amdgcn_wave_barrier();",
+    ]
+
+
 def wave_sum_lines(chunk, P, vt, target_t, posts, reads, lines, own=None):
     """Lines by which a wave (lane, wid, target j) forms hb_acc, the sum over j's synapses in
     order, through s_sum[wid][chunk] (SummedKernel).  P: prefix of the connectivity's fields;
@@ -1662,26 +1689,7 @@ def wave_sum_lines(chunk, P, vt, target_t, posts, reads, lines, own=None):
         "        // past the end -0.0, which changes no sum",
         f"        s_sum[wid][u * 64 + lane] = c_ + u * 64u + lane < hi ? _synaptic_var : ({vt})-0.0;",
         "    }",
-        "    // the wave's own LDS accesses stay in order: only the compiler must keep it",
-        "    __builtin_amdgcn_wave_barrier();",
-        f"    const unsigned int n_ = hi - c_ < {chunk}u ? hi - c_ : {chunk}u;",
-        "    // sixteen at a time, the next sixteen on their way",
-        f"    {vt} hb_x[16], hb_y[16];",
-        "    #pragma unroll",
-        "    for (int u = 0; u < 16; u++) hb_x[u] = s_sum[wid][u];",
-        "    for (unsigned int q_ = 0u; q_ < n_; q_ += 32u) {",
-        "        #pragma unroll",
-        "        for (int u = 0; u < 16; u++) hb_y[u] = s_sum[wid][q_ + 16u + u];",
-        "        #pragma unroll",
-        "        for (int u = 0; u < 16; u++) hb_acc += hb_x[u];",
-        "        if (q_ + 16u >= n_) break;",
-        f"        const unsigned int z_ = q_ + 32u < {chunk}u ? q_ + 32u : 0u;",
-        "        #pragma unroll",
-        "        for (int u = 0; u < 16; u++) hb_x[u] = s_sum[wid][z_ + u];",
-        "        #pragma unroll",
-        "        for (int u = 0; u < 16; u++) hb_acc += hb_y[u];",
-        "    }",
-        "    __builtin_amdgcn_wave_barrier();",
+    ] + ["    " + x for x in chain_lines(chunk, vt, "wid", f"(hi - c_ < {chunk}u ? hi - c_ : {chunk}u)")] + [
         "}",
     ]
 

@@ -837,15 +837,14 @@ class Network:
         self.resident = None
         self.in_launch = None  # what runs many steps in a launch, or None
         for g in groups:
-            g.pull = None
+            g.pull = g.own_sum = None
         # heavy updates rather over the whole chip than in one workgroup (GroupStep.takes)
         if ((_resident.GroupStep.too_heavy(groups) and self._build_pull(groups, paths))
                 or self._build_resident(groups, paths) or self._build_targets(groups, paths)
-                or self._build_pull(groups, paths)):
+                or self._build_pull(groups, paths) or self._build_sums(groups, paths)):
             self._built = True
             return
         for g in groups:
-            g.own_sum = None
             if self._sums_itself(g, groups, paths):
                 g.block, g.npt, g.tile, g.share = 256, 1, 4, 64
                 g.own_sum = True  # (built with its synapses)
@@ -1009,6 +1008,7 @@ class Network:
             s.pull_bits = bits
             args[f"bits{r}"], args[f"events{r}"] = bits.data_ptr(), s.events_dev.data_ptr()
         R = g.pull = _chip.ChipSteps(g, self._group_scalars(g), ops, fields, n_words, self._reset_mode(g))
+        R.grid, R.threads = n_words, 64 * R.waves
         R.xch = zeros(4 * n_words, "long long")
         args["xch"] = R.xch.data_ptr()
         R.args = args
@@ -1130,6 +1130,9 @@ class Network:
     def _run_chip(self, n_steps):
         """Launches the steps over the whole chip for n_steps steps on the current stream."""
         R, g = self.in_launch, self.in_launch.group
+        if isinstance(R, _chip.SumSteps):
+            for v, t in g.copies.items():
+                t[: g.N].copy_(g._dev[v])
         v = {"step0": self.t_step, "dt": self.dt, "n_steps": n_steps, "N": g.N, "status": self.status.data_ptr(), **R.args}
         for n in g.vars:
             v[f"a_{n}"] = g._dev[n].data_ptr()
@@ -1142,7 +1145,7 @@ class Network:
                 setattr(a, name, v[name])
         R.xch.zero_()  # no step's number
         buf = bytes(a)
-        _lib.check(L.hb_launch_together(R.fn, R.n_words, 64 * R.waves, 0, self.device.stream, buf), "steps over the chip")
+        _lib.check(L.hb_launch_together(R.fn, R.grid, R.threads, 0, self.device.stream, buf), "steps over the chip")
         self.clock.fill_(self.t_step + n_steps)
 
     def _run_targets(self, n_steps):
@@ -1176,7 +1179,7 @@ class Network:
         """Launches the resident step for n_steps steps on the current stream."""
         if isinstance(self.in_launch, _targets.TargetSteps):
             return self._run_targets(n_steps)
-        if isinstance(self.in_launch, _chip.ChipSteps):
+        if isinstance(self.in_launch, (_chip.ChipSteps, _chip.SumSteps)):
             return self._run_chip(n_steps)
         R, g = self.resident, self.resident.group
         v = {"clock": self.clock.data_ptr(), "step_off": 0, "dt": self.dt, "n_steps": n_steps, "N": g.N,
@@ -1649,13 +1652,15 @@ class Network:
         variables, and the synapses' by target."""
         for g in self.groups:
             if getattr(g, "own_sum", None) is not None:
-                for v, t in g.copies.items():
-                    t.view(2, g.N)[self.t_step & 1].copy_(g._dev[v])
+                if self.in_launch is None:
+                    for v, t in g.copies.items():
+                        t.view(2, g.N)[self.t_step & 1].copy_(g._dev[v])
                 c = self.summed_syn[0].csr
                 for n, t in g.by_target.items():
                     _torch().index_select(c["syn"][n], 0, c["post_syn"], out=t)
 
-    def _build_summed(self, s):
+    @staticmethod
+    def _check_summed(net, s):
         g = s.target
         for tv, (pre_r, post_r) in s.summed_reads.items():
             for grp, names in ((s.source, pre_r), (g, post_r)):
@@ -1664,12 +1669,59 @@ class Network:
                         raise ValueError(f"summed variable of {s.name} reads {gv!r}, not a variable of {grp.name}")
                     # the fold of a step's events and deferred resets happen at the start of the next
                     # group update: a summed variable computed before it would read stale values
-                    if any(p.target is grp and p.target_var == gv for p in self.paths) or (
-                            self._reset_mode(grp) == "deferred"):
+                    if any(p.target is grp and p.target_var == gv for p in net.paths) or (
+                            net._reset_mode(grp) == "deferred"):
                         raise NotImplementedError(f"summed variable reading {gv!r}, which synapses or a deferred "
                                                   "reset also update")
-            if any(p.target is g and p.target_var == tv for p in self.paths):
+            if any(p.target is g and p.target_var == tv for p in net.paths):
                 raise NotImplementedError(f"{tv!r} is both a summed variable and the target of a pathway")
+
+    def _make_own_sum(self, s):
+        """The group's own sum s (kernels.OwnSum) with what its fields hold."""
+        g = s.target
+        (tv, sp), (pre_r, post_r) = next(iter(s.summed.items())), next(iter(s.summed_reads.values()))
+        var_types = {n: g.vars[gv] for x in (pre_r, post_r) for n, gv in x.items()}
+        used = {n: ct for n, ct in s.syn_ctypes().items() if n in identifiers(sp.vector)}
+        host = {"dt": self.dt}
+        host.update(getattr(s, "namespace", {}) or {})
+        sc = scalar_values(sp, host, g.float_t)
+        g.own_sum = OwnSum(sp.vector, used, pre_r, post_r, var_types, tv, g.vars[tv], sc, g.float_t, *s.tgt_range)
+        g.copies = {gv: zeros(2 * g.N, g.vars[gv]) for gv in g.own_sum.shared}
+        g.by_target = {n: _torch().empty_like(s.csr["syn"][n]) for n in used}
+        g.sum_args = {f"z_x_{gv}": t.data_ptr() for gv, t in g.copies.items()}
+        g.sum_args.update({f"z_{n}": s.csr[n].data_ptr() for n in ("post_ptr", "post_pre")})
+        g.sum_args.update({f"z_s_{n}": t.data_ptr() for n, t in g.by_target.items()})
+        g.sum_args.update({f"z_c_{n}": val for n, (val, _) in sc.items()})
+
+    def _build_sums(self, groups, paths):
+        """Builds the steps of a group that is a summed variable of itself, many in a launch
+        (chip.SumSteps), when the network takes them."""
+        g = groups[0]
+        if not self._sums_itself(g, groups, paths) or g.su is None:
+            return False
+        s = self.summed_syn[0]
+        pre_r = next(iter(s.summed_reads.values()))[0]
+        if not _chip.SumSteps.takes(g.N, [g.vars[v] for v in set(pre_r.values())]):
+            return False
+        self._check_summed(self, s)
+        self._monitors(g)
+        self._make_own_sum(s)
+        ptr_ = s.csr["post_ptr"].long()
+        R = _chip.SumSteps(g, self._group_scalars(g), g.own_sum, int((ptr_[1:] - ptr_[:-1]).max()))
+        R.xch = zeros(2 * R.n_words * g.N, "long long")
+        R.args = {"xch": R.xch.data_ptr(), **g.sum_args}
+        R.fn = self.device.function(R.source, R.kernel_name)
+        R.cls = R.struct.ctypes_struct()
+        R.threads = 64 * R.WAVES
+        g.flush_fn = None
+        self._step_in_launches(R)
+        return True
+
+    def _build_summed(self, s):
+        g = s.target
+        self._check_summed(self, s)
+        if g.own_sum is not None:
+            return self._make_own_sum(s)
         s.summed_kernels = []
         types_syn = s.syn_ctypes()
         for tv, sp in sorted(s.summed.items()):
@@ -1681,15 +1733,6 @@ class Network:
             host.update(getattr(s, "namespace", {}) or {})
             sc = scalar_values(sp, host, g.float_t)
             t0, t1 = s.tgt_range
-            if g.own_sum is not None:
-                g.own_sum = OwnSum(sp.vector, used, pre_r, post_r, var_types, tv, g.vars[tv], sc, g.float_t, t0, t1)
-                g.copies = {gv: zeros(2 * g.N, g.vars[gv]) for gv in g.own_sum.shared}
-                g.sum_args = {f"z_x_{gv}": t.data_ptr() for gv, t in g.copies.items()}
-                g.sum_args.update({f"z_{n}": s.csr[n].data_ptr() for n in ("post_ptr", "post_pre")})
-                g.by_target = {n: _torch().empty_like(s.csr["syn"][n]) for n in used}
-                g.sum_args.update({f"z_s_{n}": t.data_ptr() for n, t in g.by_target.items()})
-                g.sum_args.update({f"z_c_{n}": val for n, (val, _) in sc.items()})
-                continue
             K = SummedKernel(f"{s.name}_{tv}", sp.vector, used, pre_r, post_r, var_types, g.vars[tv], sc, g.float_t,
                              lanes=SummedKernel.lanes_for(s.csr["n_syn"], t1 - t0))
             fn = self.device.function(K.source, K.kernel_name)

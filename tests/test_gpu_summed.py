@@ -104,3 +104,42 @@ def test_a_groups_own_sum_equals_two_launches(n, t, float_t, when):
     assert len(want[2]) > 0
     for x, y in zip(got, want):
         assert np.array_equal(x, y)
+
+
+@pytest.mark.parametrize("n, t, float_t, when", [(1, (0, 1), "double", "start"), (20, (0, 20), "float", "end"),
+                                                 (257, (3, 250), "double", "end"), (384, (0, 384), "double", "start"),
+                                                 (385, (0, 385), "double", "end"), (768, (0, 768), "float", "start")])
+def test_own_sums_in_a_launch_and_launch_by_launch(n, t, float_t, when, monkeypatch):
+    """All steps in a launch (up to 768 words, synapses in registers up to 512 a target), the group's
+    own sum launch by launch and a launch for the sum: the same."""
+    from brian2_amd import Model, Network, NeuronGroup, SpikeMonitor, StateMonitor, Synapses, chip
+    from brian2_amd.kernels import SummedKernel
+
+    monkeypatch.setattr(SummedKernel, "lanes_for", staticmethod(lambda n_syn, n_tgt: 64))
+
+    def run(**options):
+        rng = np.random.default_rng(n)
+        m = Model.load("gap")
+        G = NeuronGroup(n, m, float_t=float_t)
+        G.v = 1.3 * rng.random(n)
+        S = Synapses(G, G[t[0]:t[1]], summed={"Igap": m.summed["Igap"]})
+        i, j = np.nonzero(rng.random((n, t[1] - t[0])) < 0.97)
+        S.connect(i, j)
+        S.set("w", 6.0 / n * rng.random(len(i)))
+        mons = [SpikeMonitor(G), StateMonitor(G, ["v", "Igap"], record=sorted({0, n - 1}), when=when)]
+        net = Network(G, S, *mons, dt=1e-4, **options)
+        net.run(1)
+        net.run(90)
+        net.run(30, dt=5e-5)
+        return net, [G.get("v"), G.get("Igap"), mons[0].i, mons[0].step, mons[1].values()]
+
+    a, got = run()
+    assert (a.in_launch is not None) == (n != 385)
+    b, want = run(tile=256)
+    assert b.in_launch is None
+    monkeypatch.setattr(chip.SumSteps, "takes", classmethod(lambda *x: False))
+    c, alone = run()
+    assert c.in_launch is None and c.groups[0].own_sum is not None
+    assert n == 1 or len(want[2]) > 0
+    for x, y, z in zip(got, want, alone):
+        assert np.array_equal(x, y) and np.array_equal(z, y)
