@@ -138,6 +138,21 @@ def zeros(n, ct):
     return _torch().zeros(max(int(n), 1), dtype=torch_dtype(ct), device="cuda")
 
 
+def copy_all(pairs):
+    """Device tensors (to, from): the small ones of a type in one launch (fifteen of a small network
+    31 us against 89 with a launch each), the others, whose time is their bytes', one by one."""
+    by = {}
+    for to, fr in pairs:
+        if to.numel() > 1 << 15:
+            to.copy_(fr)
+            continue
+        tos, frs = by.setdefault(to.dtype, ([], []))
+        tos.append(to)
+        frs.append(fr)
+    for tos, frs in by.values():
+        _torch()._foreach_copy_(tos, frs)
+
+
 def ptr(t):
     return ctypes.c_void_p(t.data_ptr()) if t is not None else ctypes.c_void_p(0)
 
@@ -1860,12 +1875,12 @@ class Network:
     def restore(self, name="default"):
         """Returns the network to the state kept by store(name)."""
         snap = self._stored[name]
-        for o, a in self._mutable():
-            (o[a] if isinstance(o, dict) else getattr(o, a)).copy_(snap["tensors"][(id(o), a)])
+        pairs = [(o[a] if isinstance(o, dict) else getattr(o, a), snap["tensors"][(id(o), a)]) for o, a in self._mutable()]
         for g in self.groups:
             if isinstance(g, NeuronGroup):
-                for n, t in g._dev.items():
-                    t.copy_(snap["state"][id(g)][n])
+                pairs += [(t, snap["state"][id(g)][n]) for n, t in g._dev.items()]
+        copy_all(pairs)
+        for g in self.groups:
             m = getattr(g, "smon", None)
             if m is not None:
                 i, s, t, d = snap["monitors"][id(m)]
