@@ -183,11 +183,12 @@ class LIFNetwork:
 
     # ------------------------------------------------------------------ kernels
     def _shape(self):
-        """Threads of a trial's workgroup and neurons per thread: eight waves at most, two per
-        SIMD.  1000 neurons, 2000 steps with 4 / 8 / 16 waves, ms: 256 trials forward 2.08 /
-        2.00 / 2.15, backward 4.28 / 4.04 / 4.02; 9 trials, double weights, 600 steps forward
-        0.61 / 0.53 / 0.50, backward 0.99 / 0.93 / 0.84."""
-        self.block = 64 * min(8, -(-self.N // 64))
+        """Threads of a trial's workgroup and neurons per thread: eight waves at most with float
+        weights, sixteen with double ones, whose rows are twice the loads of a thread.  500
+        steps forward and backward with 4 / 8 / 16 waves, ms: float weights, 9 trials of 1000
+        neurons 1.53 / 1.39 / 1.40, 256 trials 1.53 / 1.41 / 1.44; double weights, 9 trials of
+        777 neurons 1.65 / 1.48 / 1.37, 256 trials of 1000 1.82 / 1.66 / 1.56."""
+        self.block = 64 * min(8 if self.wt == "float" else 16, -(-self.N // 64))
         self.per_thread = -(-self.N // self.block)
         # steps of a block of the backward pass: what its LDS holds (16 bytes per neuron and step,
         # 2 per possible event), a raster word per thread, at most 8
