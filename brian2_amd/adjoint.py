@@ -28,8 +28,9 @@ dt*dt/du, dt*dt/dv at the crossing step; lam_v = A lam_u, lam_I = B lam_u +
 beta lam_I'; weight gradients are event-based: dL/dw_ij += lam_I'_j at every
 step where source i spiked.  Spikes themselves carry no gradient (a
 perturbation that creates or deletes no spike leaves them unchanged).  The
-state is checkpointed every `ckpt_every` steps; the backward pass recomputes
-each segment forward from its checkpoint, then walks it in reverse.  Weight
+state is kept at the start of every block of a few steps (runs whose states
+would take more than KEEP_BYTES: every `ckpt_every` steps); the backward pass
+recomputes a block forward from there, then walks it in reverse.  Weight
 gradients accumulate per trial (no atomics) and are summed over trials in a
 fixed order.
 """
@@ -49,6 +50,7 @@ S_RATE, S_POISSON, S_CONN_IN, S_CONN_REC, S_W_IN, S_W_REC, S_V0_LIF, S_TARGET = 
 LIF = dict(N=1000, NE=800, n_in=200, tau_m=0.02, tau_s=0.005, theta=0.01, bias=0.0105, p=0.1,
            rate_lo=5.0, rate_hi=50.0, w_scale=0.5e-3, n_steps=2000, n_readout=10, t_ref=0.01, c_v=0.1)
 BLOCK = 1024
+KEEP_BYTES = 4 << 30  # up to which the forward pass keeps the states at every block of the backward pass
 
 
 def _torch():
@@ -195,6 +197,10 @@ class LIFNetwork:
         words = sum(self._words())
         step = 16 * self.block * self.per_thread + 2 * 64 * words
         self.sub = max(1, min(8, self.block // words, (LDS_BYTES - 4096) // step))
+        # the states at the blocks' starts: kept by the forward pass, or recomputed from the
+        # intervals' checkpoints (_bwd_source)
+        self.n_sub = -(-self.C // self.sub)
+        self.keep = 16 * self.B * self.S * self.n_sub * self.N <= KEEP_BYTES
 
     def _kernels(self):
         """Loads the model's statements and generates both kernel sources."""
@@ -209,11 +215,12 @@ class LIFNetwork:
         self.bwd_source = self._bwd_source()
 
     @classmethod
-    def sources(cls, config=None, weight_dtype="float"):
+    def sources(cls, config=None, weight_dtype="float", trials=256, ckpt_every=100):
         """The generated kernel sources (no device needed)."""
         self = cls.__new__(cls)
         self.c = dict(LIF if config is None else config)
         self.N, self.dt, self.wt = self.c["N"], 1e-4, weight_dtype
+        self.B, self.C, self.S = trials, ckpt_every, self.c["n_steps"] // ckpt_every
         self._shape()
         self._kernels()
         return self.fwd_source, self.bwd_source
@@ -368,7 +375,7 @@ template <typename V> struct hb_rows {{
         which the backward pass knows every spike.  Bound by the chain of a step: update,
         barrier, words, one row fetch (L2).  256 trials of 1000 neurons (fp32 weights):
         2.05 us per step with ordered compactions and a barrier per row (ten barriers a
-        step), 1.00 now and 0.05 for the draws."""
+        step), 1.05 now and 0.05 for the draws."""
         ps = self._struct("hba_fwd", False)
         self.fwd_struct = ps
         NIW, NSW = self._words()
@@ -419,9 +426,10 @@ template <typename V> struct hb_rows {{
             "            hb_ahead(k + 32);",
             "            if (k > 0) hb_flush(k - 32, 32);",
             "        }",
-            "        if (c == 0)",
+            f"        if (c % {self.sub} == 0)  // a block of the backward pass" if self.keep else "        if (c == 0)",
             "            HB_EACH_Q if (HB_J < N) {",
-            "                const size_t co = ((size_t)sg * gridDim.x + b) * N + HB_J;",
+            f"                const size_t co = (((size_t)b * p.n_seg + sg) * {self.n_sub} + c / {self.sub}) * N + HB_J;" if self.keep
+            else "                const size_t co = ((size_t)sg * gridDim.x + b) * N + HB_J;",
             "                p.ckpt_v[co] = v[q]; p.ckpt_I[co] = I[q];",
             "            }",
             "        bool cond[HB_Q], fs_any = false;",
@@ -539,15 +547,17 @@ template <typename V> struct hb_rows {{
         With the raster the recomputation of an interval is each thread's own: no spike has
         to be exchanged, and the rows of a step are fetched while the step before it is
         computed.  The steps are taken in blocks of SUB: a block's raster words become a
-        list of its events in LDS (step and source, in order; a word per thread).  From the
-        interval's checkpoint the states at every block's start are kept (sub_v, sub_I);
-        from the last block to the first, its steps' states are recomputed into LDS (a
-        column per neuron) and walked in reverse.  The adjoint of I is kept in the
+        list of its events in LDS (step and source, in order; a word per thread).  The states
+        at every block's start come from the forward pass (256 trials of 1000 neurons, 2000
+        steps: 1 GB) or, beyond KEEP_BYTES, from a first run through the interval from its
+        checkpoint (sub_v, sub_I); from the last block to the first, its steps' states are
+        recomputed into LDS (a column per neuron) and walked in reverse.  The adjoint of I is kept in the
         state's place, and the block's weight gradients follow: a wave adds it to the
         synapses of its sources that spiked, in descending step order.
         Bound by the latency of the rows and of the gradients.  256 trials: 5.05 us per
         step with the recomputation through a history of 16 bytes per neuron and step in
-        memory, 2.02 now."""
+        memory, 2.02 with the first run through the interval, 1.36 with the states kept (the
+        forward pass 1.00 to 1.05)."""
         ps = self._struct("hba_bwd", True)
         self.bwd_struct = ps
         NIW, NSW = self._words()
@@ -688,28 +698,54 @@ template <typename V> struct hb_rows {{
             f"                for (int y = {GP} * 64 + lane; y < gn[u]; y += 64) g[e - lane + y] += s_hi[gs[u]][post[e - lane + y]];",
             "            }",
             "    };",
-            "    unsigned long long w_next = hb_word(p.n_seg - 1, 0);  // of the block to come (read ahead)",
-            "    for (int sg = p.n_seg - 1; sg >= 0; sg--) {",
-            "        const size_t co = ((size_t)sg * gridDim.x + b) * N + threadIdx.x;",
-            f"        HB_EACH_Q {{ v[q] = HB_J < N ? p.ckpt_v[co + q * {T}] : 0.0; I[q] = HB_J < N ? p.ckpt_I[co + q * {T}] : 0.0; }}",
-            "        const size_t so = (size_t)b * n_sub * N + threadIdx.x;",
-            "        for (int sb = 0; sb < n_sub - 1; sb++) {",
-            "            const int n_ev = hb_list(w_next);",
-            "            w_next = hb_word(sg, sb + 1);",
-            "            HB_EACH_Q if (HB_J < N) {",
-            f"                p.sub_v[so + (size_t)sb * N + q * {T}] = v[q]; p.sub_I[so + (size_t)sb * N + q * {T}] = I[q];",
-            "            }",
-            f"            hb_steps(sg * C + sb * {SB}, {SB}, n_ev, [](const int) {{}});",
-            "        }",
-            "        for (int sb = n_sub - 1; sb >= 0; sb--) {",
-            f"            const int k0 = sg * C + sb * {SB}, n = hb_len(sb);",
-            "            const int n_ev = hb_list(w_next);",
-            "            w_next = sb > 0 ? hb_word(sg, sb - 1) : hb_word(sg - 1, 0);",
-            "            if (sb < n_sub - 1)",
-            "                HB_EACH_Q {",
-            f"                    v[q] = HB_J < N ? p.sub_v[so + (size_t)sb * N + q * {T}] : 0.0;",
-            f"                    I[q] = HB_J < N ? p.sub_I[so + (size_t)sb * N + q * {T}] : 0.0;",
-            "                }",
+        ]
+        if self.keep:
+            k += [
+                "    unsigned long long w_next = hb_word(p.n_seg - 1, n_sub - 1);  // of the block to come (read ahead)",
+                "    // the states at the start of the block to come, read a block ahead",
+                "    double v_next[HB_Q], I_next[HB_Q];",
+                "    auto hb_state = [&](const int sg, const int sb) __attribute__((always_inline)) {",
+                "        const size_t so = (((size_t)b * p.n_seg + (sg > 0 ? sg : 0)) * n_sub + sb) * N;",
+                "        HB_EACH_Q {",
+                "            const int j = HB_J < N ? HB_J : N - 1;",
+                "            v_next[q] = p.ckpt_v[so + j]; I_next[q] = p.ckpt_I[so + j];",
+                "        }",
+                "    };",
+                "    hb_state(p.n_seg - 1, n_sub - 1);",
+                "    for (int sg = p.n_seg - 1; sg >= 0; sg--) {",
+                "        for (int sb = n_sub - 1; sb >= 0; sb--) {",
+                f"            const int k0 = sg * C + sb * {SB}, n = hb_len(sb);",
+                "            const int n_ev = hb_list(w_next);",
+                "            w_next = sb > 0 ? hb_word(sg, sb - 1) : hb_word(sg - 1, n_sub - 1);",
+                "            HB_EACH_Q { v[q] = HB_J < N ? v_next[q] : 0.0; I[q] = HB_J < N ? I_next[q] : 0.0; }",
+                "            hb_state(sb > 0 ? sg : sg - 1, sb > 0 ? sb - 1 : n_sub - 1);",
+            ]
+        else:
+            k += [
+                "    unsigned long long w_next = hb_word(p.n_seg - 1, 0);  // of the block to come (read ahead)",
+                "    for (int sg = p.n_seg - 1; sg >= 0; sg--) {",
+                "        const size_t co = ((size_t)sg * gridDim.x + b) * N + threadIdx.x;",
+                f"        HB_EACH_Q {{ v[q] = HB_J < N ? p.ckpt_v[co + q * {T}] : 0.0; I[q] = HB_J < N ? p.ckpt_I[co + q * {T}] : 0.0; }}",
+                "        const size_t so = (size_t)b * n_sub * N + threadIdx.x;",
+                "        for (int sb = 0; sb < n_sub - 1; sb++) {",
+                "            const int n_ev = hb_list(w_next);",
+                "            w_next = hb_word(sg, sb + 1);",
+                "            HB_EACH_Q if (HB_J < N) {",
+                f"                p.sub_v[so + (size_t)sb * N + q * {T}] = v[q]; p.sub_I[so + (size_t)sb * N + q * {T}] = I[q];",
+                "            }",
+                f"            hb_steps(sg * C + sb * {SB}, {SB}, n_ev, [](const int) {{}});",
+                "        }",
+                "        for (int sb = n_sub - 1; sb >= 0; sb--) {",
+                f"            const int k0 = sg * C + sb * {SB}, n = hb_len(sb);",
+                "            const int n_ev = hb_list(w_next);",
+                "            w_next = sb > 0 ? hb_word(sg, sb - 1) : hb_word(sg - 1, 0);",
+                "            if (sb < n_sub - 1)",
+                "                HB_EACH_Q {",
+                f"                    v[q] = HB_J < N ? p.sub_v[so + (size_t)sb * N + q * {T}] : 0.0;",
+                f"                    I[q] = HB_J < N ? p.sub_I[so + (size_t)sb * N + q * {T}] : 0.0;",
+                "                }",
+            ]
+        k += [
             "            hb_steps(k0, n - 1, n_ev, [&](const int s) { HB_EACH_Q { s_hv[s][HB_J] = v[q]; s_hi[s][HB_J] = I[q]; } });",
             "            HB_EACH_Q { s_hv[n - 1][HB_J] = v[q]; s_hi[n - 1][HB_J] = I[q]; }",
             "            g_c = n_ev > 0 ? (n_ev - 1) & ~63 : 0;",
@@ -795,7 +831,7 @@ template <typename V> struct hb_rows {{
         B, N, R = self.B, self.N, self.R
         v = self.v0.clone()
         I = torch.zeros_like(v)
-        ckpt_v = torch.empty((self.S, B, N), dtype=torch.float64, device="cuda")
+        ckpt_v = torch.empty((B, self.S, self.n_sub, N) if self.keep else (self.S, B, N), dtype=torch.float64, device="cuda")
         ckpt_I = torch.empty_like(ckpt_v)
         fs_step = torch.full((B, R), -1, dtype=torch.int32, device="cuda")
         fs_vprev = torch.zeros((B, R), dtype=torch.float64, device="cuda")
@@ -848,7 +884,7 @@ template <typename V> struct hb_rows {{
         c, B, N = self.c, self.B, self.N
         sc, consts = saved["scalars"]
         lin = saved["lin"] or linear_map(self.su, consts, self.dt)
-        sub_v = torch.empty((B, -(-self.C // self.sub), N), dtype=torch.float64, device="cuda")
+        sub_v = torch.empty((1,) if self.keep else (B, self.n_sub, N), dtype=torch.float64, device="cuda")
         sub_I = torch.empty_like(sub_v)
         # (a pathway without synapses keeps a place to read)
         g_in = torch.zeros((B, max(1, self.n_syn_in)), dtype=torch.float64, device="cuda")

@@ -167,3 +167,23 @@ def test_shapes_at_the_edges_of_words_blocks_and_batches(n, n_in, p, rate, steps
             assert _rel(got, want.grad.numpy()) < 1e-9
     assert abs(g_m - float(tm.grad)) <= 1e-9 * abs(float(tm.grad))
     assert abs(g_s - float(ts.grad)) <= 1e-9 * abs(float(ts.grad))
+
+
+@pytest.mark.parametrize("n, every, wt", [(65, 7, "float"), (513, 25, "double"), (1000, 100, "float")])
+def test_kept_and_recomputed_states_give_the_same_gradients(n, every, wt, monkeypatch):
+    """The states at the blocks' starts from the forward pass, and recomputed from the
+    intervals' checkpoints (as for runs whose states would be too large to keep)."""
+    from brian2_amd import adjoint
+
+    c = dict(adjoint.LIF, N=n, NE=n * 4 // 5, n_steps=every * 4, tau_m=0.004, bias=0.012, rate_hi=400.0)
+    out = []
+    for keep in (True, False):
+        if not keep:
+            monkeypatch.setattr(adjoint, "KEEP_BYTES", 0)
+        net = adjoint.LIFNetwork(trials=2, config=c, weight_dtype=wt, ckpt_every=every)
+        assert net.keep == keep
+        loss, saved = net.forward(net.w_in0, net.w_rec0, c["tau_m"], c["tau_s"])
+        g = net.backward(saved)
+        out.append([np.float64(loss), g[0].cpu().numpy(), g[1].cpu().numpy(), g[2], g[3]])
+    assert np.abs(out[0][2]).max() > 0
+    assert all(np.array_equal(a, b) for a, b in zip(*out))
