@@ -206,7 +206,7 @@ class BatchedCUBA:
             "int* const s_pre = (int*)(s_bit + (N + 63) / 64);",
         ]
         store = ("if (hb_sn + {r} < hb_sc) {{ p.spk_i[hb_so + hb_sn + {r}] = {i}; "
-                 "p.spk_step[hb_so + hb_sn + {r}] = (int)step; }}")
+                 "p.spk_step[hb_so + hb_sn + {r}] = (int)hb_step; }}")
         record = [
             "// the record keeps a step's spikes in ascending order",
             "if (hb_nsp <= 64) {",

@@ -388,9 +388,9 @@ class SumSteps:
             "    bool hb_cond = false;",
         ]
         sl = [f"{ct} hb_s_{v}[{U}];" for v, ct in own.syn_arrays.items()] + [f"int hb_p[{U}];"]
-        ld = ["#pragma unroll", f"for (int u = 0; u < {U}; u++) {{",
-              "    const unsigned int q_ = hb_c + u * 64u + hb_lane, k_ = q_ < hb_hi ? q_ : hb_hi - 1u;"]
-        ld += [f"    hb_s_{v}[u] = p.z_s_{v}[k_];" for v in own.syn_arrays] + ["    hb_p[u] = p.z_post_pre[k_];", "}"]
+        ld = ["#pragma unroll", f"for (int hb_u = 0; hb_u < {U}; hb_u++) {{",
+              "    const unsigned int q_ = hb_c + hb_u * 64u + hb_lane, k_ = q_ < hb_hi ? q_ : hb_hi - 1u;"]
+        ld += [f"    hb_s_{v}[hb_u] = p.z_s_{v}[k_];" for v in own.syn_arrays] + ["    hb_p[hb_u] = p.z_post_pre[k_];", "}"]
         if kept:
             k += ["    " + x for x in sl]
             k += ["    if (hb_hi > hb_lo) {", "        const unsigned int hb_c = hb_lo;"] + ["        " + x for x in ld] + ["    }"]
@@ -450,17 +450,17 @@ class SumSteps:
         ]
         if not kept:
             k += ["                " + x for x in sl + ld]
-        k += ["                #pragma unroll", f"                for (int u = 0; u < {U}; u++) {{",
-              "                    const int _presynaptic_idx = hb_p[u], _postsynaptic_idx = i;",
+        k += ["                #pragma unroll", f"                for (int hb_u = 0; hb_u < {U}; hb_u++) {{",
+              "                    const int _presynaptic_idx = hb_p[hb_u], _postsynaptic_idx = i;",
               "                    (void)_presynaptic_idx; (void)_postsynaptic_idx;"]
-        k += [f"                    const {ct} {v} = hb_s_{v}[u];" for v, ct in own.syn_arrays.items()]
+        k += [f"                    const {ct} {v} = hb_s_{v}[hb_u];" for v, ct in own.syn_arrays.items()]
         k += [f"                    const {own.var_types[n]} {n} = s_x_{v}[hb_s & 1][_presynaptic_idx];"
               for n, v in sorted(own.pre_reads.items())]
         k += [f"                    const {own.var_types[n]} {n} = {v};" for n, v in sorted(own.post_reads.items())]
         k += ["                    " + x for x in own.code]
         k += [
             "                    // past the end -0.0, which changes no sum",
-            f"                    s_sum[hb_wave][u * 64 + hb_lane] = hb_c + u * 64u + hb_lane < hb_hi ? _synaptic_var : ({own.vt})-0.0;",
+            f"                    s_sum[hb_wave][hb_u * 64 + hb_lane] = hb_c + hb_u * 64u + hb_lane < hb_hi ? _synaptic_var : ({own.vt})-0.0;",
             "                }",
         ]
         k += ["                " + x for x in chain_lines(CH, own.vt, "hb_wave", f"(hb_hi - hb_c < {CH}u ? hb_hi - hb_c : {CH}u)")]

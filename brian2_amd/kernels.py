@@ -1660,36 +1660,36 @@ def wave_sum_lines(chunk, P, vt, target_t, posts, reads, lines, own=None):
     storage by source is read)."""
     U = chunk // 64
     decl = ["unsigned int hb_e[{U}];"] if own is None else [f"{ct} hb_s_{v}[{{U}}];" for v, ct in own.items()]
-    load = [f"hb_e[u] = {P}post_syn[k_];"] if own is None else [f"hb_s_{v}[u] = {P}s_{v}[k_];" for v in own]
-    at = ["const unsigned int e = hb_e[u];", "const int _idx = (int)e;", "(void)_idx;"] if own is None else []
+    load = [f"hb_e[hb_u] = {P}post_syn[k_];"] if own is None else [f"hb_s_{v}[hb_u] = {P}s_{v}[k_];" for v in own]
+    at = ["const unsigned int e = hb_e[hb_u];", "const int _idx = (int)e;", "(void)_idx;"] if own is None else []
     return [
         "const int _postsynaptic_idx = j;",
         "(void)_postsynaptic_idx;",
-        f"const unsigned int lo = {P}post_ptr[j], hi = {P}post_ptr[j + 1];",
+        f"const unsigned int hb_lo = {P}post_ptr[j], hb_hi = {P}post_ptr[j + 1];",
     ] + posts + [
         f"{target_t} hb_acc = ({target_t})0;",
-        f"for (unsigned int c_ = lo; c_ < hi; c_ += {chunk}u) {{",
+        f"for (unsigned int c_ = hb_lo; c_ < hb_hi; c_ += {chunk}u) {{",
         "    // positions and sources, then the variables: loads at a clamped index, so that those",
         "    // of a chunk are issued together (one under a condition is waited for in its branch)",
     ] + ["    " + x.format(U=U) for x in decl] + [
         f"    int hb_p[{U}];",
         "    #pragma unroll",
-        f"    for (int u = 0; u < {U}; u++) {{",
-        "        const unsigned int q_ = c_ + u * 64u + lane;",
-        "        const unsigned int k_ = q_ < hi ? q_ : hi - 1u;",
+        f"    for (int hb_u = 0; hb_u < {U}; hb_u++) {{",
+        "        const unsigned int q_ = c_ + hb_u * 64u + lane;",
+        "        const unsigned int k_ = q_ < hb_hi ? q_ : hb_hi - 1u;",
     ] + ["        " + x for x in load] + [
-        f"        hb_p[u] = {P}post_pre[k_];",
+        f"        hb_p[hb_u] = {P}post_pre[k_];",
         "    }",
         "    #pragma unroll",
-        f"    for (int u = 0; u < {U}; u++) {{",
+        f"    for (int hb_u = 0; hb_u < {U}; hb_u++) {{",
     ] + ["        " + x for x in at] + [
-        "        const int _presynaptic_idx = hb_p[u];",
+        "        const int _presynaptic_idx = hb_p[hb_u];",
         "        (void)_presynaptic_idx;",
     ] + ["        " + x for x in reads + lines] + [
         "        // past the end -0.0, which changes no sum",
-        f"        s_sum[wid][u * 64 + lane] = c_ + u * 64u + lane < hi ? _synaptic_var : ({vt})-0.0;",
+        f"        s_sum[wid][hb_u * 64 + lane] = c_ + hb_u * 64u + lane < hb_hi ? _synaptic_var : ({vt})-0.0;",
         "    }",
-    ] + ["    " + x for x in chain_lines(chunk, vt, "wid", f"(hi - c_ < {chunk}u ? hi - c_ : {chunk}u)")] + [
+    ] + ["    " + x for x in chain_lines(chunk, vt, "wid", f"(hb_hi - c_ < {chunk}u ? hb_hi - c_ : {chunk}u)")] + [
         "}",
     ]
 
@@ -1732,7 +1732,7 @@ class OwnSum:
 
     def lines(self, T):
         TN = T // 64
-        reads = [f"const {ct} {v} = hb_s_{v}[u];" for v, ct in self.syn_arrays.items()]
+        reads = [f"const {ct} {v} = hb_s_{v}[hb_u];" for v, ct in self.syn_arrays.items()]
         reads += [f"const {self.var_types[n]} {n} = p.z_x_{v}[hb_at + _presynaptic_idx];" for n, v in sorted(self.pre_reads.items())]
         posts = [f"const {self.var_types[n]} {n} = p.a_{v}[j];" for n, v in sorted(self.post_reads.items())]
         k = [

@@ -92,8 +92,8 @@ class ResidentKernel:
     events      further lines per event
     record      lines run for a step's spikes (s_spk[0 .. hb_nsp), any order) by every
                 thread; may contain barriers
-    begin/start lines that set hb_recq[q] of neuron i, and lines run before its every step
-                with hb_rec = hb_recq[q] (state monitors)
+    begin/start lines that set hb_recq[hb_q] of neuron i, and lines run before its every step
+                with hb_rec = hb_recq[hb_q] (state monitors)
     finish      lines run once at the end by every thread
     resident    neurons per thread in registers
     bound       C expression of timestep_bound(K, dt) when K >= 1 is the refractory period
@@ -128,7 +128,7 @@ class ResidentKernel:
         pt = {v: ("unsigned char" if ct == "bool" else ct) for v, ct in var_types.items()}
         load = {v: (f"p.a_{v}[hb_off + i] != 0" if ct == "bool" else f"p.a_{v}[hb_off + i]") for v, ct in var_types.items()}
         save = {v: (f"{v} ? 1 : 0" if ct == "bool" else v) for v, ct in var_types.items()}
-        regs = ", ".join(f"r_{v}[q]" for v in held)
+        regs = ", ".join(f"r_{v}[hb_q]" for v in held)
         held_args, all_args = ", ".join(held), ", ".join(var_types)
         mem_load = " ".join(f"{ct} {v} = {load[v]};" for v, ct in var_types.items())
         mem_save = " ".join(f"p.a_{v}[hb_off + i] = ({pt[v]})({save[v]});" for v in var_types)
@@ -181,7 +181,7 @@ class ResidentKernel:
         row = "s_rp[{}]" if rows_in_lds else "hb_rp[{}]"
         k += [
             f"    unsigned short* const s_spk = (unsigned short*){lds};",
-            "    __shared__ int s_n[3];  // spikes of steps s % 3: added to, read, cleared in turn",
+            "    __shared__ int s_n[3];  // spikes of steps hb_s % 3: added to, read, cleared in turn",
         ]
         k += ["    " + x for x in shared]
         if released:
@@ -203,13 +203,13 @@ class ResidentKernel:
         # the update of a neuron in registers, and of one in memory where they differ
         for fn, vs in (("hb_update", held), ("hb_update_mem", var_types)):
             reg = released and fn == "hb_update"
-            lines = ["not_refractory = s >= hb_rel;" if reg and _REFRACTORY.fullmatch(x.strip()) else x for x in update]
+            lines = ["not_refractory = hb_s >= hb_rel;" if reg and _REFRACTORY.fullmatch(x.strip()) else x for x in update]
             k += [
                 "    // one step of neuron i after the events of the step before: whether it spikes",
-                f"    auto {fn} = [&](const int i, const int s, const double t, {decl(vs)}"
+                f"    auto {fn} = [&](const int i, const int hb_s, const double t, {decl(vs)}"
                 f"{', const int hb_rel' if reg else ''}) __attribute__((always_inline)) {{",
                 "        const int _idx = i;",
-                "        (void)_idx; (void)s; (void)t;",
+                "        (void)_idx; (void)hb_s; (void)t;",
                 "        bool hb_cond = false;",
             ]
             k += ["        bool not_refractory;"] if reg else []
@@ -237,24 +237,24 @@ class ResidentKernel:
         for v, ct in held.items():
             k.append(f"    {ct} r_{v}[{R}];")
         if released:
-            k.append(f"    int r_rel[{R}];")
+            k.append(f"    int hb_rels[{R}];")
         if start:
             k.append(f"    int hb_recq[{R}];")
         k += [
             f"    unsigned long long hb_act[{R}];  // lanes with a neuron (scalars)",
             "    #pragma unroll",
-            f"    for (int q = 0; q < {R}; q++) {{",
-            "        const int i = q * T + (int)threadIdx.x;",
+            f"    for (int hb_q = 0; hb_q < {R}; hb_q++) {{",
+            "        const int i = hb_q * T + (int)threadIdx.x;",
             "        const bool act = i < N;",
-            "        hb_act[q] = __builtin_amdgcn_ballot_w64(act);",
+            "        hb_act[hb_q] = __builtin_amdgcn_ballot_w64(act);",
         ]
         for v, ct in held.items():
-            k.append(f"        r_{v}[q] = act ? {load[v]} : ({ct})0;")
+            k.append(f"        r_{v}[hb_q] = act ? {load[v]} : ({ct})0;")
         if released:
-            k.append(f"        r_rel[q] = act ? {first} : 0x7fffffff;")
+            k.append(f"        hb_rels[hb_q] = act ? {first} : 0x7fffffff;")
         k += ["        " + x for x in begin]
         k.append("        // waited for here: a wait inside the loop would be for the step's stores as well")
-        k += [f'        asm volatile("" : "+v"(r_{v}[q]));' for v, ct in held.items() if ct != "bool"]
+        k += [f'        asm volatile("" : "+v"(r_{v}[hb_q]));' for v, ct in held.items() if ct != "bool"]
         k.append("    }")
         if counts_in_lds:
             k.append(f"    for (int i = threadIdx.x; i < {W} * hb_np; i += T) s_cnt[i] = 0u;")
@@ -271,16 +271,16 @@ class ResidentKernel:
         k += [
             "    int hb_cur = 0, hb_old = 2;",
             "    double hb_k = (double)hb_step0;  // the step (exact)",
-            "    for (int s = 0; s < p.n_steps; s++, hb_k += 1.0) {",
-            "        const long long step = hb_step0 + s;",
-            "        const double t = hb_k * dt;  // (double)step * dt",
-            "        (void)step;",
+            "    for (int hb_s = 0; hb_s < p.n_steps; hb_s++, hb_k += 1.0) {",
+            "        const long long hb_step = hb_step0 + hb_s;",
+            "        const double t = hb_k * dt;  // (double)hb_step * dt",
+            "        (void)hb_step;",
         ]
         k += [f"        unsigned int hb_c{w}[{R}], hb_o{w} = 0u;" for w in range(W)]
-        k += ["        #pragma unroll", f"        for (int q = 0; q < {R}; q++) {{  // all reads in flight together",
-              "            const int i = q * T + (int)threadIdx.x;"]
-        k += [f"            hb_c{w}[q] = {read.format(w=w)};" for w in range(W)]
-        k += [f"            hb_o{w} |= hb_c{w}[q];" for w in range(W)]
+        k += ["        #pragma unroll", f"        for (int hb_q = 0; hb_q < {R}; hb_q++) {{  // all reads in flight together",
+              "            const int i = hb_q * T + (int)threadIdx.x;"]
+        k += [f"            hb_c{w}[hb_q] = {read.format(w=w)};" for w in range(W)]
+        k += [f"            hb_o{w} |= hb_c{w}[hb_q];" for w in range(W)]
         k.append("        }")
         more = " | ".join(f"(hb_o{w} & 0xfffefffeu)" for w in range(W))
         same = len({v for v, _, _ in pathways}) < len(pathways)
@@ -289,29 +289,29 @@ class ResidentKernel:
         last = {v: r for r, (v, _, _) in enumerate(pathways)}
         rest = " | ".join(f"hb_o{w}" for w in range(W)) if same else more
         k += [f"        if (__builtin_amdgcn_ballot_w64(({rest}) != 0u) != 0ull) {{  // more events than one of a pathway",
-              "            #pragma unroll", f"            for (int q = 0; q < {R}; q++) {{"]
-        k += [f"                {held[v]}& {v} = r_{v}[q];" for v in dict.fromkeys(v for v, _, _ in pathways)]
+              "            #pragma unroll", f"            for (int hb_q = 0; hb_q < {R}; hb_q++) {{"]
+        k += [f"                {held[v]}& {v} = r_{v}[hb_q];" for v in dict.fromkeys(v for v, _, _ in pathways)]
         for r_, (var, op, val) in enumerate(pathways):
-            k.append(f"                for (unsigned int n_ = {field(r_, 'hb_c{w}[q]')}; n_ > "
+            k.append(f"                for (unsigned int n_ = {field(r_, 'hb_c{w}[hb_q]')}; n_ > "
                      f"{1 if last[var] == r_ else 0}u; n_--) {var} {op} {val};")
         k += ["            }", "        }",
               f"        unsigned long long hb_b[{R}], hb_any = 0ull;  // the wave's spikes (scalars)",
               "        #pragma unroll",
-              f"        for (int q = 0; q < {R}; q++) {{  // lanes without a neuron compute on zeros",
-              "            const int i = q * T + (int)threadIdx.x;"]
+              f"        for (int hb_q = 0; hb_q < {R}; hb_q++) {{  // lanes without a neuron compute on zeros",
+              "            const int i = hb_q * T + (int)threadIdx.x;"]
         for r_, (var, op, val) in enumerate(pathways):
             if last[var] == r_:
-                k += [f"            {{ {held[var]} x_ = r_{var}[q]; x_ {op} {val}; "
-                      f"r_{var}[q] = {field(r_, 'hb_c{w}[q]')} != 0u ? x_ : r_{var}[q]; }}"]
+                k += [f"            {{ {held[var]} x_ = r_{var}[hb_q]; x_ {op} {val}; "
+                      f"r_{var}[hb_q] = {field(r_, 'hb_c{w}[hb_q]')} != 0u ? x_ : r_{var}[hb_q]; }}"]
         k += ["            " + x for x in clears]
         if start:
-            k += ["            if (i < N) {"] + [f"                const {ct}& {v} = r_{v}[q];" for v, ct in held.items()]
-            k += ["                const int hb_rec = hb_recq[q];"]
+            k += ["            if (i < N) {"] + [f"                const {ct}& {v} = r_{v}[hb_q];" for v, ct in held.items()]
+            k += ["                const int hb_rec = hb_recq[hb_q];"]
             k += ["                " + x for x in start] + ["            }"]
         k += [
-            f"            hb_b[q] = __builtin_amdgcn_ballot_w64(hb_update(i, s, t, {regs}"
-            f"{', r_rel[q]' if released else ''})) & hb_act[q];",
-            "            hb_any |= hb_b[q];",
+            f"            hb_b[hb_q] = __builtin_amdgcn_ballot_w64(hb_update(i, hb_s, t, {regs}"
+            f"{', hb_rels[hb_q]' if released else ''})) & hb_act[hb_q];",
+            "            hb_any |= hb_b[hb_q];",
             "        }",
             "        if (hb_any != 0ull) {",
             "            int hb_x = (int)threadIdx.x;  // hidden: see the end",
@@ -321,31 +321,31 @@ class ResidentKernel:
             k += [
                 "            // the release step of a neuron that spikes now: K steps on, or one beside it by rounding",
                 f"            const double k_ = hb_k + (double)({period});",
-                f"            const int rel_ = s + (int)({period}) + (hb_free(t, k_ - 1.0) ? -1 : hb_free(t, k_) ? 0 : 1);",
+                f"            const int rel_ = hb_s + (int)({period}) + (hb_free(t, k_ - 1.0) ? -1 : hb_free(t, k_) ? 0 : 1);",
             ]
-        k += ["            #pragma unroll", f"            for (int q = 0; q < {R}; q++) {{",
-              "                const int i = q * T + hb_x;", "                const unsigned long long b_ = hb_b[q];"]
+        k += ["            #pragma unroll", f"            for (int hb_q = 0; hb_q < {R}; hb_q++) {{",
+              "                const int i = hb_q * T + hb_x;", "                const unsigned long long b_ = hb_b[hb_q];"]
         k += ["                " + x for x in put]
         if released:
-            k.append("                        r_rel[q] = rel_; p.a_lastspike[hb_off + i] = t;")
+            k.append("                        hb_rels[hb_q] = rel_; p.a_lastspike[hb_off + i] = t;")
         k += [f"                        hb_spike(i, t, {regs});", "                    }", "                }",
               "            }", "        }",
               f"        for (int j0 = {R} * T; j0 < N; j0 += T) {{  // neurons beyond the registers",
               "            const int i = j0 + (int)threadIdx.x;",
-              "            bool sp = false;",
+              "            bool hb_sp = false;",
               "            if (i < N) {",
               f"                {mem_load}"]
         k += ["                " + x for x in reads + each_event() + clears]
         if start:
             k += ["                {"] + ["                " + x for x in self._search(begin)]
             k += ["                " + x for x in start] + ["                }"]
-        k += [f"                sp = {'hb_update_mem' if released else 'hb_update'}(i, s, t, {all_args});",
-              "                if (sp) {"]
+        k += [f"                hb_sp = {'hb_update_mem' if released else 'hb_update'}(i, hb_s, t, {all_args});",
+              "                if (hb_sp) {"]
         if released:
             k.append("                    not_refractory = false; lastspike = t;")
         k += [f"                    hb_spike(i, t, {held_args});", "                }",
               f"                {mem_save}", "            }",
-              "            const unsigned long long b_ = __builtin_amdgcn_ballot_w64(sp);"]
+              "            const unsigned long long b_ = __builtin_amdgcn_ballot_w64(hb_sp);"]
         k += ["            " + x for x in put] + ["                }", "            }"]
         k += ["        }"] + ["        " + x for x in fence] + [
             "        __syncthreads();",
@@ -429,18 +429,18 @@ class ResidentKernel:
             "    int hb_x = (int)threadIdx.x;",
             '    asm volatile("" : "+v"(hb_x));',
             "    #pragma unroll",
-            f"    for (int q = 0; q < {R}; q++) {{",
-            "        const int i = q * T + hb_x;",
+            f"    for (int hb_q = 0; hb_q < {R}; hb_q++) {{",
+            "        const int i = hb_q * T + hb_x;",
             "        if (i < N) {",
         ]
         k += ["            " + x for x in reads]
-        k += [f"            {held[v]}& {v} = r_{v}[q];" for v in dict.fromkeys(v for v, _, _ in pathways)]
+        k += [f"            {held[v]}& {v} = r_{v}[hb_q];" for v in dict.fromkeys(v for v, _, _ in pathways)]
         k += ["            " + x for x in each_event() + clears]
         for v, ct in held.items():
-            val = f"r_{v}[q] ? 1 : 0" if ct == "bool" else f"r_{v}[q]"
+            val = f"r_{v}[hb_q] ? 1 : 0" if ct == "bool" else f"r_{v}[hb_q]"
             k.append(f"            p.a_{v}[hb_off + i] = ({pt[v]})({val});")
         if released:
-            k.append("            p.a_not_refractory[hb_off + i] = p.n_steps - 1 >= r_rel[q] ? 1 : 0;")
+            k.append("            p.a_not_refractory[hb_off + i] = p.n_steps - 1 >= hb_rels[hb_q] ? 1 : 0;")
         k += [
             "        }",
             "    }",
@@ -456,7 +456,7 @@ class ResidentKernel:
     @staticmethod
     def _search(begin):
         """The begin lines for a neuron outside the registers (hb_rec instead of hb_recq[q])."""
-        return ["int hb_recm[1]; { const int q = 0; const bool act = true;"] + [
+        return ["int hb_recm[1]; { const int hb_q = 0; const bool act = true;"] + [
             x.replace("hb_recq", "hb_recm") for x in begin] + ["}", "const int hb_rec = hb_recm[0];"]
 
     def lds_bytes(self, N, threads, extra=0):
@@ -602,7 +602,7 @@ class GroupStep:
         # the record is the last waves' work: the first ones have the spikes' synapses
         each = "for (int j = T - 1 - (int)threadIdx.x; j < {n}; j += T) {{"
         if g.smon:
-            add = ["if (o_ < (unsigned long long)p.mon_cap) { p.mon_i[o_] = id_; p.mon_step[o_] = (int)step; }",
+            add = ["if (o_ < (unsigned long long)p.mon_cap) { p.mon_i[o_] = id_; p.mon_step[o_] = (int)hb_step; }",
                    "atomicAdd(&p.mon_count[id_ - p.mon_start], 1);"]
             if g.smon.range == (0, g.N):
                 prologue.append("unsigned long long hb_mn = p.mon_n[0];")
@@ -621,25 +621,25 @@ class GroupStep:
                        "    if (hb_mn > (unsigned long long)p.mon_cap) atomicOr(p.status, 2);", "}"]
         if g.rmon:
             record += [
-                "if (p.rate_cnt && step - p.rate_row0 >= 0 && step - p.rate_row0 < p.rate_rows) {",
+                "if (p.rate_cnt && hb_step - p.rate_row0 >= 0 && hb_step - p.rate_row0 < p.rate_rows) {",
                 "    " + each.format(n="hb_nsp"),
                 "        const int id_ = (int)s_spk[j];",
-                "        if (id_ >= p.rate_start && id_ < p.rate_stop) atomicAdd(&p.rate_cnt[step - p.rate_row0], 1);",
+                "        if (id_ >= p.rate_start && id_ < p.rate_stop) atomicAdd(&p.rate_cnt[hb_step - p.rate_row0], 1);",
                 "    }",
                 "}",
             ]
         if g.stmon:  # recorded neurons: their place in rec_idx, or -1
             begin += [
-                "hb_recq[q] = -1;",
+                "hb_recq[hb_q] = -1;",
                 "if (act) {",
                 "    int lo = 0, hi = p.n_rec;",
                 "    while (lo < hi) { const int m = (lo + hi) >> 1; if (p.rec_idx[m] < i) lo = m + 1; else hi = m; }",
-                "    if (lo < p.n_rec && p.rec_idx[lo] == i) hb_recq[q] = lo;",
+                "    if (lo < p.n_rec && p.rec_idx[lo] == i) hb_recq[hb_q] = lo;",
                 "}",
             ]
             nv = len(g.stmon.variables)
-            start += ["if (hb_rec >= 0 && step - p.rec_row0 >= 0 && step - p.rec_row0 < p.rec_rows) {",
-                      f"    double* const o_ = p.rec_buf + (size_t)(step - p.rec_row0) * {nv} * p.n_rec + hb_rec;"]
+            start += ["if (hb_rec >= 0 && hb_step - p.rec_row0 >= 0 && hb_step - p.rec_row0 < p.rec_rows) {",
+                      f"    double* const o_ = p.rec_buf + (size_t)(hb_step - p.rec_row0) * {nv} * p.n_rec + hb_rec;"]
             start += [f"    o_[(size_t){a} * p.n_rec] = (double){v};" for a, v in enumerate(g.stmon.variables)] + ["}"]
         finish += [f"if (hb_ev{r}) atomicAdd(&p.events[{r}], hb_ev{r});" for r in range(len(ops))]
         finish.append("if (threadIdx.x == 0) p.clock[0] = hb_step0 + p.n_steps;")

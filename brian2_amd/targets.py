@@ -17,7 +17,7 @@ class TargetSteps:
 
     The wave's lanes hold the next 64 entries of the generator's list, the following 64 being
     on their way.  A step: the neuron's update (all lanes alike), the entries of this step, a
-    lane each, with the on_pre statements on that source's synapse (s_at: its place in LDS),
+    lane each, with the on_pre statements on that source's synapse (hb_map: its place in LDS),
     their values added up in the entries' order, the on_post statements on all synapses if
     the neuron spikes, its reset.  No lane waits for memory but at the start, the end and for
     a spike's record.
@@ -77,13 +77,13 @@ class TargetSteps:
         types.update({n: ct for n, (_, ct) in post_scalars.items()})
         post = _rename(translate_block(on_post, {}, types, set(), g.float_t), {n: f"p.q_{n}" for n in post_scalars})
         pre = onpre_lines(on_pre, target_index, syn_arrays, pre_scalars, g.float_t, f"hb_gv = ({val_t})", val_t)
-        load = [f"{ct} {v} = s_{v}[k];" for v, ct in syn_arrays.items()]
-        save = [f"s_{v}[k] = {v};" for v in syn_arrays if v in plastic]
+        load = [f"{ct} {v} = s_{v}[hb_k];" for v, ct in syn_arrays.items()]
+        save = [f"s_{v}[hb_k] = {v};" for v in syn_arrays if v in plastic]
 
         k = [source_header(64), ps.c_decl()]
         k.append(f'extern "C" __global__ void __launch_bounds__(64) {self.kernel_name}(const {ps.name} p) {{')
         k += [
-            "    const int lane = threadIdx.x, i = blockIdx.x, N = p.N, _idx = i;",
+            "    const int hb_lane = threadIdx.x, i = blockIdx.x, N = p.N, _idx = i;",
             "    const double dt = p.dt;",
             "    (void)dt; (void)N; (void)_idx;",
             "    extern __shared__ __align__(16) unsigned char hb_lds[];",
@@ -93,27 +93,27 @@ class TargetSteps:
             k.append(f"    {ct}* const s_{v} = ({ct}*)({at});")
             at = f"s_{v} + p.deg"
         k += [
-            f"    unsigned short* const s_at = (unsigned short*)({at});  // a source's synapse, or 0xffff",
-            "    const unsigned int first = p.post_ptr[i];",
-            "    const int deg = (int)(p.post_ptr[i + 1] - first);",
-            "    for (int x = lane; x < p.n_src; x += 64) s_at[x] = 0xffff;",
+            f"    unsigned short* const hb_map = (unsigned short*)({at});  // a source's synapse, or 0xffff",
+            "    const unsigned int hb_first = p.post_ptr[i];",
+            "    const int hb_deg = (int)(p.post_ptr[i + 1] - hb_first);",
+            "    for (int x = hb_lane; x < p.n_src; x += 64) hb_map[x] = 0xffff;",
             "    __syncthreads();",
-            "    for (int k = lane; k < deg; k += 64) {",
-            "        const unsigned int e = p.post_syn[first + k];",
-        ] + [f"        s_{v}[k] = p.s_{v}[e];" for v in syn_arrays] + [
-            "        s_at[p.post_pre[first + k] - p.src0] = (unsigned short)k;",
+            "    for (int hb_k = hb_lane; hb_k < hb_deg; hb_k += 64) {",
+            "        const unsigned int e = p.post_syn[hb_first + hb_k];",
+        ] + [f"        s_{v}[hb_k] = p.s_{v}[e];" for v in syn_arrays] + [
+            "        hb_map[p.post_pre[hb_first + hb_k] - p.src0] = (unsigned short)hb_k;",
             "    }",
             "    __syncthreads();",
         ]
         for v, ct in g.vars.items():
             k.append(f"    {ct} {v} = p.a_{v}[i]{' != 0' if ct == 'bool' else ''};")
         k += [
-            "    auto hb_entries = [&](const long long x0, int& tb, int& id) {",
-            "        const long long x = x0 + lane < p.gen_n ? x0 + lane : p.gen_n - 1;",
-            "        tb = x >= 0 ? p.gen_tb[x] : 0; id = x >= 0 ? p.gen_idx[x] : 0;",
-            "        if (x0 + lane >= p.gen_n) tb = 0x7fffffff;",
+            "    auto hb_entries = [&](const long long x0, int& hb_tb, int& hb_id) {",
+            "        const long long x = x0 + hb_lane < p.gen_n ? x0 + hb_lane : p.gen_n - 1;",
+            "        hb_tb = x >= 0 ? p.gen_tb[x] : 0; hb_id = x >= 0 ? p.gen_idx[x] : 0;",
+            "        if (x0 + hb_lane >= p.gen_n) hb_tb = 0x7fffffff;",
             "    };",
-            f"    auto hb_lane = [](const {val_t} x, const int l) {{  // lane l's value",
+            f"    auto hb_from = [](const {val_t} x, const int l) {{  // lane l's value",
         ] + (["        return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), l));"]
              if val_t == "float" else [
             "        const long long b = __builtin_bit_cast(long long, x);",
@@ -121,14 +121,14 @@ class TargetSteps:
             "        const unsigned int hi = (unsigned int)__builtin_amdgcn_readlane((int)(b >> 32), l);",
             "        return __builtin_bit_cast(double, (unsigned long long)hi << 32 | lo);"]) + [
             "    };",
-            "    long long at = p.gen_at;",
-            "    int tb, id, tb2, id2;",
-            "    hb_entries(at, tb, id);",
-            "    hb_entries(at + 64, tb2, id2);",
+            "    long long hb_at = p.gen_at;",
+            "    int hb_tb, hb_id, hb_tb2, hb_id2;",
+            "    hb_entries(hb_at, hb_tb, hb_id);",
+            "    hb_entries(hb_at + 64, hb_tb2, hb_id2);",
             "    unsigned long long hb_ev = 0ull;",
-            "    for (int s = 0; s < p.n_steps; s++) {",
-            "        const long long step = p.step0 + s;",
-            "        const double t = (double)step * dt;",
+            "    for (int hb_s = 0; hb_s < p.n_steps; hb_s++) {",
+            "        const long long hb_step = p.step0 + hb_s;",
+            "        const double t = (double)hb_step * dt;",
             "        (void)t;",
             "        bool hb_cond = false;",
         ]
@@ -140,48 +140,48 @@ class TargetSteps:
             if g.uses_refractory:
                 k.append("        if (hb_cond) { not_refractory = false; lastspike = t; }")
         k += [
-            "        const bool spiked = __builtin_amdgcn_ballot_w64(hb_cond) != 0ull;",
+            "        const bool hb_spiked = __builtin_amdgcn_ballot_w64(hb_cond) != 0ull;",
             "        for (;;) {  // this step's entries",
-            "            const bool on = tb == (int)step;",
-            "            if (__builtin_amdgcn_ballot_w64(on) != 0ull) {",
-            "                const int k = on && id >= p.src0 && id < p.src0 + p.n_src ? (int)s_at[id - p.src0] : 0xffff;",
+            "            const bool hb_on = hb_tb == (int)hb_step;",
+            "            if (__builtin_amdgcn_ballot_w64(hb_on) != 0ull) {",
+            "                const int hb_k = hb_on && hb_id >= p.src0 && hb_id < p.src0 + p.n_src ? (int)hb_map[hb_id - p.src0] : 0xffff;",
             f"                {val_t} hb_gv = 0;",
-            "                if (k != 0xffff) {",
-            "                    const int _idx = k;",
+            "                if (hb_k != 0xffff) {",
+            "                    const int _idx = hb_k;",
             "                    (void)_idx;",
         ]
         k += ["                    " + x for x in load + pre + save]
         k += [
             "                }",
-            "                unsigned long long m = __builtin_amdgcn_ballot_w64(k != 0xffff);",
-            "                hb_ev += (unsigned long long)__popcll(m);",
-            f"                for (; m; m &= m - 1ull) {{ const {val_t} hb_v = hb_lane(hb_gv, __builtin_ctzll(m)); "
+            "                unsigned long long hb_m = __builtin_amdgcn_ballot_w64(hb_k != 0xffff);",
+            "                hb_ev += (unsigned long long)__popcll(hb_m);",
+            f"                for (; hb_m; hb_m &= hb_m - 1ull) {{ const {val_t} hb_v = hb_from(hb_gv, __builtin_ctzll(hb_m)); "
             f"{target_var} {op} hb_v; }}",
             "                __syncthreads();",
             "            }",
-            "            if (__builtin_amdgcn_readlane(tb, 63) > (int)step) break;",
-            "            tb = tb2; id = id2; at += 64;",
-            "            hb_entries(at + 64, tb2, id2);",
+            "            if (__builtin_amdgcn_readlane(hb_tb, 63) > (int)hb_step) break;",
+            "            hb_tb = hb_tb2; hb_id = hb_id2; hb_at += 64;",
+            "            hb_entries(hb_at + 64, hb_tb2, hb_id2);",
             "        }",
-            "        if (spiked) {",
+            "        if (hb_spiked) {",
         ]
         if g.smon:
             k += [
-                "            if (lane == 0 && i >= p.mon_start && i < p.mon_stop) {",
+                "            if (hb_lane == 0 && i >= p.mon_start && i < p.mon_stop) {",
                 "                const unsigned long long o = atomicAdd(p.mon_n, 1ull);",
-                "                if (o < (unsigned long long)p.mon_cap) { p.mon_i[o] = i; p.mon_step[o] = (int)step; }",
+                "                if (o < (unsigned long long)p.mon_cap) { p.mon_i[o] = i; p.mon_step[o] = (int)hb_step; }",
                 "                else atomicOr(p.status, 2);",
                 "                p.mon_count[i - p.mon_start] += 1;",
                 "            }",
             ]
-        k += ["            for (int k = lane; k < deg; k += 64) {", "                const int _idx = k;", "                (void)_idx;"]
+        k += ["            for (int hb_k = hb_lane; hb_k < hb_deg; hb_k += 64) {", "                const int _idx = hb_k;", "                (void)_idx;"]
         k += ["                " + x for x in load + post + save]
         k += ["            }", "            __syncthreads();"]
         if g.rs is not None:
             k += ["            {"] + ["                " + x for x in block("rs", g.rs)] + ["            }"]
-        k += ["        }", "    }", "    for (int k = lane; k < deg; k += 64) {",
-              "        const unsigned int e = p.post_syn[first + k];"]
-        k += [f"        p.s_{v}[e] = s_{v}[k];" for v in syn_arrays if v in plastic] + ["    }", "    if (lane == 0) {"]
+        k += ["        }", "    }", "    for (int hb_k = hb_lane; hb_k < hb_deg; hb_k += 64) {",
+              "        const unsigned int e = p.post_syn[hb_first + hb_k];"]
+        k += [f"        p.s_{v}[e] = s_{v}[hb_k];" for v in syn_arrays if v in plastic] + ["    }", "    if (hb_lane == 0) {"]
         for v, ct in g.vars.items():
             k.append(f"        p.a_{v}[i] = {v}{' ? 1 : 0' if ct == 'bool' else ''};")
         k += ["        p.events[i] += hb_ev;", "    }", "}"]

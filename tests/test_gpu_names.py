@@ -1,0 +1,87 @@
+"""Models whose variables have the names that generated code might use itself: the same
+results as under their own names, in every form of the steps that holds the state in registers."""
+import json
+import os
+import re
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _model(name, names):
+    """The model with its variables renamed (the generator's names kept apart)."""
+    from brian2_amd import Model, runtime
+
+    with open(os.path.join(runtime.SPEC_DIR, f"{name}.json")) as f:
+        text = f.read()
+    for old, new in names.items():
+        text = re.sub(rf"(?<![\w.])(_?){old}((?:_pre|_post)?)(?!\w)", rf"\1{new}\2", text)
+    return Model(json.loads(text))
+
+
+def _group(n, name, names, when, **options):
+    from brian2_amd import Network, NeuronGroup, SpikeMonitor, StateMonitor, Synapses, synth
+
+    rng = np.random.default_rng(n)
+    m = _model(name, names)
+    G = NeuronGroup(n, m, name="g")
+    v = names.get("v", "v")
+    mons = [SpikeMonitor(G), StateMonitor(G, [v], record=[0, n - 1], when=when)]
+    if name == "gap":
+        G.set(v, 1.3 * rng.random(n))
+        S = Synapses(G, G, summed={names["Igap"]: m.summed[names["Igap"]]}, name="s")
+        i, j = np.repeat(np.arange(n), n), np.tile(np.arange(n), n)
+        S.connect(i, j)
+        S.set(names["w"], 6.0 / n * rng.random(n * n))
+        syn = [S]
+    else:
+        G.set(v, synth.cuba_v0(3, n) if name == "cuba" else -0.06 + 0.05 * rng.random(n))
+        syn = []
+        for k, (a, b) in {"exc": (0, n * 4 // 5), "inh": (n * 4 // 5, n)}.items():
+            S = Synapses(G[a:b], G, m.pathways[k], name=k)
+            S.connect(*np.nonzero(rng.random((b - a, n)) < 0.1))
+            syn.append(S)
+    net = Network(G, *syn, *mons, dt=1e-4, **options)
+    net.run(150)
+    return net, [G.get(names.get(x, x)) for x in ("v",)] + [mons[0].i, mons[0].step, mons[1].values()]
+
+
+@pytest.mark.parametrize("name, names, when, chip", [
+    ("cuba", {"v": "s", "ge": "q", "gi": "step"}, "start", False),
+    ("cobahh", {"m": "hi", "n": "w", "h": "x", "ge": "lane", "gi": "s", "v": "step"}, "end", True),
+    ("gap", {"v": "x", "Igap": "u", "w": "lo"}, "start", True),
+])
+def test_awkward_names(name, names, when, chip):
+    net, got = _group(700 if name == "cuba" else 100, name, names, when)
+    own = {"Igap": "Igap", "w": "w"} if name == "gap" else {}
+    _, want = _group(700 if name == "cuba" else 100, name, own, when, tile=256)
+    assert net.in_launch is not None and (net.resident is None) == chip
+    assert len(want[1]) > 0
+    for x, y in zip(got, want):
+        assert np.array_equal(x, y)
+
+
+def test_awkward_names_of_targets():
+    from brian2_amd import Network, NeuronGroup, SpikeGeneratorGroup, SpikeMonitor, Synapses
+
+    out = []
+    for names, options in (({"ge": "m", "v": "s", "w": "k", "Apre": "at", "Apost": "id"}, {}), ({}, {"tile": 256})):
+        rng = np.random.default_rng(2)
+        model = _model("stdp", names)
+        step, idx = np.nonzero(rng.random((300, 200)) < 0.02)
+        src = SpikeGeneratorGroup(200, idx, timebins=step)
+        G = NeuronGroup(5, model, name="g")
+        G.set(names.get("v", "v"), -0.06 + 0.006 * rng.random(5))
+        S = Synapses(src, G, model.pathways["pre"], on_post=model.pathways["post"], name="s")
+        S.connect(np.repeat(np.arange(200), 5), np.tile(np.arange(5), 200))
+        S.set(names.get("w", "w"), 0.01 * rng.random(1000))
+        mon = SpikeMonitor(G)
+        net = Network(src, G, S, mon, dt=1e-4, **options)
+        net.run(300)
+        assert (net.resident is not None) == (not options)
+        out.append([G.get(names.get("v", "v")), mon.i, mon.step] + [S.get(names.get(x, x)) for x in ("w", "Apre", "Apost")])
+    assert len(out[1][1]) > 0
+    for x, y in zip(*out):
+        assert np.array_equal(x, y)
