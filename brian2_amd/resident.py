@@ -319,9 +319,12 @@ class ResidentKernel:
         ]
         if released:
             k += [
-                "            // the release step of a neuron that spikes now: K steps on, or one beside it by rounding",
+                "            // the release step of a neuron that spikes now: K steps on, or one beside it by rounding;",
+                "            // beyond 32 bits (K is 64 of them) a step that no launch reaches",
                 f"            const double k_ = hb_k + (double)({period});",
-                f"            const int rel_ = hb_s + (int)({period}) + (hb_free(t, k_ - 1.0) ? -1 : hb_free(t, k_) ? 0 : 1);",
+                f"            const long long far_ = hb_s + ({period} < 0x7fffffffll ? (long long)({period}) : 0x7fffffffll);",
+                "            const int rel_ = (far_ < 0x7ffffffell ? (int)far_ : 0x7ffffffe) "
+                "+ (hb_free(t, k_ - 1.0) ? -1 : hb_free(t, k_) ? 0 : 1);",
             ]
         k += ["            #pragma unroll", f"            for (int hb_q = 0; hb_q < {R}; hb_q++) {{",
               "                const int i = hb_q * T + hb_x;", "                const unsigned long long b_ = hb_b[hb_q];"]

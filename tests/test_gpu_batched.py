@@ -147,3 +147,35 @@ def test_resident_forms_at_the_edges_of_a_workgroup(variant, monkeypatch):
         assert len(i) > 0 and np.array_equal(i, c["mon"].i) and np.array_equal(s, c["mon"].step), net.N
         for x in ("v", "ge", "gi", "lastspike", "not_refractory"):
             assert np.array_equal(B.get(x, k), c["G"].get(x)), (net.N, x)
+
+
+@pytest.mark.parametrize("steps", [2**31 - 2, 3 * 10**9])
+def test_refractory_periods_beyond_32_bits(steps):
+    """Neurons that fire once: the sweep equals the plain path's staged launches."""
+    from brian2_amd import Model, batched, synth
+
+    def model():
+        m = Model.load("cuba")
+        m.group["stateupdate"].scalar[0]["expr"] = f"timestep({steps!r} * dt, dt)"
+        return m
+
+    B = batched.BatchedCUBA([batched.SweepNetwork(600, 480, 7, {"we": 1.62e-3})], model=model())
+    B.block, B.steps_per_launch = 1024, 50
+    B.build()
+    B.state["v"][::2] = -0.0495
+    B.state["lastspike"].fill_(-1e7)
+    B.run(150)
+    c = synth.cuba_network(N=600, NE=480, seed=7, we=1.62e-3, network_options={"tile": 256})
+    spec = c["G"].su
+    spec.scalar = [dict(st) for st in spec.scalar]
+    spec.scalar[0]["expr"] = f"timestep({steps!r} * dt, dt)"
+    v = c["G"].get("v")
+    v[::2] = -0.0495
+    c["G"].v = v
+    c["G"].lastspike = -1e7
+    c["net"].run(150)
+    i, s = B.spikes(0)
+    assert len(i) >= 300 and np.bincount(i).max() == 1
+    assert np.array_equal(i, c["mon"].i) and np.array_equal(s, c["mon"].step)
+    for x in ("v", "ge", "gi", "lastspike", "not_refractory"):
+        assert np.array_equal(B.get(x, 0), c["G"].get(x)), x

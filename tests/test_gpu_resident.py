@@ -127,3 +127,29 @@ def test_networks_that_are_not_taken():
               synth.cobahh_network(N=1000), synth.cuba_network(N=9000)):
         c["net"].run(2)
         assert c["net"].resident is None
+
+
+@pytest.mark.parametrize("steps", [2**31 - 2, 2**31 - 1, 2**31, 3 * 10**9])
+def test_refractory_periods_beyond_32_bits(steps):
+    """Neurons that fire once: a period whose steps, or whose release step counted from a
+    launch's beginning, take more than 32 bits."""
+    from brian2_amd import Model, Network, NeuronGroup, SpikeMonitor, Synapses
+
+    out = []
+    for options in ({}, {"tile": 256}):
+        m = Model.load("cuba")
+        m.group["stateupdate"].scalar[0]["expr"] = f"timestep({steps!r} * dt, dt)"
+        G = NeuronGroup(200, m, name="g")
+        G.v = np.linspace(-0.06, -0.04, 200)
+        G.lastspike = -1e7
+        S = Synapses(G, G, _const_spec("ge", "+=", 1.62e-3))
+        S.connect(*np.nonzero(np.random.default_rng(1).random((200, 200)) < 0.2))
+        mon = SpikeMonitor(G)
+        net = Network(G, S, mon, dt=1e-4, **options)
+        for k in (100, 1, 99):
+            net.run(k)
+        assert (net.resident is not None) == (not options)
+        out.append([mon.i, mon.step] + [G.get(v) for v in STATE])
+    assert len(out[1][0]) > 100 and np.bincount(out[1][0]).max() == 1
+    for x, y in zip(*out):
+        assert np.array_equal(x, y)
