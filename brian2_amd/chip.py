@@ -204,8 +204,7 @@ class ChipSteps:
             "        }",
             "    };",
             "    // the events of the step before step hb_s of the launch, applied (hb_ok: no workgroup missing)",
-            "    auto hb_events = [&](const int hb_s, const double t) {",
-            "        (void)t;",
+            "    auto hb_events = [&](const int hb_s) {",
             f"        unsigned int hb_n[{R}];",
         ]
         if W > 1:
@@ -226,11 +225,12 @@ class ChipSteps:
         for r, (var, op, val, _, _) in enumerate(self.pathways):
             k.append(f"        for (unsigned int n_ = hb_n[{r}]; n_ > 0u; n_--) {var} {op} {val};")
         if mode == "deferred":
-            k += ["        if (hb_cond) { // reset of the step before, after its propagation"]
+            k += ["        if (hb_cond) { // reset of the step before, after its propagation, at its time",
+                  "            const double t = (double)(p.step0 + hb_s - 1) * dt;", "            (void)t;"]
             k += ["            " + x for x in block("rs", g.rs)] + ["        }"]
         k += ["    };", "    for (int hb_s = 0; hb_s < p.n_steps; hb_s++) {", "        const long long hb_step = p.step0 + hb_s;",
               "        const double t = (double)hb_step * dt;", "        (void)t;",
-              "        if (hb_s > 0) { hb_events(hb_s, t); if (!hb_ok) return; }"]
+              "        if (hb_s > 0) { hb_events(hb_s); if (!hb_ok) return; }"]
         if g.stmon:
             row = "(hb_step - p.rec_row0)" if g.stmon.when == "start" else "(hb_step - 1 - p.rec_row0)"
             k += ["        " + x for x in record_lines(g, first, row)]
@@ -292,7 +292,8 @@ class ChipSteps:
             "    }",
             "    {  // the last step's events, and the state back to memory",
             "        const long long hb_step = p.step0 + p.n_steps;",
-            "        hb_events(p.n_steps, (double)hb_step * dt);",
+            "        hb_events(p.n_steps);",
+            "        (void)hb_step;",
             "        if (!hb_ok) return;",
         ]
         if g.stmon and g.stmon.when == "end":

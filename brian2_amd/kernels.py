@@ -726,7 +726,9 @@ class NeuronKernel:
             body.append(f"{'bool' if ct == 'bool' else ct} {v} = hb_a_{v}[q];")
         body.append("bool hb_cond = false;")
         if self.reset_mode == "deferred":
-            body.append("if (p.spiked[i]) { // reset of the previous step (after its propagation)")
+            body.append("if (p.spiked[i]) { // reset of the previous step (after its propagation), at its time")
+            body.append("    const double t = (double)(step - 1) * p.dt;")
+            body.append("    (void)t;")
             body += ["    " + x for x in self._block("rs", self.rs, {})]
             body.append("}")
         if self.statemon and (not self.flush or self.statemon_when == "end"):

@@ -91,3 +91,35 @@ def test_parts_of_an_update():
                      "blocks": {"None": {"scalar": [], "vector": code, "conditional_write": {}}}})
     assert split_update(spec, 4) == [[0, 1], [2, 5]]
     assert split_update(spec, 1) == [[0, 1, 2, 5]]
+
+
+@pytest.mark.parametrize("n, delay, options, form", [(300, 0.0, {}, "chip"), (300, 0.0, {"tile": 256}, "staged"),
+                                                     (300, 0.0, {"tile": 64, "npt": 2}, "staged"),
+                                                     (6000, 3e-4, {}, "fused")])
+def test_a_reset_that_follows_the_events_has_its_steps_time(n, delay, options, form):
+    """A reset that writes a variable of the pathways runs behind them; the time that it reads
+    is that of the spike, in the steps of a run and at its end."""
+    from brian2_amd import Model, Network, NeuronGroup, SpikeMonitor, Synapses
+
+    rng = np.random.default_rng(4)
+    m = Model.load("cuba")
+    rs = m.group["reset"]
+    rs.vector = rs.vector + [dict(var="ge", op="=", expr="0.0", dtype="float64"),
+                             dict(var="tlast", op="=", expr="t", dtype="float64")]
+    rs.variables = dict(rs.variables, t=m.group["stateupdate"].variables["t"])
+    G = NeuronGroup(n, m, name="g", variables={"tlast": "float64"})
+    G.v = -0.06 + 0.02 * rng.random(n)
+    G.tlast = -1.0
+    S = Synapses(G, G, _const_spec(*E))
+    S.connect(*np.nonzero(rng.random((n, n)) < 30.0 / n))
+    S.set_delay(delay)
+    mon = SpikeMonitor(G)
+    net = Network(G, S, mon, dt=1e-4, **options)
+    want = np.full(n, -1.0)
+    for k in (1, 60, 139):
+        net.run(k)
+        want[mon.i] = mon.step * 1e-4
+        assert (G.pull is not None) == (form == "chip") and (getattr(G, "fused", None) is not None) == (form == "fused")
+        assert np.array_equal(G.get("tlast"), want)
+        assert np.array_equal(G.get("lastspike")[want >= 0], want[want >= 0])
+    assert (want >= 0).sum() > n // 4 and (want == 199 * 1e-4).any() == (199 in mon.step)
