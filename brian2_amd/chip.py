@@ -50,12 +50,13 @@ def place_lines(first):
     ]
 
 
-def record_lines(g, first, row):
-    """The recorded variables' values to row `row`, by the threads for which `first` holds."""
+def record_lines(g, first, row, was={}):
+    """The recorded variables' values to row `row`, by the threads for which `first` holds
+    (was: {variable: what holds its value at that point})."""
     nv = len(g.stmon.variables)
     return [f"if ({first} && hb_rec >= 0 && {row} >= 0 && {row} < p.rec_rows) {{",
             f"    double* const o_ = p.rec_buf + (size_t)({row}) * {nv} * p.n_rec + hb_rec;"] + [
-        f"    o_[(size_t){a} * p.n_rec] = (double){v};" for a, v in enumerate(g.stmon.variables)] + ["}"]
+        f"    o_[(size_t){a} * p.n_rec] = (double){was.get(v, v)};" for a, v in enumerate(g.stmon.variables)] + ["}"]
 
 
 class ChipSteps:
@@ -445,6 +446,8 @@ class SumSteps:
             "        }",
             "        __syncthreads();  // (two sets of values in turn: one barrier is enough)",
             "        if (s_late[hb_s & 1] != 0) return;",
+            f"        const {own.target_t} hb_was = {own.target};  // before this step's sum",
+            "        (void)hb_was;",
             "        if (hb_sums) {",
             f"            {own.target_t} hb_acc = ({own.target_t})0;",
             f"            for (unsigned int hb_c = hb_lo; hb_c < hb_hi; hb_c += {CH}u) {{",
@@ -468,8 +471,7 @@ class SumSteps:
         k += ["            }", f"            {own.target} = hb_acc;", "        }"]
         if g.stmon:
             row = "(hb_step - p.rec_row0)" if g.stmon.when == "start" else "(hb_step - 1 - p.rec_row0)"
-            rec = ["        " + x for x in record_lines(g, first, row)]
-            k += rec
+            k += ["        " + x for x in record_lines(g, first, row, {own.target: "hb_was"})]
         k += ["        hb_cond = false;", "        {"] + ["            " + x for x in block("su", g.su)] + ["        }"]
         if g.th is not None:
             k += ["        {"] + ["            " + x for x in block("th", g.th, {"_cond": "bool"})]

@@ -550,7 +550,7 @@ class NeuronKernel:
     def __init__(self, name, N, arrays, float_t, stateupdate=None, threshold=None, reset=None,
                  reset_mode="none", scalars=None, fold=None, lds_cap=0, val_t="double",
                  spikemon=None, statemon=None, flush=False, uses_refractory=False, statemon_when="start",
-                 tile=256, npt=1, ratemon=None, waves_per_eu=0, ring_parts=None, share=1, summed=None):
+                 tile=256, npt=1, ratemon=None, waves_per_eu=0, ring_parts=None, share=1, summed=None, sums_before=()):
         self.name = name
         self.N = N
         self.arrays = arrays          # {var: ctype} of the group's state arrays
@@ -581,6 +581,9 @@ class NeuronKernel:
         if npt < 1 or tile * npt > 65536:
             raise ValueError("a tile holds at most 65536 neurons")
         self.summed = summed          # OwnSum: a summed variable of this group formed here, or None
+        # recorded variables that a launch before this one has summed anew: a monitor's row has the
+        # step's start or the last step's end, which is their value before (p.was_<variable>)
+        self.sums_before = [v for v in sums_before if not flush and statemon and v in statemon]
         if share < 1 or tile % share or (share > 1 and (npt > 1 or (fold and tile // share < 64))):
             raise ValueError("share divides the tile's threads, of one neuron each")
         if summed is not None and share != 64:
@@ -614,6 +617,8 @@ class NeuronKernel:
             ps.val("stg_stride", "unsigned long long")
         if self.summed:
             self.summed.fields(ps)
+        for v in self.sums_before:
+            ps.ptr(f"was_{v}", self.arrays[v])
         if self.reset_mode == "deferred":
             ps.ptr("spiked", "unsigned char")
         ps.ptr("status", "int")
@@ -684,7 +689,12 @@ class NeuronKernel:
                 k.append(f"        hb_a_{v}[q] = act ? p.a_{v}[i] : ({ct})0;")
         k.append("        hb_condq[q] = false;")
         k.append("    }")
+        was = {v: f"p.was_{v}[i]" for v in self.sums_before}
         if self.summed:
+            v = self.summed.target
+            k.append(f"    const {self.summed.target_t} hb_was = hb_a_{v}[0];  // before this step's sum")
+            k.append("    (void)hb_was;")
+            was[v] = "hb_was"
             k += self.summed.lines(T)
         if self.fold:
             fk, U, W = fold[1], fold[2], fold[3]
@@ -744,7 +754,7 @@ class NeuronKernel:
                 "    if (lo < hb_rhi && p.rec_idx[lo] == i && row >= 0 && row < p.rec_rows) {",
             ]
             for a_, v in enumerate(self.statemon):
-                body.append(f"        p.rec_buf[((size_t)row * {nv} + {a_}) * p.n_rec + lo] = (double){v};")
+                body.append(f"        p.rec_buf[((size_t)row * {nv} + {a_}) * p.n_rec + lo] = (double){was.get(v, v)};")
             body += ["    }", "}"]
         if not self.flush:
             if self.su is not None:
@@ -773,6 +783,7 @@ class NeuronKernel:
             if v in kept:
                 body.append(("if (hb_cond) " if v in at_spikes else "")
                             + (f"p.a_{v}[i] = {v} ? 1 : 0;" if ct == "bool" else f"p.a_{v}[i] = {v};"))
+        body += [f"p.was_{v}[i] = {v};" for v in self.sums_before]
         if self.summed:
             body += [f"p.z_x_{v}[(size_t)((step + 1) & 1) * N + i] = {v};" for v in self.summed.shared]
         body.append("hb_condq[q] = hb_cond;")

@@ -853,6 +853,7 @@ class Network:
         self.in_launch = None  # what runs many steps in a launch, or None
         for g in groups:
             g.pull = g.own_sum = None
+            g.was = {}
         # heavy updates rather over the whole chip than in one workgroup (GroupStep.takes)
         if ((_resident.GroupStep.too_heavy(groups) and self._build_pull(groups, paths))
                 or self._build_resident(groups, paths) or self._build_targets(groups, paths)
@@ -1368,6 +1369,8 @@ class Network:
             g.spiked = zeros(g.N, "bool")
         self._monitors(g)
 
+        sums_before = sorted({v for s in self.summed_syn if s.target is g and g.own_sum is None for v in s.summed})
+
         def step_kernel(waves):
             return NeuronKernel(g.name, g.N, g.vars, g.float_t, g.su, g.th, g.rs, mode, scalars, fold,
                                 getattr(g, "lds_cap", 0), getattr(g, "val_t", "double"),
@@ -1376,7 +1379,7 @@ class Network:
                                 uses_refractory=g.uses_refractory,
                                 statemon_when=g.stmon.when if g.stmon else "start", tile=g.block, npt=g.npt,
                                 ratemon=g.rmon.range if g.rmon else None, waves_per_eu=waves,
-                                ring_parts=g.ring_parts, share=g.share, summed=g.own_sum)
+                                ring_parts=g.ring_parts, share=g.share, summed=g.own_sum, sums_before=sums_before)
 
         # two workgroups of 1024 threads per CU need at most 64 VGPRs: keep that build only
         # if the compiler fits it without spilling
@@ -1392,6 +1395,7 @@ class Network:
                 g.fn = D.function(K.source, K.kernel_name)
         g.kernel = K
         g.struct_cls = K.struct.ctypes_struct()
+        g.was = {v: zeros(g.N, g.vars[v]) for v in K.sums_before}
         if g.smon:
             self._alloc_spike_monitor(g, g.smon)
         if g.stmon:
@@ -1497,6 +1501,7 @@ class Network:
             v[f"{tg}_{n}"] = val
         if g.own_sum is not None:
             v.update(g.sum_args)
+        v.update({f"was_{n}": t.data_ptr() for n, t in g.was.items()})
         if g.incoming:
             v.update(stg_rec=g.stg_rec.data_ptr(), stg_ord=g.stg_ord.data_ptr(),
                      tile_off=g.tile_off.data_ptr(), tile_cnt=g.tile_cnt.data_ptr(), n_tiles=g.n_tiles,
@@ -1664,8 +1669,10 @@ class Network:
 
     def _copy_read_state(self):
         """What the groups' own sums read, as it is between runs, to its copies: the sources'
-        variables, and the synapses' by target."""
+        variables, and the synapses' by target.  And the recorded sums' values before a step."""
         for g in self.groups:
+            for v, t in getattr(g, "was", {}).items():
+                t.copy_(g._dev[v])
             if getattr(g, "own_sum", None) is not None:
                 if self.in_launch is None:
                     for v, t in g.copies.items():

@@ -143,3 +143,54 @@ def test_own_sums_in_a_launch_and_launch_by_launch(n, t, float_t, when, monkeypa
     assert n == 1 or len(want[2]) > 0
     for x, y, z in zip(got, want, alone):
         assert np.array_equal(x, y) and np.array_equal(z, y)
+
+
+@pytest.mark.parametrize("when", ["start", "end"])
+@pytest.mark.parametrize("form", ["all steps in a launch", "its own step", "a wave per target", "a thread per target",
+                                  "another group"])
+def test_recorded_sums_are_those_of_the_monitors_point(form, when, monkeypatch):
+    """A step forms the sums first.  A monitor at the step's start has the sum of the step before,
+    one at its end the step's own: the sequential fold of the states recorded beside it, however
+    the steps are cut into runs."""
+    from brian2_amd import Model, Network, NeuronGroup, StateMonitor, Synapses, chip
+    from brian2_amd.kernels import SummedKernel
+
+    n = 70
+    if form == "its own step":
+        monkeypatch.setattr(chip.SumSteps, "takes", classmethod(lambda *x: False))
+    if form == "a thread per target":
+        monkeypatch.setattr(SummedKernel, "lanes_for", staticmethod(lambda *x: 1))
+    rng = np.random.default_rng(9)
+    pre, post = np.nonzero(rng.random((n, n - 5)) < 0.7)  # five neurons that are no targets
+    v0, w = 1.3 * rng.random(n), 6.0 / n * rng.random(len(pre))
+    rows = []
+    for pieces in ((40,), (1, 19, 20)):
+        m = Model.load("gap")
+        H = NeuronGroup(n, m, name="h")
+        H.v = v0
+        H.Igap = 0.25
+        G = H
+        if form == "another group":
+            G = NeuronGroup(n, Model.load("gap"), name="g")
+            G.v = v0[::-1]
+        S = Synapses(G, H[:n - 5], summed={"Igap": m.summed["Igap"]})
+        S.connect(pre, post)
+        S.set("w", w)
+        mons = {x: StateMonitor(x, ["v", "Igap"], record=np.arange(n), when=when) for x in {G, H}}
+        net = Network(*{G, H}, S, *mons.values(), dt=1e-4, **({"tile": 256} if form == "a wave per target" else {}))
+        for k in pieces:
+            net.run(k)
+        assert (net.in_launch is not None) == (form == "all steps in a launch")
+        assert (H.own_sum is not None) == (form in ("all steps in a launch", "its own step"))
+        (vh, ih), vg = mons[H].values(), mons[G].values()[0]
+        rows.append(ih)
+        # the states that step s's sums read: recorded at its start, or at the end of step s - 1
+        for s in range(39):
+            want = np.full(n, 0.25)
+            want[:n - 5] = 0.0
+            for i, j, x in zip(pre, post, w):
+                want[j] = want[j] + x * (vg[i, s] - vh[j, s])
+            assert np.array_equal(ih[:, s + 1], want), s
+        if when == "start":
+            assert np.array_equal(ih[:, 0], np.full(n, 0.25))
+    assert np.array_equal(*rows)
