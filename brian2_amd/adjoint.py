@@ -28,14 +28,16 @@ dt*dt/du, dt*dt/dv at the crossing step; lam_v = A lam_u, lam_I = B lam_u +
 beta lam_I'; weight gradients are event-based: dL/dw_ij += lam_I'_j at every
 step where source i spiked.  Spikes themselves carry no gradient (a
 perturbation that creates or deletes no spike leaves them unchanged).  The
-state is kept at the start of every block of a few steps (runs whose states
-would take more than KEEP_BYTES: every `ckpt_every` steps); the backward pass
-recomputes a block forward from there, then walks it in reverse.  Weight
+state is kept at the start of every block of a few steps (or, where that is
+too much memory, of every `ckpt_every` steps or not at all: LIFNetwork._form);
+the backward pass recomputes a block forward from there, then walks it in
+reverse.  Weight
 gradients accumulate per trial (no atomics) and are summed over trials in a
 fixed order.
 """
 import ctypes
 import os
+import weakref
 
 import numpy as np
 
@@ -50,7 +52,7 @@ S_RATE, S_POISSON, S_CONN_IN, S_CONN_REC, S_W_IN, S_W_REC, S_V0_LIF, S_TARGET = 
 LIF = dict(N=1000, NE=800, n_in=200, tau_m=0.02, tau_s=0.005, theta=0.01, bias=0.0105, p=0.1,
            rate_lo=5.0, rate_hi=50.0, w_scale=0.5e-3, n_steps=2000, n_readout=10, t_ref=0.01, c_v=0.1)
 BLOCK = 1024
-KEEP_BYTES = 4 << 30  # up to which the forward pass keeps the states at every block of the backward pass
+KEEP_BYTES = 4 << 30  # that a network's losses hold for their backward passes at most, all together
 
 
 def _torch():
@@ -135,9 +137,13 @@ def _linear_map(torch, spec, consts, dt):
 
 
 class LIFNetwork:
-    """Trials of the differentiable LIF network on the device (see module doc)."""
+    """Trials of the differentiable LIF network on the device (see module doc).
 
-    def __init__(self, trials=256, seed=SEED, config=None, weight_dtype="float", ckpt_every=100):
+    keep_bytes: device memory that the network's losses may hold for their backward passes,
+    all together (default KEEP_BYTES); a loss beyond that is simulated again by its backward
+    pass (_form)."""
+
+    def __init__(self, trials=256, seed=SEED, config=None, weight_dtype="float", ckpt_every=100, keep_bytes=None):
         torch = _torch()
         self.c = dict(LIF if config is None else config)
         c = self.c
@@ -152,6 +158,8 @@ class LIFNetwork:
         self.seed = int(seed)
         self.dt = 1e-4
         self.wt = weight_dtype
+        self.keep_bytes = KEEP_BYTES if keep_bytes is None else int(keep_bytes)
+        self._held = []  # weak references to the tensors held for backward passes
         self._shape()
         self._kernels()
         inp = lif_inputs(self.B, seed, c)
@@ -181,7 +189,7 @@ class LIFNetwork:
         self.targets = dev(inp["targets"], np.float64)
         self._inp_fn = self.D.function(self.fwd_source, "lif_inputs")
         self._fwd_fn = self.D.function(self.fwd_source, "lif_forward")
-        self._bwd_fn = self.D.function(self.bwd_source, "lif_backward")
+        self._bwd_fns = {self.keep: self.D.function(self.bwd_source, "lif_backward")}
 
     # ------------------------------------------------------------------ kernels
     def _shape(self):
@@ -197,10 +205,31 @@ class LIFNetwork:
         words = sum(self._words())
         step = 16 * self.block * self.per_thread + 2 * 64 * words
         self.sub = max(1, min(8, self.block // words, (LDS_BYTES - 4096) // step))
-        # the states at the blocks' starts: kept by the forward pass, or recomputed from the
-        # intervals' checkpoints (_bwd_source)
         self.n_sub = -(-self.C // self.sub)
-        self.keep = 16 * self.B * self.S * self.n_sub * self.N <= KEEP_BYTES
+        # whether the states at the blocks' starts are kept, if there is room (_form)
+        self.keep = self._bytes(self.sub) <= self.keep_bytes
+
+    def _bytes(self, every):
+        """What a loss holds with the state kept at every so many steps of an interval: the
+        states, and every spike."""
+        return self.B * (16 * self.S * -(-self.C // every) * self.N + 8 * self.T * sum(self._words()))
+
+    def _form(self, held=True):
+        """Steps of an interval from one kept state to the next: of a block (`sub`), of the
+        whole interval (`C`), or 0, no state.
+
+        The blocks' states (256 trials of 1000 neurons and 2000 steps: 1.11 GB with the spikes)
+        are for a few losses at a time: together with those of other losses alive they stay
+        within keep_bytes, and take a quarter of the device's free memory at most (asked for
+        from 64 MB on).  A loss beyond that holds the intervals' states (0.16 GB), then
+        nothing but its weights; the only loss alive always holds the intervals'.  held: whether
+        the states are held from the forward pass to the backward pass."""
+        self._held = [r for r in self._held if r() is not None]
+        alive = [t for t in (r() for r in self._held) if t is not None] if held else []
+        now, need = sum(t.numel() * t.element_size() for t in alive), self._bytes(self.sub)
+        if now + need <= self.keep_bytes and (need < 64 << 20 or 4 * need <= _torch().cuda.mem_get_info()[0]):
+            return self.sub
+        return self.C if now == 0 or now + self._bytes(self.C) <= self.keep_bytes else 0
 
     def _kernels(self):
         """Loads the model's statements and generates both kernel sources."""
@@ -212,7 +241,7 @@ class LIFNetwork:
             raise NotImplementedError("threshold 'v > theta' and reset 'v = 0' expected")
         self.su_code = self._su_lines()
         self.fwd_source = self._fwd_source()
-        self.bwd_source = self._bwd_source()
+        self.bwd_source = self._bwd_source(self.keep)
 
     @classmethod
     def sources(cls, config=None, weight_dtype="float", trials=256, ckpt_every=100):
@@ -220,7 +249,8 @@ class LIFNetwork:
         self = cls.__new__(cls)
         self.c = dict(LIF if config is None else config)
         self.N, self.dt, self.wt = self.c["N"], 1e-4, weight_dtype
-        self.B, self.C, self.S = trials, ckpt_every, self.c["n_steps"] // ckpt_every
+        self.B, self.C, self.T, self.S = trials, ckpt_every, self.c["n_steps"], self.c["n_steps"] // ckpt_every
+        self.keep_bytes = KEEP_BYTES
         self._shape()
         self._kernels()
         return self.fwd_source, self.bwd_source
@@ -261,6 +291,8 @@ class LIFNetwork:
         ps.ptr("ckpt_I", "double", const=backward)
         ps.ptr("fs_step", "int", const=backward)
         if not backward:
+            ps.val("every", "int")    # steps from one kept state to the next, in an interval (0: none)
+            ps.val("n_keep", "int")   # kept states of an interval
             ps.ptr("r_dt", "unsigned long long", const=True)
             ps.ptr("v", "double")
             ps.ptr("I", "double")
@@ -416,7 +448,8 @@ template <typename V> struct hb_rows {{
             "        }",
             "    };",
             "    hb_ahead(0);",
-            "    for (int k = 0, c = 0, sg = 0; k < T; k++) {",
+            "    size_t kept = (size_t)b * p.n_seg * p.n_keep * N;  // place of the next kept state",
+            "    for (int k = 0, c = 0, left = 0; k < T; k++, left--) {  // left: steps to it",
             "        if ((k & 31) == 0) {",
             "            #pragma unroll",
             "            for (int a = 0; a < AHEAD; a++) {",
@@ -426,12 +459,11 @@ template <typename V> struct hb_rows {{
             "            hb_ahead(k + 32);",
             "            if (k > 0) hb_flush(k - 32, 32);",
             "        }",
-            f"        if (c % {self.sub} == 0)  // a block of the backward pass" if self.keep else "        if (c == 0)",
-            "            HB_EACH_Q if (HB_J < N) {",
-            f"                const size_t co = (((size_t)b * p.n_seg + sg) * {self.n_sub} + c / {self.sub}) * N + HB_J;" if self.keep
-            else "                const size_t co = ((size_t)sg * gridDim.x + b) * N + HB_J;",
-            "                p.ckpt_v[co] = v[q]; p.ckpt_I[co] = I[q];",
-            "            }",
+            "        if (left == 0 && p.every > 0) {",
+            "            HB_EACH_Q if (HB_J < N) { p.ckpt_v[kept + HB_J] = v[q]; p.ckpt_I[kept + HB_J] = I[q]; }",
+            "            kept += N;",
+            "            left = p.every;",
+            "        }",
             "        bool cond[HB_Q], fs_any = false;",
             "        double v_prev[HB_Q];",
             "        unsigned long long mine[HB_Q], word = 0ull;",
@@ -505,7 +537,7 @@ template <typename V> struct hb_rows {{
             "            n_spk += __builtin_amdgcn_readlane(x_, 63);",
             "        }",
             "        if (++c == p.n_steps) { // an interval's sum",
-            "            c = 0; sg++;",
+            "            c = 0; left = 1;",
         ]
         k += self._sum_lines(["l2[q]"], "l2_all", 1)
         k += [
@@ -541,16 +573,15 @@ template <typename V> struct hb_rows {{
         ]
         return "\n".join(k) + "\n"
 
-    def _bwd_source(self):
+    def _bwd_source(self, keep):
         """Backward pass of a trial per workgroup, all intervals in one launch.
 
         With the raster the recomputation of an interval is each thread's own: no spike has
         to be exchanged, and the rows of a step are fetched while the step before it is
         computed.  The steps are taken in blocks of SUB: a block's raster words become a
         list of its events in LDS (step and source, in order; a word per thread).  The states
-        at every block's start come from the forward pass (256 trials of 1000 neurons, 2000
-        steps: 1 GB) or, beyond KEEP_BYTES, from a first run through the interval from its
-        checkpoint (sub_v, sub_I); from the last block to the first, its steps' states are
+        at every block's start come from the forward pass (keep) or from a first run through
+        the interval from its checkpoint (sub_v, sub_I); from the last block to the first, its steps' states are
         recomputed into LDS (a column per neuron) and walked in reverse.  The adjoint of I is kept in the
         state's place, and the block's weight gradients follow: a wave adds it to the
         synapses of its sources that spiked, in descending step order.
@@ -699,7 +730,7 @@ template <typename V> struct hb_rows {{
             "            }",
             "    };",
         ]
-        if self.keep:
+        if keep:
             k += [
                 "    unsigned long long w_next = hb_word(p.n_seg - 1, n_sub - 1);  // of the block to come (read ahead)",
                 "    // the states at the start of the block to come, read a block ahead",
@@ -724,7 +755,7 @@ template <typename V> struct hb_rows {{
             k += [
                 "    unsigned long long w_next = hb_word(p.n_seg - 1, 0);  // of the block to come (read ahead)",
                 "    for (int sg = p.n_seg - 1; sg >= 0; sg--) {",
-                "        const size_t co = ((size_t)sg * gridDim.x + b) * N + threadIdx.x;",
+                "        const size_t co = ((size_t)b * p.n_seg + sg) * N + threadIdx.x;",
                 f"        HB_EACH_Q {{ v[q] = HB_J < N ? p.ckpt_v[co + q * {T}] : 0.0; I[q] = HB_J < N ? p.ckpt_I[co + q * {T}] : 0.0; }}",
                 "        const size_t so = (size_t)b * n_sub * N + threadIdx.x;",
                 "        for (int sb = 0; sb < n_sub - 1; sb++) {",
@@ -818,54 +849,63 @@ template <typename V> struct hb_rows {{
             v[f"su_{n}"] = x
         return v
 
-    def forward(self, w_in, w_rec, tau_m, tau_s, record_spikes=False, spike_cap=200000, linearise=False):
+    def forward(self, w_in, w_rec, tau_m, tau_s, record_spikes=False, spike_cap=200000, linearise=False, keep=True):
         """Runs all trials; returns (loss, saved) where saved holds what the backward
-        pass needs (checkpoints, first-spike records).  linearise: with the neurons' linear
+        pass needs (states, spikes, first-spike records).  linearise: with the neurons' linear
         map, which the host then forms while the device runs the steps.  With that, the
         scalars formed once and fewer copies back, 9 trials take 2.24 ms forward and
-        backward instead of 2.74."""
+        backward instead of 2.74.  keep: whether a backward pass will follow (without states
+        and spikes it simulates again)."""
         torch = _torch()
         w_in = w_in.detach().to(self.w_in0.dtype).contiguous()
         w_rec = w_rec.detach().to(self.w_rec0.dtype).contiguous()
         sc, consts = self._scalars(tau_m, tau_s)
-        B, N, R = self.B, self.N, self.R
-        v = self.v0.clone()
-        I = torch.zeros_like(v)
-        ckpt_v = torch.empty((B, self.S, self.n_sub, N) if self.keep else (self.S, B, N), dtype=torch.float64, device="cuda")
-        ckpt_I = torch.empty_like(ckpt_v)
-        fs_step = torch.full((B, R), -1, dtype=torch.int32, device="cuda")
-        fs_vprev = torch.zeros((B, R), dtype=torch.float64, device="cuda")
-        fs_u = torch.zeros_like(fs_vprev)
-        l2 = torch.zeros(B, dtype=torch.float64, device="cuda")
-        vals = self._base_vals(sc)
         dense = torch.zeros(self.dense_size, dtype=w_in.dtype, device="cuda")
         dense[self.in_at] = w_in
         dense[self.rec_at] = w_rec
-        raster = torch.empty((B, self.T, sum(self._words())), dtype=torch.int64, device="cuda")
-        vals.update(dense=dense.data_ptr(), raster=raster.data_ptr(), r_dt=self.r_dt.data_ptr(), v=v.data_ptr(),
-                    I=I.data_ptr(), ckpt_v=ckpt_v.data_ptr(), ckpt_I=ckpt_I.data_ptr(), fs_step=fs_step.data_ptr(),
-                    fs_vprev=fs_vprev.data_ptr(), fs_u=fs_u.data_ptr(), l2=l2.data_ptr())
+        saved = dict(w_in=w_in, w_rec=w_rec, dense=dense, tau_m=tau_m, tau_s=tau_s, scalars=(sc, consts))
+        spk = None
         if record_spikes:
-            spk_i = torch.zeros((B, spike_cap), dtype=torch.int32, device="cuda")
-            spk_step = torch.zeros_like(spk_i)
-            spk_n = torch.zeros(B, dtype=torch.int64, device="cuda")
-            vals.update(spk_i=spk_i.data_ptr(), spk_step=spk_step.data_ptr(), spk_n=spk_n.data_ptr(),
-                        spk_cap=spike_cap)
+            spk_i = torch.zeros((self.B, spike_cap), dtype=torch.int32, device="cuda")
+            spk = (spk_i, torch.zeros_like(spk_i), torch.zeros(self.B, dtype=torch.int64, device="cuda"), spike_cap)
+        sim = self._simulate(dense, sc, self._form() if keep else 0, spk)
+        saved.update(sim)
+        if sim["every"]:
+            self._held += [weakref.ref(sim[n]) for n in ("ckpt_v", "ckpt_I", "raster")]
+        else:
+            saved["raster"] = None
+        saved["lin"] = linear_map(self.su, consts, self.dt) if linearise else None
+        loss, saved["parts"] = self._loss(*(sim[n] for n in ("fs_step", "fs_vprev", "fs_u", "l2")))
+        if record_spikes:
+            si, ss, n = (x.cpu().numpy() for x in spk[:3])
+            if (n > spike_cap).any():
+                raise _lib.HipBrianError("spike record buffer overflow")
+            saved["spikes"] = [(si[b, :n[b]].copy(), ss[b, :n[b]].astype(np.int64)) for b in range(self.B)]
+        return loss, saved
+
+    def _simulate(self, dense, sc, every, spk=None):
+        """Runs all trials with the states kept as `every` says (_form); spk: (indices, steps,
+        numbers, room) of the spike records.  Returns what the steps leave."""
+        torch = _torch()
+        B, N, R = self.B, self.N, self.R
+        v = self.v0.clone()
+        n_keep = -(-self.C // every) if every else 0
+        ckpt_v = torch.empty((B, self.S, n_keep, N), dtype=torch.float64, device="cuda")
+        fs_vprev = torch.zeros((B, R), dtype=torch.float64, device="cuda")
+        out = dict(v=v, I=torch.zeros_like(v), ckpt_v=ckpt_v, ckpt_I=torch.empty_like(ckpt_v),
+                   fs_step=torch.full((B, R), -1, dtype=torch.int32, device="cuda"), fs_vprev=fs_vprev,
+                   fs_u=torch.zeros_like(fs_vprev), l2=torch.zeros(B, dtype=torch.float64, device="cuda"),
+                   raster=torch.empty((B, self.T, sum(self._words())), dtype=torch.int64, device="cuda"))
+        vals = self._base_vals(sc)
+        vals.update(every=every, n_keep=n_keep, dense=dense.data_ptr(), r_dt=self.r_dt.data_ptr(),
+                    **{n: t.data_ptr() for n, t in out.items()})
+        if spk is not None:
+            vals.update(spk_i=spk[0].data_ptr(), spk_step=spk[1].data_ptr(), spk_n=spk[2].data_ptr(), spk_cap=spk[3])
         cls = self.fwd_struct.ctypes_struct()
         waves = B * -(-self.T // 16) * self._words()[0]  # of lif_inputs
         self._launch(self._inp_fn, cls, vals, -(-waves // (self.block // 64)))
         self._launch(self._fwd_fn, cls, vals)
-        lin = linear_map(self.su, consts, self.dt) if linearise else None
-        loss, parts = self._loss(fs_step, fs_vprev, fs_u, l2)
-        saved = dict(w_in=w_in, w_rec=w_rec, dense=dense, raster=raster, tau_m=tau_m, tau_s=tau_s, ckpt_v=ckpt_v, ckpt_I=ckpt_I,
-                     fs_step=fs_step, fs_vprev=fs_vprev, fs_u=fs_u, v=v, I=I, parts=parts, lin=lin, scalars=(sc, consts))
-        if record_spikes:
-            n = spk_n.cpu().numpy()
-            if (n > spike_cap).any():
-                raise _lib.HipBrianError("spike record buffer overflow")
-            si, ss = spk_i.cpu().numpy(), spk_step.cpu().numpy()
-            saved["spikes"] = [(si[b, :n[b]].copy(), ss[b, :n[b]].astype(np.int64)) for b in range(B)]
-        return loss, saved
+        return dict(out, every=every)
 
     def _loss(self, fs_step, fs_vprev, fs_u, l2):
         c, B, N, T = self.c, self.B, self.N, self.T
@@ -884,15 +924,19 @@ template <typename V> struct hb_rows {{
         c, B, N = self.c, self.B, self.N
         sc, consts = saved["scalars"]
         lin = saved["lin"] or linear_map(self.su, consts, self.dt)
-        sub_v = torch.empty((1,) if self.keep else (B, self.n_sub, N), dtype=torch.float64, device="cuda")
+        sim = saved if saved["every"] else self._simulate(saved["dense"], sc, self._form(held=False))
+        keep = sim["every"] == self.sub
+        if keep not in self._bwd_fns:
+            self._bwd_fns[keep] = self.D.function(self._bwd_source(keep), "lif_backward")
+        sub_v = torch.empty((1,) if keep else (B, self.n_sub, N), dtype=torch.float64, device="cuda")
         sub_I = torch.empty_like(sub_v)
         # (a pathway without synapses keeps a place to read)
         g_in = torch.zeros((B, max(1, self.n_syn_in)), dtype=torch.float64, device="cuda")
         g_rec = torch.zeros((B, max(1, self.n_syn_rec)), dtype=torch.float64, device="cuda")
         gacc = torch.zeros((B, 4), dtype=torch.float64, device="cuda")
         vals = self._base_vals(sc)
-        vals.update(dense=saved["dense"].data_ptr(), raster=saved["raster"].data_ptr(),
-                    ckpt_v=saved["ckpt_v"].data_ptr(), ckpt_I=saved["ckpt_I"].data_ptr(),
+        vals.update(dense=saved["dense"].data_ptr(), raster=sim["raster"].data_ptr(),
+                    ckpt_v=sim["ckpt_v"].data_ptr(), ckpt_I=sim["ckpt_I"].data_ptr(),
                     fs_step=saved["fs_step"].data_ptr(), A=lin["A"], B=lin["B"], beta=lin["beta"],
                     coef_fs=grad_out / (B * c["t_ref"] ** 2),
                     coef_v=grad_out * c["c_v"] / (N * self.T * c["theta"] ** 2) / B,
@@ -900,7 +944,7 @@ template <typename V> struct hb_rows {{
                     post_rec=self.post_rec.data_ptr(), sub_v=sub_v.data_ptr(),
                     sub_I=sub_I.data_ptr(), n_syn_in=g_in.shape[1], n_syn_rec=g_rec.shape[1], g_in=g_in.data_ptr(),
                     g_rec=g_rec.data_ptr(), gacc=gacc.data_ptr())
-        self._launch(self._bwd_fn, self.bwd_struct.ctypes_struct(), vals)
+        self._launch(self._bwd_fns[keep], self.bwd_struct.ctypes_struct(), vals)
         gw_in = g_in.sum(0)[:self.n_syn_in]
         gw_rec = g_rec.sum(0)[:self.n_syn_rec]
         ga = gacc.sum(0).cpu().numpy()
@@ -915,12 +959,13 @@ def _make_function():
 
     class LIFLoss(torch.autograd.Function):
         """loss = LIFLoss.apply(net, w_in, w_rec, tau_m, tau_s): forward on the device,
-        backward by the exact adjoint (weights and time constants)."""
+        backward by the exact adjoint (weights and time constants).  recording: whether
+        autograd records operations around the call (inside it, it never does)."""
 
         @staticmethod
-        def forward(ctx, net, w_in, w_rec, tau_m, tau_s):
-            loss, saved = net.forward(w_in, w_rec, float(tau_m), float(tau_s),
-                                      linearise=any(ctx.needs_input_grad))
+        def forward(ctx, net, w_in, w_rec, tau_m, tau_s, recording=True):
+            grad = recording and any(ctx.needs_input_grad)
+            loss, saved = net.forward(w_in, w_rec, float(tau_m), float(tau_s), linearise=grad, keep=grad)
             ctx.net, ctx.saved = net, saved
             ctx.dtypes = (w_in.dtype, w_rec.dtype, tau_m.dtype, tau_s.dtype)
             return torch.tensor(loss, dtype=torch.float64, device=w_in.device)
@@ -930,7 +975,7 @@ def _make_function():
             g_in, g_rec, g_m, g_s = ctx.net.backward(ctx.saved, float(grad))
             d = ctx.dtypes
             return (None, g_in.to(d[0]), g_rec.to(d[1]), torch.tensor(g_m, dtype=d[2], device=grad.device),
-                    torch.tensor(g_s, dtype=d[3], device=grad.device))
+                    torch.tensor(g_s, dtype=d[3], device=grad.device), None)[:len(ctx.needs_input_grad)]
 
     return LIFLoss
 
@@ -943,4 +988,4 @@ def lif_loss(net, w_in, w_rec, tau_m, tau_s):
     global _FN
     if _FN is None:
         _FN = _make_function()
-    return _FN.apply(net, w_in, w_rec, tau_m, tau_s)
+    return _FN.apply(net, w_in, w_rec, tau_m, tau_s, _torch().is_grad_enabled())

@@ -187,3 +187,73 @@ def test_kept_and_recomputed_states_give_the_same_gradients(n, every, wt, monkey
         out.append([np.float64(loss), g[0].cpu().numpy(), g[1].cpu().numpy(), g[2], g[3]])
     assert np.abs(out[0][2]).max() > 0
     assert all(np.array_equal(a, b) for a, b in zip(*out))
+
+
+def _leaves(net):
+    import torch
+
+    w = [x.clone().requires_grad_(True) for x in (net.w_in0, net.w_rec0)]
+    return w + [torch.tensor(net.c[k], dtype=torch.float64, requires_grad=True) for k in ("tau_m", "tau_s")]
+
+
+def test_losses_alive_together_hold_bounded_memory():
+    """Losses that are summed before their backward pass: what they hold beside their weights stays
+    within 4 GiB; a loss without a backward pass holds nothing and keeps no states on the way."""
+    import torch
+
+    from brian2_amd import adjoint
+
+    net = adjoint.LIFNetwork(trials=64)
+    states = 16 * 64 * 1000 * 2000 // 8  # of the blocks of the backward pass
+    leaves = _leaves(net)
+    before = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    with torch.no_grad():
+        a = adjoint.lif_loss(net, *leaves)
+    b = adjoint.lif_loss(net, *(x.detach() for x in leaves))
+    assert torch.cuda.max_memory_allocated() - before < states // 4
+    assert torch.cuda.memory_allocated() - before < 1 << 20
+    losses = [adjoint.lif_loss(net, *leaves) for _ in range(24)]
+    assert float(a) == float(b) == float(losses[0]) == float(losses[-1])
+    assert torch.cuda.memory_allocated() - before < (4 << 30) + len(losses) * (8 << 20)
+    first, last = (torch.autograd.grad(x, leaves) for x in (losses[0], losses[-1]))
+    assert all(torch.equal(x, y) for x, y in zip(first, last)) and float(last[1].abs().max()) > 0
+    torch.autograd.backward([sum(losses)])
+    assert all(torch.allclose(x.grad.double(), len(losses) * y.double(), rtol=1e-5, atol=0.0)
+               for x, y in zip(leaves, first))
+    del losses
+    assert torch.cuda.memory_allocated() - before < 32 << 20
+
+
+@pytest.mark.parametrize("n, steps, every, wt", [(65, 56, 7, "float"), (300, 96, 8, "float"), (513, 100, 25, "double")])
+def test_every_form_of_what_is_held_gives_the_same_gradients(n, steps, every, wt):
+    """The blocks' states, the intervals' states and a second simulation; the room that a loss
+    took is there again when it is gone."""
+    import torch
+
+    from brian2_amd import adjoint
+
+    c = dict(adjoint.LIF, N=n, NE=n * 4 // 5, n_steps=steps, tau_m=0.004, bias=0.012, rate_hi=400.0)
+    net = adjoint.LIFNetwork(trials=3, config=c, weight_dtype=wt, ckpt_every=every)
+    net.keep_bytes = net._bytes(net.sub) + net._bytes(net.C)
+    leaves = _leaves(net)
+    with torch.no_grad():
+        values = [float(adjoint.lif_loss(net, *leaves))]
+    for _ in range(2):
+        losses = [adjoint.lif_loss(net, *leaves) for _ in range(4)]
+        held = [x.grad_fn.saved["every"] for x in losses]
+        # (an interval of one block has the same states in both forms)
+        assert held == [net.sub, net.sub if net.sub >= every else every, 0, 0]
+        values += [float(x) for x in losses]
+        with torch.no_grad():
+            for x in leaves[:2]:  # as an optimizer's step between the passes
+                x.mul_(2.0)
+        grads = [torch.autograd.grad(x, leaves) for x in reversed(losses)]
+        with torch.no_grad():
+            for x in leaves[:2]:
+                x.mul_(0.5)
+        for g in grads[1:]:
+            assert all(torch.equal(x, y) for x, y in zip(g, grads[0]))
+        assert float(grads[0][1].abs().max()) > 0
+        del losses
+    assert len(set(values)) == 1
