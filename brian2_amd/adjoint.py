@@ -167,7 +167,9 @@ class LIFNetwork:
         self.D = Device.get()
         dev = lambda a, dt: torch.from_numpy(np.ascontiguousarray(a).astype(dt)).to("cuda")  # noqa: E731
         # U < rate dt for a U of 53 bits over 2^53: the bits below ceil(rate dt 2^53), exactly
-        self.r_dt = dev(np.ceil(np.ldexp(inp["rates"] * self.dt, 53)), np.int64)
+        # (never for a rate below 0 or without a value, always from 1 / dt on)
+        bound = np.ceil(np.ldexp(inp["rates"] * self.dt, 53))
+        self.r_dt = dev(np.where(bound > 0.0, np.minimum(bound, 2.0 ** 53), 0.0), np.int64)
         self.n_syn_in, self.n_syn_rec = len(inp["pre_in"]), len(inp["pre_rec"])
         # places of the synapses in the dense matrix; first synapse and synapses of each row
         niw, nsw = self._words()

@@ -257,3 +257,19 @@ def test_every_form_of_what_is_held_gives_the_same_gradients(n, steps, every, wt
         assert float(grads[0][1].abs().max()) > 0
         del losses
     assert len(set(values)) == 1
+
+
+@pytest.mark.parametrize("rates, same_as", [((-50.0, -1.0), (0.0, 0.0)), ((float("nan"), 1.0), (0.0, 0.0)),
+                                            ((1.5e4, 3e7), (1e4, 1e4))])
+def test_rates_outside_of_a_probabilitys_range(rates, same_as):
+    """A draw is compared with rate dt: a rate below 0 or NaN never spikes, one of 1 / dt and more
+    always."""
+    from brian2_amd import adjoint
+
+    out = []
+    for lo, hi in (rates, same_as):
+        c = dict(adjoint.LIF, N=100, NE=80, n_steps=200, rate_lo=lo, rate_hi=hi, tau_m=0.004, bias=0.012)
+        net = adjoint.LIFNetwork(trials=2, config=c)
+        loss, saved = net.forward(net.w_in0, net.w_rec0, c["tau_m"], c["tau_s"], record_spikes=True)
+        out.append([np.float64(loss)] + [x for pair in saved["spikes"] for x in pair])
+    assert len(out[0][1]) > 0 and all(np.array_equal(x, y) for x, y in zip(*out))
