@@ -330,13 +330,14 @@ class SumSteps:
     @classmethod
     def takes(cls, n, types):
         """Whether a group of n neurons, whose sum reads variables of these types of its sources,
-        is stepped this way: with few values to exchange, as everyone reads them all.
+        is stepped this way: with few values to exchange, as everyone reads them all (and, where
+        the sum reads none, with as few workgroups, which run all at once).
 
         us per step all-to-all against a launch each, fp64 / fp32 (two words or one per neuron):
         50 neurons 3.4 against 4.4 / 2.3 against 4.2, 150 4.1 against 5.5 / 3.3 against 5.0, 300
         5.6 against 5.9 / 4.4 against 5.5, 500 7.5 against 7.2 / 5.7 against 6.9, 1000 13.4
         against 11.0 / 10.2 against 10.1."""
-        return n * sum(2 if ct == "double" else 1 for ct in types) <= cls.WORDS
+        return n * max(1, sum(2 if ct == "double" else 1 for ct in types)) <= cls.WORDS
 
     def __init__(self, group, scalars, own, max_degree):
         g = self.group = group

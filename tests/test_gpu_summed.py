@@ -194,3 +194,28 @@ def test_recorded_sums_are_those_of_the_monitors_point(form, when, monkeypatch):
         if when == "start":
             assert np.array_equal(ih[:, 0], np.full(n, 0.25))
     assert np.array_equal(*rows)
+
+
+@pytest.mark.parametrize("n, own", [(300, True), (768, True), (769, False), (40001, False)])
+def test_sums_that_read_nothing_of_their_sources(n, own):
+    """The sum of a target's weights, say: as with a launch of its own, whatever the size."""
+    from brian2_amd import Model, Network, NeuronGroup, Synapses
+
+    out = []
+    for options in ({}, {"tile": 256}):
+        rng = np.random.default_rng(n)
+        m = Model.load("gap")
+        sp = m.summed["Igap"]
+        sp.vector = [dict(sp.vector[0], expr="w")]
+        G = NeuronGroup(n, m)
+        G.v = 1.3 * rng.random(n)
+        S = Synapses(G, G, summed={"Igap": sp})
+        post = np.repeat(np.arange(n), 24)
+        S.connect(rng.integers(0, n, len(post)), post)
+        S.set("w", rng.random(len(post)) / 24)
+        net = Network(G, S, dt=1e-4, **options)
+        net.run(1)
+        net.run(20)
+        assert (net.in_launch is not None) == (own and not options)
+        out.append([G.get("v"), G.get("Igap")])
+    assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
