@@ -43,6 +43,8 @@ L = _lib.lib
 PULL_NEURONS = 16384  # neurons of a group whose step counts its events itself
 PULL_WORDS = 1 << 23  # words of a pathway's bit matrix (64 MB)
 RESIDENT_STEPS = 2000  # steps of one launch of the resident step (some ms)
+LATE = _chip.LATE
+TRIES = 20  # launches in a row that end so (some seconds each)
 S_POISSON_GROUP = 17  # generator stream of PoissonGroup draws (hb_rng.h)
 SPEC_DIR = os.path.join(os.path.dirname(os.path.abspath(__file__)), "specs")
 
@@ -111,6 +113,12 @@ class Device:
         r, sc, lds = ctypes.c_int(), ctypes.c_int64(), ctypes.c_int64()
         _lib.check(L.hb_function_info(fn, ctypes.byref(r), ctypes.byref(sc), ctypes.byref(lds)), "hb_function_info")
         return r.value, sc.value, lds.value
+
+    def together(self, fn, threads):
+        """Workgroups of a generated kernel that the device runs at once."""
+        n = ctypes.c_int()
+        _lib.check(L.hb_function_together(fn, threads, 0, ctypes.byref(n)), "hb_function_together")
+        return n.value
 
     def spills(self, fn):
         """Whether a generated kernel spills vector registers to memory: by the code object's
@@ -1023,13 +1031,10 @@ class Network:
             s.events_dev = _torch().zeros(n_words, dtype=_torch().int64, device="cuda")
             s.pull_bits = bits
             args[f"bits{r}"], args[f"events{r}"] = bits.data_ptr(), s.events_dev.data_ptr()
-        R = g.pull = _chip.ChipSteps(g, self._group_scalars(g), ops, fields, n_words, self._reset_mode(g))
-        R.grid, R.threads = n_words, 64 * R.waves
-        R.xch = zeros(4 * n_words, "long long")
-        args["xch"] = R.xch.data_ptr()
-        R.args = args
-        R.fn = self.device.function(R.source, R.kernel_name)
-        R.cls = R.struct.ctypes_struct()
+        R = _chip.ChipSteps(g, self._group_scalars(g), ops, fields, n_words, self._reset_mode(g))
+        if not self._together(R, n_words, 64 * R.waves, 4 * n_words, args):
+            return False
+        g.pull = R
         for s in paths:
             s.fused_into = None
         g.flush_fn = None
@@ -1058,6 +1063,18 @@ class Network:
         if int(ones[bits.view(torch.uint8).int()].sum()) != n:
             return None
         return s.src_range[0] + a, b - a, bits
+
+    def _together(self, R, grid, threads, words, args):
+        """The kernel of R and what its workgroups, which wait for each other, exchange through;
+        whether the device runs all of them at once."""
+        R.grid, R.threads = grid, threads
+        R.fn = self.device.function(R.source, R.kernel_name)
+        if grid > self.device.together(R.fn, threads):
+            return False
+        R.cls = R.struct.ctypes_struct()
+        R.xch = zeros(_chip.here_at(words) + _chip.HERE, "long long")
+        R.args = {**args, "xch": R.xch.data_ptr()}
+        return True
 
     def _step_in_launches(self, R):
         """The network's steps come from R, many in a launch: its monitors, and an empty plan."""
@@ -1159,7 +1176,7 @@ class Network:
         for name, _ in R.cls._fields_:
             if name in v:
                 setattr(a, name, v[name])
-        R.xch.zero_()  # no step's number
+        R.xch.zero_()  # no step's number, nobody here
         buf = bytes(a)
         _lib.check(L.hb_launch_together(R.fn, R.grid, R.threads, 0, self.device.stream, buf), "steps over the chip")
         self.clock.fill_(self.t_step + n_steps)
@@ -1730,11 +1747,8 @@ class Network:
         self._make_own_sum(s)
         ptr_ = s.csr["post_ptr"].long()
         R = _chip.SumSteps(g, self._group_scalars(g), g.own_sum, int((ptr_[1:] - ptr_[:-1]).max()))
-        R.xch = zeros(2 * R.n_words * g.N, "long long")
-        R.args = {"xch": R.xch.data_ptr(), **g.sum_args}
-        R.fn = self.device.function(R.source, R.kernel_name)
-        R.cls = R.struct.ctypes_struct()
-        R.threads = 64 * R.WAVES
+        if not self._together(R, R.grid, 64 * R.WAVES, 2 * R.n_words * g.N, g.sum_args):
+            return False
         g.flush_fn = None
         self._step_in_launches(R)
         return True
@@ -2111,7 +2125,7 @@ class Network:
                 if self.in_launch is None:
                     self._set_launch_args(g.launch_index, self._launch_args(g))
         self._copy_read_state()
-        done = 0
+        done = late = 0
         timers = []
         if timing:  # HIP events on the plan's stream around each chunk's launches
             _lib.check(L.hb_plan_timing(self._plan, 1, None, None), "hb_plan_timing")
@@ -2138,8 +2152,17 @@ class Network:
             done += k
             self.t_step += k
             st = int(self.status.cpu().item())  # synchronises
+            if st == LATE:  # nothing has happened: once more
+                done -= k
+                self.t_step -= k
+                self.clock.fill_(self.t_step)
+                self.status.zero_()
+                late += 1
+                if late < TRIES:
+                    continue
             if st:
                 raise _lib.HipBrianError(self._status_message(st))
+            late = 0
         if timing:
             ms, nr = ctypes.c_double(), ctypes.c_int64()
             _lib.check(L.hb_plan_timing(self._plan, 0, ctypes.byref(ms), ctypes.byref(nr)), "hb_plan_timing")
@@ -2248,6 +2271,9 @@ class Network:
             msg.append("spike monitor buffer overflow")
         if st & 16:
             msg.append("a workgroup did not hear from the others (their launch was interrupted)")
+        if st & LATE:
+            msg.append("the workgroups of a launch did not come to run at once (other work holds the device); "
+                       "the network is as it was before the launch")
         if st & 8:
             msg.append("synapse data names a target index outside the target group")
         return "; ".join(msg) or f"device status {st}"

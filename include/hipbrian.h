@@ -85,6 +85,9 @@ int hb_launch(void* fn, unsigned grid, unsigned block, unsigned shmem, void* str
               size_t argsize);
 /* The same for a kernel whose workgroups wait for each other: a cooperative launch,
  * which runs all of them at once or fails.  Not for a captured graph. */
+/* hb_function_together: the workgroups of that shape which the device runs at once when nothing
+ * else runs (0: no cooperative launches). */
+int hb_function_together(void* fn, unsigned block, unsigned shmem, int* workgroups);
 int hb_launch_together(void* fn, unsigned grid, unsigned block, unsigned shmem, void* stream, const void* args);
 
 /* ---- step plans (Network.run hot loop + Clock.advance) ------------------ */

@@ -123,3 +123,83 @@ def test_a_reset_that_follows_the_events_has_its_steps_time(n, delay, options, f
         assert np.array_equal(G.get("tlast"), want)
         assert np.array_equal(G.get("lastspike")[want >= 0], want[want >= 0])
     assert (want >= 0).sum() > n // 4 and (want == 199 * 1e-4).any() == (199 in mon.step)
+
+
+def _waiting_network(form, **options):
+    from brian2_amd import Model, Network, NeuronGroup, PopulationRateMonitor, SpikeMonitor, StateMonitor, Synapses, synth
+
+    if form == "chip":
+        c = synth.cobahh_network(N=1000, record=[3, 70], network_options=options)
+        return c["net"], c["G"], c["mon"], c["state"]
+    rng = np.random.default_rng(2)
+    m = Model.load("gap")
+    G = NeuronGroup(100, m)
+    G.v = 1.3 * rng.random(100)
+    S = Synapses(G, G, summed={"Igap": m.summed["Igap"]})
+    S.connect(np.repeat(np.arange(100), 100), np.tile(np.arange(100), 100))
+    S.set("w", 0.06 * rng.random(10000))
+    mon, state = SpikeMonitor(G), StateMonitor(G, ["v"], record=[3, 70])
+    return Network(G, S, mon, state, PopulationRateMonitor(G), dt=1e-4, **options), G, mon, state
+
+
+@pytest.mark.parametrize("form", ["chip", "sums"])
+def test_a_launch_whose_workgroups_do_not_all_run_changes_nothing(form, monkeypatch):
+    """A launch that misses a workgroup (one more is expected than there are, few polls) ends
+    without a step and is made again; after too many of them a run fails, and the next goes on."""
+    import torch
+
+    from brian2_amd import chip, runtime
+    from brian2_amd._lib import HipBrianError
+
+    def results(x):
+        net, G, mon, state = x
+        return [G.get(v) for v in G.vars] + [mon.i, mon.step, mon.count, state.values(), state.t_]
+
+    a, b = _waiting_network(form), _waiting_network(form)
+    for x in (a, b):
+        x[0].run(60)
+    launches, zero = [], torch.Tensor.zero_
+
+    def run(x):
+        if x is b[0].in_launch.xch:
+            launches.append(1)
+            zero(x)
+            if len(launches) in missing:
+                x[-2], x[-1] = 1, chip.SPINS - 3
+            return x
+        return zero(x)
+
+    a[0].run(50)
+    a[0].run(70)
+    monkeypatch.setattr(torch.Tensor, "zero_", run)
+    missing = {1, 2, 4}
+    b[0].run(50)
+    b[0].run(70)
+    assert len(launches) == 5
+    assert all(np.array_equal(x, y) for x, y in zip(results(a), results(b)))
+    monkeypatch.setattr(runtime, "TRIES", 2)
+    before = [b[1].get(v) for v in b[1].vars] + [b[2].i, b[0].t_step]
+    missing = set(range(100))
+    with pytest.raises(HipBrianError, match="did not come to run"):
+        b[0].run(40)
+    assert all(np.array_equal(x, y) for x, y in zip(before, [b[1].get(v) for v in b[1].vars] + [b[2].i, b[0].t_step]))
+    missing = set()
+    a[0].run(40)
+    b[0].run(40)
+    assert all(np.array_equal(x, y) for x, y in zip(results(a), results(b)))
+
+
+@pytest.mark.parametrize("form", ["chip", "sums"])
+def test_networks_whose_workgroups_do_not_fit_at_once(form, monkeypatch):
+    """As many workgroups as the device says it runs at once, and no more."""
+    from brian2_amd import runtime
+
+    x, y = _waiting_network(form), _waiting_network(form)
+    x[0].run(120)
+    assert x[0].in_launch is not None
+    assert x[0].device.together(x[0].in_launch.fn, x[0].in_launch.threads) % x[0].device.n_cu == 0
+    monkeypatch.setattr(runtime.Device, "together", lambda self, fn, threads: x[0].in_launch.grid - 1)
+    y[0].run(120)
+    assert y[0].in_launch is None or y[0].resident is not None
+    assert len(x[2].i) > 0 and np.array_equal(x[2].i, y[2].i) and np.array_equal(x[2].step, y[2].step)
+    assert all(np.array_equal(x[1].get(v), y[1].get(v)) for v in x[1].vars)
