@@ -14,6 +14,7 @@ import ctypes
 import hashlib
 import json
 import os
+import re
 
 import numpy as np
 
@@ -66,6 +67,16 @@ def torch_dtype(ct):
             "bool": torch.uint8, "unsigned long long": torch.int64, "unsigned int": torch.int32}[ct]
 
 
+def plain_names(source, objects):
+    """A generated source whose identifiers step_<name>, hbp_<name> and the like of the objects
+    named have their numbers instead (@0, @1)."""
+    if not objects:
+        return source
+    own = r"(?<!\w)((?:step|flush|fused|gather|carry|post|summed|resident|chip|sums|targets|hbb_step|hbb_gather|hb_syn|hb[a-z])_)"
+    return re.sub(own + "(" + "|".join(re.escape(x) for x in objects) + r")(?!\w)",
+                  lambda m: f"{m.group(1)}@{objects.index(m.group(2))}", source)
+
+
 # ---------------------------------------------------------------------------
 class Device:
     """One HIP context per process (device 0 unless given)."""
@@ -93,9 +104,16 @@ class Device:
     def stream(self):
         return ctypes.c_void_p(_torch().cuda.current_stream().cuda_stream)
 
-    def function(self, source, name):
-        key = hashlib.sha1(source.encode()).hexdigest()
-        mod = self._modules.get(key)
+    def function(self, source, name, objects=()):
+        """Function `name` of a generated source, which is compiled once per process.
+
+        objects: names of the groups and pathways that the source's own identifiers end in.  A
+        network drawn again has other ones (neurongroup_3 instead of neurongroup) and otherwise
+        the same source: it gets the kernels that are there, under the names of the first."""
+        objects = list(dict.fromkeys(objects))
+        plain = plain_names(source, objects)
+        key = hashlib.sha1(plain.encode()).hexdigest()
+        mod, first = self._modules.get(key, (None, objects))
         if mod is None:
             mod = ctypes.c_void_p()
             log = ctypes.create_string_buffer(1 << 16)
@@ -103,7 +121,8 @@ class Device:
             if rc != 0:
                 raise _lib.HipBrianError("kernel compilation failed:\n" + _lib.last_error() + "\n--- source ---\n"
                                          + source)
-            self._modules[key] = mod
+            self._modules[key] = mod, objects
+        name = re.sub(r"@(\d+)", lambda m: first[int(m.group(1))], plain_names(name, objects))
         fn = ctypes.c_void_p()
         _lib.check(L.hb_module_function(mod, name.encode(), ctypes.byref(fn)), f"function {name}")
         return fn
@@ -1068,7 +1087,7 @@ class Network:
         """The kernel of R and what its workgroups, which wait for each other, exchange through;
         whether the device runs all of them at once."""
         R.grid, R.threads = grid, threads
-        R.fn = self.device.function(R.source, R.kernel_name)
+        R.fn = self.device.function(R.source, R.kernel_name, [R.group.name])
         if grid > self.device.together(R.fn, threads):
             return False
         R.cls = R.struct.ctypes_struct()
@@ -1112,7 +1131,7 @@ class Network:
         R = _resident.GroupStep(g, scalars, consts, g.val_t, n_syn, self.dt)
         R.group, R.scalars, R.consts = g, scalars, consts
         R.row_ptr, R.post = merged
-        R.fn = self.device.function(R.kernel.source, R.kernel.kernel_name)
+        R.fn = self.device.function(R.kernel.source, R.kernel.kernel_name, [g.name])
         R.cls = R.struct.ctypes_struct()
         R.events = _torch().zeros(len(paths), dtype=_torch().int64, device="cuda")
         for r, s in enumerate(paths):
@@ -1147,7 +1166,7 @@ class Network:
         R = _targets.TargetSteps(g, self._group_scalars(g), s.syn_ctypes(), s.plastic, s.spec.vector, s.target_index,
                                  sc[0], s.post_spec.vector, sc[1], s.target_var, s.op, g.val_t)
         R.path, R.gen = s, src
-        R.fn = self.device.function(R.source, R.kernel_name)
+        R.fn = self.device.function(R.source, R.kernel_name, [g.name])
         R.cls = R.struct.ctypes_struct()
         ptr_ = s.csr["post_ptr"].long()
         R.deg = int((ptr_[1:] - ptr_[:-1]).max())
@@ -1320,7 +1339,9 @@ class Network:
         nsrc = s.src_range[1] - s.src_range[0]
         pairs_max = nsrc * s.csr["n_seg"]
         avg = s.csr["n_syn"] / max(1, pairs_max)
-        pc = int(min(_kernels.GATHER_BLOCK, max(32, 0.95 * window / max(avg, 1e-9))))
+        # (a multiple of 16: it is a constant of the kernel, which another draw of the synapses,
+        # some more or less of them, has to find compiled)
+        pc = int(min(_kernels.GATHER_BLOCK, max(32, 0.95 * window / max(avg, 1e-9)))) // 16 * 16
         s.pairs = int(self.gather_pairs or pc)
         s.units_max = -(-pairs_max // s.pairs)
 
@@ -1405,11 +1426,11 @@ class Network:
             K = self._build_fused(g, step_kernel)
         else:
             K = step_kernel(g.waves)
-            g.fn = D.function(K.source, K.kernel_name)
+            g.fn = D.function(K.source, K.kernel_name, [g.name])
             if g.waves and D.spills(g.fn):
                 g.waves = 0
                 K = step_kernel(0)
-                g.fn = D.function(K.source, K.kernel_name)
+                g.fn = D.function(K.source, K.kernel_name, [g.name])
         g.kernel = K
         g.struct_cls = K.struct.ctypes_struct()
         g.was = {v: zeros(g.N, g.vars[v]) for v in K.sums_before}
@@ -1440,7 +1461,7 @@ class Network:
                              uses_refractory=g.uses_refractory,
                              statemon=g.stmon.variables if end_mon else None, statemon_when="end", tile=g.block,
                              npt=g.npt, waves_per_eu=g.waves, share=g.share)
-            g.flush_fn = D.function(F.source, F.kernel_name)
+            g.flush_fn = D.function(F.source, F.kernel_name, [g.name])
             g.flush_struct_cls = F.struct.ctypes_struct()
         else:
             g.flush_fn = None
@@ -1474,7 +1495,7 @@ class Network:
                                  f"{g.name}")
             blocks = [int(max(1, min(b, s.units_max))) for b, s in zip(blocks, g.incoming)]
             F = FusedStepKernel(K, [s.kernel for s in g.incoming], blocks, g.n_tiles, cfg["tiles_first"])
-            fn = D.function(F.source, F.kernel_name)
+            fn = D.function(F.source, F.kernel_name, [g.name] + [s.name for s in g.incoming])
             spills = D.spills(fn) and not cfg["allow_spills"]
             if waves and k + 1 < len(tries) and (spills or F.lds_bytes > LDS_BYTES // 2):
                 continue
@@ -1606,7 +1627,7 @@ class Network:
         self._gather_setup(s)
         if s.carry is not None:
             self._build_carry(s)  # before the gather: both write s's synaptic variables and counters
-        s.fn = self.device.function(s.kernel.source, s.kernel.kernel_name)
+        s.fn = self.device.function(s.kernel.source, s.kernel.kernel_name, [s.name])
         s.events_dev = _torch().zeros(s.grid, dtype=_torch().int64, device="cuda")
         s.args.events = s.events_dev.data_ptr()
         s.launch_index = len(self._launches)
@@ -1771,7 +1792,7 @@ class Network:
             t0, t1 = s.tgt_range
             K = SummedKernel(f"{s.name}_{tv}", sp.vector, used, pre_r, post_r, var_types, g.vars[tv], sc, g.float_t,
                              lanes=SummedKernel.lanes_for(s.csr["n_syn"], t1 - t0))
-            fn = self.device.function(K.source, K.kernel_name)
+            fn = self.device.function(K.source, K.kernel_name, [f"{s.name}_{tv}"])
             cls = K.struct.ctypes_struct()
             v = {"clock": self.clock.data_ptr(), "step_off": 0, "dt": self.dt, "t0": t0, "t1": t1,
                  "post_ptr": s.csr["post_ptr"].data_ptr(), "post_syn": s.csr["post_syn"].data_ptr(),
@@ -1798,7 +1819,7 @@ class Network:
         K = PostPathKernel(s.name, s.post_spec.vector, s.syn_ctypes(), s.plastic, sc, s.target.float_t,
                            s.post_delay_steps, ring_parts=s.target.ring_parts)
         s.post_kernel = K
-        s.post_fn = self.device.function(K.source, K.kernel_name)
+        s.post_fn = self.device.function(K.source, K.kernel_name, [s.name])
         cls = K.struct.ctypes_struct()
         g = s.target
         v = {"clock": self.clock.data_ptr(), "step_off": 0, "dt": self.dt, "ring_spk": g.ring_spk.data_ptr(),
@@ -2065,7 +2086,7 @@ class Network:
         s.carry_ptr = dev(c["ptr"].astype(np.uint32).view(np.int32))
         s.carry_events = _torch().zeros(1, dtype=_torch().int64, device="cuda")
         K = _kernels.CarryKernel(s.kernel)
-        fn = self.device.function(K.source, K.kernel_name)
+        fn = self.device.function(K.source, K.kernel_name, [s.name])
         cls = K.struct.ctypes_struct()
         g = s.target
         v = {"clock": self.clock.data_ptr(), "step_off": 0, "t0": c["t0"], "n_slots": len(c["ptr"]) - 1,

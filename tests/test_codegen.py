@@ -316,3 +316,16 @@ def test_mod_renders_as_the_cython_target():
     assert "hb_imod" in c and t == "int"
     c, t = R("a // b", a="double", b="double")
     assert c.startswith("floor(")
+
+
+def test_sources_are_the_same_but_for_the_names_of_their_objects():
+    """plain_names: only a generated identifier that ends in an object's name, only as a whole."""
+    from brian2_amd.runtime import plain_names
+
+    a = "struct hbp_g { double a_v; }; step_g(hbp_g p) { hbb_gather_s_1(p); g + a_g + my_step_g + step_gg; hb_syn_s x; }"
+    b = a.replace("hbp_g", "hbp_neurons").replace(" step_g(", " step_neurons(").replace("gather_s_1", "gather_t").replace(
+        "hb_syn_s ", "hb_syn_exp ")
+    assert plain_names(a, ["g", "s", "s_1"]) == plain_names(b, ["neurons", "exp", "t"]) != a
+    assert "g + a_g + my_step_g + step_gg" in plain_names(a, ["g", "s", "s_1"])
+    assert plain_names("exp(x) + log(x)", ["exp"]) != plain_names("log(x) + log(x)", ["log"])
+    assert plain_names(a, []) == a

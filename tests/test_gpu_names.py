@@ -85,3 +85,54 @@ def test_awkward_names_of_targets():
     assert len(out[1][1]) > 0
     for x, y in zip(*out):
         assert np.array_equal(x, y)
+
+
+def _drawn(kind, seed, names=None):
+    """A network of a seed's draw, and what a run leaves."""
+    from brian2_amd import Model, Network, NeuronGroup, SpikeGeneratorGroup, SpikeMonitor, StateMonitor, Synapses, synth
+
+    rng = np.random.default_rng(seed)
+    if kind in ("cuba", "staged"):
+        c = synth.cuba_network(N=700, seed=seed, network_options={"tile": 256} if kind == "staged" else {})
+        net, G = c["net"], c["G"]
+    elif kind == "cobahh":
+        c = synth.cobahh_network(N=700, seed=seed)
+        net, G = c["net"], c["G"]
+    elif kind in ("fused", "separate"):
+        c = synth.cuba_synw_network(N=6000, K=1000, seed=seed, network_options={"fuse": kind == "fused"})
+        net, G = c["net"], c["G"]
+    elif kind == "targets":
+        m = Model.load("stdp")
+        step, idx = np.nonzero(rng.random((100, 50)) < 0.1)
+        src = SpikeGeneratorGroup(50, idx, timebins=step)
+        G = NeuronGroup(3, m)
+        G.v = -0.055
+        S = Synapses(src, G, m.pathways["pre"], on_post=m.pathways["post"])
+        S.connect(np.repeat(np.arange(50), 3), np.tile(np.arange(3), 50))
+        S.set("w", 0.05 * rng.random(150))
+        net = Network(src, G, S, SpikeMonitor(G), dt=1e-4)
+    else:
+        m = Model.load("gap")
+        n = 60 if kind == "sums" else 1000
+        G = NeuronGroup(n, m)
+        G.v = 1.3 * rng.random(n)
+        S = Synapses(G, G, summed={"Igap": m.summed["Igap"]})
+        S.connect(rng.integers(0, n, 40 * n), np.repeat(np.arange(n), 40))
+        S.set("w", rng.random(40 * n) / 40)
+        net = Network(G, S, dt=1e-4, **({"tile": 128} if kind == "summed" else {}))
+    net.run(150)
+    return net, [G.get(v) for v in G.vars]
+
+
+@pytest.mark.parametrize("kind", ["cuba", "staged", "cobahh", "fused", "separate", "targets", "sums", "own sum", "summed"])
+def test_a_network_drawn_again_finds_its_kernels_compiled(kind):
+    """Names that the package gives (neurongroup_3) and the draw of the synapses compile nothing
+    anew, and the kernels found are the right ones."""
+    from brian2_amd import runtime
+
+    net, first = _drawn(kind, 1)
+    modules = len(runtime.Device.get()._modules)
+    for seed in (2, 3, 1):
+        net, out = _drawn(kind, seed)
+        assert len(runtime.Device.get()._modules) == modules, seed
+    assert all(np.array_equal(x, y) for x, y in zip(first, out))
