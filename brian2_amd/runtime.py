@@ -10,6 +10,7 @@ State lives in device memory as torch tensors (one per variable, structure of
 arrays); kernels are generated per group/pathway, compiled with hiprtc and
 replayed per step from a hipGraph-captured plan.
 """
+import copy
 import ctypes
 import hashlib
 import json
@@ -813,6 +814,7 @@ class Network:
             raise ValueError("gather_blocks: a list of positive workgroup counts, one per pathway into the group")
         self.t_step = 0
         self._built = False
+        self._apart = False  # a launch per code object, whatever could be one (profile)
         for o in objs:
             self.add(o)
 
@@ -872,7 +874,7 @@ class Network:
             g.ring_parts = tuple(sorted(cuts))
             g.ring_spk = zeros(g.ring_slots * g.N, "int")
             g.ring_cnt = zeros(g.ring_slots * len(g.ring_parts), "int")
-            if isinstance(g, NeuronGroup):
+            if isinstance(g, NeuronGroup) and g._dev is None:
                 g._dev = {n: dev(g._host[n], ct) for n, ct in g.vars.items()}
         for g in groups:
             g.incoming = [s for s in paths if s.target is g]
@@ -882,7 +884,8 @@ class Network:
             g.pull = g.own_sum = None
             g.was = {}
         # heavy updates rather over the whole chip than in one workgroup (GroupStep.takes)
-        if ((_resident.GroupStep.too_heavy(groups) and self._build_pull(groups, paths))
+        if not self._apart and (
+                (_resident.GroupStep.too_heavy(groups) and self._build_pull(groups, paths))
                 or self._build_resident(groups, paths) or self._build_targets(groups, paths)
                 or self._build_pull(groups, paths) or self._build_sums(groups, paths)):
             self._built = True
@@ -2232,7 +2235,8 @@ class Network:
 
     def profile(self, n_steps):
         """Runs n_steps as individual launches timed with HIP events (advances the
-        simulation).  Returns [(kind, name, total_ms)] per launch of the step."""
+        simulation).  Returns [(kind, name, total_ms)] per launch of the step; a network whose
+        runs take many steps in a launch is run with the launches of its code objects instead."""
         if not self._built:
             self._build()
         for g in self.groups:
@@ -2244,8 +2248,7 @@ class Network:
             if getattr(g, "rmon", None) is not None:
                 raise NotImplementedError("profile() of a network with a PopulationRateMonitor")
         if self.in_launch is not None:
-            self.run(n_steps, timing=True)
-            return [("resident", self.in_launch.group.name, self.last_run_gpu_ms)]
+            return self._profile_apart(int(n_steps))
         self._copy_read_state()
         ms = (ctypes.c_float * len(self._launches))()
         _lib.check(L.hb_plan_profile(self._plan, self.device.stream, int(n_steps), ms), "hb_plan_profile")
@@ -2261,6 +2264,35 @@ class Network:
             else:
                 kind = "fused" if getattr(obj, "fused", None) is not None else "step"
                 out.append((kind, obj.name, float(ms[obj.launch_index])))
+        return out
+
+    def _profile_apart(self, n_steps):
+        """profile() by a network of a launch per code object, of the same state: copies of the
+        objects that share their device tensors.  Its records and counts are added to this one's."""
+        self._drain_monitors()
+        twin = Network(dt=self.dt, graph_steps=self.graph_steps, bucket_mem_frac=self.bucket_mem_frac)
+        twin._apart, twin.t_step = True, self.t_step
+        of = {id(o): copy.copy(o) for o in self.objs}
+        for x in of.values():
+            if isinstance(x, Synapses):
+                x.source, x.target, x.csr, x._events_base = of[id(x.source)], of[id(x.target)], dict(x.csr), 0
+            elif isinstance(x, SpikeMonitor):
+                x.source, x._i, x._step, x._t = of[id(x.source)], [], [], []
+            twin.add(x)
+        out = twin.profile(n_steps)
+        twin.run(0)  # folds the last step's events
+        twin._drain_monitors()
+        for o in self.objs:
+            x = of[id(o)]
+            if isinstance(o, SpikeMonitor):
+                o.count_dev += x.count_dev
+                for a in ("_i", "_step", "_t"):
+                    setattr(o, a, getattr(o, a) + getattr(x, a))
+            elif isinstance(o, Synapses) and o.spec is not None:
+                o.events_dev.view(-1)[:1] += x.n_events
+        self.t_step += n_steps
+        self.clock.fill_(self.t_step)
+        _lib.check(L.hb_plan_destroy(twin._plan), "hb_plan_destroy")
         return out
 
     @staticmethod

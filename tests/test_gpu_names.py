@@ -136,3 +136,31 @@ def test_a_network_drawn_again_finds_its_kernels_compiled(kind):
         net, out = _drawn(kind, seed)
         assert len(runtime.Device.get()._modules) == modules, seed
     assert all(np.array_equal(x, y) for x, y in zip(first, out))
+
+
+@pytest.mark.parametrize("kind, launches", [("cuba", ["step", "gather", "gather"]), ("cobahh", ["step", "gather", "gather"]),
+                                            ("targets", ["step", "step", "gather"]), ("sums", ["step"])])
+def test_profiles_of_networks_that_step_in_one_launch(kind, launches):
+    """profile() times the code objects one by one, as for any network, and leaves what a run
+    would: state, records, counts, and what a snapshot restores."""
+    a, b = _drawn(kind, 5)[0], _drawn(kind, 5)[0]
+    assert b.in_launch is not None
+
+    def results(net):
+        out = [g._dev[v].cpu().numpy() for g in net.groups for v in g.vars] + [net.n_events, net.t_step]
+        out += [s.get(v) for s in net.paths for v in s.syn_vars]
+        return out + [x for m in net.smons for x in (m.i, m.step, m.t_, m.count)]
+
+    assert kind == "sums" or len(results(b)[-4]) > 0
+    a.run(60)
+    b.store()
+    for _ in range(2):
+        prof = b.profile(60)
+        assert [k for k, _, _ in prof] == launches and all(ms > 0.0 for _, _, ms in prof)
+        assert [n for _, n, _ in prof] == [o.name for o in list(b.groups) + list(b.paths)]
+        assert all(np.array_equal(x, y) for x, y in zip(results(a), results(b)))
+        b.restore()
+    b.profile(60)
+    a.run(40)
+    b.run(40)
+    assert b.in_launch is not None and all(np.array_equal(x, y) for x, y in zip(results(a), results(b)))
