@@ -187,6 +187,7 @@ class ResidentKernel:
         if released:
             k += [
                 f"    const double hb_tb = {bound};",
+                f"    const unsigned int hb_far = {period} < 0x7fffffffll ? (unsigned int)({period}) : 0x7fffffffu;  // K",
                 "    // a neuron that last spiked at time x is not refractory from the step k on (a double:",
                 "    // exact) at which (k * dt - x) + 1e-3 * dt >= hb_tb, which grows with k",
                 "    auto hb_free = [&](const double x, const double k) { return (k * dt - x) + 1e-3 * dt >= hb_tb; };",
@@ -322,8 +323,8 @@ class ResidentKernel:
                 "            // the release step of a neuron that spikes now: K steps on, or one beside it by rounding;",
                 "            // beyond 32 bits (K is 64 of them) a step that no launch reaches",
                 f"            const double k_ = hb_k + (double)({period});",
-                f"            const long long far_ = hb_s + ({period} < 0x7fffffffll ? (long long)({period}) : 0x7fffffffll);",
-                "            const int rel_ = (far_ < 0x7ffffffell ? (int)far_ : 0x7ffffffe) "
+                "            const unsigned int far_ = (unsigned int)hb_s + hb_far;",
+                "            const int rel_ = (int)(far_ < 0x7ffffffeu ? far_ : 0x7ffffffeu) "
                 "+ (hb_free(t, k_ - 1.0) ? -1 : hb_free(t, k_) ? 0 : 1);",
             ]
         k += ["            #pragma unroll", f"            for (int hb_q = 0; hb_q < {R}; hb_q++) {{",
