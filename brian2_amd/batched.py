@@ -241,7 +241,7 @@ class BatchedCUBA:
             "}",
             "hb_sn += hb_nsp;",
         ]
-        finish = ["if (threadIdx.x == 0) { p.spk_n[net] = hb_sn; if (hb_sn > hb_sc) atomicOr(p.status, 2); }"]
+        finish = ["if (threadIdx.x == 0) { p.spk_n[net] = hb_sn; if (hb_sc && hb_sn > hb_sc) atomicOr(p.status, 2); }"]
         return ResidentKernel(
             "batched_step", self._struct(), self.vars, update,
             [(self.exc_var, "+=", "pe_val"), (self.inh_var, "+=", "pi_val")], prologue,

@@ -179,3 +179,13 @@ def test_refractory_periods_beyond_32_bits(steps):
     assert np.array_equal(i, c["mon"].i) and np.array_equal(s, c["mon"].step)
     for x in ("v", "ge", "gi", "lastspike", "not_refractory"):
         assert np.array_equal(B.get(x, 0), c["G"].get(x)), x
+
+
+def test_a_sweep_without_records_counts_its_spikes():
+    """record_spikes=False: no room for records and no complaint about it; the numbers of spikes
+    and the states are those of a sweep that records."""
+    (_, A), (nets, B) = _sweep(3), _sweep(3, record_spikes=False)
+    A.run(400)
+    B.run(400)
+    assert A.spk_n.sum().item() > 0 and np.array_equal(A.spk_n.cpu().numpy(), B.spk_n.cpu().numpy())
+    assert all(np.array_equal(A.get(v, k), B.get(v, k)) for v in ("v", "ge", "gi") for k in range(len(nets)))
