@@ -50,7 +50,6 @@ _SIGS = {
     "hb_module_unload": ([_vp], _i),
     "hb_module_function": ([_vp, _cp, _P(_vp)], _i),
     "hb_function_together": ([_vp, ctypes.c_uint, ctypes.c_uint, _P(_i)], _i),
-    "hb_launch_together": ([_vp, ctypes.c_uint, ctypes.c_uint, ctypes.c_uint, _vp, _vp], _i),
     "hb_launch": ([_vp, ctypes.c_uint, ctypes.c_uint, ctypes.c_uint, _vp, _vp, _sz], _i),
     "hb_function_info": ([_vp, _P(_i), _P(_i64), _P(_i64)], _i),
     "hb_function_spills": ([_vp, _P(_i), _P(_i)], _i),

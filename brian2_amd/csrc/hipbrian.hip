@@ -294,22 +294,11 @@ extern "C" int hb_launch(void* fn, unsigned grid, unsigned block, unsigned shmem
 extern "C" int hb_function_together(void* fn, unsigned block, unsigned shmem, int* workgroups) {
     const hb_fn* f = (const hb_fn*)fn;
     if (!f || !f->mfn) return set_err("hb_function_together: not a generated kernel");
-    int dev = 0, can = 0, cus = 0, per_cu = 0;
+    int dev = 0, cus = 0, per_cu = 0;
     HB_HIP(hipGetDevice(&dev));
-    HB_HIP(hipDeviceGetAttribute(&can, hipDeviceAttributeCooperativeLaunch, dev));
     HB_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
     HB_HIP(hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, f->mfn, (int)block, shmem));
-    *workgroups = can ? cus * per_cu : 0;
-    return 0;
-}
-
-// A launch whose workgroups all run at once (they wait for each other), or an error.
-extern "C" int hb_launch_together(void* fn, unsigned grid, unsigned block, unsigned shmem, void* stream, const void* args) {
-    const hb_fn* f = (const hb_fn*)fn;
-    if (!f || !f->mfn) return set_err("hb_launch_together: not a generated kernel");
-    if (grid == 0) return 0;
-    void* argv[] = {const_cast<void*>(args)};
-    HB_HIP(hipModuleLaunchCooperativeKernel(f->mfn, grid, 1, 1, block, 1, 1, shmem, (hipStream_t)stream, argv));
+    *workgroups = cus * per_cu;
     return 0;
 }
 

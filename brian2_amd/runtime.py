@@ -1088,7 +1088,11 @@ class Network:
 
     def _together(self, R, grid, threads, words, args):
         """The kernel of R and what its workgroups, which wait for each other, exchange through;
-        whether the device runs all of them at once."""
+        whether the device runs all of them at once.
+
+        An ordinary launch, whose workgroups see for themselves that all of them run
+        (chip.arrival_function): a cooperative one takes the host 20 us more.  Runs of a step, 50
+        neurons with gap junctions 119 against 134 us, 4000 COBAHH neurons 87 against 105."""
         R.grid, R.threads = grid, threads
         R.fn = self.device.function(R.source, R.kernel_name, [R.group.name])
         if grid > self.device.together(R.fn, threads):
@@ -1200,7 +1204,7 @@ class Network:
                 setattr(a, name, v[name])
         R.xch.zero_()  # no step's number, nobody here
         buf = bytes(a)
-        _lib.check(L.hb_launch_together(R.fn, R.grid, R.threads, 0, self.device.stream, buf), "steps over the chip")
+        _lib.check(L.hb_launch(R.fn, R.grid, R.threads, 0, self.device.stream, buf, len(buf)), "steps over the chip")
         self.clock.fill_(self.t_step + n_steps)
 
     def _run_targets(self, n_steps):

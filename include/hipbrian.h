@@ -83,12 +83,9 @@ int hb_code_object_spills(const void* code, size_t nbytes, int* vgpr_spills, int
  * one struct by value whose bytes are `args`). */
 int hb_launch(void* fn, unsigned grid, unsigned block, unsigned shmem, void* stream, const void* args,
               size_t argsize);
-/* The same for a kernel whose workgroups wait for each other: a cooperative launch,
- * which runs all of them at once or fails.  Not for a captured graph. */
-/* hb_function_together: the workgroups of that shape which the device runs at once when nothing
- * else runs (0: no cooperative launches). */
+/* The workgroups of that shape which the device runs at once when nothing else runs (for a
+ * kernel whose workgroups wait for each other).  No counterpart in Brian. */
 int hb_function_together(void* fn, unsigned block, unsigned shmem, int* workgroups);
-int hb_launch_together(void* fn, unsigned grid, unsigned block, unsigned shmem, void* stream, const void* args);
 
 /* ---- step plans (Network.run hot loop + Clock.advance) ------------------ */
 /* A plan is the ordered list of launches of one time step.  `clock` points to a
