@@ -42,7 +42,7 @@ import weakref
 import numpy as np
 
 from . import _lib
-from .codegen import ParamStruct, source_header, translate_block
+from .codegen import ParamStruct, filled, source_header, translate_block
 from .kernels import LDS_BYTES, _rename, scalar_values
 from .runtime import Device, Model
 
@@ -836,11 +836,7 @@ template <typename V> struct hb_rows {{
         return {n: sc[n][0] for n in self.su_scalars}, consts
 
     def _launch(self, fn, cls, vals, grid=None):
-        a = cls()
-        for name, _ in cls._fields_:
-            if name in vals:
-                setattr(a, name, vals[name])
-        buf = bytes(a)
+        buf = bytes(filled(cls, vals))
         stream = ctypes.c_void_p(_torch().cuda.current_stream().cuda_stream)
         _lib.check(L.hb_launch(fn, self.B if grid is None else grid, self.block, 0, stream, buf, len(buf)), "lif launch")
 

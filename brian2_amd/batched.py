@@ -21,7 +21,7 @@ import time
 import numpy as np
 
 from . import _lib
-from .codegen import HostEval, ParamStruct, Renderer, cast_value, ctype_of, translate_block
+from .codegen import HostEval, ParamStruct, Renderer, cast_value, ctype_of, filled, translate_block
 from .kernels import _rename, identifiers
 from .resident import (
     MAX_NEURONS,
@@ -363,11 +363,8 @@ class BatchedCUBA:
             if not K.counts_in_lds and self.counts is None:
                 self.counts = zeros(int(self.n_off[-1]), "int")
             cls = K.struct.ctypes_struct()
-            a = cls()
             v.update(first=first, counts=0 if self.counts is None else self.counts.data_ptr())
-            for name, _ in cls._fields_:
-                if name in v:
-                    setattr(a, name, v[name])
+            a = filled(cls, v)
             buf = bytes(a)
             _lib.check(L.hb_plan_add(self.plan, fn, count, threads, K.lds_bytes(nmax, threads, extra), buf, len(buf),
                                      cls.step_off.offset))

@@ -429,6 +429,15 @@ class ParamStruct:
         return type(self.name, (ctypes.Structure,), {"_fields_": fields})
 
 
+def filled(cls, values):
+    """An argument struct of class cls with the values ({field: value}) of the fields it has."""
+    a = cls()
+    for name, _ in cls._fields_:
+        if name in values:
+            setattr(a, name, values[name])
+    return a
+
+
 PRELUDE = r"""
 __device__ __forceinline__ long long hb_timestep(double t, double dt) { return (long long)((t + 1e-3 * dt) / dt); }
 template <typename T> __device__ __forceinline__ T hb_clip(T v, double lo, double hi) {

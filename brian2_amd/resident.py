@@ -24,6 +24,7 @@ a second one (the counts are complete).
 import math
 import re
 
+from .chip import monitor_fields
 from .codegen import ParamStruct, Renderer, source_header
 from .kernels import _rename, group_block
 from .kernels import heavy_operations as _heavy
@@ -93,7 +94,7 @@ class ResidentKernel:
     record      lines run for a step's spikes (s_spk[0 .. hb_nsp), any order) by every
                 thread; may contain barriers
     begin/start lines that set hb_recq[hb_q] of neuron i, and lines run before its every step
-                with hb_rec = hb_recq[hb_q] (state monitors)
+                with hb_rec = hb_recq[hb_q] (state monitors; networks within the registers)
     finish      lines run once at the end by every thread
     resident    neurons per thread in registers
     bound       C expression of timestep_bound(K, dt) when K >= 1 is the refractory period
@@ -340,9 +341,6 @@ class ResidentKernel:
               "            if (i < N) {",
               f"                {mem_load}"]
         k += ["                " + x for x in reads + each_event() + clears]
-        if start:
-            k += ["                {"] + ["                " + x for x in self._search(begin)]
-            k += ["                " + x for x in start] + ["                }"]
         k += [f"                hb_sp = {'hb_update_mem' if released else 'hb_update'}(i, hb_s, t, {all_args});",
               "                if (hb_sp) {"]
         if released:
@@ -457,12 +455,6 @@ class ResidentKernel:
         k.append("}")
         self.source = "\n".join(k) + "\n"
 
-    @staticmethod
-    def _search(begin):
-        """The begin lines for a neuron outside the registers (hb_rec instead of hb_recq[q])."""
-        return ["int hb_recm[1]; { const int hb_q = 0; const bool act = true;"] + [
-            x.replace("hb_recq", "hb_recm") for x in begin] + ["}", "const int hb_rec = hb_recm[0];"]
-
     def lds_bytes(self, N, threads, extra=0):
         """Dynamic LDS of a workgroup of that many threads for a network of N neurons."""
         b = 2 * N + extra
@@ -550,27 +542,7 @@ class GroupStep:
         ps.ptr("events", "unsigned long long")
         ps.ptr("counts", "unsigned int")
         ps.ptr("status", "int")
-        if g.smon:
-            ps.ptr("mon_i", "int")
-            ps.ptr("mon_step", "int")
-            ps.ptr("mon_n", "unsigned long long")
-            ps.ptr("mon_count", "int")
-            ps.val("mon_cap", "long long")
-            ps.val("mon_start", "int")
-            ps.val("mon_stop", "int")
-        if g.rmon:
-            ps.ptr("rate_cnt", "int")
-            ps.val("rate_row0", "long long")
-            ps.val("rate_rows", "long long")
-            ps.val("rate_start", "int")
-            ps.val("rate_stop", "int")
-        if g.stmon:
-            ps.ptr("rec_idx", "int", const=True)
-            ps.ptr("rec_buf", "double")
-            ps.val("rec_row0", "long long")
-            ps.val("rec_rows", "long long")
-            ps.val("n_rec", "int")
-            ps.val("pad_rec", "int")
+        monitor_fields(ps, g)
         self.struct = ps
 
         def block(tag, spec, extra=()):

@@ -24,7 +24,7 @@ from . import chip as _chip
 from . import kernels as _kernels
 from . import resident as _resident
 from . import targets as _targets
-from .codegen import Renderer, ctype_of
+from .codegen import Renderer, ctype_of, filled
 from .kernels import (
     LDS_BYTES,
     CodeSpec,
@@ -1198,12 +1198,8 @@ class Network:
         for (tg, n), (val, _) in R.scalars.items():
             v[f"{tg}_{n}"] = val
         v.update(self._monitor_args(g))
-        a = R.cls()
-        for name, _ in R.cls._fields_:
-            if name in v:
-                setattr(a, name, v[name])
         R.xch.zero_()  # no step's number, nobody here
-        buf = bytes(a)
+        buf = bytes(filled(R.cls, v))
         _lib.check(L.hb_launch(R.fn, R.grid, R.threads, 0, self.device.stream, buf, len(buf)), "steps over the chip")
         self.clock.fill_(self.t_step + n_steps)
 
@@ -1226,11 +1222,7 @@ class Network:
             for n, (val, _) in sc.items():
                 v[f"{x}_{n}"] = val
         v.update(self._monitor_args(g))
-        a = R.cls()
-        for name, _ in R.cls._fields_:
-            if name in v:
-                setattr(a, name, v[name])
-        buf = bytes(a)
+        buf = bytes(filled(R.cls, v))
         _lib.check(L.hb_launch(R.fn, g.N, 64, R.lds, self.device.stream, buf, len(buf)), "targets' steps")
         self.clock.fill_(self.t_step + n_steps)
 
@@ -1252,11 +1244,7 @@ class Network:
             for n, (val, _) in sc.items():
                 v[f"c{r}_{n}"] = val
         v.update(self._monitor_args(g))
-        a = R.cls()
-        for name, _ in R.cls._fields_:
-            if name in v:
-                setattr(a, name, v[name])
-        buf = bytes(a)
+        buf = bytes(filled(R.cls, v))
         _lib.check(L.hb_launch(R.fn, 1, R.threads, R.lds_bytes, self.device.stream, buf, len(buf)), "resident step")
 
     @staticmethod
@@ -1554,11 +1542,7 @@ class Network:
         if getattr(g, "spiked", None) is not None:
             v["spiked"] = g.spiked.data_ptr()
         v.update(self._monitor_args(g, flush))
-        s = cls()
-        for name, _ in cls._fields_:
-            if name in v:
-                setattr(s, name, v[name])
-        return s
+        return filled(cls, v)
 
     def _build_spikegen(self, g):
         fn = ctypes.c_void_p()
@@ -1688,10 +1672,7 @@ class Network:
             s.syn_count_dev = zeros(s.csr["n_syn"], "int")
         if s.count_events:
             v["syn_count"] = s.syn_count_dev.data_ptr()
-        a = cls()
-        for name, _ in cls._fields_:
-            if name in v:
-                setattr(a, name, v[name])
+        a = filled(cls, v)
         s.args, s.grid = a, grid
 
     def _sums_itself(self, g, groups, paths):
@@ -1812,10 +1793,7 @@ class Network:
                 v[f"a_{n}"] = g._dev[gv].data_ptr()
             for n, (val, ct) in sc.items():
                 v[f"c_{n}"] = val
-            a = cls()
-            for name, _ in cls._fields_:
-                if name in v:
-                    setattr(a, name, v[name])
+            a = filled(cls, v)
             s.summed_kernels.append(K)
             self._add_launch(fn, K.grid(t1 - t0), K.BLOCK, a, cls)
 
@@ -1836,10 +1814,7 @@ class Network:
             v[f"s_{n}"] = s.csr["syn"][n].data_ptr()
         for n, (val, ct) in sc.items():
             v[f"c_{n}"] = val
-        a = cls()
-        for name, _ in cls._fields_:
-            if name in v:
-                setattr(a, name, v[name])
+        a = filled(cls, v)
         s.post_launch_index = len(self._launches)
         self._add_launch(s.post_fn, int(min(256, max(1, g.N))), K.BLOCK, a, cls)
 
@@ -2108,10 +2083,7 @@ class Network:
                 v[f"s_{n}"] = s.csr["syn"][n].data_ptr()
         if s.count_events:
             v["syn_count"] = s.syn_count_dev.data_ptr()
-        a = cls()
-        for name, _ in cls._fields_:
-            if name in v:
-                setattr(a, name, v[name])
+        a = filled(cls, v)
         most = int(np.diff(c["ptr"]).max())
         grid = max(1, min(4 * self.device.n_cu, -(-most // K.BLOCK)))
         s.carry_index = len(self._launches)

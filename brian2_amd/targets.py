@@ -6,6 +6,7 @@ know nothing of each other: a neuron, its synapses and the generator's list are 
 step needs.  So a wave takes one target through all the steps of a launch, with the
 synapses' variables in LDS.
 """
+from .chip import monitor_fields
 from .codegen import ParamStruct, source_header, translate_block
 from .kernels import LDS_BYTES, _rename, group_block, onpre_lines
 
@@ -58,14 +59,7 @@ class TargetSteps:
         ps.val("pad", "int")
         ps.ptr("events", "unsigned long long")
         ps.ptr("status", "int")
-        if g.smon:
-            ps.ptr("mon_i", "int")
-            ps.ptr("mon_step", "int")
-            ps.ptr("mon_n", "unsigned long long")
-            ps.ptr("mon_count", "int")
-            ps.val("mon_cap", "long long")
-            ps.val("mon_start", "int")
-            ps.val("mon_stop", "int")
+        monitor_fields(ps, g)  # (a spike monitor's, if any)
         self.struct = ps
         self.kernel_name = f"targets_{g.name}"
 
