@@ -29,6 +29,7 @@ from .resident import (
     lds_plan,
     neurons_in_registers,
     refractory_form,
+    releasable,
     timestep_bound,
 )
 from .runtime import Device, Model, dev, ptr, zeros
@@ -121,7 +122,7 @@ class BatchedCUBA:
         self.bounds = {}
         for k, (tg, n) in enumerate(names):
             steps = table[:, k]
-            if self.scalar_types[(tg, n)] == "long long" and tg == "su" and np.all(steps >= 1):
+            if self.scalar_types[(tg, n)] == "long long" and tg == "su" and np.all(releasable(steps)):
                 self.bounds[f"{tg}_{n}"] = f"tb_{n}"
                 of = {int(x): timestep_bound(int(x), self.dt) for x in np.unique(steps)}
                 table = np.column_stack([table, [of[int(x)] for x in steps]])

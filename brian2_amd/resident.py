@@ -52,6 +52,13 @@ def timestep_bound(k, dt):
     return y
 
 
+def releasable(k):
+    """Whether the step at which a refractory period of k steps ends may be kept, in 32 bits and
+    counted from a launch's first step (a longer period, of neurons that fire once say, is
+    compared by its lastspike)."""
+    return (k >= 1) & (k < 1 << 30)
+
+
 def refractory_form(update, spike, var_types):
     """The name compared with in the refractoriness test `timestep(t - lastspike, dt) >= K`,
     when that test is the only use of lastspike and the only assignment of not_refractory
@@ -97,8 +104,8 @@ class ResidentKernel:
                 with hb_rec = hb_recq[hb_q] (state monitors; networks within the registers)
     finish      lines run once at the end by every thread
     resident    neurons per thread in registers
-    bound       C expression of timestep_bound(K, dt) when K >= 1 is the refractory period
-                in steps, so that the release step may be kept (refractory_form)
+    bound       C expression of timestep_bound(K, dt) when K is the refractory period in
+                steps and releasable, so that the release step may be kept (refractory_form)
     rows_in_lds, counts_in_lds   where row pointers and counts are kept
 
     What bounds it.  A step is a chain: the update of R neurons per thread, a barrier, the
@@ -188,7 +195,6 @@ class ResidentKernel:
         if released:
             k += [
                 f"    const double hb_tb = {bound};",
-                f"    const unsigned int hb_far = {period} < 0x7fffffffll ? (unsigned int)({period}) : 0x7fffffffu;  // K",
                 "    // a neuron that last spiked at time x is not refractory from the step k on (a double:",
                 "    // exact) at which (k * dt - x) + 1e-3 * dt >= hb_tb, which grows with k",
                 "    auto hb_free = [&](const double x, const double k) { return (k * dt - x) + 1e-3 * dt >= hb_tb; };",
@@ -321,12 +327,9 @@ class ResidentKernel:
         ]
         if released:
             k += [
-                "            // the release step of a neuron that spikes now: K steps on, or one beside it by rounding;",
-                "            // beyond 32 bits (K is 64 of them) a step that no launch reaches",
+                "            // the release step of a neuron that spikes now: K steps on, or one beside it by rounding",
                 f"            const double k_ = hb_k + (double)({period});",
-                "            const unsigned int far_ = (unsigned int)hb_s + hb_far;",
-                "            const int rel_ = (int)(far_ < 0x7ffffffeu ? far_ : 0x7ffffffeu) "
-                "+ (hb_free(t, k_ - 1.0) ? -1 : hb_free(t, k_) ? 0 : 1);",
+                f"            const int rel_ = hb_s + (int)({period}) + (hb_free(t, k_ - 1.0) ? -1 : hb_free(t, k_) ? 0 : 1);",
             ]
         k += ["            #pragma unroll", f"            for (int hb_q = 0; hb_q < {R}; hb_q++) {{",
               "                const int i = hb_q * T + hb_x;", "                const unsigned long long b_ = hb_b[hb_q];"]
@@ -561,7 +564,7 @@ class GroupStep:
         name = refractory_form(update, spike, g.vars)
         if name is not None and not recorded & {"lastspike", "not_refractory"}:
             value, ct = scalars.get(("su", name[len("p.su_"):]), (0, None))
-            if ct == "long long" and value >= 1:
+            if ct == "long long" and releasable(value):
                 self.bound = timestep_bound(value, dt)
         ops, events = [], []
         for r, (s, sc) in enumerate(pathways):

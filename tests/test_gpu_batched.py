@@ -149,7 +149,7 @@ def test_resident_forms_at_the_edges_of_a_workgroup(variant, monkeypatch):
             assert np.array_equal(B.get(x, k), c["G"].get(x)), (net.N, x)
 
 
-@pytest.mark.parametrize("steps", [2**31 - 2, 3 * 10**9])
+@pytest.mark.parametrize("steps", [2**30 - 1, 2**30, 2**31 - 2, 3 * 10**9])
 def test_refractory_periods_beyond_32_bits(steps):
     """Neurons that fire once: the sweep equals the plain path's staged launches."""
     from brian2_amd import Model, batched, synth

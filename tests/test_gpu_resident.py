@@ -129,7 +129,7 @@ def test_networks_that_are_not_taken():
         assert c["net"].resident is None
 
 
-@pytest.mark.parametrize("steps", [2**31 - 2, 2**31 - 1, 2**31, 3 * 10**9])
+@pytest.mark.parametrize("steps", [2**30 - 1, 2**30, 2**31 - 2, 2**31, 3 * 10**9])
 def test_refractory_periods_beyond_32_bits(steps):
     """Neurons that fire once: a period whose steps, or whose release step counted from a
     launch's beginning, take more than 32 bits."""
