@@ -44,7 +44,7 @@ from .kernels import (
 L = _lib.lib
 PULL_NEURONS = 16384  # neurons of a group whose step counts its events itself
 PULL_WORDS = 1 << 23  # words of a pathway's bit matrix (64 MB)
-RESIDENT_STEPS = 2000  # steps of one launch of the resident step (some ms)
+RESIDENT_STEPS = 2000  # steps of one launch at most (some ms); a spike monitor's room may allow fewer
 LATE = _chip.LATE
 TRIES = 20  # launches in a row that end so (some seconds each)
 S_POISSON_GROUP = 17  # generator stream of PoissonGroup draws (hb_rng.h)
