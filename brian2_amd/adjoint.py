@@ -851,8 +851,8 @@ template <typename V> struct hb_rows {{
         """Runs all trials; returns (loss, saved) where saved holds what the backward
         pass needs (states, spikes, first-spike records).  linearise: with the neurons' linear
         map, which the host then forms while the device runs the steps.  With that, the
-        scalars formed once and fewer copies back, 9 trials take 2.24 ms forward and
-        backward instead of 2.74.  keep: whether a backward pass will follow (without states
+        scalars formed once and fewer copies back, 9 trials took 2.24 ms forward and
+        backward instead of 2.74 (1.84 with what came since).  keep: whether a backward pass will follow (without states
         and spikes it simulates again)."""
         torch = _torch()
         w_in = w_in.detach().to(self.w_in0.dtype).contiguous()
